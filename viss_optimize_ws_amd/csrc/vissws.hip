@@ -76,6 +76,7 @@ struct Ctx {
   RowRec* d_rows = nullptr;
   double4* d_rowt = nullptr; /* half-row (u, v, w) * 1024 for the plain Viss phase */
   double2* d_tab = nullptr;  /* the plain kernels' sine table (VW_TAB_N entries) */
+  double2* d_tabc = nullptr; /* the plain recon's cosine table                   */
   double* d_ant8 = nullptr;
   struct SegSet {
     RowRec* rows;
@@ -674,8 +675,9 @@ int create_device(Ctx* c) {
       (rc = dalloc(c, &c->d_B, np)) || (rc = dalloc(c, &c->d_Bf, np)) ||
       (rc = dalloc(c, &c->d_Cacc, np * (size_t)c->nsky)) || (rc = dalloc(c, &c->d_Wacc, np)))
     return rc;
-  if ((rc = dalloc(c, &c->d_tab, (size_t)VW_TAB_N))) return rc;
+  if ((rc = dalloc(c, &c->d_tab, (size_t)VW_TAB_N)) || (rc = dalloc(c, &c->d_tabc, (size_t)VW_TAB_N))) return rc;
   k_tab_build<<<(VW_TAB_N + 255) / 256, 256, 0, c->st>>>(c->d_tab);
+  k_tab_build_cos<<<(VW_TAB_N + 255) / 256, 256, 0, c->st>>>(c->d_tabc);
   k_pix2lmn<<<blocks_for(c->npix), 256, 0, c->st>>>(c->nside, c->npix, c->d_l, c->d_m, c->d_n, c->d_nm1);
   KC();
   if (c->TP == 256) k_tile_cone<256><<<(unsigned)c->ntile, 256, 0, c->st>>>(c->d_l, c->d_m, c->d_n, c->npix, c->ntile, c->d_cone);
@@ -1236,7 +1238,7 @@ int enq_recon_set_one(Ctx* c, bool img, double* acc, uint32_t* wacc) {
       if (rc) return rc;
     }
     ReconArgs a{};
-    a.tab = c->d_tab;
+    a.tab = kind == VW_KIND_GENERIC ? c->d_tab : c->d_tabc;
     a.l = img ? c->d_gl : c->d_l;
     a.m = img ? c->d_gm : c->d_m;
     a.n = img ? c->d_gn : c->d_n;

@@ -426,6 +426,14 @@ __global__ void k_tab_build(double2* __restrict__ tab) {
   vw_sincos_turn((double)i / (double)VW_TAB_N, &e[1], &e[0]);
   tab[i] = make_double2(e[0], e[1]);
 }
+/* the plain recon's table: entry k = (cos, -a sin)(2 pi k / N), a = 2 pi / N */
+__global__ void k_tab_build_cos(double2* __restrict__ tab) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= VW_TAB_N) return;
+  double s, c;
+  vw_sincos_turn((double)i / (double)VW_TAB_N, &s, &c);
+  tab[i] = make_double2(c, -VW_SHORT_S1 * s);
+}
 __device__ __forceinline__ void vw_tab_fill(double2* tab, const double2* __restrict__ src) {
   for (int i = threadIdx.x; i < VW_TAB_N; i += blockDim.x) tab[i] = src[i];
 }
@@ -1401,13 +1409,17 @@ __global__ __launch_bounds__(1024) void k_groups(const int64_t* __restrict__ ks,
 }
 
 /* Per-group records as SoA (uniform loads of four groups per array in one
- * scalar load): cell centre, visibility (representative or group mean), the
- * representative's antenna frames and member range. */
+ * scalar load): cell centre, visibility (representative or group mean) in
+ * polar form, the representative's antenna frames and member range.  The
+ * one-sky recon adds Re(V exp(2 pi j x)) = |V| cos(2 pi (x + arg)), arg in
+ * turns: the argument rides in the phase's first multiply-add, so a term
+ * needs one cosine and one product instead of sine, cosine and two. */
 struct GRec {
-  double ugu, vgu, vr, vi;
+  double ugu, vgu; /* wavelengths; x1024 in the plain form          */
+  double arg, amp; /* visibility: argument (as ugu, vgu), magnitude */
 };
 struct GroupSoA {
-  GRec* rec;    /* cell centre (wavelengths; x1024 in the plain form) and visibility, 32 B */
+  GRec* rec;    /* 32 B */
   double* ant;  /* [q][10]: representative's antenna frames a and b    */
   int32_t *gia, *gib, *grep;
 };
@@ -1451,8 +1463,11 @@ __global__ void k_group_data(const int64_t* __restrict__ gkeys, const int32_t* _
   GRec gr;
   gr.ugu = ugu * uv_scale; /* 1024 for the plain table sincos, 1 for the mixed form (exact) */
   gr.vgu = vgu * uv_scale;
-  gr.vr = vr;
-  gr.vi = vi;
+  /* finite parts give a finite magnitude (the finite-value filter reads it);
+   * a NaN part, or two infinite ones, make every term NaN */
+  gr.amp = isfinite(vr) && isfinite(vi) ? fmin(hypot(vr, vi), 0x1.fffffffffffffp1023)
+                                        : (isinf(vr) != isinf(vi) && !isnan(vr) && !isnan(vi) ? INFINITY : NAN);
+  gr.arg = (atan2(vi, vr) * VW_INV_TWOPI) * uv_scale;
   g.rec[q] = gr;
   g.grep[q] = (int32_t)hr;
   RowRec r = rows[hr];
@@ -1548,7 +1563,8 @@ __global__ __launch_bounds__(256) void k_group_cls_tile(const double* __restrict
 /* reconstruction                                                       */
 /* ------------------------------------------------------------------ */
 struct ReconArgs {
-  const double2* tab; /* the sine table (plain forms), built once per context */
+  const double2* tab;  /* plain forms, built once per context: the sine table of the generic kind, the
+                        * cosine table of the others */
   const double *l, *m, *n;
   int64_t pt0, npts, TP; /* points [pt0, pt0 + npts) of this pass, pt0 = tile0 * TP */
   const uint32_t* gcls; /* [ntile_out][nq_pad]: per group (representative kind) */
@@ -1594,15 +1610,15 @@ __device__ __forceinline__ void vw_ant_vis(const double* __restrict__ ant8, int 
  * folded with Kahan compensation (mixed form, one point) */
 struct ReconAccF32 {
   float s = 0.f, c = 0.f, b = 0.f;
-  __device__ void term(double ugu, double vgu, float vrf, float vif, double lp, double mp) {
+  /* b + amp cos(2 pi (ugu lp + vgu mp + arg)) */
+  __device__ float term(double ugu, double vgu, double arg, float amp, double lp, double mp) const {
     /* the fraction in [0, 1) turns: one v_fract_f64 */
-    const double x = vw_recon_phase(ugu, vgu, lp, mp);
+    const double x = fma(vgu, mp, fma(ugu, lp, arg));
     const float f = (float)__builtin_amdgcn_fract(x);
-    const float sn = __builtin_amdgcn_sinf(f), cs = __builtin_amdgcn_cosf(f);
-    b = fmaf(vrf, cs, fmaf(-vif, sn, b));
+    return fmaf(amp, __builtin_amdgcn_cosf(f), b);
   }
-  /* the same, kept only where use holds: a select, not a branch */
-  __device__ void term_if(bool use, double ugu, double vgu, float vrf, float vif, double lp, double mp) {
+  /* the (re, im) form of a term, kept only where use holds: a select, not a branch */
+  __device__ void term_ri(bool use, double ugu, double vgu, float vrf, float vif, double lp, double mp) {
     const double x = vw_recon_phase(ugu, vgu, lp, mp);
     const float f = (float)__builtin_amdgcn_fract(x);
     const float sn = __builtin_amdgcn_sinf(f), cs = __builtin_amdgcn_cosf(f);
@@ -1619,10 +1635,25 @@ struct ReconAccF32 {
   __device__ double value() const { return ((double)s - (double)c) + (double)b; }
 };
 
-/* the PPL points of one lane and one group.  Plain: (ugu, vgu) arrive
- * scaled by 1024; all table indices and reads come before the polynomials
- * so the LDS reads overlap the arithmetic; a point with use[k] false keeps
- * its sum. */
+/* cos(2 pi (k + f) / N) = ec (1 - a^2 f^2 / 2) + A f (1 - a^2 f^2 / 6) from the
+ * table entry (ec, A = -a sin) as a cubic in f: five operations.  The square's
+ * coefficient is Taylor's times (1 - (2 sqrt 2 - 2) Y^2 / 12), Y = pi / N = the
+ * largest |a f|: with the constant term fixed that spreads the omitted
+ * y^4 / 24 (3.8e-12 at Y) over the interval, 6.4e-13 at most. */
+#define VW_COS_C2 (VW_SHORT_C2 * (1.0 - 6.4976e-7))
+#define VW_COS_S3 (-(VW_SHORT_S1 * VW_SHORT_S1) / 6.0)
+__device__ __forceinline__ double vw_tab_cos(double f, const double2& e) {
+  return fma(f, fma(f, fma(f, VW_COS_S3 * e.y, VW_COS_C2 * e.x), e.y), e.x);
+}
+
+/* the PPL points of one lane and one group.  Plain: (ugu, vgu, arg) arrive
+ * scaled by 1024; all table indices and reads come before the polynomials so
+ * the LDS reads overlap the arithmetic; a point with use[k] false keeps its
+ * sum.  A plain term is 11 FP64 instructions (phase 2, split 3, cosine 5, sum
+ * 1) where the (re, im) form takes 15; a mixed term saves the sine and a
+ * product, 16.2 -> 11.5 issue slots of an FP32 FMA.  Both are bound by VALU
+ * issue: one 64-epoch segment at Nside 256 with 32 antennas, plain, 34.7 ->
+ * 30.6 ms, its mixed form 16.1 -> 15.0 ms a segment. */
 template <int PPL, bool MIXED>
 struct ReconLane {
   double d[PPL];
@@ -1631,11 +1662,38 @@ struct ReconLane {
 #pragma unroll
     for (int k = 0; k < PPL; ++k) d[k] = 0.0;
   }
-  __device__ __forceinline__ void add(double ugu, double vgu, const double* vr, const double* vi, const bool* use,
-                                      const double* lp, const double* mp, const double2* tab) {
+  template <bool MASK>
+  __device__ __forceinline__ void add(const GRec& g, const bool* use, const double* lp, const double* mp,
+                                      const double2* tab) {
+    if (MIXED) {
+      const float amp = (float)g.amp;
+#pragma unroll
+      for (int k = 0; k < PPL; ++k) {
+        const float t = f[k].term(g.ugu, g.vgu, g.arg, amp, lp[k], mp[k]);
+        f[k].b = !MASK || use[k] ? t : f[k].b;
+      }
+    } else {
+      double fr[PPL];
+      int ix[PPL];
+#pragma unroll
+      for (int k = 0; k < PPL; ++k) fr[k] = vw_tab_split(fma(g.vgu, mp[k], fma(g.ugu, lp[k], g.arg)), &ix[k]);
+      double2 e[PPL];
+#pragma unroll
+      for (int k = 0; k < PPL; ++k) e[k] = tab[ix[k]];
+#pragma unroll
+      for (int k = 0; k < PPL; ++k) {
+        const double t = fma(g.amp, vw_tab_cos(fr[k], e[k]), d[k]);
+        d[k] = !MASK || use[k] ? t : d[k];
+      }
+    }
+  }
+  /* the (re, im) form, a value per point: averages over the members that
+   * each point sees */
+  __device__ __forceinline__ void add_ri(double ugu, double vgu, const double* vr, const double* vi, const bool* use,
+                                         const double* lp, const double* mp, const double2* tab) {
     if (MIXED) {
 #pragma unroll
-      for (int k = 0; k < PPL; ++k) f[k].term_if(use[k], ugu, vgu, (float)vr[k], (float)vi[k], lp[k], mp[k]);
+      for (int k = 0; k < PPL; ++k) f[k].term_ri(use[k], ugu, vgu, (float)vr[k], (float)vi[k], lp[k], mp[k]);
     } else {
       double fr[PPL];
       int ix[PPL];
@@ -1746,15 +1804,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(
           const int cls = (int)((cw >> (8 * j)) & 0xffu);
           if ((int)q < (int)q0 || (int)q >= (int)qb_ || cls == VW_CLS_HIDDEN) continue;
           const GRec g = blk[q - q16];
-          if (KIND == VW_KIND_REP_FINITE && !(isfinite(g.vr) && isfinite(g.vi))) continue;
-          double vr[PPL], vi[PPL];
-#pragma unroll
-          for (int k = 0; k < PPL; ++k) { vr[k] = g.vr; vi[k] = g.vi; }
+          if (KIND == VW_KIND_REP_FINITE && !isfinite(g.amp)) continue;
           if (cls == VW_CLS_VISIBLE) {
-            bool all[PPL];
-#pragma unroll
-            for (int k = 0; k < PPL; ++k) all[k] = true;
-            acc.add(g.ugu, g.vgu, vr, vi, all, lp, mp, tab);
+            acc.template add<false>(g, nullptr, lp, mp, tab);
             wu += 1;
           } else {
             const double* d = a.g.ant + q * 10;
@@ -1766,7 +1818,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(
               vis[k] = vw_vis2<true>(ok[k], pl[k], pm[k], pn[k], ax, ay, az, ai, ac, bx, by, bz, bi, bc);
               wl[k] += vis[k] ? 1 : 0;
             }
-            acc.add(g.ugu, g.vgu, vr, vi, vis, lp, mp, tab);
+            acc.template add<true>(g, vis, lp, mp, tab);
           }
           if (MIXED && ++nblk == 32) {
             nblk = 0;
@@ -1822,7 +1874,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(
         ai[k] = si[k] * invc;
         wl[k] += use[k] ? 1 : 0;
       }
-      acc.add(ugu, vgu, ar, ai, use, lp, mp, tab);
+      acc.add_ri(ugu, vgu, ar, ai, use, lp, mp, tab);
       if (MIXED && ++nblk == 32) {
         nblk = 0;
         acc.fold();
