@@ -1,0 +1,52 @@
+"""The recon's group masks (16 groups a word, 64 a ballot, 256 a wave) and its
+polar terms at the edges of those blocks, against the CPU FP64 oracle (needs
+a GPU).  Tolerances as in _lockstep: 1e-9 plain, 1e-4 mixed, weights and groups
+bit-exact."""
+import numpy as np
+import pytest
+
+from _lockstep import MIXED_TOL, PLAIN_TOL, config, rel_err, run_both
+
+pytestmark = pytest.mark.gpu
+
+
+# (antennas, epochs): 1, 15, 16, 17 | 63, 64, 65 | 255, 256, 257 | 1,025 rows, about as many groups
+ROWS = [(2, 1), (6, 1), (2, 16), (2, 17), (7, 3), (2, 64), (2, 65), (6, 17), (2, 256), (2, 257), (2, 1025)]
+
+
+@pytest.mark.parametrize("mixed", [0, 1])
+@pytest.mark.parametrize("n_ant,n_epochs", ROWS)
+def test_group_count_edges(n_ant, n_epochs, mixed):
+    if mixed and (n_ant, n_epochs) == (2, 1):
+        pytest.skip("one row spans no plane: the fitted slopes are rounding noise, phases pass 2^30 turns, and the "
+                    "mixed visibility's own 3e-7 decides nothing but is compared with FP64's")
+    cfg = config(nside=16, n_ant=n_ant, n_epochs=n_epochs, segs=1, img_n=37, precision=mixed, orbit_seed=5)
+    (C, W, img, wi), (Co, Wo, imgo, wio) = run_both(cfg, np.random.default_rng(2).lognormal(0.0, 1.0, 12 * 256))
+    tol = MIXED_TOL if mixed else PLAIN_TOL
+    assert np.array_equal(W, Wo) and np.array_equal(wi, wio)
+    assert rel_err(C, Co) <= tol and rel_err(img, imgo) <= tol
+
+
+@pytest.mark.parametrize("kw", [dict(bl_max_m=2e6), dict(bl_max_m=2e6, recon_mode=1), dict(bl_max_m=2e6, blockage=0),
+                                dict(recon_mode=1, occ_mode=1), dict(bl_max_m=1e5, occ_mode=1, precision=1),
+                                dict(bl_max_m=2e6, blockage=0, precision=1), dict(tile_pix=512, nside=4)])
+def test_rows_outside_the_grid_and_kinds(kw):
+    """a grid smaller than the baselines makes the key-0 group, which no output
+    point counts; both recon modes, the three kinds"""
+    base = dict(nside=16, n_ant=6, n_epochs=40, segs=3, img_n=40, freq_hz=1e7)
+    base.update(kw)
+    cfg = config(**base)
+    seen = []
+
+    def chk(g, o, k, d):
+        seen.append(d["ig"]["nuniq"] - d["ig"]["nkeys"])
+        for key in ("nuniq", "nkeys", "res", "fa", "fb"):
+            assert d["ig"][key] == d["io"][key]
+
+    sky = np.random.default_rng(4).lognormal(0.0, 1.0, 12 * base["nside"] ** 2)
+    (C, W, img, wi), (Co, Wo, imgo, wio) = run_both(cfg, sky, chk)
+    if "bl_max_m" in kw:
+        assert max(seen) == 1
+    tol = MIXED_TOL if base.get("precision") else PLAIN_TOL
+    assert np.array_equal(W, Wo) and np.array_equal(wi, wio)
+    assert rel_err(C, Co) <= tol and rel_err(img, imgo) <= tol

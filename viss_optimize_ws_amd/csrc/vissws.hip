@@ -754,7 +754,7 @@ int create_device(Ctx* c) {
   {
     const size_t nq = (size_t)c->nq_pad;
     GroupSoA& g = c->gs;
-    if ((rc = dalloc(c, &g.rec, nq)) || (rc = dalloc(c, &g.ant, 10 * nq)) ||
+    if ((rc = dalloc(c, &g.rec, nq)) || (rc = dalloc(c, &g.v, nq)) || (rc = dalloc(c, &g.ant, 10 * nq)) ||
         (rc = dalloc(c, &g.gia, nq)) || (rc = dalloc(c, &g.gib, nq)) || (rc = dalloc(c, &g.grep, nq)))
       return rc;
     int64_t rp = 1;
@@ -843,18 +843,17 @@ void launch_classify(Ctx* c, const uint8_t* bits, int64_t nt, uint8_t* cls, hipS
 }
 
 /* class table of a tile pass into the class scratch: cone bits per
- * (tile, antenna frame), then per (tile, half row) or (tile, group) */
+ * (tile, antenna frame), then per (tile, half row) or (tile, group in the
+ * batched recon's work order) */
 int enq_classes(Ctx* c, const double* cone, int64_t ntile_all, int64_t tile0, int64_t nt, bool groups,
-                uint8_t* bits, uint8_t* cls, hipStream_t st, bool work_order = false) {
+                uint8_t* bits, uint8_t* cls, hipStream_t st) {
   const int64_t nfr = (int64_t)c->tlen * c->A;
   if (c->nfr_pad <= VW_GCLS_LDS_MAX) {
     /* one block per tile makes the tile's cone bits in LDS: no bit table */
     const size_t lds = (size_t)c->nfr_pad;
     if (groups)
       k_group_cls_tile<<<(unsigned)nt, 256, lds, st>>>(cone, ntile_all, tile0, c->d_ant8, nfr,
-                                                       work_order ? c->d_oia : c->gs.gia,
-                                                       work_order ? c->d_oib : c->gs.gib, c->d_info, c->nq_pad,
-                                                       (uint32_t*)cls);
+                                                       c->d_oia, c->d_oib, c->d_info, c->nq_pad, (uint32_t*)cls);
     else
       k_classify_tile<<<(unsigned)nt, 256, lds, st>>>(cone, ntile_all, tile0, c->d_ant8, nfr, c->d_rows, c->nh,
                                                       c->nh_pad, (uint32_t*)cls);
@@ -867,12 +866,32 @@ int enq_classes(Ctx* c, const double* cone, int64_t ntile_all, int64_t tile0, in
   if (groups) {
     const int nqb = (int)((c->nq_pad + VW_GCLS_BLOCK - 1) / VW_GCLS_BLOCK);
     const unsigned nb = (unsigned)(nt * nqb);
-    const int32_t* ia = work_order ? c->d_oia : c->gs.gia;
-    const int32_t* ib = work_order ? c->d_oib : c->gs.gib;
     /* frame rows here are longer than the LDS staging limit */
-    k_group_cls<false><<<nb, 256, 0, st>>>(bits, c->nfr_pad, nqb, ia, ib, c->d_info, c->nq_pad, (uint32_t*)cls);
+    k_group_cls<false><<<nb, 256, 0, st>>>(bits, c->nfr_pad, nqb, c->d_oia, c->d_oib, c->d_info, c->nq_pad,
+                                           (uint32_t*)cls);
   } else
     launch_classify(c, bits, nt, cls, st);
+  KC();
+  return VW_OK;
+}
+
+/* the one-sky recon's group masks of a tile pass ([nt][nq_pad / 16] words) into
+ * the class scratch */
+int enq_group_masks(Ctx* c, const double* cone, int64_t ntile_all, int64_t tile0, int64_t nt, uint8_t* bits,
+                    uint32_t* gmask, hipStream_t st) {
+  const int64_t nfr = (int64_t)c->tlen * c->A;
+  if (c->nfr_pad <= VW_GCLS_LDS_MAX) {
+    k_group_mask<true><<<(unsigned)nt, 256, (size_t)c->nfr_pad, st>>>(cone, ntile_all, tile0, c->d_ant8, nfr, nullptr,
+                                                                       c->nfr_pad, c->gs.gia, c->gs.gib, c->d_info,
+                                                                       c->nq_pad, gmask);
+    KC();
+    return VW_OK;
+  }
+  if (nt * c->nfr_pad > c->bits_cap) return c->fail(VW_ERR_RANGE, "internal: cone bit buffer too small");
+  k_ant_bits<<<blocks_for(nt * c->nfr_pad), 256, 0, st>>>(cone, ntile_all, tile0, nt, c->d_ant8, nfr, c->nfr_pad, bits);
+  KC();
+  k_group_mask<false><<<(unsigned)nt, 256, 0, st>>>(cone, ntile_all, tile0, c->d_ant8, nfr, bits, c->nfr_pad, c->gs.gia,
+                                                    c->gs.gib, c->d_info, c->nq_pad, gmask);
   KC();
   return VW_OK;
 }
@@ -1173,7 +1192,7 @@ int enq_recon_set_batch(Ctx* c, bool img) {
     const int64_t pt0 = tile0 * c->TP;
     const int64_t np = std::min(nt * c->TP, npts_all - pt0);
     if (rep) {
-      int rc = enq_classes(c, cone, ntile_all, tile0, nt, true, bits, cls, st, true);
+      int rc = enq_classes(c, cone, ntile_all, tile0, nt, true, bits, cls, st);
       if (rc) return rc;
     }
     const ReconBShape s = reconb_shape(c, np, c->rb_target);
@@ -1234,7 +1253,8 @@ int enq_recon_set_one(Ctx* c, bool img, double* acc, uint32_t* wacc) {
     const int64_t pt0 = tile0 * c->TP;
     const int64_t np = std::min(nt * c->TP, npts_all - pt0);
     if (kind != VW_KIND_AVG) {
-      int rc = enq_classes(c, cone, ntile_all, tile0, nt, kind == VW_KIND_REP, bits, cls, st);
+      int rc = kind == VW_KIND_REP ? enq_group_masks(c, cone, ntile_all, tile0, nt, bits, (uint32_t*)cls, st)
+                                   : enq_classes(c, cone, ntile_all, tile0, nt, false, bits, cls, st);
       if (rc) return rc;
     }
     ReconArgs a{};
@@ -1245,7 +1265,7 @@ int enq_recon_set_one(Ctx* c, bool img, double* acc, uint32_t* wacc) {
     a.pt0 = pt0;
     a.npts = np;
     a.TP = c->TP;
-    a.gcls = (const uint32_t*)cls;
+    a.gmask = (const uint32_t*)cls;
     a.nq_pad = c->nq_pad;
     a.rcls = (const uint32_t*)cls;
     a.nh_pad = c->nh_pad;

@@ -45,7 +45,8 @@ struct DevInfo {
   int64_t nuniq;
   int64_t first_nz;
   int64_t wtotal;
-  int64_t pad;
+  int32_t polar; /* 1: the plain recon's polar terms may be used (vw_polar_ok) */
+  int32_t pad;
 };
 
 #define VW_FULLMASK 0xffffffffffffffffULL
@@ -1280,6 +1281,16 @@ __global__ void k_conj_fill(const double2* __restrict__ vraw, const RowRec* __re
 /* ------------------------------------------------------------------ */
 /* segment parameters, keys, stable grouping                            */
 /* ------------------------------------------------------------------ */
+/* The polar terms round the phase after adding the visibility's argument, the
+ * (re, im) terms without it: they differ by the rounding of phases of up to
+ * umax (2 + |fa| + |fb|) turns.  Below 2^22 turns that is under 1e-9 of the
+ * maps; it stays below for baselines of 14,000 km at 30 MHz.  Beyond it, and for
+ * the unbounded slopes of rows that span no plane, the plain recon keeps the
+ * (re, im) terms and their rounding. */
+__device__ __forceinline__ int vw_polar_ok(const vw_segparams& sp) {
+  return (double)sp.half * sp.du * (2.0 + fabs(sp.fa) + fabs(sp.fb)) <= 4194304.0;
+}
+
 __global__ __launch_bounds__(256) void k_segparams(const RowRec* __restrict__ rows, int64_t nh, int P,
                                                    double bl_max, double lambda, DevInfo* __restrict__ info) {
   __shared__ double s[5][256];
@@ -1306,7 +1317,12 @@ __global__ __launch_bounds__(256) void k_segparams(const RowRec* __restrict__ ro
       for (int k = 0; k < 5; ++k) s[k][t] = s[k][t] + s[k][t + st];
     __syncthreads();
   }
-  if (t == 0) vw_segparams_from_sums(s[0][0], s[1][0], s[2][0], s[3][0], s[4][0], bl_max, lambda, &info->sp);
+  if (t == 0) {
+    vw_segparams sp;
+    vw_segparams_from_sums(s[0][0], s[1][0], s[2][0], s[3][0], s[4][0], bl_max, lambda, &sp);
+    info->sp = sp;
+    info->polar = vw_polar_ok(sp);
+  }
 }
 
 /* mode row -> (half row, conjugate flag) */
@@ -1420,6 +1436,7 @@ struct GRec {
 };
 struct GroupSoA {
   GRec* rec;    /* 32 B */
+  double2* v;   /* the visibility as (re, im), for segments without polar terms */
   double* ant;  /* [q][10]: representative's antenna frames a and b    */
   int32_t *gia, *gib, *grep;
 };
@@ -1469,6 +1486,7 @@ __global__ void k_group_data(const int64_t* __restrict__ gkeys, const int32_t* _
                                         : (isinf(vr) != isinf(vi) && !isnan(vr) && !isnan(vi) ? INFINITY : NAN);
   gr.arg = (atan2(vi, vr) * VW_INV_TWOPI) * uv_scale;
   g.rec[q] = gr;
+  g.v[q] = make_double2(vr, vi);
   g.grep[q] = (int32_t)hr;
   RowRec r = rows[hr];
   g.gia[q] = r.ia;
@@ -1480,18 +1498,18 @@ __global__ void k_group_data(const int64_t* __restrict__ gkeys, const int32_t* _
   d[5] = qb[0]; d[6] = qb[1]; d[7] = qb[2]; d[8] = qb[3]; d[9] = qb[7];
 }
 
-/* class of (output tile, group) from the representative's antennas: entry j
- * of a tile's row pairs frames ia[j] and ib[j] (the groups' own arrays, or
- * for the batched recon the same arrays in its work order, which puts the
- * groups past nuniq last, so in both entries j >= nuniq are hidden).  A
+/* class of (output tile, group) from the representative's antennas, for the
+ * batched recon: entry j of a tile's row pairs frames ia[j] and ib[j] (in the
+ * work order, which puts the groups past nuniq last: entries j >= nuniq are
+ * hidden).  A
  * block covers VW_GCLS_BLOCK entries of one tile's row, four a thread
  * written as one class word (byte e = entry 4 i + e).  Each thread issues
  * its index loads first, then the block stages that tile's frame row of
  * cone bits in LDS (STAGE; nfr_pad bytes of dynamic LDS; longer rows are
  * gathered from global memory), so the loads overlap.  Blocks that start
  * past the 64-entry block holding entry nuniq - 1 write nothing: the recon
- * kernels read the classes of entries below nuniq only, in words of 4 (one
- * sky) or blocks of 32 (batched) aligned to their size. */
+ * kernel reads the classes of entries below nuniq only, in aligned blocks of
+ * 32. */
 template <bool STAGE>
 __global__ __launch_bounds__(256) void k_group_cls(const uint8_t* __restrict__ bits, int64_t nfr_pad, int nqb,
                                                    const int32_t* __restrict__ ia, const int32_t* __restrict__ ib,
@@ -1559,6 +1577,55 @@ __global__ __launch_bounds__(256) void k_group_cls_tile(const double* __restrict
   }
 }
 
+/* The one-sky recon's form of the same classes: per (tile, 16 groups) one
+ * word, bit j = group j is visible from the whole tile, bit 16 + j = partly;
+ * groups below first_nz (the key-0 group) and past nuniq have neither bit, so
+ * the recon walks set bits and needs no range test.  TILE: one block per tile
+ * makes the tile's cone bits in LDS (frame rows up to VW_GCLS_LDS_MAX bytes);
+ * else they come from the bit table of the pass.  A wave takes 4 x 64 groups
+ * at a time, a lane one group of each 64 (coalesced index loads, all issued
+ * before the gathers), and writes the masks of ballots.  Words of entries
+ * below nuniq rounded up to 64 are written: the recon reads no others. */
+template <bool TILE>
+__global__ __launch_bounds__(256) void k_group_mask(const double* __restrict__ cone, int64_t ntile, int64_t tile0,
+                                                    const double* __restrict__ ant8, int64_t nfr,
+                                                    const uint8_t* __restrict__ bits, int64_t nfr_pad,
+                                                    const int32_t* __restrict__ ia, const int32_t* __restrict__ ib,
+                                                    const DevInfo* __restrict__ info, int64_t nq_pad,
+                                                    uint32_t* __restrict__ gmask) {
+  extern __shared__ uint4 sbits[];
+  const int64_t tr = blockIdx.x;
+  const int nu = vw_rfl((int)info->nuniq), q0 = vw_rfl((int)info->first_nz);
+  const int qend = (nu + 63) / 64 * 64; /* <= nq_pad, a multiple of 64 */
+  const uint8_t* b = TILE ? (const uint8_t*)sbits : bits + tr * nfr_pad;
+  if (TILE) {
+    vw_tile_bits_lds((uint8_t*)sbits, cone, ntile, tile0 + tr, ant8, nfr);
+    __syncthreads();
+  }
+  const int wave = vw_rfl((int)(threadIdx.x >> 6)), lane = threadIdx.x & 63;
+  uint32_t* out = gmask + tr * (nq_pad >> 4);
+  for (int j0 = 256 * wave; j0 < qend; j0 += 1024) {
+    int av[4], bv[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const int q = j0 + 64 * e + lane;
+      /* indices past nuniq are not frames: frame 0 stands in for them */
+      av[e] = q < nu ? ia[q] : 0;
+      bv[e] = q < nu ? ib[q] : 0;
+    }
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const int q = j0 + 64 * e + lane;
+      const bool in = q >= q0 && q < nu;
+      const int c = vw_pair_class(b[av[e]], b[bv[e]]);
+      const uint64_t v = __ballot(in && c == VW_CLS_VISIBLE), m = __ballot(in && c == VW_CLS_MIXED);
+      if (lane < 4 && j0 + 64 * e < qend)
+        out[((j0 + 64 * e) >> 4) + lane] =
+            (uint32_t)((v >> (16 * lane)) & 0xffffu) | ((uint32_t)((m >> (16 * lane)) & 0xffffu) << 16);
+    }
+  }
+}
+
 /* ------------------------------------------------------------------ */
 /* reconstruction                                                       */
 /* ------------------------------------------------------------------ */
@@ -1567,7 +1634,7 @@ struct ReconArgs {
                         * cosine table of the others */
   const double *l, *m, *n;
   int64_t pt0, npts, TP; /* points [pt0, pt0 + npts) of this pass, pt0 = tile0 * TP */
-  const uint32_t* gcls; /* [ntile_out][nq_pad]: per group (representative kind) */
+  const uint32_t* gmask; /* [ntile_out][nq_pad / 16] mask words of 16 groups (representative kinds) */
   int64_t nq_pad;
   const uint32_t* rcls; /* [ntile_out][nh_pad]: per half row (generic kind)     */
   int64_t nh_pad;
@@ -1606,10 +1673,11 @@ __device__ __forceinline__ void vw_ant_vis(const double* __restrict__ ant8, int 
              bi, bc);
 }
 
-/* FP64 phase and turn reduction, hardware FP32 sin/cos, FP32 block sums
- * folded with Kahan compensation (mixed form, one point) */
+/* FP64 phase and turn reduction, hardware FP32 sin/cos, FP32 sums over blocks
+ * of at most 32 groups, added up in FP64 (mixed form, one point) */
 struct ReconAccF32 {
-  float s = 0.f, c = 0.f, b = 0.f;
+  float b = 0.f;
+  double s = 0.0;
   /* b + amp cos(2 pi (ugu lp + vgu mp + arg)) */
   __device__ float term(double ugu, double vgu, double arg, float amp, double lp, double mp) const {
     /* the fraction in [0, 1) turns: one v_fract_f64 */
@@ -1626,13 +1694,10 @@ struct ReconAccF32 {
     b = use ? nb : b;
   }
   __device__ void fold() {
-    float y = b - c;
-    float t = s + y;
-    c = (t - s) - y;
-    s = t;
+    s += (double)b;
     b = 0.f;
   }
-  __device__ double value() const { return ((double)s - (double)c) + (double)b; }
+  __device__ double value() const { return s + (double)b; }
 };
 
 /* cos(2 pi (k + f) / N) = ec (1 - a^2 f^2 / 2) + A f (1 - a^2 f^2 / 6) from the
@@ -1712,6 +1777,22 @@ struct ReconLane {
       }
     }
   }
+  /* the (re, im) form of a group's terms, point after point (plain form,
+   * segments without polar terms); use == nullptr: every point */
+  __device__ __forceinline__ void add_one(const GRec& g, const double2& v, const bool* use, const double* lp,
+                                          const double* mp, const double2* tab) {
+#pragma unroll
+    for (int k = 0; k < PPL; ++k) {
+      int ix;
+      const double fr = vw_tab_split(vw_recon_phase(g.ugu, g.vgu, lp[k], mp[k]), &ix);
+      const double2 e = tab[ix];
+      double sy, cy, sn, cs;
+      vw_tab_poly_short(fr, &sy, &cy);
+      vw_tab_rotate(e.x, e.y * (-1.0 / VW_SHORT_S1), sy, cy, &sn, &cs);
+      const double t = vw_recon_add(d[k], v.x, v.y, sn, cs);
+      d[k] = use == nullptr || use[k] ? t : d[k];
+    }
+  }
   __device__ void fold() {
     if (MIXED) {
 #pragma unroll
@@ -1747,6 +1828,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(
   /* group counts fit 32 bits; uniform values keep the range tests scalar */
   const int64_t nu = vw_rfl((int)a.info->nuniq);
   const int64_t q0 = vw_rfl((int)a.info->first_nz);
+  const bool polar = vw_rfl(a.info->polar) != 0;
   /* group range of this chunk, aligned to 16 groups */
   const int64_t base = q0 & ~(int64_t)15;
   const int64_t span = ((nu - base) + a.nchunk - 1) / a.nchunk;
@@ -1776,56 +1858,72 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(
 
   if (VW_KIND_IS_REP(KIND) || KIND == VW_KIND_AVG) {
     /* records pass through a per-wave LDS ring in blocks of 16 (512 B: one
-     * double per lane, loaded one block ahead); each group is then read
-     * with a uniform LDS address.  Class words (4 groups each) are scalar
-     * loads fetched one word ahead.  Blocks start at multiples of 16 and
-     * nq_pad is a multiple of 64, so every block lies inside the records. */
+     * double per lane, loaded one block ahead); each group is then read with
+     * a uniform LDS address.  The mask words of 16 groups are scalar loads
+     * fetched one block ahead; the set bits are walked, the groups visible
+     * from the whole tile first, so that a hidden group costs nothing and
+     * each kind of term has one place in the code (the sums stay in their
+     * registers): a class byte per group tested in turn, with a fourfold
+     * unrolled site per class, cost a dozen scalar instructions a group and
+     * eight moves a term.  Nside 256, 32 antennas, 1024^2 image, one 64-epoch
+     * segment: 30.6 -> 29.6 ms plain, 15.0 -> 12.7 ms mixed; Nside 128 mixed
+     * day 10.8 -> 10.0 ms.  Blocks start at multiples of 16 and nq_pad is a multiple of
+     * 64, so every block lies inside the records and the masks. */
     double* ring = gring[vw_rfl((int)(threadIdx.x >> 6))];
     const double* recd = (const double*)a.g.rec;
+    const uint32_t* mrow = VW_KIND_IS_REP(KIND) ? a.gmask + tile * (a.nq_pad >> 4) : nullptr;
     double stage = (qa_ < qb_) ? recd[qa_ * 4 + lane] : 0.0;
-    uint32_t ncw = 0x01010101u; /* AVG: every group counts, no class */
-    if (VW_KIND_IS_REP(KIND) && qa_ < qb_) ncw = (uint32_t)vw_rfl((int)a.gcls[(tile * a.nq_pad + qa_) >> 2]);
+    uint32_t nmw = 0;
+    if (VW_KIND_IS_REP(KIND) && qa_ < qb_) nmw = (uint32_t)vw_rfl((int)mrow[qa_ >> 4]);
     int buf = 0;
-    for (int64_t q16 = qa_; q16 < qb_; q16 += 16, buf ^= 1) {
+    for (int q16 = (int)qa_; q16 < (int)qb_; q16 += 16, buf ^= 1) {
       ring[buf * 64 + lane] = stage;
       __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
       __builtin_amdgcn_wave_barrier();
       __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-      if (q16 + 16 < qb_) stage = recd[(q16 + 16) * 4 + lane];
+      uint32_t mw = nmw;
+      if (q16 + 16 < (int)qb_) {
+        stage = recd[(int64_t)(q16 + 16) * 4 + lane];
+        if (VW_KIND_IS_REP(KIND)) nmw = (uint32_t)vw_rfl((int)mrow[(q16 + 16) >> 4]);
+      }
+      if (KIND == VW_KIND_AVG) { /* every group of nonzero key, no classes */
+        const int lo = (int)q0 > q16 ? (int)q0 - q16 : 0, hi = (int)qb_ - q16 < 16 ? (int)qb_ - q16 : 16;
+        mw = ((1u << hi) - 1u) & ~((1u << lo) - 1u);
+      }
       const GRec* blk = (const GRec*)(ring + buf * 64);
-      const int64_t qe = q16 + 16 < qb_ ? q16 + 16 : qb_;
-      for (int64_t q4 = q16; q4 < qe; q4 += 4) {
-        const uint32_t cw = ncw;
-        if (VW_KIND_IS_REP(KIND) && q4 + 4 < qb_)
-          ncw = (uint32_t)vw_rfl((int)a.gcls[(tile * a.nq_pad + q4 + 4) >> 2]);
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          const int64_t q = q4 + j;
-          const int cls = (int)((cw >> (8 * j)) & 0xffu);
-          if ((int)q < (int)q0 || (int)q >= (int)qb_ || cls == VW_CLS_HIDDEN) continue;
-          const GRec g = blk[q - q16];
+      uint32_t vis = mw & 0xffffu, part = mw >> 16;
+      if (KIND != VW_KIND_REP_FINITE) wu += (uint32_t)__builtin_popcount(vis);
+      while (vis) {
+        const int j = __builtin_ctz(vis);
+        vis &= vis - 1;
+        const GRec g = blk[j];
+        if (KIND == VW_KIND_REP_FINITE) {
+          if (!isfinite(g.amp)) continue;
+          wu += 1;
+        }
+        if (MIXED || polar) acc.template add<false>(g, nullptr, lp, mp, tab);
+        else acc.add_one(g, a.g.v[q16 + j], nullptr, lp, mp, tab);
+      }
+      if (VW_KIND_IS_REP(KIND)) {
+        while (part) {
+          const int j = __builtin_ctz(part);
+          part &= part - 1;
+          const GRec g = blk[j];
           if (KIND == VW_KIND_REP_FINITE && !isfinite(g.amp)) continue;
-          if (cls == VW_CLS_VISIBLE) {
-            acc.template add<false>(g, nullptr, lp, mp, tab);
-            wu += 1;
-          } else {
-            const double* d = a.g.ant + q * 10;
-            const double ax = d[0], ay = d[1], az = d[2], ai = d[3], ac = d[4];
-            const double bx = d[5], by = d[6], bz = d[7], bi = d[8], bc = d[9];
-            bool vis[PPL];
+          const double* d = a.g.ant + (int64_t)(q16 + j) * 10;
+          const double ax = d[0], ay = d[1], az = d[2], ai = d[3], ac = d[4];
+          const double bx = d[5], by = d[6], bz = d[7], bi = d[8], bc = d[9];
+          bool use[PPL];
 #pragma unroll
-            for (int k = 0; k < PPL; ++k) {
-              vis[k] = vw_vis2<true>(ok[k], pl[k], pm[k], pn[k], ax, ay, az, ai, ac, bx, by, bz, bi, bc);
-              wl[k] += vis[k] ? 1 : 0;
-            }
-            acc.template add<true>(g, vis, lp, mp, tab);
+          for (int k = 0; k < PPL; ++k) {
+            use[k] = vw_vis2<true>(ok[k], pl[k], pm[k], pn[k], ax, ay, az, ai, ac, bx, by, bz, bi, bc);
+            wl[k] += use[k] ? 1 : 0;
           }
-          if (MIXED && ++nblk == 32) {
-            nblk = 0;
-            acc.fold();
-          }
+          if (MIXED || polar) acc.template add<true>(g, use, lp, mp, tab);
+          else acc.add_one(g, a.g.v[q16 + j], use, lp, mp, tab);
         }
       }
+      if (MIXED && buf) acc.fold(); /* every 32 groups */
     }
   } else {
     /* generic representative sets (viss_recon_kernel.cuh:603-614, isfinite filter) */
