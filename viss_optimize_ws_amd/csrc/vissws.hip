@@ -754,7 +754,7 @@ int create_device(Ctx* c) {
   {
     const size_t nq = (size_t)c->nq_pad;
     GroupSoA& g = c->gs;
-    if ((rc = dalloc(c, &g.rec, nq)) || (rc = dalloc(c, &g.v, nq)) || (rc = dalloc(c, &g.ant, 10 * nq)) ||
+    if ((rc = dalloc(c, &g.rec, nq)) || (rc = dalloc(c, &g.v, nq)) || (rc = dalloc(c, &g.ant, 10 * nq)) || (rc = dalloc(c, &g.ant32, 8 * nq)) ||
         (rc = dalloc(c, &g.gia, nq)) || (rc = dalloc(c, &g.gib, nq)) || (rc = dalloc(c, &g.grep, nq)))
       return rc;
     int64_t rp = 1;

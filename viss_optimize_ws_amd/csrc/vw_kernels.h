@@ -1424,6 +1424,29 @@ __global__ __launch_bounds__(1024) void k_groups(const int64_t* __restrict__ ks,
   }
 }
 
+/* Occlusion in FP32, exact where it decides.  d = s . u - cosphi with every
+ * operand rounded to FP32 is within 4e-7 of the FP64 test's difference
+ * (operands 2^-24 relative each, |s| = |u| = 1, three roundings of sums below
+ * 2, the threshold), so outside +-VW_VIS_EPS its sign is the FP64 test's
+ * result; closer in, the caller evaluates the FP64 test.  A frame that is not
+ * finite (an antenna at the origin) fails the FP64 test everywhere: threshold
+ * 2 here. */
+#define VW_VIS_EPS 1e-6f
+__device__ __forceinline__ void vw_frame32(const double* __restrict__ q8, float* __restrict__ f) {
+  const bool ok = isfinite(q8[4]) && isfinite(q8[5]) && isfinite(q8[6]) && isfinite(q8[7]);
+  f[0] = ok ? (float)q8[4] : 0.f;
+  f[1] = ok ? (float)q8[5] : 0.f;
+  f[2] = ok ? (float)q8[6] : 0.f;
+  f[3] = ok ? (float)q8[7] : 2.f;
+}
+/* the smaller of the two endpoints' differences: above VW_VIS_EPS both see
+ * the direction, below -VW_VIS_EPS one does not */
+__device__ __forceinline__ float vw_vis32(float l, float m, float n, const float* f) {
+  const float a = fmaf(n, f[2], fmaf(m, f[1], fmaf(l, f[0], -f[3])));
+  const float b = fmaf(n, f[6], fmaf(m, f[5], fmaf(l, f[4], -f[7])));
+  return fminf(a, b);
+}
+
 /* Per-group records as SoA (uniform loads of four groups per array in one
  * scalar load): cell centre, visibility (representative or group mean) in
  * polar form, the representative's antenna frames and member range.  The
@@ -1438,6 +1461,7 @@ struct GroupSoA {
   GRec* rec;    /* 32 B */
   double2* v;   /* the visibility as (re, im), for segments without polar terms */
   double* ant;  /* [q][10]: representative's antenna frames a and b    */
+  float* ant32; /* [q][8]: their unit vectors and thresholds in FP32 (vw_frame32) */
   int32_t *gia, *gib, *grep;
 };
 
@@ -1496,6 +1520,8 @@ __global__ void k_group_data(const int64_t* __restrict__ gkeys, const int32_t* _
   double* d = g.ant + q * 10;
   d[0] = qa[0]; d[1] = qa[1]; d[2] = qa[2]; d[3] = qa[3]; d[4] = qa[7];
   d[5] = qb[0]; d[6] = qb[1]; d[7] = qb[2]; d[8] = qb[3]; d[9] = qb[7];
+  vw_frame32(qa, g.ant32 + q * 8);
+  vw_frame32(qb, g.ant32 + q * 8 + 4);
 }
 
 /* class of (output tile, group) from the representative's antennas, for the
@@ -1803,14 +1829,17 @@ struct ReconLane {
 };
 
 #ifndef VW_RECON_WAVES_PLAIN
-#define VW_RECON_WAVES_PLAIN 4
+#define VW_RECON_WAVES_PLAIN 5
 #endif
 #ifndef VW_RECON_WAVES_MIXED
 #define VW_RECON_WAVES_MIXED 5
 #endif
+#ifndef VW_RECON_WAVES_GENERIC
+#define VW_RECON_WAVES_GENERIC 4
+#endif
 template <int PPL, bool MIXED, int KIND>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(
-    MIXED && KIND != VW_KIND_GENERIC ? VW_RECON_WAVES_MIXED : VW_RECON_WAVES_PLAIN))) void k_recon(ReconArgs a) {
+    KIND == VW_KIND_GENERIC ? VW_RECON_WAVES_GENERIC : MIXED ? VW_RECON_WAVES_MIXED : VW_RECON_WAVES_PLAIN))) void k_recon(ReconArgs a) {
   __shared__ double2 tab[MIXED ? 1 : VW_TAB_N];
   __shared__ double gring[4][2 * 64]; /* per wave: two blocks of 16 group records */
   if (!MIXED) {
@@ -1837,6 +1866,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(
   const int64_t qb_ = vw_rfl((int)(qa_ + spanA < nu ? qa_ + spanA : nu));
 
   double pl[PPL], pm[PPL], pn[PPL], lp[PPL], mp[PPL];
+  float fl[PPL], fm[PPL], fn[PPL]; /* FP32 directions (partly visible tiles) */
   bool ok[PPL];
 #pragma unroll
   for (int k = 0; k < PPL; ++k) {
@@ -1848,6 +1878,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(
     pn[k] = a.n[pp];
     lp[k] = fma(sp.fa, pn[k], pl[k]);
     mp[k] = fma(sp.fb, pn[k], pm[k]);
+    fl[k] = (float)pl[k];
+    fm[k] = (float)pm[k];
+    fn[k] = (float)pn[k];
   }
   ReconLane<PPL, MIXED> acc;
   uint32_t wl[PPL];
@@ -1910,15 +1943,30 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(
           part &= part - 1;
           const GRec g = blk[j];
           if (KIND == VW_KIND_REP_FINITE && !isfinite(g.amp)) continue;
-          const double* d = a.g.ant + (int64_t)(q16 + j) * 10;
-          const double ax = d[0], ay = d[1], az = d[2], ai = d[3], ac = d[4];
-          const double bx = d[5], by = d[6], bz = d[7], bi = d[8], bc = d[9];
+          float fr[8];
+#pragma unroll
+          for (int e = 0; e < 8; ++e) fr[e] = a.g.ant32[(int64_t)(q16 + j) * 8 + e];
+          float vd[PPL], near_ = 4.f;
           bool use[PPL];
 #pragma unroll
           for (int k = 0; k < PPL; ++k) {
-            use[k] = vw_vis2<true>(ok[k], pl[k], pm[k], pn[k], ax, ay, az, ai, ac, bx, by, bz, bi, bc);
-            wl[k] += use[k] ? 1 : 0;
+            vd[k] = vw_vis32(fl[k], fm[k], fn[k], fr);
+            near_ = fminf(near_, fabsf(vd[k]));
+            use[k] = vd[k] > 0.f;
           }
+          if (__ballot(near_ <= VW_VIS_EPS)) { /* a point on the horizon: the FP64 test */
+            const double* d = a.g.ant + (int64_t)(q16 + j) * 10;
+#pragma unroll
+            for (int k = 0; k < PPL; ++k) {
+              int ln = lane; /* opaque: the addresses are formed here, not kept in registers across the loop */
+              __asm__ volatile("" : "+v"(ln));
+              const int64_t pp = a.pt0 + (ok[k] ? pbase + ln + 64 * k : 0);
+              use[k] = vw_vis2<true>(ok[k], a.l[pp], a.m[pp], a.n[pp], d[0], d[1], d[2], d[3], d[4], d[5], d[6], d[7],
+                                     d[8], d[9]);
+            }
+          }
+#pragma unroll
+          for (int k = 0; k < PPL; ++k) wl[k] += use[k] ? 1 : 0;
           if (MIXED || polar) acc.template add<true>(g, use, lp, mp, tab);
           else acc.add_one(g, a.g.v[q16 + j], use, lp, mp, tab);
         }
