@@ -76,7 +76,6 @@ struct Ctx {
   RowRec* d_rows = nullptr;
   double4* d_rowt = nullptr; /* half-row (u, v, w) * 1024 for the plain Viss phase */
   double2* d_tab = nullptr;  /* the plain kernels' sine table (VW_TAB_N entries) */
-  double2* d_tabc = nullptr; /* the plain recon's cosine table                   */
   double* d_ant8 = nullptr;
   struct SegSet {
     RowRec* rows;
@@ -675,9 +674,8 @@ int create_device(Ctx* c) {
       (rc = dalloc(c, &c->d_B, np)) || (rc = dalloc(c, &c->d_Bf, np)) ||
       (rc = dalloc(c, &c->d_Cacc, np * (size_t)c->nsky)) || (rc = dalloc(c, &c->d_Wacc, np)))
     return rc;
-  if ((rc = dalloc(c, &c->d_tab, (size_t)VW_TAB_N)) || (rc = dalloc(c, &c->d_tabc, (size_t)VW_TAB_N))) return rc;
+  if ((rc = dalloc(c, &c->d_tab, (size_t)VW_TAB_N))) return rc;
   k_tab_build<<<(VW_TAB_N + 255) / 256, 256, 0, c->st>>>(c->d_tab);
-  k_tab_build_cos<<<(VW_TAB_N + 255) / 256, 256, 0, c->st>>>(c->d_tabc);
   k_pix2lmn<<<blocks_for(c->npix), 256, 0, c->st>>>(c->nside, c->npix, c->d_l, c->d_m, c->d_n, c->d_nm1);
   KC();
   if (c->TP == 256) k_tile_cone<256><<<(unsigned)c->ntile, 256, 0, c->st>>>(c->d_l, c->d_m, c->d_n, c->npix, c->ntile, c->d_cone);
@@ -1140,7 +1138,8 @@ int enq_group_data(Ctx* c, const double2* vh) {
   int64_t nr = full ? 2 * c->nh : c->nh;
   k_group_data<<<blocks_for(nr), 256, 0, c->stB>>>(c->d_gkeys, c->d_goff, c->d_idx_sorted, vh, c->d_rows,
                                                   c->d_ant8, c->P, full ? 1 : 0, c->cfg.blockage, c->cfg.occ_mode,
-                                                  c->cfg.precision == VW_PREC_MIXED ? 1.0 : VW_TAB_SCALE, c->d_info,
+                                                  c->cfg.precision == VW_PREC_PLAIN && c->generic ? VW_TAB_SCALE : 1.0,
+                                                  c->d_info,
                                                   c->gs);
   KC();
   return VW_OK;
@@ -1258,7 +1257,7 @@ int enq_recon_set_one(Ctx* c, bool img, double* acc, uint32_t* wacc) {
       if (rc) return rc;
     }
     ReconArgs a{};
-    a.tab = kind == VW_KIND_GENERIC ? c->d_tab : c->d_tabc;
+    a.tab = c->d_tab;
     a.l = img ? c->d_gl : c->d_l;
     a.m = img ? c->d_gm : c->d_m;
     a.n = img ? c->d_gn : c->d_n;

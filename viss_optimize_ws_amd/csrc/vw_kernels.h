@@ -427,14 +427,6 @@ __global__ void k_tab_build(double2* __restrict__ tab) {
   vw_sincos_turn((double)i / (double)VW_TAB_N, &e[1], &e[0]);
   tab[i] = make_double2(e[0], e[1]);
 }
-/* the plain recon's table: entry k = (cos, -a sin)(2 pi k / N), a = 2 pi / N */
-__global__ void k_tab_build_cos(double2* __restrict__ tab) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= VW_TAB_N) return;
-  double s, c;
-  vw_sincos_turn((double)i / (double)VW_TAB_N, &s, &c);
-  tab[i] = make_double2(c, -VW_SHORT_S1 * s);
-}
 __device__ __forceinline__ void vw_tab_fill(double2* tab, const double2* __restrict__ src) {
   for (int i = threadIdx.x; i < VW_TAB_N; i += blockDim.x) tab[i] = src[i];
 }
@@ -1454,8 +1446,8 @@ __device__ __forceinline__ float vw_vis32(float l, float m, float n, const float
  * turns: the argument rides in the phase's first multiply-add, so a term
  * needs one cosine and one product instead of sine, cosine and two. */
 struct GRec {
-  double ugu, vgu; /* wavelengths; x1024 in the plain form          */
-  double arg, amp; /* visibility: argument (as ugu, vgu), magnitude */
+  double ugu, vgu; /* wavelengths; x1024 for the plain generic kind  */
+  double arg, amp; /* visibility: argument in turns, magnitude        */
 };
 struct GroupSoA {
   GRec* rec;    /* 32 B */
@@ -1502,13 +1494,12 @@ __global__ void k_group_data(const int64_t* __restrict__ gkeys, const int32_t* _
     vi = si / (double)(s1 - s0);
   }
   GRec gr;
-  gr.ugu = ugu * uv_scale; /* 1024 for the plain table sincos, 1 for the mixed form (exact) */
+  gr.ugu = ugu * uv_scale; /* 1024 for the plain generic kind's table sincos, else 1 (exact) */
   gr.vgu = vgu * uv_scale;
   /* finite parts give a finite magnitude (the finite-value filter reads it);
-   * a NaN part, or two infinite ones, make every term NaN */
-  gr.amp = isfinite(vr) && isfinite(vi) ? fmin(hypot(vr, vi), 0x1.fffffffffffffp1023)
-                                        : (isinf(vr) != isinf(vi) && !isnan(vr) && !isnan(vi) ? INFINITY : NAN);
-  gr.arg = (atan2(vi, vr) * VW_INV_TWOPI) * uv_scale;
+   * a part that is not finite makes every term NaN */
+  gr.amp = isfinite(vr) && isfinite(vi) ? fmin(hypot(vr, vi), 0x1.fffffffffffffp1020) : NAN;
+  gr.arg = atan2(vi, vr) * VW_INV_TWOPI;
   g.rec[q] = gr;
   g.v[q] = make_double2(vr, vi);
   g.grep[q] = (int32_t)hr;
@@ -1656,8 +1647,7 @@ __global__ __launch_bounds__(256) void k_group_mask(const double* __restrict__ c
 /* reconstruction                                                       */
 /* ------------------------------------------------------------------ */
 struct ReconArgs {
-  const double2* tab;  /* plain forms, built once per context: the sine table of the generic kind, the
-                        * cosine table of the others */
+  const double2* tab;  /* the sine table (plain), built once per context */
   const double *l, *m, *n;
   int64_t pt0, npts, TP; /* points [pt0, pt0 + npts) of this pass, pt0 = tile0 * TP */
   const uint32_t* gmask; /* [ntile_out][nq_pad / 16] mask words of 16 groups (representative kinds) */
@@ -1726,36 +1716,42 @@ struct ReconAccF32 {
   __device__ double value() const { return s + (double)b; }
 };
 
-/* cos(2 pi (k + f) / N) = ec (1 - a^2 f^2 / 2) + A f (1 - a^2 f^2 / 6) from the
- * table entry (ec, A = -a sin) as a cubic in f: five operations.  The square's
- * coefficient is Taylor's times (1 - (2 sqrt 2 - 2) Y^2 / 12), Y = pi / N = the
- * largest |a f|: with the constant term fixed that spreads the omitted
- * y^4 / 24 (3.8e-12 at Y) over the interval, 6.4e-13 at most. */
-#define VW_COS_C2 (VW_SHORT_C2 * (1.0 - 6.4976e-7))
-#define VW_COS_S3 (-(VW_SHORT_S1 * VW_SHORT_S1) / 6.0)
-__device__ __forceinline__ double vw_tab_cos(double f, const double2& e) {
-  return fma(f, fma(f, fma(f, VW_COS_S3 * e.y, VW_COS_C2 * e.x), e.y), e.x);
+/* cos(2 pi x) without a table.  q = fract(x) and r = q - 1/2 give cos(2 pi x) =
+ * -cos(2 pi r) = -T4(c), c = cos(pi r / 2), T4(c) = 8 (u^2 - u) + 1 with u = c^2.
+ * c is even in r, and r^2 = w + 1/4 with w = q^2 - q, one multiply-add, so c is a
+ * polynomial in w on [-1/4, 0]: degree 5, the minimax fit to |T4'(c)| times the
+ * error, which leaves 1.9e-13 of the cosine.  Seven operations to v = u^2 - u,
+ * with cos(2 pi x) = -8 v - 1; the -1 is summed per group, not per point. */
+__device__ __forceinline__ double vw_cos_v(double x) {
+  const double q = __builtin_amdgcn_fract(x);
+  const double w = fma(q, q, -q);
+  double c = fma(w, -0x1.a1f326935c708p-16, 0x1.d198ac4ebf5c1p-11);
+  c = fma(w, c, -0x1.4705ad44bdfc1p-6);
+  c = fma(w, c, 0x1.e82ab50a06c0cp-3);
+  c = fma(w, c, -0x1.1c5831ae32c64p+0);
+  c = fma(w, c, 0x1.6a09e667f13cap-1);
+  const double u = c * c;
+  return fma(u, u, -u);
 }
 
-/* the PPL points of one lane and one group.  Plain: (ugu, vgu, arg) arrive
- * scaled by 1024; all table indices and reads come before the polynomials so
- * the LDS reads overlap the arithmetic; a point with use[k] false keeps its
- * sum.  A plain term is 11 FP64 instructions (phase 2, split 3, cosine 5, sum
- * 1) where the (re, im) form takes 15; a mixed term saves the sine and a
- * product, 16.2 -> 11.5 issue slots of an FP32 FMA.  Both are bound by VALU
- * issue: one 64-epoch segment at Nside 256 with 32 antennas, plain, 34.7 ->
- * 30.6 ms, its mixed form 16.1 -> 15.0 ms a segment. */
+/* the PPL points of one lane and one group; a point with use[k] false keeps
+ * its sum.  A plain term is 12 FP64 instructions (phase 2, cosine 9, sum 1)
+ * and nothing else: sine and cosine from the 1024-entry LDS table took 15 and
+ * a 16-byte read at a random entry, whose bank conflicts (8 lanes a phase on 8
+ * bank groups, 20 cycles of the CU's one LDS pipe a read) had become the bound.
+ * A mixed term saves the sine and a product of the (re, im) form, 16.2 -> 11.5
+ * issue slots of an FP32 FMA.  Both are bound by VALU issue. */
 template <int PPL, bool MIXED>
 struct ReconLane {
   double d[PPL];
+  double ones = 0.0; /* minus the magnitudes of the groups that every point sees (plain polar terms) */
   ReconAccF32 f[PPL];
   __device__ ReconLane() {
 #pragma unroll
     for (int k = 0; k < PPL; ++k) d[k] = 0.0;
   }
   template <bool MASK>
-  __device__ __forceinline__ void add(const GRec& g, const bool* use, const double* lp, const double* mp,
-                                      const double2* tab) {
+  __device__ __forceinline__ void add(const GRec& g, const bool* use, const double* lp, const double* mp) {
     if (MIXED) {
       const float amp = (float)g.amp;
 #pragma unroll
@@ -1764,16 +1760,12 @@ struct ReconLane {
         f[k].b = !MASK || use[k] ? t : f[k].b;
       }
     } else {
-      double fr[PPL];
-      int ix[PPL];
-#pragma unroll
-      for (int k = 0; k < PPL; ++k) fr[k] = vw_tab_split(fma(g.vgu, mp[k], fma(g.ugu, lp[k], g.arg)), &ix[k]);
-      double2 e[PPL];
-#pragma unroll
-      for (int k = 0; k < PPL; ++k) e[k] = tab[ix[k]];
+      const double a8 = -8.0 * g.amp;
+      if (!MASK) ones -= g.amp;
 #pragma unroll
       for (int k = 0; k < PPL; ++k) {
-        const double t = fma(g.amp, vw_tab_cos(fr[k], e[k]), d[k]);
+        const double v = vw_cos_v(fma(g.vgu, mp[k], fma(g.ugu, lp[k], g.arg)));
+        const double t = fma(a8, v, MASK ? d[k] - g.amp : d[k]);
         d[k] = !MASK || use[k] ? t : d[k];
       }
     }
@@ -1804,17 +1796,18 @@ struct ReconLane {
     }
   }
   /* the (re, im) form of a group's terms, point after point (plain form,
-   * segments without polar terms); use == nullptr: every point */
+   * segments without polar terms) with the sine table in global memory; use ==
+   * nullptr: every point */
   __device__ __forceinline__ void add_one(const GRec& g, const double2& v, const bool* use, const double* lp,
-                                          const double* mp, const double2* tab) {
+                                          const double* mp, const double2* __restrict__ gtab) {
 #pragma unroll
     for (int k = 0; k < PPL; ++k) {
       int ix;
-      const double fr = vw_tab_split(vw_recon_phase(g.ugu, g.vgu, lp[k], mp[k]), &ix);
-      const double2 e = tab[ix];
+      const double fr = vw_tab_split(vw_recon_phase(g.ugu, g.vgu, lp[k], mp[k]) * VW_TAB_SCALE, &ix);
+      const double2 e = gtab[ix];
       double sy, cy, sn, cs;
       vw_tab_poly_short(fr, &sy, &cy);
-      vw_tab_rotate(e.x, e.y * (-1.0 / VW_SHORT_S1), sy, cy, &sn, &cs);
+      vw_tab_rotate(e.x, e.y, sy, cy, &sn, &cs);
       const double t = vw_recon_add(d[k], v.x, v.y, sn, cs);
       d[k] = use == nullptr || use[k] ? t : d[k];
     }
@@ -1825,7 +1818,7 @@ struct ReconLane {
       for (int k = 0; k < PPL; ++k) f[k].fold();
     }
   }
-  __device__ double value(int k) const { return MIXED ? f[k].value() : d[k]; }
+  __device__ double value(int k) const { return MIXED ? f[k].value() : d[k] + ones; }
 };
 
 #ifndef VW_RECON_WAVES_PLAIN
@@ -1840,9 +1833,10 @@ struct ReconLane {
 template <int PPL, bool MIXED, int KIND>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(
     KIND == VW_KIND_GENERIC ? VW_RECON_WAVES_GENERIC : MIXED ? VW_RECON_WAVES_MIXED : VW_RECON_WAVES_PLAIN))) void k_recon(ReconArgs a) {
-  __shared__ double2 tab[MIXED ? 1 : VW_TAB_N];
+  constexpr bool TABLE = !MIXED && KIND == VW_KIND_GENERIC;
+  __shared__ double2 tab[TABLE ? VW_TAB_N : 1];
   __shared__ double gring[4][2 * 64]; /* per wave: two blocks of 16 group records */
-  if (!MIXED) {
+  if (TABLE) {
     vw_tab_fill(tab, a.tab);
     __syncthreads();
   }
@@ -1934,8 +1928,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(
           if (!isfinite(g.amp)) continue;
           wu += 1;
         }
-        if (MIXED || polar) acc.template add<false>(g, nullptr, lp, mp, tab);
-        else acc.add_one(g, a.g.v[q16 + j], nullptr, lp, mp, tab);
+        if (MIXED || polar) acc.template add<false>(g, nullptr, lp, mp);
+        else acc.add_one(g, a.g.v[q16 + j], nullptr, lp, mp, a.tab);
       }
       if (VW_KIND_IS_REP(KIND)) {
         while (part) {
@@ -1967,8 +1961,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(
           }
 #pragma unroll
           for (int k = 0; k < PPL; ++k) wl[k] += use[k] ? 1 : 0;
-          if (MIXED || polar) acc.template add<true>(g, use, lp, mp, tab);
-          else acc.add_one(g, a.g.v[q16 + j], use, lp, mp, tab);
+          if (MIXED || polar) acc.template add<true>(g, use, lp, mp);
+          else acc.add_one(g, a.g.v[q16 + j], use, lp, mp, a.tab);
         }
       }
       if (MIXED && buf) acc.fold(); /* every 32 groups */
