@@ -38,10 +38,10 @@ def test_automatic_form_matches_the_oracle(n_ant, tp, budget):
 
 
 def test_automatic_form_keeps_rows_for_long_baselines_and_nan():
-    """30 MHz (1.4e6 turns) and a sky with a NaN pixel give the row form's bits"""
+    """100 MHz (4.7e6 turns) and a sky with a NaN pixel give the row form's bits"""
     kw = dict(nside=16, n_ant=16, n_epochs=5, segs=1, img_n=0)
     sky = np.random.default_rng(1).lognormal(0.0, 1.0, 12 * 256)
-    long = config(freq_hz=3e7, **kw), config(freq_hz=3e7, viss_form=1, **kw)
+    long = config(freq_hz=1e8, **kw), config(freq_hz=1e8, viss_form=1, **kw)
     assert np.array_equal(_viss(long[0], sky), _viss(long[1], sky))
     bad = sky.copy()
     bad[17] = np.nan

@@ -251,11 +251,12 @@ int sync(Ctx* c) {
  * 0.741 / 1.512 1.410, 32 1.650 0.758 / 2.939 1.409.  So 13-16 and 22-32.
  * Both forms hold the same sums; each row's phase is rounded where the row form
  * rounds it, by up to 2^-53 of the longest baseline in turns several times
- * over.  Up to 2^19 turns (14,000 km at 10 MHz: 4.7e5) that is 3e-10 of the
- * visibilities; longer baselines keep the row form and its rounding.  So do
+ * over.  At 4.7e5 turns (14,000 km at 10 MHz) that is 1.4e-10 of the
+ * visibilities, at 1.4e6 (30 MHz) 4.7e-10; longer baselines keep the row form
+ * and its rounding.  So do
  * skies that are not finite: a product with a masked weight would spread a NaN
  * to rows that do not see its pixel (enq_viss). */
-#define VW_FACT_MAX_TURNS 524288.0
+#define VW_FACT_MAX_TURNS 1.5e6
 bool fact_auto_plain(const vw_config* cfg, double lambda) {
   if (cfg->viss_form != VW_VISS_AUTO || cfg->precision != VW_PREC_PLAIN || cfg->geometry != VW_GEOM_CIRCULAR) return false;
   if (!((cfg->n_ant >= 13 && cfg->n_ant <= 16) || (cfg->n_ant >= 22 && cfg->n_ant <= 32))) return false;
