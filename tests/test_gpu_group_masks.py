@@ -50,3 +50,29 @@ def test_rows_outside_the_grid_and_kinds(kw):
     tol = MIXED_TOL if base.get("precision") else PLAIN_TOL
     assert np.array_equal(W, Wo) and np.array_equal(wi, wio)
     assert rel_err(C, Co) <= tol and rel_err(img, imgo) <= tol
+
+
+# rows at the edges of the grouping's blocks: 64 and 256 (ranks), 128 (radix blocks, above 8,192), 4,096 (run scan)
+@pytest.mark.parametrize("rows", [63, 65, 257, 4095, 4096, 4097, 8192, 8193, 8320, 8321, 12289])
+@pytest.mark.parametrize("full", [0, 1])
+def test_grouping_edges(rows, full):
+    """keys, offsets, order and representatives bit-exact; 1 MHz and one-second
+    epochs put many rows in a cell, so equal keys keep their order"""
+    cfg = config(nside=4, n_ant=2, n_epochs=rows, segs=1, img_n=0, freq_hz=1e6, dt_s=1.0, recon_mode=full, occ_mode=1)
+    sky = np.ones(12 * 16)
+    from oracle.oracle import Oracle
+    from viss_optimize_ws_amd import Pipeline
+
+    with Pipeline(cfg) as g, Oracle(cfg) as o:
+        for x in (g, o):
+            x.set_sky(sky)
+            x.gen_segment(0, rows)
+            x.viss_half()
+            x.conj_fill()
+            x.recon_segment()
+        a, b = g.groups(), o.groups()
+    for k in ("fa", "fb", "denom", "du", "res", "half", "nuniq", "nkeys"):
+        assert a[0][k] == b[0][k], k
+    for x, y in zip(a[1:], b[1:]):
+        assert np.array_equal(x, y)
+    assert a[0]["nuniq"] <= rows * (1 + full)

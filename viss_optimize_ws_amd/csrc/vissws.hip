@@ -117,6 +117,7 @@ struct Ctx {
   int64_t nq_pad = 0;
   bool generic = false; /* recon needs per-row classes of the image tiles */
   DevInfo* d_info = nullptr;
+  double* d_sums = nullptr; /* partial sums of the w-plane fit [5][256] */
   /* sky batch (nsky > 1): packed sky operand, Viss chunk partials, packed
    * group visibilities, recon partials of both output sets */
   bool batch = false;
@@ -486,7 +487,7 @@ constexpr int RECON_PPL = VW_RECON_PPL;
 struct ReconShape {
   int64_t pwaves, nchunk;
 };
-ReconShape recon_shape(int64_t npts) {
+ReconShape recon_shape(int64_t npts, int64_t nq = INT64_MAX) {
   ReconShape r;
   r.pwaves = (npts + 64 * RECON_PPL - 1) / (64 * RECON_PPL);
   const int64_t target_waves = VW_RECON_TARGET_WAVES;
@@ -496,6 +497,10 @@ ReconShape recon_shape(int64_t npts) {
    * recon -4 to -5% per launch); the largest keep the target's count */
   const int64_t lo = std::min<int64_t>(VW_RECON_MIN_CHUNKS, 2 * target_waves / r.pwaves);
   r.nchunk = std::max(r.nchunk, lo);
+  /* ranges are multiples of 16 groups: more of them than the segment's nq rows
+   * can fill would only write and fold zeros (128 ranges for 448 rows at Nside
+   * 32, 28 of them with work) */
+  r.nchunk = std::min(r.nchunk, std::max<int64_t>(1, nq / 16 + (nq % 16 != 0)));
   return r;
 }
 
@@ -768,7 +773,7 @@ int create_device(Ctx* c) {
       (rc = dalloc(c, &c->d_keys, 2 * mh)) || (rc = dalloc(c, &c->d_keys_sorted, 2 * mh)) ||
       (rc = dalloc(c, &c->d_gkeys, 2 * mh + 1)) || (rc = dalloc(c, &c->d_idx_sorted, 2 * mh)) ||
       (rc = dalloc(c, &c->d_goff, 2 * mh + 2)) || (rc = dalloc(c, &c->d_rank, 2 * mh)) ||
-      (rc = dalloc(c, &c->d_info, 1)) ||
+      (rc = dalloc(c, &c->d_info, 1)) || (rc = dalloc(c, &c->d_sums, 5 * 256)) ||
       (rc = dalloc(c, &c->d_out, (size_t)c->npix * c->nsky)) || (rc = dalloc(c, &c->d_wout, (size_t)c->npix)) ||
       (rc = dalloc(c, &c->d_iout, (size_t)std::max<int64_t>(1, (int64_t)c->cfg.img_n * c->cfg.img_n) * c->nsky)) ||
       (rc = dalloc(c, &c->d_iwout, (size_t)std::max<int64_t>(1, (int64_t)c->cfg.img_n * c->cfg.img_n))))
@@ -975,8 +980,8 @@ int enq_viss_fact(Ctx* c, int64_t tile0, int64_t nt) {
  * the Viss stream; 1: its groups on the grouping stream): a stable radix
  * sort of the antenna-direction pair keys */
 /* stable LSD radix sort of n (key, value) pairs over `passes` 8-bit digits
- * from bit 0 with the memset-free kernels of vw_batch.h; the pairs move
- * between (k0, v0) and (k1, v1) and the sorted pairs end in (k1, v1) */
+ * (an even number) from bit 0 with the memset-free kernels of vw_batch.h; the
+ * pairs move between (k0, v0) and (k1, v1) and the sorted pairs end in (k0, v0) */
 template <typename K, typename V>
 int enq_rsort(Ctx* c, int which, hipStream_t st, K* k0, V* v0, K* k1, V* v1, int64_t n, int passes) {
   const int64_t nblk = (n + VW_RS_BLOCK - 1) / VW_RS_BLOCK;
@@ -994,12 +999,6 @@ int enq_rsort(Ctx* c, int which, hipStream_t st, K* k0, V* v0, K* k1, V* v1, int
                                                        ka[cur ^ 1], va[cur ^ 1]);
     KC();
   }
-  if (cur == 0) { /* an even number of passes ends in (k0, v0) */
-    k_copy<K><<<blocks_for(n), 256, 0, st>>>(k0, k1, n);
-    KC();
-    k_copy<V><<<blocks_for(n), 256, 0, st>>>(v0, v1, n);
-    KC();
-  }
   return VW_OK;
 }
 
@@ -1007,14 +1006,14 @@ int enq_order(Ctx* c, int which) {
   hipStream_t st = which == 0 ? c->st : c->stB;
   const int64_t n = which == 0 ? c->nh_pad : c->nq_pad;
   if (which == 0)
-    k_row_keys<<<blocks_for(n), 256, 0, st>>>(c->d_rows, c->d_ant8, c->nh, n, c->d_okey[0], c->d_oidx[0]);
+    k_row_keys<<<blocks_for(n), 256, 0, st>>>(c->d_rows, c->d_ant8, c->nh, n, c->d_okey[0], c->d_order[0]);
   else
     k_group_keys<<<blocks_for(n), 256, 0, st>>>(c->gs.gia, c->gs.gib, c->d_ant8, c->d_info, n, c->d_okey[1],
-                                                c->d_oidx[1]);
+                                                c->d_order[1]);
   KC();
   /* keys below 2^13: two 8-bit digits */
-  return enq_rsort<int32_t, int32_t>(c, which, st, c->d_okey[which], c->d_oidx[which], c->d_okey2[which],
-                                     c->d_order[which], n, 2);
+  return enq_rsort<int32_t, int32_t>(c, which, st, c->d_okey[which], c->d_order[which], c->d_okey2[which],
+                                     c->d_oidx[which], n, 2);
 }
 
 /* one tile pass of the batched Viss: classes, the product kernel, the fold */
@@ -1126,25 +1125,26 @@ int enq_conj(Ctx* c) {
 int enq_group_keys(Ctx* c) {
   bool full = c->cfg.recon_mode == VW_RECON_FULL;
   int64_t nr = full ? 2 * c->nh : c->nh;
-  k_segparams<<<1, 256, 0, c->stB>>>(c->d_rows, c->nh, c->P, c->bl_max, c->lambda, c->d_info);
+  const bool rsort = nr > VW_RANK_MAX;
+  k_segsums<<<4, 64, 0, c->stB>>>(c->d_rows, c->nh, c->P, c->d_sums);
   KC();
-  k_keys<<<blocks_for(nr), 256, 0, c->stB>>>(c->d_rows, nr, c->P, full ? 1 : 0, c->d_info, c->d_keys);
+  /* the radix sort's pairs start and end in the sorted arrays */
+  k_keys<<<blocks_for(nr), 256, 0, c->stB>>>(c->d_sums, c->d_rows, nr, c->P, full ? 1 : 0, c->bl_max, c->lambda,
+                                             c->d_info, rsort ? c->d_keys_sorted : c->d_keys,
+                                             rsort ? c->d_idx_sorted : c->d_rank, rsort ? 1 : 0);
   KC();
-  if (nr > VW_RANK_MAX) {
+  if (rsort) {
     /* long segments: stable LSD radix sort of the (key, row index) pairs
      * over the eight bytes of the non-negative int64 keys */
-    k_iota<<<blocks_for(nr), 256, 0, c->stB>>>(nr, c->d_rank);
-    KC();
-    int rc = enq_rsort<int64_t, int32_t>(c, 1, c->stB, c->d_keys, c->d_rank, c->d_keys_sorted, c->d_idx_sorted, nr, 8);
+    int rc = enq_rsort<int64_t, int32_t>(c, 1, c->stB, c->d_keys_sorted, c->d_idx_sorted, c->d_keys, c->d_rank, nr, 8);
     if (rc) return rc;
   } else {
     /* stable rank by (key, row): a grid of (256 rows) x (jblk rows) compare
-     * tiles sized for about 2,048 workgroups, then a scatter */
-    k_fill0<<<blocks_for(nr), 256, 0, c->stB>>>((uint32_t*)c->d_rank, nr);
-    KC();
+     * tiles sized for about 2,048 workgroups of at least 64 compares a thread
+     * (256 at the least took 20 us for 448 rows as for 3,840), then a scatter */
     const int64_t gx = blocks_for(nr);
-    const int64_t gy = std::max<int64_t>(1, std::min<int64_t>(gx, (2048 + gx - 1) / gx));
-    const int64_t jblk = ((nr + gy - 1) / gy + 255) / 256 * 256;
+    const int64_t gy = std::max<int64_t>(1, std::min<int64_t>((nr + 63) / 64, (2048 + gx - 1) / gx));
+    const int64_t jblk = ((nr + gy - 1) / gy + 63) / 64 * 64;
     dim3 grid((unsigned)gx, (unsigned)((nr + jblk - 1) / jblk));
     k_rank_count<<<grid, 256, 0, c->stB>>>(c->d_keys, nr, jblk, c->d_rank);
     KC();
@@ -1306,7 +1306,7 @@ int enq_recon_set_one(Ctx* c, bool img, double* acc, uint32_t* wacc) {
     /* representatives are filtered for finite values except in the uv-mirror
      * recon with occ_mode 2 */
     const bool rep_finite = !(c->cfg.recon_mode == VW_RECON_MIRROR && c->cfg.occ_mode == 2);
-    ReconShape rs = recon_shape(np);
+    ReconShape rs = recon_shape(np, c->cfg.recon_mode == VW_RECON_FULL ? 2 * c->nh : c->nh);
     if (rs.nchunk * np > c->rpart_cap) return c->fail(VW_ERR_RANGE, "internal: recon partial buffer too small");
     a.pwaves = rs.pwaves;
     a.nchunk = rs.nchunk;

@@ -786,10 +786,9 @@ __global__ void k_fill0(uint32_t* __restrict__ p, int64_t n) {
  * k_rs_scan turns the digit-major table [256][nblk] into exclusive offsets
  * within each digit plus the digit totals, k_rs_scatter places each block's
  * elements at the digit's base (the scan of the totals) plus the block's
- * offset: lane b walks the block's digits in order and moves the elements of
- * digit b to consecutive positions, so equal digits keep their input order
- * (stable). */
-#define VW_RS_BLOCK 128 /* short serial walks in the scatter (one lane per digit) */
+ * offset plus the element's place among the block's equal digits, in input
+ * order (stable). */
+#define VW_RS_BLOCK 128
 template <typename K>
 __global__ __launch_bounds__(256) void k_rs_hist(const K* __restrict__ keys, int64_t n, int shift,
                                                  int32_t* __restrict__ hist, int64_t nblk) {
@@ -829,39 +828,59 @@ __global__ __launch_bounds__(256) void k_rs_scan(int32_t* __restrict__ a, int64_
   }
   if (threadIdx.x == 255) tot[blockIdx.x] = t[255];
 }
+/* Each of the first two waves holds 64 elements, one a lane; the lanes of equal
+ * digit find each other by eight ballots, so an element's place among its
+ * wave's equals is a population count and the second wave starts after the
+ * first one's count.  (One lane per digit walking the block's 128 digits took
+ * 13-15 us a pass.) */
 template <typename K, typename V>
 __global__ __launch_bounds__(256) void k_rs_scatter(const K* __restrict__ kin, const V* __restrict__ vin, int64_t n,
                                                     int shift, const int32_t* __restrict__ offs, int64_t nblk,
                                                     const int32_t* __restrict__ tot, K* __restrict__ kout,
                                                     V* __restrict__ vout) {
-  __shared__ uint8_t d[VW_RS_BLOCK];
-  __shared__ int32_t base[256];
+  static_assert(VW_RS_BLOCK == 128, "two waves of elements");
+  __shared__ int32_t pos0[256]; /* where the block's elements of a digit start   */
+  __shared__ int32_t cnt0[256]; /* elements of a digit in the block's first wave */
+  __shared__ int32_t wsum[4];
   const int64_t b = blockIdx.x;
-  const int64_t i0 = b * VW_RS_BLOCK;
-  const int cnt = (int)(i0 + VW_RS_BLOCK < n ? VW_RS_BLOCK : n - i0);
-  for (int j = threadIdx.x; j < cnt; j += 256) d[j] = (uint8_t)((kin[i0 + j] >> shift) & 255);
-  /* digit bases: exclusive scan of the digit totals */
-  base[threadIdx.x] = tot[threadIdx.x];
-  __syncthreads();
-  for (int o = 1; o < 256; o <<= 1) {
-    const int32_t v = threadIdx.x >= (unsigned)o ? base[threadIdx.x - o] : 0;
-    __syncthreads();
-    base[threadIdx.x] += v;
-    __syncthreads();
+  const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+  const int64_t i = b * VW_RS_BLOCK + t;
+  const bool mine = t < VW_RS_BLOCK && i < n;
+  K key = 0;
+  V val = 0;
+  if (mine) { key = kin[i]; val = vin[i]; }
+  const int32_t off = offs[(int64_t)t * nblk + b]; /* digit t's elements in earlier blocks */
+  /* digit bases: exclusive scan of the digit totals, one digit a thread */
+  const int32_t tt = tot[t];
+  int32_t inc = tt;
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    const int32_t v = __shfl_up(inc, o, 64);
+    if (lane >= o) inc += v;
   }
-  const int bin = threadIdx.x;
-  int64_t pos = (bin ? base[bin - 1] : 0) + offs[(int64_t)bin * nblk + b];
-  for (int j = 0; j < cnt; ++j)
-    if (d[j] == bin) {
-      kout[pos] = kin[i0 + j];
-      vout[pos] = vin[i0 + j];
-      ++pos;
-    }
-}
-template <typename T>
-__global__ void k_copy(const T* __restrict__ a, T* __restrict__ b, int64_t n) {
-  int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) b[i] = a[i];
+  if (lane == 63) wsum[wave] = inc;
+  cnt0[t] = 0;
+  __syncthreads();
+  int32_t before = 0;
+#pragma unroll
+  for (int wv = 0; wv < 3; ++wv) before += wv < wave ? wsum[wv] : 0;
+  pos0[t] = before + inc - tt + off;
+  /* the lanes with this lane's digit (lanes without an element: none) */
+  const int d = (int)((key >> shift) & 255);
+  uint64_t same = __ballot(mine);
+#pragma unroll
+  for (int bit = 0; bit < 8; ++bit) {
+    const uint64_t m = __ballot((d >> bit) & 1);
+    same &= ((d >> bit) & 1) ? m : ~m;
+  }
+  const uint64_t lower = same & ((1ull << lane) - 1);
+  if (wave == 0 && mine && lower == 0) cnt0[d] = __popcll(same);
+  __syncthreads();
+  if (mine) {
+    const int32_t p = pos0[d] + (wave == 1 ? cnt0[d] : 0) + __popcll(lower);
+    kout[p] = key;
+    vout[p] = val;
+  }
 }
 
 #endif

@@ -1313,38 +1313,44 @@ __device__ __forceinline__ int vw_polar_ok(const vw_segparams& sp) {
   return (double)sp.half * sp.du * (2.0 + fabs(sp.fa) + fabs(sp.fb)) <= 4194304.0;
 }
 
-__global__ __launch_bounds__(256) void k_segparams(const RowRec* __restrict__ rows, int64_t nh, int P,
-                                                   double bl_max, double lambda, DevInfo* __restrict__ info) {
-  __shared__ double s[5][256];
-  const int t = threadIdx.x;
+/* The five sums of the w-plane fit over the full rows, in 256 strided partial
+ * sums (partial t: full rows t, t + 256, ... in order) that a pairwise tree
+ * folds: the order every build of this path and its oracle use.  A full row's
+ * products are its half row's (the signs cancel).  One wave per 64 partials on
+ * four CUs, VW_SEG_BATCH rows' loads in flight before they are added in order;
+ * one workgroup with a 64-bit division and a load waited for per row took 86 us
+ * for 31,744 half rows. */
+#define VW_SEG_BATCH 16
+__global__ __launch_bounds__(64) void k_segsums(const RowRec* __restrict__ rows, int64_t nh, int P,
+                                                double* __restrict__ sums) {
+  const int t = blockIdx.x * 64 + threadIdx.x;
+  const int64_t n = 2 * nh;
   double a0 = 0.0, a1 = 0.0, a2 = 0.0, a3 = 0.0, a4 = 0.0;
-  for (int64_t i = t; i < 2 * nh; i += 256) {
-    int64_t g = i / (2 * P);
-    int jj = (int)(i - g * 2 * P);
-    bool neg = jj >= P;
-    int64_t h = g * P + (neg ? jj - P : jj);
-    double sg = neg ? -1.0 : 1.0;
-    RowRec r = rows[h];
-    double u = sg * r.u, v = sg * r.v, w = sg * r.w;
-    a0 = a0 + u * u;
-    a1 = a1 + v * v;
-    a2 = a2 + u * v;
-    a3 = a3 + u * w;
-    a4 = a4 + v * w;
+  const int64_t gstep = (int64_t)(256 / (2 * P)) * P; /* full row i -> i + 256: epochs (as half rows) and pairs */
+  const int jstep = 256 % (2 * P);
+  int64_t gP = (int64_t)(t / (2 * P)) * P; /* first half row of the epoch of full row i */
+  int jj = t % (2 * P);
+  for (int64_t i = t; i < n; i += 256 * VW_SEG_BATCH) {
+    double u[VW_SEG_BATCH], v[VW_SEG_BATCH], w[VW_SEG_BATCH];
+#pragma unroll
+    for (int e = 0; e < VW_SEG_BATCH; ++e) {
+      const RowRec& r = rows[i + 256 * e < n ? gP + (jj >= P ? jj - P : jj) : 0];
+      u[e] = r.u; v[e] = r.v; w[e] = r.w;
+      jj += jstep;
+      gP += gstep;
+      if (jj >= 2 * P) { jj -= 2 * P; gP += P; }
+    }
+#pragma unroll
+    for (int e = 0; e < VW_SEG_BATCH; ++e)
+      if (i + 256 * e < n) {
+        a0 = a0 + u[e] * u[e];
+        a1 = a1 + v[e] * v[e];
+        a2 = a2 + u[e] * v[e];
+        a3 = a3 + u[e] * w[e];
+        a4 = a4 + v[e] * w[e];
+      }
   }
-  s[0][t] = a0; s[1][t] = a1; s[2][t] = a2; s[3][t] = a3; s[4][t] = a4;
-  __syncthreads();
-  for (int st = 128; st > 0; st >>= 1) {
-    if (t < st)
-      for (int k = 0; k < 5; ++k) s[k][t] = s[k][t] + s[k][t + st];
-    __syncthreads();
-  }
-  if (t == 0) {
-    vw_segparams sp;
-    vw_segparams_from_sums(s[0][0], s[1][0], s[2][0], s[3][0], s[4][0], bl_max, lambda, &sp);
-    info->sp = sp;
-    info->polar = vw_polar_ok(sp);
-  }
+  sums[t] = a0; sums[256 + t] = a1; sums[512 + t] = a2; sums[768 + t] = a3; sums[1024 + t] = a4;
 }
 
 /* mode row -> (half row, conjugate flag) */
@@ -1356,16 +1362,41 @@ __device__ __forceinline__ int64_t vw_row_half(int64_t r, int P, bool full, bool
   return g * P + (jj >= P ? jj - P : jj);
 }
 
-__global__ void k_keys(const RowRec* __restrict__ rows, int64_t nr, int P, int full, const DevInfo* __restrict__ info,
-                       int64_t* __restrict__ keys) {
-  int64_t r = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (r >= nr) return;
+/* segment parameters from the partial sums (every workgroup folds them, the
+ * first writes them), then the uv-grid key of each row and, in idx, its index
+ * (iota, for the radix sort) or zero (for k_rank_count) */
+__global__ __launch_bounds__(256) void k_keys(const double* __restrict__ sums, const RowRec* __restrict__ rows,
+                                              int64_t nr, int P, int full, double bl_max, double lambda,
+                                              DevInfo* __restrict__ info, int64_t* __restrict__ keys,
+                                              int32_t* __restrict__ idx, int iota) {
+  __shared__ double s[5][256];
+  __shared__ vw_segparams ssp;
+  const int t = threadIdx.x;
+#pragma unroll
+  for (int k = 0; k < 5; ++k) s[k][t] = sums[256 * k + t];
+  const int64_t r = (int64_t)blockIdx.x * 256 + t;
   bool neg;
-  int64_t h = vw_row_half(r, P, full != 0, &neg);
-  double sg = neg ? -1.0 : 1.0;
-  RowRec rec = rows[h];
-  vw_segparams sp = info->sp;
+  const int64_t h = vw_row_half(r < nr ? r : 0, P, full != 0, &neg);
+  const RowRec rec = rows[h];
+  __syncthreads();
+  for (int st = 128; st > 0; st >>= 1) {
+    if (t < st)
+      for (int k = 0; k < 5; ++k) s[k][t] = s[k][t] + s[k][t + st];
+    __syncthreads();
+  }
+  if (t == 0) {
+    vw_segparams_from_sums(s[0][0], s[1][0], s[2][0], s[3][0], s[4][0], bl_max, lambda, &ssp);
+    if (blockIdx.x == 0) {
+      info->sp = ssp;
+      info->polar = vw_polar_ok(ssp);
+    }
+  }
+  __syncthreads();
+  if (r >= nr) return;
+  const vw_segparams sp = ssp;
+  const double sg = neg ? -1.0 : 1.0;
   keys[r] = vw_grid_key(sg * rec.u, sg * rec.v, &sp, full ? 0 : 1);
+  idx[r] = iota ? (int32_t)r : 0;
 }
 
 /* Stable order by (key, row index): all-pairs rank counted over a 2-D grid
@@ -1398,11 +1429,6 @@ __global__ __launch_bounds__(256) void k_rank_count(const int64_t* __restrict__ 
 /* segments longer than this many rows are ordered by a radix sort */
 #define VW_RANK_MAX 8192
 
-__global__ void k_iota(int64_t n, int32_t* __restrict__ out) {
-  int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) out[i] = (int32_t)i;
-}
-
 __global__ void k_rank_scatter(const int64_t* __restrict__ keys, const int32_t* __restrict__ rank, int64_t nr,
                                int32_t* __restrict__ idx_sorted, int64_t* __restrict__ keys_sorted) {
   int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -1411,38 +1437,66 @@ __global__ void k_rank_scatter(const int64_t* __restrict__ keys, const int32_t* 
   keys_sorted[rank[i]] = keys[i];
 }
 
-/* run boundaries -> keys, offsets, nuniq (single workgroup) */
+/* run boundaries -> keys, offsets, nuniq (single workgroup): 4,096 sorted keys
+ * at a time, four consecutive ones a thread, the next ones loaded while these
+ * are counted; boundary counts are scanned in the waves, then over the 16 waves.
+ * (A run of nr / 1024 keys a thread, walked twice from global memory, took 82 us
+ * for 31,744 rows.) */
 __global__ __launch_bounds__(1024) void k_groups(const int64_t* __restrict__ ks, int64_t nr, int blockage,
                                                  int64_t* __restrict__ gkeys, int32_t* __restrict__ goff,
                                                  DevInfo* __restrict__ info) {
-  __shared__ int64_t sc[1024];
-  const int t = threadIdx.x;
-  int64_t per = (nr + 1023) / 1024;
-  int64_t b = t * per, e = b + per < nr ? b + per : nr;
-  int64_t c = 0;
-  for (int64_t k = b; k < e; ++k) c += (k == 0 || ks[k] != ks[k - 1]);
-  sc[t] = c;
-  __syncthreads();
-  for (int s = 1; s < 1024; s <<= 1) {
-    int64_t v = t >= s ? sc[t - s] : 0;
-    __syncthreads();
-    sc[t] += v;
-    __syncthreads();
-  }
-  int64_t g = sc[t] - c; /* exclusive */
-  for (int64_t k = b; k < e; ++k) {
-    if (k == 0 || ks[k] != ks[k - 1]) {
-      gkeys[g] = ks[k];
-      goff[g] = (int32_t)k;
-      ++g;
+  __shared__ int32_t wtot[2][16];
+  const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+  int64_t k[4], prev;
+  auto load = [&](int64_t i0) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) k[e] = i0 + e < nr ? ks[i0 + e] : 0;
+    prev = i0 > 0 && i0 <= nr ? ks[i0 - 1] : 0;
+  };
+  int64_t i = 4 * t;
+  load(i);
+  int32_t base = 0; /* groups before this block of 4,096 keys */
+  int buf = 0;
+  for (int64_t b0 = 0; b0 < nr; b0 += 4096, i += 4096, buf ^= 1) {
+    int64_t c[4];
+    int f[4], cnt = 0;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      c[e] = k[e];
+      f[e] = i + e < nr && (i + e == 0 || k[e] != (e ? k[e > 0 ? e - 1 : 0] : prev)) ? 1 : 0;
+      cnt += f[e];
     }
+    if (b0 + 4096 < nr) load(i + 4096);
+    int inc = cnt;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const int v = __shfl_up(inc, o, 64);
+      if (lane >= o) inc += v;
+    }
+    if (lane == 63) wtot[buf][wave] = inc;
+    __syncthreads();
+    int32_t before = 0, all = 0;
+#pragma unroll
+    for (int wv = 0; wv < 16; ++wv) {
+      const int32_t x = wtot[buf][wv];
+      before += wv < wave ? x : 0;
+      all += x;
+    }
+    int32_t g = base + before + inc - cnt;
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      if (f[e]) {
+        gkeys[g] = c[e];
+        goff[g] = (int32_t)(i + e);
+        ++g;
+      }
+    base += all;
   }
-  if (t == 1023) {
-    int64_t nu = sc[1023];
-    goff[nu] = (int32_t)nr;
-    info->nuniq = nu;
-    info->first_nz = (nu > 0 && ks[0] == 0) ? 1 : 0;
-    if (!blockage) info->wtotal += nu;
+  if (t == 0) {
+    goff[base] = (int32_t)nr;
+    info->nuniq = base;
+    info->first_nz = (base > 0 && ks[0] == 0) ? 1 : 0;
+    if (!blockage) info->wtotal += base;
   }
 }
 
