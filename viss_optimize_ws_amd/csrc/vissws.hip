@@ -58,7 +58,7 @@ struct Ctx {
    * buffers alternate between two sets) */
   hipStream_t stB = nullptr;
   hipStream_t st2 = nullptr;
-  hipEvent_t ev_fork = nullptr, ev_join = nullptr, ev_conj = nullptr;
+  hipEvent_t ev_fork = nullptr, ev_join = nullptr, ev_conj = nullptr, ev_gen = nullptr;
   hipEvent_t ev_recon[2] = {nullptr, nullptr}; /* recon done with segment buffer set b */
   int cur = 1;                                  /* buffer set of the current segment   */
   std::vector<void*> allocs;
@@ -67,6 +67,7 @@ struct Ctx {
   double* d_B = nullptr;
   float* d_Bf = nullptr;
   int64_t* d_gidx = nullptr;
+  int32_t* d_ginv = nullptr; /* point of each image pixel, -1 outside the disk */
   double *d_gl = nullptr, *d_gm = nullptr, *d_gn = nullptr, *d_gcone = nullptr;
   double* d_pos = nullptr;
   int64_t* d_t1s = nullptr;
@@ -681,6 +682,30 @@ int create_batch(Ctx* c) {
   return VW_OK;
 }
 
+/* accumulators and the running key total cleared in one launch (no memset nodes) */
+int enq_reset_fill(Ctx* c) {
+  ClearArgs a{};
+  int64_t most = 0;
+  auto add = [&](void* p, int64_t words) {
+    if (!p || !words) return;
+    a.p[a.cnt] = (uint32_t*)p;
+    a.n[a.cnt++] = words;
+    most = std::max(most, words);
+  };
+  add(c->d_Cacc, 2 * c->npix * c->nsky);
+  add(c->d_Wacc, c->npix);
+  add(c->d_Gacc, 2 * c->ngp * c->nsky);
+  add(c->d_GWacc, c->ngp);
+  add(c->d_info, (int64_t)(sizeof(DevInfo) / 4));
+  if (c->sky_sched) {
+    add(c->d_Wsky, c->npix * c->nsky);
+    add(c->d_GWsky, c->ngp * c->nsky);
+  }
+  k_clear<<<(unsigned)std::min<int64_t>(blocks_for(most, 1024), 4096), 256, 0, c->st>>>(a);
+  KC();
+  return VW_OK;
+}
+
 int create_device(Ctx* c) {
   int ndev = 0;
   if (hipGetDeviceCount(&ndev) != hipSuccess || ndev <= 0) return c->fail(VW_ERR_DEVICE, "no HIP device");
@@ -694,6 +719,7 @@ int create_device(Ctx* c) {
   HC(hipEventCreateWithFlags(&c->ev_fork, hipEventDisableTiming));
   HC(hipEventCreateWithFlags(&c->ev_join, hipEventDisableTiming));
   HC(hipEventCreateWithFlags(&c->ev_conj, hipEventDisableTiming));
+  HC(hipEventCreateWithFlags(&c->ev_gen, hipEventDisableTiming));
   for (int b = 0; b < 2; ++b) HC(hipEventCreateWithFlags(&c->ev_recon[b], hipEventDisableTiming));
   int rc;
   const size_t np = (size_t)c->npix;
@@ -716,6 +742,11 @@ int create_device(Ctx* c) {
         (rc = dalloc(c, &c->d_Gacc, ng * (size_t)c->nsky)) || (rc = dalloc(c, &c->d_GWacc, ng)))
       return rc;
     HC(hipMemcpyAsync(c->d_gidx, c->gidx.data(), sizeof(int64_t) * ng, hipMemcpyHostToDevice, c->st));
+    const size_t NN = (size_t)c->cfg.img_n * c->cfg.img_n;
+    if ((rc = dalloc(c, &c->d_ginv, NN))) return rc;
+    HC(hipMemsetAsync(c->d_ginv, 0xff, sizeof(int32_t) * NN, c->st));
+    k_grid_inv<<<blocks_for(c->ngp), 256, 0, c->st>>>(c->ngp, c->d_gidx, c->d_ginv);
+    KC();
     k_grid_points<<<blocks_for(c->ngp), 256, 0, c->st>>>(c->cfg.img_n, c->ngp, c->d_gidx, c->d_gl, c->d_gm, c->d_gn);
     KC();
     if (c->TP == 256) k_tile_cone<256><<<(unsigned)c->ngt, 256, 0, c->st>>>(c->d_gl, c->d_gm, c->d_gn, c->ngp, c->ngt, c->d_gcone);
@@ -818,13 +849,7 @@ int create_device(Ctx* c) {
       return rc;
   }
   if (c->batch && (rc = create_batch(c))) return rc;
-  HC(hipMemsetAsync(c->d_info, 0, sizeof(DevInfo), c->st));
-  HC(hipMemsetAsync(c->d_Cacc, 0, sizeof(double) * np * c->nsky, c->st));
-  HC(hipMemsetAsync(c->d_Wacc, 0, sizeof(uint32_t) * np, c->st));
-  if (c->ngp) {
-    HC(hipMemsetAsync(c->d_Gacc, 0, sizeof(double) * c->ngp * c->nsky, c->st));
-    HC(hipMemsetAsync(c->d_GWacc, 0, sizeof(uint32_t) * c->ngp, c->st));
-  }
+  if ((rc = enq_reset_fill(c))) return rc;
   if ((rc = upload_day(c))) return rc;
   HC(hipStreamSynchronize(c->st));
   return VW_OK;
@@ -842,17 +867,11 @@ int enq_gen(Ctx* c, int t0, int tlen) {
   HC(hipStreamWaitEvent(c->st, c->ev_recon[c->cur], 0));
   ev_begin(c, ST_GEN);
   int64_t na = (int64_t)tlen * c->A;
-  k_seg_ant<<<blocks_for(na), 256, 0, c->st>>>(c->d_pos, c->T, c->A, t0, tlen, c->per_ant ? c->cfg.occ_radius_km : 0.0,
-                                               c->cosphi_glob, c->d_ant8);
+  k_seg_gen<<<blocks_for(std::max(na, c->nh)), 256, 0, c->st>>>(
+      c->d_pos, c->T, c->A, c->P, t0, tlen, c->per_ant ? c->cfg.occ_radius_km : 0.0, c->cosphi_glob, c->d_pa, c->d_pb,
+      c->lambda, c->d_ant8, c->vfact ? c->d_aph : nullptr,
+      c->vfact && c->cfg.precision == VW_PREC_PLAIN ? c->d_aphl : nullptr, c->d_rows, c->d_rowt);
   KC();
-  k_seg_rows<<<blocks_for(c->nh), 256, 0, c->st>>>(c->d_pos, c->T, c->A, c->P, t0, c->nh, c->d_pa, c->d_pb, c->lambda,
-                                                   c->d_rows, c->d_rowt);
-  KC();
-  if (c->vfact) {
-    k_ant_phase<<<blocks_for(na), 256, 0, c->st>>>(c->d_pos, c->T, c->A, t0, tlen, c->lambda, c->d_aph,
-                                                   c->cfg.precision == VW_PREC_PLAIN ? c->d_aphl : nullptr);
-    KC();
-  }
   ev_end(c, ST_GEN);
   c->have_seg = true;
   c->have_viss = c->have_conj = c->have_groups = false;
@@ -903,23 +922,27 @@ int enq_classes(Ctx* c, const double* cone, int64_t ntile_all, int64_t tile0, in
   return VW_OK;
 }
 
-/* the one-sky recon's group masks of a tile pass ([nt][nq_pad / 16] words) into
- * the class scratch */
-int enq_group_masks(Ctx* c, const double* cone, int64_t ntile_all, int64_t tile0, int64_t nt, uint8_t* bits,
-                    uint32_t* gmask, hipStream_t st) {
+/* the one-sky recon's group masks of a pass ([nt][nq_pad / 16] words per output
+ * set) into the sets' class scratch */
+int enq_group_masks(Ctx* c, const ReconSets& sets, uint8_t* const* bits) {
   const int64_t nfr = (int64_t)c->tlen * c->A;
+  const unsigned nb = (unsigned)(sets.s[0].nt + sets.s[1].nt);
   if (c->nfr_pad <= VW_GCLS_LDS_MAX) {
-    k_group_mask<true><<<(unsigned)nt, 256, (size_t)c->nfr_pad, st>>>(cone, ntile_all, tile0, c->d_ant8, nfr, nullptr,
-                                                                       c->nfr_pad, c->gs.gia, c->gs.gib, c->d_info,
-                                                                       c->nq_pad, gmask);
+    k_group_mask<true><<<nb, 256, (size_t)c->nfr_pad, c->stB>>>(sets, c->d_ant8, nfr, c->nfr_pad, c->gs.gia, c->gs.gib,
+                                                                 c->d_info, c->nq_pad);
     KC();
     return VW_OK;
   }
-  if (nt * c->nfr_pad > c->bits_cap) return c->fail(VW_ERR_RANGE, "internal: cone bit buffer too small");
-  k_ant_bits<<<blocks_for(nt * c->nfr_pad), 256, 0, st>>>(cone, ntile_all, tile0, nt, c->d_ant8, nfr, c->nfr_pad, bits);
-  KC();
-  k_group_mask<false><<<(unsigned)nt, 256, 0, st>>>(cone, ntile_all, tile0, c->d_ant8, nfr, bits, c->nfr_pad, c->gs.gia,
-                                                    c->gs.gib, c->d_info, c->nq_pad, gmask);
+  for (int i = 0; i < 2; ++i) {
+    const ReconSet& S = sets.s[i];
+    if (!S.nt) continue;
+    if (S.nt * c->nfr_pad > c->bits_cap) return c->fail(VW_ERR_RANGE, "internal: cone bit buffer too small");
+    k_ant_bits<<<blocks_for(S.nt * c->nfr_pad), 256, 0, c->stB>>>(S.cone, S.ntile, S.tile0, S.nt, c->d_ant8, nfr,
+                                                                  c->nfr_pad, bits[i]);
+    KC();
+  }
+  k_group_mask<false><<<nb, 256, 0, c->stB>>>(sets, c->d_ant8, nfr, c->nfr_pad, c->gs.gia, c->gs.gib, c->d_info,
+                                              c->nq_pad);
   KC();
   return VW_OK;
 }
@@ -934,7 +957,7 @@ void launch_viss(const VissArgs& a, unsigned nb, hipStream_t st) {
 
 /* one tile pass of the antenna-factorized Viss: cone bits per (tile, frame),
  * the product blocks, then their fold into the raw half sums */
-int enq_viss_fact(Ctx* c, int64_t tile0, int64_t nt) {
+int enq_viss_fact(Ctx* c, int64_t tile0, int64_t nt, double2* vh) {
   const bool mixed = c->cfg.precision == VW_PREC_MIXED;
   const int G = vissf_groups(c->A);
   VissFShape s = viss_fshape(c, c->tlen, nt, c->fpart_cap / ((int64_t)c->tlen * vissf_blocks(G) * 256));
@@ -971,7 +994,7 @@ int enq_viss_fact(Ctx* c, int64_t tile0, int64_t nt) {
   k_vissf_fold<<<(unsigned)(c->tlen * (nent / 32)), 256, 0, c->st>>>(c->d_fpart, s.nchunk, nent, c->d_fesum);
   KC();
   k_vissf_rows<<<blocks_for(c->nh), 256, 0, c->st>>>(c->d_fesum, c->nh, c->P, G, c->d_pa, c->d_pb, tile0 > 0 ? 1 : 0,
-                                                     c->d_vraw);
+                                                     c->d_vraw, c->d_rows, vh);
   KC();
   return VW_OK;
 }
@@ -1047,7 +1070,9 @@ int enq_viss_batch(Ctx* c, int64_t tile0, int64_t nt) {
   return VW_OK;
 }
 
-int enq_viss(Ctx* c, bool count) {
+/* the Viss of the current segment; fill: the conjugate fill's phase correction
+ * with the last fold (whole steps of one sky; the full rows are not formed) */
+int enq_viss(Ctx* c, bool count, bool fill = false) {
   if (!c->have_seg || !c->have_sky) return c->fail(VW_ERR_STATE, "vw_viss_half needs vw_set_sky and vw_gen_segment");
   if (count && c->batch) return c->fail(VW_ERR_ARG, "per-row counts come from the one-sky form (nsky = 1)");
   if (count && !c->d_cpart) {
@@ -1060,13 +1085,14 @@ int enq_viss(Ctx* c, bool count) {
   ev_begin(c, ST_VISS);
   for (int64_t tile0 = 0; tile0 < c->ntile; tile0 += c->vtpp) {
     const int64_t nt = std::min(c->vtpp, c->ntile - tile0);
+    double2* vh = fill && !c->batch && tile0 + nt == c->ntile ? c->d_vh : nullptr;
     if (c->batch) {
       if (tile0 == 0 && (rc = enq_order(c, 0))) return rc;
       if ((rc = enq_viss_batch(c, tile0, nt))) return rc;
       continue;
     }
     if (c->vfact && !count && !(c->fact_auto && !c->sky_finite)) {
-      if ((rc = enq_viss_fact(c, tile0, nt))) return rc;
+      if ((rc = enq_viss_fact(c, tile0, nt, vh))) return rc;
       continue;
     }
     VissShape s = viss_shape(c, c->nh, nt, count, c->nchunk_max);
@@ -1095,12 +1121,16 @@ int enq_viss(Ctx* c, bool count) {
     ev_end(c, ST_VISSK);
     k_viss_reduce<<<blocks_for(c->nh), 256, 0, c->st>>>(c->d_part, s.nchunk, c->nh, c->nh_pad, tile0 > 0 ? 1 : 0,
                                                         c->d_vraw, count ? c->d_cpart : nullptr,
-                                                        count ? c->d_counts : nullptr);
+                                                        count ? c->d_counts : nullptr, c->d_rows, vh);
     KC();
   }
   ev_end(c, ST_VISS);
   c->have_viss = true;
   c->have_conj = c->have_groups = false;
+  if (fill && !c->batch) {
+    HC(hipEventRecord(c->ev_conj, c->st));
+    c->have_conj = true;
+  }
   return VW_OK;
 }
 
@@ -1170,13 +1200,13 @@ int enq_group_data(Ctx* c, const double2* vh) {
   return VW_OK;
 }
 
-int enq_group(Ctx* c) {
+int enq_group(Ctx* c, bool keys_done) {
   if (!c->have_conj) return c->fail(VW_ERR_STATE, "vw_recon_segment needs vw_conj_fill");
   bool full = c->cfg.recon_mode == VW_RECON_FULL;
   HC(hipStreamWaitEvent(c->stB, c->ev_conj, 0));
   ev_begin(c, ST_GROUP, c->stB);
   int rcg;
-  if ((rcg = enq_group_keys(c)) || (rcg = enq_group_data(c, c->d_vh))) return rcg;
+  if ((!keys_done && (rcg = enq_group_keys(c))) || (rcg = enq_group_data(c, c->d_vh))) return rcg;
   if (c->batch) {
     int rc;
     if ((rc = enq_order(c, 1))) return rc;
@@ -1196,8 +1226,7 @@ int enq_group(Ctx* c) {
 
 template <bool MIXED, int KIND>
 void launch_recon(const ReconArgs& a, hipStream_t st) {
-  int64_t waves = a.pwaves * a.nchunk;
-  k_recon<RECON_PPL, MIXED, KIND><<<blocks_for(waves, 4), 256, 0, st>>>(a);
+  k_recon<RECON_PPL, MIXED, KIND><<<(unsigned)(a.sets.s[0].nblk + a.sets.s[1].nblk), 256, 0, st>>>(a);
 }
 
 /* batched recon of one output set: per tile pass the (tile, group) classes,
@@ -1255,43 +1284,64 @@ int enq_recon_set_batch(Ctx* c, bool img) {
   return VW_OK;
 }
 
-/* one-sky recon of one output set into the accumulators acc / wacc (per
- * tile pass: classes, the recon kernel, the ordered fold of its chunks) */
-int enq_recon_set_one(Ctx* c, bool img, double* acc, uint32_t* wacc) {
-  /* each output set has its own stream and scratch */
-  hipStream_t st = img ? c->st2 : c->stB;
-  uint8_t* cls = img ? c->d_cls2 : c->d_cls;
-  uint8_t* bits = img ? c->d_bits2 : c->d_bits;
+/* one-sky recon of the wanted output sets (0: HEALPix map, 1: lm image) into
+ * their accumulators.  Per tile pass one launch each of the classes, the recon
+ * kernel and the ordered fold of its chunks covers both sets: two streams with
+ * a launch per set cost three more launches, a fork and a join a segment. */
+int enq_recon_one(Ctx* c, double* const (&acc)[2], uint32_t* const (&wacc)[2]) {
   int kind;
   if (!c->cfg.blockage) kind = VW_KIND_AVG;
   else if (!c->generic) kind = VW_KIND_REP;
   else kind = VW_KIND_GENERIC;
   const bool mixed = c->cfg.precision == VW_PREC_MIXED;
-  const int64_t npts_all = img ? c->ngp : c->npix;
-  const int64_t ntile_all = img ? c->ngt : c->ntile;
-  const double* cone = img ? c->d_gcone : c->d_cone;
+  const bool full = c->cfg.recon_mode == VW_RECON_FULL;
   const int64_t kind_w = kind == VW_KIND_GENERIC ? c->nh_pad : c->nq_pad;
-  const int64_t otpp = recon_pass_tiles(c, ntile_all, kind_w);
-  for (int64_t tile0 = 0; tile0 < ntile_all; tile0 += otpp) {
-    const int64_t nt = std::min(otpp, ntile_all - tile0);
-    const int64_t pt0 = tile0 * c->TP;
-    const int64_t np = std::min(nt * c->TP, npts_all - pt0);
-    if (kind != VW_KIND_AVG) {
-      int rc = kind == VW_KIND_REP ? enq_group_masks(c, cone, ntile_all, tile0, nt, bits, (uint32_t*)cls, st)
-                                   : enq_classes(c, cone, ntile_all, tile0, nt, false, bits, cls, st);
-      if (rc) return rc;
-    }
+  const bool want[2] = {c->cfg.healpix_out != 0, c->ngp > 0};
+  uint8_t* const bits[2] = {c->d_bits, c->d_bits2};
+  for (int64_t pass = 0;; ++pass) {
     ReconArgs a{};
+    int64_t npts_all = 0;
+    for (int i = 0; i < 2; ++i) {
+      ReconSet& S = a.sets.s[i];
+      S.ntile = i ? c->ngt : c->ntile;
+      if (!want[i]) continue;
+      const int64_t otpp = recon_pass_tiles(c, S.ntile, kind_w);
+      S.tile0 = pass * otpp;
+      if (S.tile0 >= S.ntile) continue;
+      S.nt = std::min(otpp, S.ntile - S.tile0);
+      S.l = i ? c->d_gl : c->d_l;
+      S.m = i ? c->d_gm : c->d_m;
+      S.n = i ? c->d_gn : c->d_n;
+      S.cone = i ? c->d_gcone : c->d_cone;
+      S.pt0 = S.tile0 * c->TP;
+      S.npts = std::min(S.nt * c->TP, (i ? c->ngp : c->npix) - S.pt0);
+      S.cls = (uint32_t*)(i ? c->d_cls2 : c->d_cls);
+      S.bits = bits[i];
+      const ReconShape rs = recon_shape(S.npts, full ? 2 * c->nh : c->nh);
+      if (rs.nchunk * S.npts > c->rpart_cap) return c->fail(VW_ERR_RANGE, "internal: recon partial buffer too small");
+      S.nchunk = rs.nchunk;
+      S.pwaves = rs.pwaves;
+      S.nblk = blocks_for(rs.nchunk * rs.pwaves, 4);
+      S.part = i ? c->d_rpart2 : c->d_rpart;
+      S.wpart = i ? c->d_rwpart2 : c->d_rwpart;
+      S.acc = acc[i];
+      S.wacc = wacc[i];
+      npts_all += S.npts;
+    }
+    if (!npts_all) return VW_OK;
+    int rc;
+    if (kind == VW_KIND_REP) {
+      if ((rc = enq_group_masks(c, a.sets, bits))) return rc;
+    } else if (kind == VW_KIND_GENERIC) {
+      for (int i = 0; i < 2; ++i) {
+        const ReconSet& S = a.sets.s[i];
+        if (S.nt && (rc = enq_classes(c, S.cone, S.ntile, S.tile0, S.nt, false, bits[i], (uint8_t*)S.cls, c->stB)))
+          return rc;
+      }
+    }
     a.tab = c->d_tab;
-    a.l = img ? c->d_gl : c->d_l;
-    a.m = img ? c->d_gm : c->d_m;
-    a.n = img ? c->d_gn : c->d_n;
-    a.pt0 = pt0;
-    a.npts = np;
     a.TP = c->TP;
-    a.gmask = (const uint32_t*)cls;
     a.nq_pad = c->nq_pad;
-    a.rcls = (const uint32_t*)cls;
     a.nh_pad = c->nh_pad;
     a.g = c->gs;
     a.goff = c->d_goff;
@@ -1301,58 +1351,53 @@ int enq_recon_set_one(Ctx* c, bool img, double* acc, uint32_t* wacc) {
     a.ant8 = c->d_ant8;
     a.info = c->d_info;
     a.P = c->P;
-    a.full = c->cfg.recon_mode == VW_RECON_FULL;
+    a.full = full;
     a.occ_mode = c->cfg.occ_mode;
     /* representatives are filtered for finite values except in the uv-mirror
      * recon with occ_mode 2 */
-    const bool rep_finite = !(c->cfg.recon_mode == VW_RECON_MIRROR && c->cfg.occ_mode == 2);
-    ReconShape rs = recon_shape(np, c->cfg.recon_mode == VW_RECON_FULL ? 2 * c->nh : c->nh);
-    if (rs.nchunk * np > c->rpart_cap) return c->fail(VW_ERR_RANGE, "internal: recon partial buffer too small");
-    a.pwaves = rs.pwaves;
-    a.nchunk = rs.nchunk;
-    a.pstride = np;
-    a.part = img ? c->d_rpart2 : c->d_rpart;
-    a.wpart = img ? c->d_rwpart2 : c->d_rwpart;
-    ev_begin(c, ST_RECONK, st);
+    const bool rep_finite = full || c->cfg.occ_mode != 2;
+    ev_begin(c, ST_RECONK, c->stB);
     if (mixed) {
-      if (kind == VW_KIND_REP && rep_finite) launch_recon<true, VW_KIND_REP_FINITE>(a, st);
-      else if (kind == VW_KIND_REP) launch_recon<true, VW_KIND_REP>(a, st);
-      else if (kind == VW_KIND_GENERIC) launch_recon<true, VW_KIND_GENERIC>(a, st);
-      else launch_recon<true, VW_KIND_AVG>(a, st);
+      if (kind == VW_KIND_REP && rep_finite) launch_recon<true, VW_KIND_REP_FINITE>(a, c->stB);
+      else if (kind == VW_KIND_REP) launch_recon<true, VW_KIND_REP>(a, c->stB);
+      else if (kind == VW_KIND_GENERIC) launch_recon<true, VW_KIND_GENERIC>(a, c->stB);
+      else launch_recon<true, VW_KIND_AVG>(a, c->stB);
     } else {
-      if (kind == VW_KIND_REP && rep_finite) launch_recon<false, VW_KIND_REP_FINITE>(a, st);
-      else if (kind == VW_KIND_REP) launch_recon<false, VW_KIND_REP>(a, st);
-      else if (kind == VW_KIND_GENERIC) launch_recon<false, VW_KIND_GENERIC>(a, st);
-      else launch_recon<false, VW_KIND_AVG>(a, st);
+      if (kind == VW_KIND_REP && rep_finite) launch_recon<false, VW_KIND_REP_FINITE>(a, c->stB);
+      else if (kind == VW_KIND_REP) launch_recon<false, VW_KIND_REP>(a, c->stB);
+      else if (kind == VW_KIND_GENERIC) launch_recon<false, VW_KIND_GENERIC>(a, c->stB);
+      else launch_recon<false, VW_KIND_AVG>(a, c->stB);
     }
     KC();
-    ev_end(c, ST_RECONK, st);
-    k_recon_reduce<<<blocks_for(np), 256, 0, st>>>(a.part, a.wpart, a.nchunk, a.pstride, pt0, np, c->cfg.blockage,
-                                                      acc, wacc);
+    ev_end(c, ST_RECONK, c->stB);
+    k_recon_reduce<<<blocks_for(a.sets.s[0].npts) + blocks_for(a.sets.s[1].npts), 256, 0, c->stB>>>(a.sets,
+                                                                                                    c->cfg.blockage);
     KC();
   }
-  return VW_OK;
 }
 
-int enq_recon_set(Ctx* c, bool img) {
-  if (c->batch) return enq_recon_set_batch(c, img);
-  return enq_recon_set_one(c, img, img ? c->d_Gacc : c->d_Cacc, img ? c->d_GWacc : c->d_Wacc);
-}
-
-int enq_recon(Ctx* c) {
+/* the recon stage of the current segment after its groups' keys (keys_done) or
+ * from the start */
+int enq_recon(Ctx* c, bool keys_done = false) {
   int rc;
-  if ((rc = enq_group(c))) return rc;
+  if ((rc = enq_group(c, keys_done))) return rc;
   ev_begin(c, ST_RECON, c->stB);
-  if (c->ngp) {
-    /* the image set runs on its own stream beside the HEALPix set; both
-     * read the groups and write disjoint accumulators */
-    HC(hipEventRecord(c->ev_fork, c->stB));
-    HC(hipStreamWaitEvent(c->st2, c->ev_fork, 0));
-    if ((rc = enq_recon_set(c, true))) return rc;
-    HC(hipEventRecord(c->ev_join, c->st2));
+  if (c->batch) {
+    if (c->ngp) {
+      /* the image set runs on its own stream beside the HEALPix set; both
+       * read the groups and write disjoint accumulators */
+      HC(hipEventRecord(c->ev_fork, c->stB));
+      HC(hipStreamWaitEvent(c->st2, c->ev_fork, 0));
+      if ((rc = enq_recon_set_batch(c, true))) return rc;
+      HC(hipEventRecord(c->ev_join, c->st2));
+    }
+    if (c->cfg.healpix_out && (rc = enq_recon_set_batch(c, false))) return rc;
+    if (c->ngp) HC(hipStreamWaitEvent(c->stB, c->ev_join, 0));
+  } else {
+    double* const acc[2] = {c->d_Cacc, c->d_Gacc};
+    uint32_t* const wacc[2] = {c->d_Wacc, c->d_GWacc};
+    if ((rc = enq_recon_one(c, acc, wacc))) return rc;
   }
-  if (c->cfg.healpix_out && (rc = enq_recon_set(c, false))) return rc;
-  if (c->ngp) HC(hipStreamWaitEvent(c->stB, c->ev_join, 0));
   ev_end(c, ST_RECON, c->stB);
   /* the segment's buffer set is free for the segment after next */
   HC(hipEventRecord(c->ev_recon[c->cur], c->stB));
@@ -1368,10 +1413,16 @@ int enq_recon(Ctx* c) {
 int enq_step(Ctx* c) {
   int rc;
   if (!c->sky_sched) {
-    for (int s = 0; s < c->segs; ++s)
-      if ((rc = enq_gen(c, c->seg_t0[s], c->seg_tlen[s])) || (rc = enq_viss(c, false)) || (rc = enq_conj(c)) ||
-          (rc = enq_recon(c)))
-        return rc;
+    for (int s = 0; s < c->segs; ++s) {
+      if ((rc = enq_gen(c, c->seg_t0[s], c->seg_tlen[s]))) return rc;
+      /* the groups' keys and order need the rows only: beside the Viss */
+      HC(hipEventRecord(c->ev_gen, c->st));
+      HC(hipStreamWaitEvent(c->stB, c->ev_gen, 0));
+      ev_begin(c, ST_GROUP, c->stB);
+      if ((rc = enq_group_keys(c))) return rc;
+      ev_end(c, ST_GROUP, c->stB);
+      if ((rc = enq_viss(c, false, true)) || (c->batch && (rc = enq_conj(c))) || (rc = enq_recon(c, true))) return rc;
+    }
     return VW_OK;
   }
   const int64_t day_rows = (int64_t)c->T * c->P;
@@ -1392,16 +1443,9 @@ int enq_step(Ctx* c) {
     for (const int32_t sk : u.skies) {
       if ((rc = enq_group_data(c, c->d_vday + sk * day_rows + (int64_t)u.t0 * c->P))) return rc;
       ev_begin(c, ST_RECON, c->stB);
-      if (c->ngp) {
-        HC(hipEventRecord(c->ev_fork, c->stB));
-        HC(hipStreamWaitEvent(c->st2, c->ev_fork, 0));
-        if ((rc = enq_recon_set_one(c, true, c->d_Gacc + sk * c->ngp, c->d_GWsky + sk * c->ngp))) return rc;
-        HC(hipEventRecord(c->ev_join, c->st2));
-      }
-      if (c->cfg.healpix_out &&
-          (rc = enq_recon_set_one(c, false, c->d_Cacc + sk * c->npix, c->d_Wsky + sk * c->npix)))
-        return rc;
-      if (c->ngp) HC(hipStreamWaitEvent(c->stB, c->ev_join, 0));
+      double* const acc[2] = {c->d_Cacc + sk * c->npix, c->ngp ? c->d_Gacc + sk * c->ngp : nullptr};
+      uint32_t* const wacc[2] = {c->d_Wsky + sk * c->npix, c->ngp ? c->d_GWsky + sk * c->ngp : nullptr};
+      if ((rc = enq_recon_one(c, acc, wacc))) return rc;
       ev_end(c, ST_RECON, c->stB);
     }
     /* this buffer set is free once the segment's last recon is done */
@@ -1511,6 +1555,7 @@ VW_API void vw_destroy(void* p) {
   if (c->ev_fork) (void)hipEventDestroy(c->ev_fork);
   if (c->ev_join) (void)hipEventDestroy(c->ev_join);
   if (c->ev_conj) (void)hipEventDestroy(c->ev_conj);
+  if (c->ev_gen) (void)hipEventDestroy(c->ev_gen);
   for (int b = 0; b < 2; ++b)
     if (c->ev_recon[b]) (void)hipEventDestroy(c->ev_recon[b]);
   if (c->st2 && c->st2 != c->st) (void)hipStreamDestroy(c->st2);
@@ -1672,35 +1717,6 @@ VW_API int vw_run_all(void* p) {
   return sync(c);
 }
 
-namespace {
-/* accumulators and the running key total cleared by kernels (no memset nodes) */
-int enq_reset_fill(Ctx* c) {
-  const int64_t nC = 2 * c->npix * c->nsky; /* doubles as 32-bit words */
-  k_fill0<<<blocks_for(nC), 256, 0, c->st>>>((uint32_t*)c->d_Cacc, nC);
-  KC();
-  k_fill0<<<blocks_for(c->npix), 256, 0, c->st>>>(c->d_Wacc, c->npix);
-  KC();
-  if (c->ngp) {
-    const int64_t nG = 2 * c->ngp * c->nsky;
-    k_fill0<<<blocks_for(nG), 256, 0, c->st>>>((uint32_t*)c->d_Gacc, nG);
-    KC();
-    k_fill0<<<blocks_for(c->ngp), 256, 0, c->st>>>(c->d_GWacc, c->ngp);
-    KC();
-  }
-  k_fill0<<<1, 256, 0, c->st>>>((uint32_t*)c->d_info, (int64_t)(sizeof(DevInfo) / 4));
-  KC();
-  if (c->sky_sched) {
-    k_fill0<<<blocks_for(c->npix * c->nsky), 256, 0, c->st>>>(c->d_Wsky, c->npix * c->nsky);
-    KC();
-    if (c->ngp) {
-      k_fill0<<<blocks_for(c->ngp * c->nsky), 256, 0, c->st>>>(c->d_GWsky, c->ngp * c->nsky);
-      KC();
-    }
-  }
-  return VW_OK;
-}
-}  // namespace
-
 /* One batched step from a graph: clear the accumulators, then every segment of
  * the schedule (as vw_reset_accumulators + vw_run_all).  The graph is captured
  * on the first call and replayed afterwards; a change of launch targets or of
@@ -1745,31 +1761,20 @@ VW_API int vw_finalize(void* p, double* C, uint32_t* W, double* img, uint32_t* W
   if (int rj = join_recon(c)) return rj;
   ev_begin(c, ST_FIN);
   /* normalise on the device; copy out only what was asked for */
-  if (c->cfg.healpix_out) {
-    k_normalize<<<blocks_for(c->npix), 256, 0, c->st>>>(c->d_Cacc, c->d_Wacc, c->npix, c->cfg.blockage, c->d_info,
-                                                        nullptr, c->d_out, c->d_wout);
-    KC();
-    if (c->batch) {
-      k_normalize_b<<<blocks_for(c->npix * c->nsky), 256, 0, c->st>>>(
-          c->d_Cacc, c->sky_sched ? c->d_Wsky : c->d_Wacc, c->npix, c->nsky, c->cfg.blockage, c->d_info, nullptr,
-          c->npix, c->d_out, c->sky_sched ? c->npix : 0);
-      KC();
-    }
-  }
-  if (c->ngp) {
-    int64_t NN = (int64_t)c->cfg.img_n * c->cfg.img_n;
-    HC(hipMemsetAsync(c->d_iout, 0, sizeof(double) * NN * c->nsky, c->st));
-    HC(hipMemsetAsync(c->d_iwout, 0, sizeof(uint32_t) * NN, c->st));
-    k_normalize<<<blocks_for(c->ngp), 256, 0, c->st>>>(c->d_Gacc, c->d_GWacc, c->ngp, c->cfg.blockage, c->d_info,
-                                                       c->d_gidx, c->d_iout, c->d_iwout);
-    KC();
-    if (c->batch) {
-      k_normalize_b<<<blocks_for(c->ngp * c->nsky), 256, 0, c->st>>>(
-          c->d_Gacc, c->sky_sched ? c->d_GWsky : c->d_GWacc, c->ngp, c->nsky, c->cfg.blockage, c->d_info, c->d_gidx,
-          NN, c->d_iout, c->sky_sched ? c->ngp : 0);
-      KC();
-    }
-  }
+  const int64_t NN = (int64_t)c->cfg.img_n * c->cfg.img_n;
+  FinalArgs f{};
+  f.nsky = c->nsky;
+  f.blockage = c->cfg.blockage;
+  f.info = c->d_info;
+  if (c->cfg.healpix_out)
+    f.s[0] = FinalSet{c->d_Cacc, c->sky_sched ? c->d_Wsky : c->d_Wacc, nullptr, c->npix, c->npix,
+                      c->sky_sched ? c->npix : 0, c->d_out, c->sky_sched ? nullptr : c->d_wout};
+  if (c->ngp)
+    f.s[1] = FinalSet{c->d_Gacc, c->sky_sched ? c->d_GWsky : c->d_GWacc, c->d_ginv, c->ngp, NN,
+                      c->sky_sched ? c->ngp : 0, c->d_iout, c->sky_sched ? c->d_iwout_sky : c->d_iwout};
+  const unsigned nfb = blocks_for(f.s[0].nout * c->nsky) + blocks_for(f.s[1].nout * c->nsky);
+  if (nfb) k_finalize<<<nfb, 256, 0, c->st>>>(f);
+  KC();
   ev_end(c, ST_FIN);
   if (C) {
     if (c->cfg.healpix_out)
@@ -1784,18 +1789,10 @@ VW_API int vw_finalize(void* p, double* C, uint32_t* W, double* img, uint32_t* W
     else std::memset(W, 0, sizeof(uint32_t) * c->npix * nw);
   }
   if (c->ngp) {
-    int64_t NN = (int64_t)c->cfg.img_n * c->cfg.img_n;
     if (img) HC(hipMemcpyAsync(img, c->d_iout, sizeof(double) * NN * c->nsky, hipMemcpyDeviceToHost, c->st));
-    if (Wimg && c->sky_sched) {
-      k_fill0<<<blocks_for(NN * c->nsky), 256, 0, c->st>>>(c->d_iwout_sky, NN * c->nsky);
-      KC();
-      k_scatter_w<<<blocks_for(c->ngp * c->nsky), 256, 0, c->st>>>(c->d_GWsky, c->ngp, c->nsky, c->d_gidx, NN,
-                                                                    c->d_iwout_sky);
-      KC();
-      HC(hipMemcpyAsync(Wimg, c->d_iwout_sky, sizeof(uint32_t) * NN * c->nsky, hipMemcpyDeviceToHost, c->st));
-    } else if (Wimg) {
-      HC(hipMemcpyAsync(Wimg, c->d_iwout, sizeof(uint32_t) * NN, hipMemcpyDeviceToHost, c->st));
-    }
+    if (Wimg)
+      HC(hipMemcpyAsync(Wimg, c->sky_sched ? c->d_iwout_sky : c->d_iwout, sizeof(uint32_t) * NN * nw,
+                        hipMemcpyDeviceToHost, c->st));
   }
   return sync(c);
 }
@@ -1804,17 +1801,7 @@ VW_API int vw_reset_accumulators(void* p) {
   Ctx* c = as_ctx(p);
   if (!c) return VW_ERR_ARG;
   if (int rj = join_recon(c)) return rj;
-  HC(hipMemsetAsync(c->d_Cacc, 0, sizeof(double) * c->npix * c->nsky, c->st));
-  HC(hipMemsetAsync(c->d_Wacc, 0, sizeof(uint32_t) * c->npix, c->st));
-  if (c->ngp) {
-    HC(hipMemsetAsync(c->d_Gacc, 0, sizeof(double) * c->ngp * c->nsky, c->st));
-    HC(hipMemsetAsync(c->d_GWacc, 0, sizeof(uint32_t) * c->ngp, c->st));
-  }
-  HC(hipMemsetAsync(c->d_info, 0, sizeof(DevInfo), c->st));
-  if (c->sky_sched) {
-    HC(hipMemsetAsync(c->d_Wsky, 0, sizeof(uint32_t) * c->npix * c->nsky, c->st));
-    if (c->ngp) HC(hipMemsetAsync(c->d_GWsky, 0, sizeof(uint32_t) * c->ngp * c->nsky, c->st));
-  }
+  if (int rf = enq_reset_fill(c)) return rf;
   return sync(c);
 }
 

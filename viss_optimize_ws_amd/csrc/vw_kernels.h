@@ -192,39 +192,54 @@ __global__ void k_day_positions(DayArgs a, double* __restrict__ pos) {
   pos[2 * TA + k] = z;
 }
 
-/* per (epoch, antenna) frame: px,py,pz,invn,ux,uy,uz,cosphi */
-__global__ void k_seg_ant(const double* __restrict__ pos, int T, int A, int t0, int tlen, double occ_r,
-                          double cosphi_glob, double* __restrict__ ant8) {
-  int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (k >= (int64_t)tlen * A) return;
-  int64_t TA = (int64_t)T * A;
-  int64_t src = (int64_t)t0 * A + k;
-  double px = pos[src], py = pos[TA + src], pz = pos[2 * TA + src];
-  double in, ux, uy, uz, cp;
-  vw_antenna_frame(px, py, pz, occ_r, cosphi_glob, &in, &ux, &uy, &uz, &cp);
-  double* q = ant8 + k * 8;
-  q[0] = px; q[1] = py; q[2] = pz; q[3] = in;
-  q[4] = ux; q[5] = uy; q[6] = uz; q[7] = cp;
-}
-
-__global__ void k_seg_rows(const double* __restrict__ pos, int T, int A, int P, int t0, int64_t nh,
-                           const int32_t* __restrict__ pa, const int32_t* __restrict__ pb, double lambda,
-                           RowRec* __restrict__ rows, double4* __restrict__ rowt) {
-  int64_t h = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (h >= nh) return;
-  int64_t TA = (int64_t)T * A;
-  int64_t g = h / P;
-  int j = (int)(h - g * P);
-  int64_t ka = (t0 + g) * A + pa[j], kb = (t0 + g) * A + pb[j];
-  RowRec r;
-  r.u = vw_uvw_comp(pos[ka], pos[kb], lambda);
-  r.v = vw_uvw_comp(pos[TA + ka], pos[TA + kb], lambda);
-  r.w = vw_uvw_comp(pos[2 * TA + ka], pos[2 * TA + kb], lambda);
-  r.ia = (int32_t)(g * A + pa[j]);
-  r.ib = (int32_t)(g * A + pb[j]);
-  rows[h] = r;
-  /* the plain Viss phase in 1/1024 turns (exact power-of-two scaling) */
-  rowt[h] = make_double4(r.u * VW_TAB_SCALE, r.v * VW_TAB_SCALE, r.w * VW_TAB_SCALE, 0.0);
+/* A segment's geometry in one launch: per (epoch, antenna) the frame px, py, pz,
+ * invn, ux, uy, uz, cosphi and, for the antenna-factorized Viss (aph not null),
+ * the phase coefficients (x - x_0) * 1e3 / lambda with x_0 the epoch's antenna 0
+ * and (aphl, may be null) the part that the roundings of the difference, the
+ * product and the quotient left out; per (epoch, pair) the half row. */
+__global__ void k_seg_gen(const double* __restrict__ pos, int T, int A, int P, int t0, int tlen, double occ_r,
+                          double cosphi_glob, const int32_t* __restrict__ pa, const int32_t* __restrict__ pb,
+                          double lambda, double* __restrict__ ant8, double4* __restrict__ aph,
+                          double4* __restrict__ aphl, RowRec* __restrict__ rows, double4* __restrict__ rowt) {
+  const int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  const int64_t TA = (int64_t)T * A;
+  if (k < (int64_t)tlen * A) {
+    const int64_t src = (int64_t)t0 * A + k;
+    const double x[3] = {pos[src], pos[TA + src], pos[2 * TA + src]};
+    double in, ux, uy, uz, cp;
+    vw_antenna_frame(x[0], x[1], x[2], occ_r, cosphi_glob, &in, &ux, &uy, &uz, &cp);
+    double* q = ant8 + k * 8;
+    q[0] = x[0]; q[1] = x[1]; q[2] = x[2]; q[3] = in;
+    q[4] = ux; q[5] = uy; q[6] = uz; q[7] = cp;
+    if (aph) {
+      const int64_t ref = (t0 + k / A) * A;
+      double r[3], l[3];
+#pragma unroll
+      for (int c = 0; c < 3; ++c) {
+        const double xr = pos[c * TA + ref];
+        const double d = x[c] - xr, bb = d - x[c], de = (x[c] - (d - bb)) - (xr + bb); /* d + de = x - xr */
+        const double p = d * 1e3, pe = fma(d, 1e3, -p) + de * 1e3;
+        r[c] = p / lambda;
+        l[c] = (fma(-r[c], lambda, p) + pe) / lambda;
+      }
+      aph[k] = make_double4(r[0], r[1], r[2], 0.0);
+      if (aphl) aphl[k] = make_double4(l[0], l[1], l[2], 0.0);
+    }
+  }
+  if (k < (int64_t)tlen * P) {
+    const int64_t g = k / P;
+    const int j = (int)(k - g * P);
+    const int64_t ka = (t0 + g) * A + pa[j], kb = (t0 + g) * A + pb[j];
+    RowRec r;
+    r.u = vw_uvw_comp(pos[ka], pos[kb], lambda);
+    r.v = vw_uvw_comp(pos[TA + ka], pos[TA + kb], lambda);
+    r.w = vw_uvw_comp(pos[2 * TA + ka], pos[2 * TA + kb], lambda);
+    r.ia = (int32_t)(g * A + pa[j]);
+    r.ib = (int32_t)(g * A + pb[j]);
+    rows[k] = r;
+    /* the plain Viss phase in 1/1024 turns (exact power-of-two scaling) */
+    rowt[k] = make_double4(r.u * VW_TAB_SCALE, r.v * VW_TAB_SCALE, r.w * VW_TAB_SCALE, 0.0);
+  }
 }
 
 /* reference full-row layout (orbit_online.cuh:186-231) into 9 SoA arrays */
@@ -856,11 +871,24 @@ __global__ void k_viss_adj_fold(const double* __restrict__ part, int64_t nchunk,
   g[p0 + i] = area * s;
 }
 
+/* a raw half sum, phase-corrected (vh not null: whole steps, where the
+ * correction is no stage of its own) */
+__device__ __forceinline__ void vw_store_half(double2* __restrict__ vraw, double2* __restrict__ vh,
+                                              const RowRec* __restrict__ rows, int64_t h, double re, double im) {
+  vraw[h] = make_double2(re, im);
+  if (vh) {
+    double cr, ci;
+    vw_phase_correct(re, im, rows[h].w, &cr, &ci);
+    vh[h] = make_double2(cr, ci);
+  }
+}
+
 /* partials -> raw half sums, chunks folded in ascending order; passes after
  * the first add to the running sums */
 __global__ void k_viss_reduce(const double2* __restrict__ part, int64_t nchunk, int64_t nh, int64_t nh_pad,
                               int accumulate, double2* __restrict__ vraw, const int64_t* __restrict__ cpart,
-                              int64_t* __restrict__ counts) {
+                              int64_t* __restrict__ counts, const RowRec* __restrict__ rows,
+                              double2* __restrict__ vh) {
   int64_t h = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (h >= nh) return;
   double re = 0.0, im = 0.0;
@@ -893,7 +921,7 @@ __global__ void k_viss_reduce(const double2* __restrict__ part, int64_t nchunk, 
     im = o.y + im;
     if (counts) c += counts[h];
   }
-  vraw[h] = make_double2(re, im);
+  vw_store_half(vraw, vh, rows, h, re, im);
   if (counts) counts[h] = c;
 }
 
@@ -1241,7 +1269,7 @@ __global__ __launch_bounds__(256) void k_vissf_fold(const double* __restrict__ p
  * passes after the first add to the running sums */
 __global__ void k_vissf_rows(const double* __restrict__ esum, int64_t nh, int P, int G,
                              const int32_t* __restrict__ pa, const int32_t* __restrict__ pb, int accumulate,
-                             double2* __restrict__ vraw) {
+                             double2* __restrict__ vraw, const RowRec* __restrict__ rows, double2* __restrict__ vh) {
   int64_t h = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (h >= nh) return;
   const int64_t g = h / P;
@@ -1259,31 +1287,7 @@ __global__ void k_vissf_rows(const double* __restrict__ esum, int64_t nh, int P,
     re = o.x + re;
     im = o.y + im;
   }
-  vraw[h] = make_double2(re, im);
-}
-
-/* per-frame phase coefficients of the factorized form: (x - x_0) * 1e3 /
- * lambda with x_0 the epoch's antenna 0, and (aphl, may be null) the part
- * that the roundings of the difference, the product and the quotient left out */
-__global__ void k_ant_phase(const double* __restrict__ pos, int T, int A, int t0, int tlen, double lambda,
-                            double4* __restrict__ aph, double4* __restrict__ aphl) {
-  int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (k >= (int64_t)tlen * A) return;
-  const int64_t TA = (int64_t)T * A;
-  const int64_t g = k / A;
-  const int64_t src = (int64_t)t0 * A + k, ref = (t0 + g) * A;
-  double r[3], q[3];
-#pragma unroll
-  for (int c = 0; c < 3; ++c) {
-    const double xa = pos[c * TA + src], xr = pos[c * TA + ref];
-    const double d = xa - xr, bb = d - xa, de = (xa - (d - bb)) - (xr + bb); /* d + de = xa - xr */
-    const double p = d * 1e3, pe = fma(d, 1e3, -p) + de * 1e3;
-    const double h = p / lambda;
-    r[c] = h;
-    q[c] = (fma(-h, lambda, p) + pe) / lambda;
-  }
-  aph[k] = make_double4(r[0], r[1], r[2], 0.0);
-  if (aphl) aphl[k] = make_double4(q[0], q[1], q[2], 0.0);
+  vw_store_half(vraw, vh, rows, h, re, im);
 }
 
 /* phase correction + conjugate completion (common.hpp:255-277) */
@@ -1678,6 +1682,30 @@ __global__ __launch_bounds__(256) void k_group_cls_tile(const double* __restrict
   }
 }
 
+/* The output sets of one recon launch (HEALPix map, lm image, one tile pass of
+ * each): each kernel of the recon stage takes both, the blocks of the second
+ * after those of the first. */
+struct ReconSet {
+  const double *l, *m, *n;
+  const double* cone; /* [5][ntile] */
+  int64_t ntile;      /* tiles of the whole set                                  */
+  int64_t tile0, nt;  /* tiles of this pass                                      */
+  int64_t pt0, npts;  /* its points [pt0, pt0 + npts), pt0 = tile0 * TP          */
+  uint32_t* cls;      /* [nt][nq_pad / 16] mask words of 16 groups (representative
+                       * kinds), [nt][nh_pad] row class bytes (generic kind)     */
+  const uint8_t* bits; /* [nt][nfr_pad] cone bits (long frame rows)               */
+  int64_t nchunk;     /* group ranges per point block                            */
+  int64_t pwaves;     /* point blocks (waves) per group range                    */
+  int64_t nblk;       /* workgroups of the recon kernel                          */
+  double* part;       /* [nchunk][npts]                                          */
+  uint32_t* wpart;    /* [nchunk][npts]                                          */
+  double* acc;        /* accumulators of the whole set                           */
+  uint32_t* wacc;
+};
+struct ReconSets {
+  ReconSet s[2]; /* a set without tiles or blocks is absent */
+};
+
 /* The one-sky recon's form of the same classes: per (tile, 16 groups) one
  * word, bit j = group j is visible from the whole tile, bit 16 + j = partly;
  * groups below first_nz (the key-0 group) and past nuniq have neither bit, so
@@ -1688,23 +1716,23 @@ __global__ __launch_bounds__(256) void k_group_cls_tile(const double* __restrict
  * before the gathers), and writes the masks of ballots.  Words of entries
  * below nuniq rounded up to 64 are written: the recon reads no others. */
 template <bool TILE>
-__global__ __launch_bounds__(256) void k_group_mask(const double* __restrict__ cone, int64_t ntile, int64_t tile0,
-                                                    const double* __restrict__ ant8, int64_t nfr,
-                                                    const uint8_t* __restrict__ bits, int64_t nfr_pad,
-                                                    const int32_t* __restrict__ ia, const int32_t* __restrict__ ib,
-                                                    const DevInfo* __restrict__ info, int64_t nq_pad,
-                                                    uint32_t* __restrict__ gmask) {
+__global__ __launch_bounds__(256) void k_group_mask(ReconSets sets, const double* __restrict__ ant8, int64_t nfr,
+                                                    int64_t nfr_pad, const int32_t* __restrict__ ia,
+                                                    const int32_t* __restrict__ ib, const DevInfo* __restrict__ info,
+                                                    int64_t nq_pad) {
   extern __shared__ uint4 sbits[];
-  const int64_t tr = blockIdx.x;
+  const int si = (int)blockIdx.x >= (int)sets.s[0].nt;
+  const ReconSet& S = sets.s[si];
+  const int64_t tr = blockIdx.x - (si ? sets.s[0].nt : 0);
   const int nu = vw_rfl((int)info->nuniq), q0 = vw_rfl((int)info->first_nz);
   const int qend = (nu + 63) / 64 * 64; /* <= nq_pad, a multiple of 64 */
-  const uint8_t* b = TILE ? (const uint8_t*)sbits : bits + tr * nfr_pad;
+  const uint8_t* b = TILE ? (const uint8_t*)sbits : S.bits + tr * nfr_pad;
   if (TILE) {
-    vw_tile_bits_lds((uint8_t*)sbits, cone, ntile, tile0 + tr, ant8, nfr);
+    vw_tile_bits_lds((uint8_t*)sbits, S.cone, S.ntile, S.tile0 + tr, ant8, nfr);
     __syncthreads();
   }
   const int wave = vw_rfl((int)(threadIdx.x >> 6)), lane = threadIdx.x & 63;
-  uint32_t* out = gmask + tr * (nq_pad >> 4);
+  uint32_t* out = S.cls + tr * (nq_pad >> 4);
   for (int j0 = 256 * wave; j0 < qend; j0 += 1024) {
     int av[4], bv[4];
 #pragma unroll
@@ -1732,12 +1760,8 @@ __global__ __launch_bounds__(256) void k_group_mask(const double* __restrict__ c
 /* ------------------------------------------------------------------ */
 struct ReconArgs {
   const double2* tab;  /* the sine table (plain), built once per context */
-  const double *l, *m, *n;
-  int64_t pt0, npts, TP; /* points [pt0, pt0 + npts) of this pass, pt0 = tile0 * TP */
-  const uint32_t* gmask; /* [ntile_out][nq_pad / 16] mask words of 16 groups (representative kinds) */
-  int64_t nq_pad;
-  const uint32_t* rcls; /* [ntile_out][nh_pad]: per half row (generic kind)     */
-  int64_t nh_pad;
+  ReconSets sets;
+  int64_t TP, nq_pad, nh_pad;
   GroupSoA g;
   const int32_t* goff;
   const int32_t* idx_sorted;
@@ -1746,11 +1770,6 @@ struct ReconArgs {
   const double* ant8;
   const DevInfo* info;
   int P, full, occ_mode;
-  int64_t nchunk;     /* group ranges per point block                     */
-  int64_t pwaves;     /* point blocks (waves) per group range             */
-  int64_t pstride;    /* partial row stride                               */
-  double* part;       /* [nchunk][pstride]                                */
-  uint32_t* wpart;    /* [nchunk][pstride]                                */
 };
 
 #define VW_KIND_REP 0
@@ -1925,10 +1944,13 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(
     __syncthreads();
   }
   const int lane = threadIdx.x & 63;
-  const int64_t wid = (int64_t)blockIdx.x * 4 + vw_rfl((int)(threadIdx.x >> 6));
-  const int64_t chunk = wid / a.pwaves;
-  const int64_t pw = wid - chunk * a.pwaves;
-  if (chunk >= a.nchunk) return;
+  const int si = (int)blockIdx.x >= (int)a.sets.s[0].nblk;
+  const ReconSet& S = a.sets.s[si];
+  const int64_t wid =
+      (int64_t)(blockIdx.x - (si ? (uint32_t)a.sets.s[0].nblk : 0u)) * 4 + vw_rfl((int)(threadIdx.x >> 6));
+  const int64_t chunk = wid / S.pwaves;
+  const int64_t pw = wid - chunk * S.pwaves;
+  if (chunk >= S.nchunk) return;
   const int64_t pbase = pw * 64 * PPL; /* pass-relative */
   const int64_t tile = pbase / a.TP;   /* pass-relative tile (class tables are per pass) */
   const vw_segparams sp = a.info->sp;
@@ -1938,7 +1960,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(
   const bool polar = vw_rfl(a.info->polar) != 0;
   /* group range of this chunk, aligned to 16 groups */
   const int64_t base = q0 & ~(int64_t)15;
-  const int64_t span = ((nu - base) + a.nchunk - 1) / a.nchunk;
+  const int64_t span = ((nu - base) + S.nchunk - 1) / S.nchunk;
   const int64_t spanA = (span + 15) & ~(int64_t)15;
   const int64_t qa_ = vw_rfl((int)(base + chunk * spanA));
   const int64_t qb_ = vw_rfl((int)(qa_ + spanA < nu ? qa_ + spanA : nu));
@@ -1949,11 +1971,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(
 #pragma unroll
   for (int k = 0; k < PPL; ++k) {
     int64_t p = pbase + lane + 64 * k;
-    ok[k] = p < a.npts;
-    int64_t pp = a.pt0 + (ok[k] ? p : 0);
-    pl[k] = a.l[pp];
-    pm[k] = a.m[pp];
-    pn[k] = a.n[pp];
+    ok[k] = p < S.npts;
+    int64_t pp = S.pt0 + (ok[k] ? p : 0);
+    pl[k] = S.l[pp];
+    pm[k] = S.m[pp];
+    pn[k] = S.n[pp];
     lp[k] = fma(sp.fa, pn[k], pl[k]);
     mp[k] = fma(sp.fb, pn[k], pm[k]);
     fl[k] = (float)pl[k];
@@ -1982,7 +2004,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(
      * 64, so every block lies inside the records and the masks. */
     double* ring = gring[vw_rfl((int)(threadIdx.x >> 6))];
     const double* recd = (const double*)a.g.rec;
-    const uint32_t* mrow = VW_KIND_IS_REP(KIND) ? a.gmask + tile * (a.nq_pad >> 4) : nullptr;
+    const uint32_t* mrow = VW_KIND_IS_REP(KIND) ? S.cls + tile * (a.nq_pad >> 4) : nullptr;
     double stage = (qa_ < qb_) ? recd[qa_ * 4 + lane] : 0.0;
     uint32_t nmw = 0;
     if (VW_KIND_IS_REP(KIND) && qa_ < qb_) nmw = (uint32_t)vw_rfl((int)mrow[qa_ >> 4]);
@@ -2038,8 +2060,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(
             for (int k = 0; k < PPL; ++k) {
               int ln = lane; /* opaque: the addresses are formed here, not kept in registers across the loop */
               __asm__ volatile("" : "+v"(ln));
-              const int64_t pp = a.pt0 + (ok[k] ? pbase + ln + 64 * k : 0);
-              use[k] = vw_vis2<true>(ok[k], a.l[pp], a.m[pp], a.n[pp], d[0], d[1], d[2], d[3], d[4], d[5], d[6], d[7],
+              const int64_t pp = S.pt0 + (ok[k] ? pbase + ln + 64 * k : 0);
+              use[k] = vw_vis2<true>(ok[k], S.l[pp], S.m[pp], S.n[pp], d[0], d[1], d[2], d[3], d[4], d[5], d[6], d[7],
                                      d[8], d[9]);
             }
           }
@@ -2070,7 +2092,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(
         const int32_t pos = (np < 0) ? kk : posv[kk];
         bool ng;
         const int64_t h = vw_row_half(a.idx_sorted[pos], a.P, a.full != 0, &ng);
-        const int cls = vw_cls_lookup(a.rcls, tile, a.nh_pad, h);
+        const int cls = vw_cls_lookup(S.cls, tile, a.nh_pad, h);
         if (cls == VW_CLS_HIDDEN) continue;
         bool mv[PPL];
         if (cls == VW_CLS_VISIBLE) {
@@ -2109,18 +2131,22 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(
   for (int k = 0; k < PPL; ++k) {
     if (!ok[k]) continue;
     const int64_t p = pbase + lane + 64 * k;
-    a.part[chunk * a.pstride + p] = acc.value(k);
-    a.wpart[chunk * a.pstride + p] = wu + wl[k];
+    S.part[chunk * S.npts + p] = acc.value(k);
+    S.wpart[chunk * S.npts + p] = wu + wl[k];
   }
 }
 
 /* fold group-range partials in order into the accumulators (add_inplace) for
- * points [pt0, pt0 + npts) */
-__global__ void k_recon_reduce(const double* __restrict__ part, const uint32_t* __restrict__ wpart, int64_t nchunk,
-                               int64_t pstride, int64_t pt0, int64_t npts, int weights, double* __restrict__ acc,
-                               uint32_t* __restrict__ wacc) {
-  int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (p >= npts) return;
+ * the points of a pass, both output sets */
+__global__ void k_recon_reduce(ReconSets sets, int weights) {
+  const int64_t nb0 = (sets.s[0].npts + blockDim.x - 1) / blockDim.x;
+  const int si = (int64_t)blockIdx.x >= nb0;
+  const ReconSet& S = sets.s[si];
+  const int64_t p = ((int64_t)blockIdx.x - (si ? nb0 : 0)) * blockDim.x + threadIdx.x;
+  if (p >= S.npts) return;
+  const double* __restrict__ part = S.part;
+  const uint32_t* __restrict__ wpart = S.wpart;
+  const int64_t nchunk = S.nchunk, pstride = S.npts;
   double s = part[p];
   uint32_t w = wpart[p];
   /* VW_FOLD_BATCH chunks' loads in flight at a time; the sum keeps chunk order */
@@ -2143,26 +2169,73 @@ __global__ void k_recon_reduce(const double* __restrict__ part, const uint32_t* 
     s = s + part[k * pstride + p];
     w += wpart[k * pstride + p];
   }
-  acc[pt0 + p] = acc[pt0 + p] + s;
-  if (weights) wacc[pt0 + p] += w;
+  S.acc[S.pt0 + p] = S.acc[S.pt0 + p] + s;
+  if (weights) S.wacc[S.pt0 + p] += w;
 }
 
-/* final maps: C = acc / W (blockage 1) or acc * (1/W_total) (blockage 0) */
-__global__ void k_normalize(const double* __restrict__ acc, const uint32_t* __restrict__ w, int64_t n, int blockage,
-                            const DevInfo* __restrict__ info, const int64_t* __restrict__ scatter,
-                            double* __restrict__ out, uint32_t* __restrict__ wout) {
-  int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (k >= n) return;
-  double v;
-  if (blockage) v = w[k] > 0 ? acc[k] / (double)w[k] : 0.0;
-  else {
-    int64_t wt = info->wtotal;
-    double inv = wt > 0 ? 1.0 / (double)wt : 0.0;
-    v = acc[k] * inv;
+/* Final maps of every sky of both output sets: C = acc / W (blockage 1) or
+ * acc * (1/W_total) (blockage 0), one thread per output value; inv (lm image)
+ * gives an output pixel's point, -1 outside the unit disk, which gets zeros.
+ * Weight maps: one for all skies (wstride 0, written with sky 0) or one a sky. */
+struct FinalSet {
+  const double* acc;      /* [nsky][nin]               */
+  const uint32_t* w;      /* [nin] or [nsky][nin]      */
+  const int32_t* inv;     /* [nout] or null            */
+  int64_t nin, nout;
+  int64_t wstride;        /* 0 or nin                  */
+  double* out;            /* [nsky][nout]              */
+  uint32_t* wout;         /* [nout] or [nsky][nout]; null: not wanted */
+};
+struct FinalArgs {
+  FinalSet s[2]; /* nout 0: absent */
+  int64_t nsky;
+  int blockage;
+  const DevInfo* info;
+};
+__global__ __launch_bounds__(256) void k_finalize(FinalArgs a) {
+  const int64_t nb0 = (a.nsky * a.s[0].nout + 255) / 256;
+  const int si = (int64_t)blockIdx.x >= nb0;
+  const FinalSet& S = a.s[si];
+  const int64_t k = ((int64_t)blockIdx.x - (si ? nb0 : 0)) * 256 + threadIdx.x;
+  if (k >= a.nsky * S.nout) return;
+  const int64_t sk = k / S.nout, o = k - sk * S.nout;
+  const int64_t i = S.inv ? S.inv[o] : o;
+  double v = 0.0;
+  uint32_t wi = 0;
+  if (i >= 0) {
+    wi = S.w[sk * S.wstride + i];
+    const double x = S.acc[sk * S.nin + i];
+    if (a.blockage) v = wi > 0 ? x / (double)wi : 0.0;
+    else {
+      const int64_t wt = a.info->wtotal;
+      const double r = wt > 0 ? 1.0 / (double)wt : 0.0;
+      v = x * r;
+    }
   }
-  int64_t dst = scatter ? scatter[k] : k;
-  out[dst] = v;
-  wout[dst] = w[k];
+  S.out[k] = v;
+  if (S.wout && (S.wstride || sk == 0)) S.wout[k] = wi;
+}
+
+/* point index of each image pixel (inv filled with -1 before) */
+__global__ void k_grid_inv(int64_t npts, const int64_t* __restrict__ gidx, int32_t* __restrict__ inv) {
+  const int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (k < npts) inv[gidx[k]] = (int32_t)k;
+}
+
+/* zeroes up to eight arrays of 32-bit words in one launch (kernels, not memset
+ * nodes: a captured step holds it).  Arrays start 16-byte aligned. */
+struct ClearArgs {
+  uint32_t* p[8];
+  int64_t n[8];
+  int cnt;
+};
+__global__ __launch_bounds__(256) void k_clear(ClearArgs a) {
+  const int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x, nt = (int64_t)gridDim.x * 256;
+  for (int j = 0; j < a.cnt; ++j) {
+    const int64_t n4 = a.n[j] / 4;
+    for (int64_t i = t; i < n4; i += nt) ((uint4*)a.p[j])[i] = make_uint4(0, 0, 0, 0);
+    if (t < a.n[j] - 4 * n4) a.p[j][4 * n4 + t] = 0;
+  }
 }
 
 #endif
