@@ -139,7 +139,9 @@ typedef struct {
   double *xb, *yb, *zb; /* xyzb */
 } vw_geom_host;
 
-/* Device time of the last completed stage calls (HIP events, ms). */
+/* Device time of the last completed stage calls (ms): time stamps of the stages'
+ * kernels, HIP events in batched contexts.  vw_run_all of one sky has no
+ * separate conjugate fill (conj_ms 0: part of viss_ms). */
 typedef struct {
   double gen_ms, viss_ms, conj_ms, group_ms, recon_ms, finalize_ms;
   double viss_kernel_ms;  /* the Viss summation kernel alone (sum)     */

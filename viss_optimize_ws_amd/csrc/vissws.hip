@@ -173,6 +173,16 @@ struct Ctx {
   /* timing */
   std::vector<EvPair> ev[ST_N];
   size_t ev_used[ST_N] = {};
+  /* device time stamps of the one-sky stages: host memory that the kernels
+   * write, in blocks of VW_TS_BLOCK words, reused after each synchronise */
+  std::vector<uint64_t*> ts_blk;
+  size_t ts_used = 0;
+  struct Bracket {
+    Stage s;
+    const uint64_t *from, *to;
+  };
+  std::vector<Bracket> brackets;
+  double ts_ms = 0.0; /* milliseconds a count */
   vw_timings tim{};
 
   int fail(int code, const std::string& m) {
@@ -202,7 +212,32 @@ int round_away_f(float x) { return (x >= 0.0f) ? (int)floorf(x + 0.5f) : (int)ce
 
 inline unsigned blocks_for(int64_t n, int bs = 256) { return (unsigned)((n + bs - 1) / bs); }
 
-/* event bracket for one stage launch group */
+/* the two time-stamp words of one launch (vw_ts_begin, vw_ts_end); null when
+ * nothing is to be timed (a captured graph) or no host memory is left */
+#define VW_TS_BLOCK 4096
+uint64_t* new_ts(Ctx* c) {
+  if (c->capturing) return nullptr;
+  const size_t b = c->ts_used / VW_TS_BLOCK;
+  if (b == c->ts_blk.size()) {
+    void* q = nullptr;
+    if (hipHostMalloc(&q, VW_TS_BLOCK * sizeof(uint64_t), hipHostMallocDefault) != hipSuccess) {
+      (void)hipGetLastError();
+      return nullptr;
+    }
+    c->ts_blk.push_back((uint64_t*)q);
+  }
+  uint64_t* p = c->ts_blk[b] + c->ts_used % VW_TS_BLOCK;
+  p[0] = p[1] = 0;
+  c->ts_used += 2;
+  return p;
+}
+/* stage time from the start (or, after, the end) of launch a to the end (or,
+ * before, the start) of launch b */
+void add_bracket(Ctx* c, Stage s, const uint64_t* a, const uint64_t* b, bool after = false, bool before = false) {
+  if (a && b) c->brackets.push_back({s, a + (after ? 1 : 0), b + (before ? 0 : 1)});
+}
+
+/* event bracket for one stage launch group (batched steps: few, long launches) */
 hipEvent_t ev_begin(Ctx* c, Stage s, hipStream_t stream = nullptr) {
   if (c->capturing) return nullptr; /* no timing inside a captured graph */
   auto& v = c->ev[s];
@@ -222,7 +257,7 @@ void ev_end(Ctx* c, Stage s, hipStream_t stream = nullptr) {
   c->ev_used[s]++;
 }
 
-/* after a synchronise: fold recorded brackets into the timings */
+/* after a synchronise: fold the brackets into the timings */
 void collect_timings(Ctx* c) {
   double* dst[ST_N] = {&c->tim.gen_ms, &c->tim.viss_ms, &c->tim.conj_ms, &c->tim.group_ms,
                        &c->tim.recon_ms, &c->tim.finalize_ms, &c->tim.viss_kernel_ms, &c->tim.recon_kernel_ms};
@@ -236,6 +271,13 @@ void collect_timings(Ctx* c) {
     if (s == ST_RECONK) c->tim.n_recon_launch += (int32_t)c->ev_used[s];
     c->ev_used[s] = 0;
   }
+  for (const Ctx::Bracket& k : c->brackets) {
+    if (*k.from && *k.to > *k.from) *dst[k.s] += (double)(*k.to - *k.from) * c->ts_ms;
+    if (k.s == ST_VISSK) ++c->tim.n_viss_launch;
+    if (k.s == ST_RECONK) ++c->tim.n_recon_launch;
+  }
+  c->brackets.clear();
+  c->ts_used = 0;
 }
 
 int sync(Ctx* c) {
@@ -709,6 +751,10 @@ int enq_reset_fill(Ctx* c) {
 int create_device(Ctx* c) {
   int ndev = 0;
   if (hipGetDeviceCount(&ndev) != hipSuccess || ndev <= 0) return c->fail(VW_ERR_DEVICE, "no HIP device");
+  int dev = 0, khz = 0;
+  HC(hipGetDevice(&dev));
+  HC(hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, dev));
+  c->ts_ms = khz > 0 ? 1.0 / (double)khz : 0.0;
   HC(hipStreamCreateWithFlags(&c->st, hipStreamNonBlocking));
   if (c->cfg.serial_stages) {
     c->st2 = c->stB = c->st; /* one stream: the stream waits below are no-ops */
@@ -865,35 +911,35 @@ int enq_gen(Ctx* c, int t0, int tlen) {
   /* the other buffer set: free once the recon of two segments ago is done */
   select_seg(c, c->cur ^ 1);
   HC(hipStreamWaitEvent(c->st, c->ev_recon[c->cur], 0));
-  ev_begin(c, ST_GEN);
+  uint64_t* ts = new_ts(c);
   int64_t na = (int64_t)tlen * c->A;
   k_seg_gen<<<blocks_for(std::max(na, c->nh)), 256, 0, c->st>>>(
       c->d_pos, c->T, c->A, c->P, t0, tlen, c->per_ant ? c->cfg.occ_radius_km : 0.0, c->cosphi_glob, c->d_pa, c->d_pb,
       c->lambda, c->d_ant8, c->vfact ? c->d_aph : nullptr,
-      c->vfact && c->cfg.precision == VW_PREC_PLAIN ? c->d_aphl : nullptr, c->d_rows, c->d_rowt);
+      c->vfact && c->cfg.precision == VW_PREC_PLAIN ? c->d_aphl : nullptr, c->d_rows, c->d_rowt, ts);
   KC();
-  ev_end(c, ST_GEN);
+  add_bracket(c, ST_GEN, ts, ts);
   c->have_seg = true;
   c->have_viss = c->have_conj = c->have_groups = false;
   return VW_OK;
 }
 
 /* row classes of nt tiles into cls ([nt][nh_pad] bytes) from their cone bits */
-void launch_classify(Ctx* c, const uint8_t* bits, int64_t nt, uint8_t* cls, hipStream_t st) {
+void launch_classify(Ctx* c, const uint8_t* bits, int64_t nt, uint8_t* cls, hipStream_t st, uint64_t* ts = nullptr) {
   const int nhb = (int)((c->nh_pad + VW_GCLS_BLOCK - 1) / VW_GCLS_BLOCK);
   const unsigned nb = (unsigned)(nt * nhb);
   if (c->nfr_pad <= VW_GCLS_LDS_MAX)
     k_classify<true><<<nb, 256, (size_t)c->nfr_pad, st>>>(bits, c->nfr_pad, nhb, c->d_rows, c->nh, c->nh_pad,
-                                                           (uint32_t*)cls);
+                                                           (uint32_t*)cls, ts);
   else
-    k_classify<false><<<nb, 256, 0, st>>>(bits, c->nfr_pad, nhb, c->d_rows, c->nh, c->nh_pad, (uint32_t*)cls);
+    k_classify<false><<<nb, 256, 0, st>>>(bits, c->nfr_pad, nhb, c->d_rows, c->nh, c->nh_pad, (uint32_t*)cls, ts);
 }
 
 /* class table of a tile pass into the class scratch: cone bits per
  * (tile, antenna frame), then per (tile, half row) or (tile, group in the
  * batched recon's work order) */
 int enq_classes(Ctx* c, const double* cone, int64_t ntile_all, int64_t tile0, int64_t nt, bool groups,
-                uint8_t* bits, uint8_t* cls, hipStream_t st) {
+                uint8_t* bits, uint8_t* cls, hipStream_t st, uint64_t* ts = nullptr) {
   const int64_t nfr = (int64_t)c->tlen * c->A;
   if (c->nfr_pad <= VW_GCLS_LDS_MAX) {
     /* one block per tile makes the tile's cone bits in LDS: no bit table */
@@ -903,12 +949,14 @@ int enq_classes(Ctx* c, const double* cone, int64_t ntile_all, int64_t tile0, in
                                                        c->d_oia, c->d_oib, c->d_info, c->nq_pad, (uint32_t*)cls);
     else
       k_classify_tile<<<(unsigned)nt, 256, lds, st>>>(cone, ntile_all, tile0, c->d_ant8, nfr, c->d_rows, c->nh,
-                                                      c->nh_pad, (uint32_t*)cls);
+                                                      c->nh_pad, (uint32_t*)cls, ts);
     KC();
     return VW_OK;
   }
   if (nt * c->nfr_pad > c->bits_cap) return c->fail(VW_ERR_RANGE, "internal: cone bit buffer too small");
-  k_ant_bits<<<blocks_for(nt * c->nfr_pad), 256, 0, st>>>(cone, ntile_all, tile0, nt, c->d_ant8, nfr, c->nfr_pad, bits);
+  /* the bit kernel's end stamp is overwritten by the class kernel's */
+  k_ant_bits<<<blocks_for(nt * c->nfr_pad), 256, 0, st>>>(cone, ntile_all, tile0, nt, c->d_ant8, nfr, c->nfr_pad, bits,
+                                                          ts);
   KC();
   if (groups) {
     const int nqb = (int)((c->nq_pad + VW_GCLS_BLOCK - 1) / VW_GCLS_BLOCK);
@@ -917,19 +965,19 @@ int enq_classes(Ctx* c, const double* cone, int64_t ntile_all, int64_t tile0, in
     k_group_cls<false><<<nb, 256, 0, st>>>(bits, c->nfr_pad, nqb, c->d_oia, c->d_oib, c->d_info, c->nq_pad,
                                            (uint32_t*)cls);
   } else
-    launch_classify(c, bits, nt, cls, st);
+    launch_classify(c, bits, nt, cls, st, ts);
   KC();
   return VW_OK;
 }
 
 /* the one-sky recon's group masks of a pass ([nt][nq_pad / 16] words per output
  * set) into the sets' class scratch */
-int enq_group_masks(Ctx* c, const ReconSets& sets, uint8_t* const* bits) {
+int enq_group_masks(Ctx* c, const ReconSets& sets, uint8_t* const* bits, uint64_t* ts) {
   const int64_t nfr = (int64_t)c->tlen * c->A;
   const unsigned nb = (unsigned)(sets.s[0].nt + sets.s[1].nt);
   if (c->nfr_pad <= VW_GCLS_LDS_MAX) {
     k_group_mask<true><<<nb, 256, (size_t)c->nfr_pad, c->stB>>>(sets, c->d_ant8, nfr, c->nfr_pad, c->gs.gia, c->gs.gib,
-                                                                 c->d_info, c->nq_pad);
+                                                                 c->d_info, c->nq_pad, ts);
     KC();
     return VW_OK;
   }
@@ -938,11 +986,11 @@ int enq_group_masks(Ctx* c, const ReconSets& sets, uint8_t* const* bits) {
     if (!S.nt) continue;
     if (S.nt * c->nfr_pad > c->bits_cap) return c->fail(VW_ERR_RANGE, "internal: cone bit buffer too small");
     k_ant_bits<<<blocks_for(S.nt * c->nfr_pad), 256, 0, c->stB>>>(S.cone, S.ntile, S.tile0, S.nt, c->d_ant8, nfr,
-                                                                  c->nfr_pad, bits[i]);
+                                                                  c->nfr_pad, bits[i], nullptr);
     KC();
   }
   k_group_mask<false><<<nb, 256, 0, c->stB>>>(sets, c->d_ant8, nfr, c->nfr_pad, c->gs.gia, c->gs.gib, c->d_info,
-                                              c->nq_pad);
+                                              c->nq_pad, ts);
   KC();
   return VW_OK;
 }
@@ -957,7 +1005,7 @@ void launch_viss(const VissArgs& a, unsigned nb, hipStream_t st) {
 
 /* one tile pass of the antenna-factorized Viss: cone bits per (tile, frame),
  * the product blocks, then their fold into the raw half sums */
-int enq_viss_fact(Ctx* c, int64_t tile0, int64_t nt, double2* vh) {
+int enq_viss_fact(Ctx* c, int64_t tile0, int64_t nt, double2* vh, uint64_t* tf, uint64_t* tl) {
   const bool mixed = c->cfg.precision == VW_PREC_MIXED;
   const int G = vissf_groups(c->A);
   VissFShape s = viss_fshape(c, c->tlen, nt, c->fpart_cap / ((int64_t)c->tlen * vissf_blocks(G) * 256));
@@ -966,7 +1014,7 @@ int enq_viss_fact(Ctx* c, int64_t tile0, int64_t nt, double2* vh) {
   const int64_t nfr = (int64_t)c->tlen * c->A;
   if (nt * c->nfr_pad > c->bits_cap) return c->fail(VW_ERR_RANGE, "internal: cone bit buffer too small");
   k_ant_bits<<<blocks_for(nt * c->nfr_pad), 256, 0, c->st>>>(c->d_cone, c->ntile, tile0, nt, c->d_ant8, nfr,
-                                                              c->nfr_pad, c->d_bits_v);
+                                                              c->nfr_pad, c->d_bits_v, tf);
   KC();
   VissFArgs a{};
   a.tab = c->d_tab;
@@ -977,7 +1025,6 @@ int enq_viss_fact(Ctx* c, int64_t tile0, int64_t nt, double2* vh) {
   a.tpc = s.tpc; a.nchunk = s.nchunk; a.nquad = s.nquad;
   a.check = c->cfg.viss_form == VW_VISS_ANT_CHECK ? 1 : 0;
   a.part = c->d_fpart;
-  ev_begin(c, ST_VISSK);
   const unsigned nb = (unsigned)s.nblocks;
 #define VW_VF(TP_, G_, M_) k_vissf<TP_, G_, M_><<<nb, 256, 0, c->st>>>(a)
   if (c->TP == 256) {
@@ -989,12 +1036,12 @@ int enq_viss_fact(Ctx* c, int64_t tile0, int64_t nt, double2* vh) {
   }
 #undef VW_VF
   KC();
-  ev_end(c, ST_VISSK);
+  add_bracket(c, ST_VISSK, tf, tl, true, true);
   const int64_t nent = vissf_blocks(G) * 256;
-  k_vissf_fold<<<(unsigned)(c->tlen * (nent / 32)), 256, 0, c->st>>>(c->d_fpart, s.nchunk, nent, c->d_fesum);
+  k_vissf_fold<<<(unsigned)(c->tlen * (nent / 32)), 256, 0, c->st>>>(c->d_fpart, s.nchunk, nent, c->d_fesum, tl);
   KC();
   k_vissf_rows<<<blocks_for(c->nh), 256, 0, c->st>>>(c->d_fesum, c->nh, c->P, G, c->d_pa, c->d_pb, tile0 > 0 ? 1 : 0,
-                                                     c->d_vraw, c->d_rows, vh);
+                                                     c->d_vraw, c->d_rows, vh, tl);
   KC();
   return VW_OK;
 }
@@ -1082,22 +1129,29 @@ int enq_viss(Ctx* c, bool count, bool fill = false) {
   }
   const bool mixed = c->cfg.precision == VW_PREC_MIXED;
   int rc;
-  ev_begin(c, ST_VISS);
+  if (c->batch) ev_begin(c, ST_VISS);
+  uint64_t *first = nullptr, *last = nullptr;
   for (int64_t tile0 = 0; tile0 < c->ntile; tile0 += c->vtpp) {
     const int64_t nt = std::min(c->vtpp, c->ntile - tile0);
     double2* vh = fill && !c->batch && tile0 + nt == c->ntile ? c->d_vh : nullptr;
+    uint64_t *tf = nullptr, *tl = nullptr; /* stamps of the pass's first and last launches */
+    if (!c->batch) {
+      tf = new_ts(c);
+      last = tl = new_ts(c);
+      if (tile0 == 0) first = tf;
+    }
     if (c->batch) {
       if (tile0 == 0 && (rc = enq_order(c, 0))) return rc;
       if ((rc = enq_viss_batch(c, tile0, nt))) return rc;
       continue;
     }
     if (c->vfact && !count && !(c->fact_auto && !c->sky_finite)) {
-      if ((rc = enq_viss_fact(c, tile0, nt, vh))) return rc;
+      if ((rc = enq_viss_fact(c, tile0, nt, vh, tf, tl))) return rc;
       continue;
     }
     VissShape s = viss_shape(c, c->nh, nt, count, c->nchunk_max);
     if (s.nchunk > c->nchunk_max) return c->fail(VW_ERR_RANGE, "internal: chunk buffer too small");
-    if ((rc = enq_classes(c, c->d_cone, c->ntile, tile0, nt, false, c->d_bits_v, c->d_cls_v, c->st))) return rc;
+    if ((rc = enq_classes(c, c->d_cone, c->ntile, tile0, nt, false, c->d_bits_v, c->d_cls_v, c->st, tf))) return rc;
     VissArgs a{};
     a.tab = c->d_tab;
     a.l = c->d_l; a.m = c->d_m; a.n = c->d_n; a.nm1 = c->d_nm1; a.B = c->d_B; a.Bf = c->d_Bf;
@@ -1106,7 +1160,6 @@ int enq_viss(Ctx* c, bool count, bool fill = false) {
     a.nh = c->nh; a.nh_pad = c->nh_pad;
     a.tpc = s.tpc; a.nchunk = s.nchunk; a.nrb = s.nrb; a.bpc = s.bpc;
     a.part = c->d_part; a.cpart = c->d_cpart;
-    ev_begin(c, ST_VISSK);
     unsigned nb = (unsigned)s.nblocks;
 #define VW_VISS(TP_, M_, C_) launch_viss<TP_, viss_rpw(TP_, M_, C_), M_, C_>(a, nb, c->st)
     if (c->TP == 256) {
@@ -1118,13 +1171,14 @@ int enq_viss(Ctx* c, bool count, bool fill = false) {
     }
 #undef VW_VISS
     KC();
-    ev_end(c, ST_VISSK);
+    add_bracket(c, ST_VISSK, tf, tl, true, true);
     k_viss_reduce<<<blocks_for(c->nh), 256, 0, c->st>>>(c->d_part, s.nchunk, c->nh, c->nh_pad, tile0 > 0 ? 1 : 0,
                                                         c->d_vraw, count ? c->d_cpart : nullptr,
-                                                        count ? c->d_counts : nullptr, c->d_rows, vh);
+                                                        count ? c->d_counts : nullptr, c->d_rows, vh, tl);
     KC();
   }
-  ev_end(c, ST_VISS);
+  if (c->batch) ev_end(c, ST_VISS);
+  else add_bracket(c, ST_VISS, first, last);
   c->have_viss = true;
   c->have_conj = c->have_groups = false;
   if (fill && !c->batch) {
@@ -1136,14 +1190,18 @@ int enq_viss(Ctx* c, bool count, bool fill = false) {
 
 int enq_conj(Ctx* c) {
   if (!c->have_viss) return c->fail(VW_ERR_STATE, "vw_conj_fill needs vw_viss_half");
-  ev_begin(c, ST_CONJ);
-  if (c->batch)
+  if (c->batch) {
+    ev_begin(c, ST_CONJ);
     k_conj_fill_b<<<blocks_for(c->nsky * c->nh), 256, 0, c->st>>>(c->d_vraw, c->d_rows, c->nh, c->P, c->nsky, c->d_vh,
                                                                   c->d_vfull);
-  else
-    k_conj_fill<<<blocks_for(c->nh), 256, 0, c->st>>>(c->d_vraw, c->d_rows, c->nh, c->P, c->d_vh, c->d_vfull);
-  KC();
-  ev_end(c, ST_CONJ);
+    KC();
+    ev_end(c, ST_CONJ);
+  } else {
+    uint64_t* ts = new_ts(c);
+    k_conj_fill<<<blocks_for(c->nh), 256, 0, c->st>>>(c->d_vraw, c->d_rows, c->nh, c->P, c->d_vh, c->d_vfull, ts);
+    KC();
+    add_bracket(c, ST_CONJ, ts, ts);
+  }
   HC(hipEventRecord(c->ev_conj, c->st));
   c->have_conj = true;
   c->have_groups = false;
@@ -1156,7 +1214,8 @@ int enq_group_keys(Ctx* c) {
   bool full = c->cfg.recon_mode == VW_RECON_FULL;
   int64_t nr = full ? 2 * c->nh : c->nh;
   const bool rsort = nr > VW_RANK_MAX;
-  k_segsums<<<4, 64, 0, c->stB>>>(c->d_rows, c->nh, c->P, c->d_sums);
+  uint64_t *first = new_ts(c), *last = new_ts(c);
+  k_segsums<<<4, 64, 0, c->stB>>>(c->d_rows, c->nh, c->P, c->d_sums, first);
   KC();
   /* the radix sort's pairs start and end in the sorted arrays */
   k_keys<<<blocks_for(nr), 256, 0, c->stB>>>(c->d_sums, c->d_rows, nr, c->P, full ? 1 : 0, c->bl_max, c->lambda,
@@ -1181,34 +1240,38 @@ int enq_group_keys(Ctx* c) {
     k_rank_scatter<<<blocks_for(nr), 256, 0, c->stB>>>(c->d_keys, c->d_rank, nr, c->d_idx_sorted, c->d_keys_sorted);
     KC();
   }
-  k_groups<<<1, 1024, 0, c->stB>>>(c->d_keys_sorted, nr, c->cfg.blockage, c->d_gkeys, c->d_goff, c->d_info);
+  k_groups<<<1, 1024, 0, c->stB>>>(c->d_keys_sorted, nr, c->cfg.blockage, c->d_gkeys, c->d_goff, c->d_info, last);
   KC();
+  add_bracket(c, ST_GROUP, first, last);
   return VW_OK;
 }
 
 /* group records (cell centre, representative or mean visibility from vh,
  * antenna frames) of the current groups */
-int enq_group_data(Ctx* c, const double2* vh) {
+int enq_group_data(Ctx* c, const double2* vh, uint64_t** ts_out = nullptr) {
   bool full = c->cfg.recon_mode == VW_RECON_FULL;
   int64_t nr = full ? 2 * c->nh : c->nh;
+  uint64_t* ts = new_ts(c);
   k_group_data<<<blocks_for(nr), 256, 0, c->stB>>>(c->d_gkeys, c->d_goff, c->d_idx_sorted, vh, c->d_rows,
                                                   c->d_ant8, c->P, full ? 1 : 0, c->cfg.blockage, c->cfg.occ_mode,
                                                   c->cfg.precision == VW_PREC_PLAIN && c->generic ? VW_TAB_SCALE : 1.0,
                                                   c->d_info,
-                                                  c->gs);
+                                                  c->gs, ts);
   KC();
+  add_bracket(c, ST_GROUP, ts, ts);
+  if (ts_out) *ts_out = ts;
   return VW_OK;
 }
 
-int enq_group(Ctx* c, bool keys_done) {
+int enq_group(Ctx* c, bool keys_done, uint64_t** ts_out) {
   if (!c->have_conj) return c->fail(VW_ERR_STATE, "vw_recon_segment needs vw_conj_fill");
   bool full = c->cfg.recon_mode == VW_RECON_FULL;
   HC(hipStreamWaitEvent(c->stB, c->ev_conj, 0));
-  ev_begin(c, ST_GROUP, c->stB);
   int rcg;
-  if ((!keys_done && (rcg = enq_group_keys(c))) || (rcg = enq_group_data(c, c->d_vh))) return rcg;
+  if ((!keys_done && (rcg = enq_group_keys(c))) || (rcg = enq_group_data(c, c->d_vh, ts_out))) return rcg;
   if (c->batch) {
     int rc;
+    ev_begin(c, ST_GROUP, c->stB);
     if ((rc = enq_order(c, 1))) return rc;
     k_group_order_recs<<<blocks_for(c->nq_pad), 256, 0, c->stB>>>(c->d_order[1], c->gs.rec, c->gs.ant, c->gs.gia,
                                                                   c->gs.gib, c->nq_pad, c->d_orec, c->d_oant,
@@ -1218,8 +1281,8 @@ int enq_group(Ctx* c, bool keys_done) {
         c->d_goff, c->d_idx_sorted, c->d_vh, c->nh, c->P, full ? 1 : 0, c->cfg.blockage, c->cfg.occ_mode, c->d_info,
         c->d_order[1], c->nq_pad, c->nsky, c->nsky_pad, c->d_gpk[0], c->d_gpk[1], c->d_gpk[2], c->d_gpk[3]);
     KC();
+    ev_end(c, ST_GROUP, c->stB);
   }
-  ev_end(c, ST_GROUP, c->stB);
   c->have_groups = true;
   return VW_OK;
 }
@@ -1288,7 +1351,7 @@ int enq_recon_set_batch(Ctx* c, bool img) {
  * their accumulators.  Per tile pass one launch each of the classes, the recon
  * kernel and the ordered fold of its chunks covers both sets: two streams with
  * a launch per set cost three more launches, a fork and a join a segment. */
-int enq_recon_one(Ctx* c, double* const (&acc)[2], uint32_t* const (&wacc)[2]) {
+int enq_recon_one(Ctx* c, double* const (&acc)[2], uint32_t* const (&wacc)[2], const uint64_t* ts_data) {
   int kind;
   if (!c->cfg.blockage) kind = VW_KIND_AVG;
   else if (!c->generic) kind = VW_KIND_REP;
@@ -1298,6 +1361,8 @@ int enq_recon_one(Ctx* c, double* const (&acc)[2], uint32_t* const (&wacc)[2]) {
   const int64_t kind_w = kind == VW_KIND_GENERIC ? c->nh_pad : c->nq_pad;
   const bool want[2] = {c->cfg.healpix_out != 0, c->ngp > 0};
   uint8_t* const bits[2] = {c->d_bits, c->d_bits2};
+  const uint64_t* before = ts_data; /* the launch before the recon kernel */
+  uint64_t *last = nullptr;
   for (int64_t pass = 0;; ++pass) {
     ReconArgs a{};
     int64_t npts_all = 0;
@@ -1328,14 +1393,16 @@ int enq_recon_one(Ctx* c, double* const (&acc)[2], uint32_t* const (&wacc)[2]) {
       S.wacc = wacc[i];
       npts_all += S.npts;
     }
-    if (!npts_all) return VW_OK;
+    if (!npts_all) break;
     int rc;
+    uint64_t* tm = kind == VW_KIND_AVG ? nullptr : new_ts(c);
+    if (tm) before = tm;
     if (kind == VW_KIND_REP) {
-      if ((rc = enq_group_masks(c, a.sets, bits))) return rc;
+      if ((rc = enq_group_masks(c, a.sets, bits, tm))) return rc;
     } else if (kind == VW_KIND_GENERIC) {
       for (int i = 0; i < 2; ++i) {
         const ReconSet& S = a.sets.s[i];
-        if (S.nt && (rc = enq_classes(c, S.cone, S.ntile, S.tile0, S.nt, false, bits[i], (uint8_t*)S.cls, c->stB)))
+        if (S.nt && (rc = enq_classes(c, S.cone, S.ntile, S.tile0, S.nt, false, bits[i], (uint8_t*)S.cls, c->stB, tm)))
           return rc;
       }
     }
@@ -1356,7 +1423,7 @@ int enq_recon_one(Ctx* c, double* const (&acc)[2], uint32_t* const (&wacc)[2]) {
     /* representatives are filtered for finite values except in the uv-mirror
      * recon with occ_mode 2 */
     const bool rep_finite = full || c->cfg.occ_mode != 2;
-    ev_begin(c, ST_RECONK, c->stB);
+    last = new_ts(c);
     if (mixed) {
       if (kind == VW_KIND_REP && rep_finite) launch_recon<true, VW_KIND_REP_FINITE>(a, c->stB);
       else if (kind == VW_KIND_REP) launch_recon<true, VW_KIND_REP>(a, c->stB);
@@ -1369,20 +1436,25 @@ int enq_recon_one(Ctx* c, double* const (&acc)[2], uint32_t* const (&wacc)[2]) {
       else launch_recon<false, VW_KIND_AVG>(a, c->stB);
     }
     KC();
-    ev_end(c, ST_RECONK, c->stB);
-    k_recon_reduce<<<blocks_for(a.sets.s[0].npts) + blocks_for(a.sets.s[1].npts), 256, 0, c->stB>>>(a.sets,
-                                                                                                    c->cfg.blockage);
+    k_recon_reduce<<<blocks_for(a.sets.s[0].npts) + blocks_for(a.sets.s[1].npts), 256, 0, c->stB>>>(
+        a.sets, c->cfg.blockage, last);
     KC();
+    add_bracket(c, ST_RECONK, before, last, true, true);
+    before = last;
   }
+  /* the stage: from the end of the group records */
+  add_bracket(c, ST_RECON, ts_data, last, true);
+  return VW_OK;
 }
 
 /* the recon stage of the current segment after its groups' keys (keys_done) or
  * from the start */
 int enq_recon(Ctx* c, bool keys_done = false) {
   int rc;
-  if ((rc = enq_group(c, keys_done))) return rc;
-  ev_begin(c, ST_RECON, c->stB);
+  uint64_t* ts = nullptr;
+  if ((rc = enq_group(c, keys_done, &ts))) return rc;
   if (c->batch) {
+    ev_begin(c, ST_RECON, c->stB);
     if (c->ngp) {
       /* the image set runs on its own stream beside the HEALPix set; both
        * read the groups and write disjoint accumulators */
@@ -1393,12 +1465,12 @@ int enq_recon(Ctx* c, bool keys_done = false) {
     }
     if (c->cfg.healpix_out && (rc = enq_recon_set_batch(c, false))) return rc;
     if (c->ngp) HC(hipStreamWaitEvent(c->stB, c->ev_join, 0));
+    ev_end(c, ST_RECON, c->stB);
   } else {
     double* const acc[2] = {c->d_Cacc, c->d_Gacc};
     uint32_t* const wacc[2] = {c->d_Wacc, c->d_GWacc};
-    if ((rc = enq_recon_one(c, acc, wacc))) return rc;
+    if ((rc = enq_recon_one(c, acc, wacc, ts))) return rc;
   }
-  ev_end(c, ST_RECON, c->stB);
   /* the segment's buffer set is free for the segment after next */
   HC(hipEventRecord(c->ev_recon[c->cur], c->stB));
   return VW_OK;
@@ -1418,9 +1490,7 @@ int enq_step(Ctx* c) {
       /* the groups' keys and order need the rows only: beside the Viss */
       HC(hipEventRecord(c->ev_gen, c->st));
       HC(hipStreamWaitEvent(c->stB, c->ev_gen, 0));
-      ev_begin(c, ST_GROUP, c->stB);
       if ((rc = enq_group_keys(c))) return rc;
-      ev_end(c, ST_GROUP, c->stB);
       if ((rc = enq_viss(c, false, true)) || (c->batch && (rc = enq_conj(c))) || (rc = enq_recon(c, true))) return rc;
     }
     return VW_OK;
@@ -1437,16 +1507,13 @@ int enq_step(Ctx* c) {
     /* the segment's rows and the whole day buffer are written on st */
     HC(hipEventRecord(c->ev_conj, c->st));
     HC(hipStreamWaitEvent(c->stB, c->ev_conj, 0));
-    ev_begin(c, ST_GROUP, c->stB);
     if ((rc = enq_group_keys(c))) return rc;
-    ev_end(c, ST_GROUP, c->stB);
     for (const int32_t sk : u.skies) {
-      if ((rc = enq_group_data(c, c->d_vday + sk * day_rows + (int64_t)u.t0 * c->P))) return rc;
-      ev_begin(c, ST_RECON, c->stB);
+      uint64_t* ts = nullptr;
+      if ((rc = enq_group_data(c, c->d_vday + sk * day_rows + (int64_t)u.t0 * c->P, &ts))) return rc;
       double* const acc[2] = {c->d_Cacc + sk * c->npix, c->ngp ? c->d_Gacc + sk * c->ngp : nullptr};
       uint32_t* const wacc[2] = {c->d_Wsky + sk * c->npix, c->ngp ? c->d_GWsky + sk * c->ngp : nullptr};
-      if ((rc = enq_recon_one(c, acc, wacc))) return rc;
-      ev_end(c, ST_RECON, c->stB);
+      if ((rc = enq_recon_one(c, acc, wacc, ts))) return rc;
     }
     /* this buffer set is free once the segment's last recon is done */
     HC(hipEventRecord(c->ev_recon[c->cur], c->stB));
@@ -1552,6 +1619,7 @@ VW_API void vw_destroy(void* p) {
       (void)hipEventDestroy(e.a);
       (void)hipEventDestroy(e.b);
     }
+  for (uint64_t* q : c->ts_blk) (void)hipHostFree(q);
   if (c->ev_fork) (void)hipEventDestroy(c->ev_fork);
   if (c->ev_join) (void)hipEventDestroy(c->ev_join);
   if (c->ev_conj) (void)hipEventDestroy(c->ev_conj);
@@ -1759,7 +1827,7 @@ VW_API int vw_finalize(void* p, double* C, uint32_t* W, double* img, uint32_t* W
   Ctx* c = as_ctx(p);
   if (!c) return VW_ERR_ARG;
   if (int rj = join_recon(c)) return rj;
-  ev_begin(c, ST_FIN);
+  uint64_t* ts = new_ts(c);
   /* normalise on the device; copy out only what was asked for */
   const int64_t NN = (int64_t)c->cfg.img_n * c->cfg.img_n;
   FinalArgs f{};
@@ -1773,9 +1841,11 @@ VW_API int vw_finalize(void* p, double* C, uint32_t* W, double* img, uint32_t* W
     f.s[1] = FinalSet{c->d_Gacc, c->sky_sched ? c->d_GWsky : c->d_GWacc, c->d_ginv, c->ngp, NN,
                       c->sky_sched ? c->ngp : 0, c->d_iout, c->sky_sched ? c->d_iwout_sky : c->d_iwout};
   const unsigned nfb = blocks_for(f.s[0].nout * c->nsky) + blocks_for(f.s[1].nout * c->nsky);
-  if (nfb) k_finalize<<<nfb, 256, 0, c->st>>>(f);
-  KC();
-  ev_end(c, ST_FIN);
+  if (nfb) {
+    k_finalize<<<nfb, 256, 0, c->st>>>(f, ts);
+    KC();
+    add_bracket(c, ST_FIN, ts, ts);
+  }
   if (C) {
     if (c->cfg.healpix_out)
       HC(hipMemcpyAsync(C, c->d_out, sizeof(double) * c->npix * c->nsky, hipMemcpyDeviceToHost, c->st));
@@ -2104,7 +2174,7 @@ int full_classes(Ctx* c, bool img, std::vector<uint8_t>& t, uint8_t** dev_out) {
   hipError_t e = hipMalloc(&bits, (size_t)(nt * c->nfr_pad));
   if (e == hipSuccess) {
     k_ant_bits<<<blocks_for(nt * c->nfr_pad), 256, 0, c->st>>>(img ? c->d_gcone : c->d_cone, nt, 0, nt, c->d_ant8,
-                                                               (int64_t)c->tlen * c->A, c->nfr_pad, bits);
+                                                               (int64_t)c->tlen * c->A, c->nfr_pad, bits, nullptr);
     launch_classify(c, bits, nt, d, c->st);
     e = hipGetLastError();
   }
