@@ -72,6 +72,9 @@ CASES = {
     "tp512_uneven": dict(nside=32, n_ant=12, n_epochs=40, img_n=48, nsky=40, tile_pix=512, seg_tlen=[5, 19, 16]),
     # a small class budget: several tile passes per stage, one block per wave
     "tile_passes": dict(nside=32, n_ant=8, n_epochs=16, segs=2, img_n=48, nsky=16, class_budget_bytes=64 * 1024),
+    # one tile per pass; a last 32-point block and a last 64-frame block that are partly filled
+    "tile_passes_1": dict(nside=8, n_ant=5, n_epochs=27, img_n=37, nsky=3, tile_pix=512, class_budget_bytes=1,
+                          seg_tlen=[13, 14]),
     # a segment of 8,400 rows: grouping by the batched contexts' own radix sort
     # (equal weights mean equal groups)
     "long_segment": dict(nside=16, n_ant=16, n_epochs=72, img_n=32, nsky=20, seg_tlen=[70, 2]),

@@ -138,7 +138,10 @@ struct Ctx {
   int32_t *d_okey[2] = {}, *d_oidx[2] = {}, *d_okey2[2] = {}, *d_order[2] = {};
   double2* d_orec = nullptr; /* (ugu, vgu) of the group at each work-order position */
   int32_t *d_oia = nullptr, *d_oib = nullptr; /* its representative's antenna frames */
-  double* d_oant = nullptr;  /* its representative's antenna frames [position][10]    */
+  /* occlusion bits [32-point block of a pass][nfr_pad] of the Viss and of the
+   * recon's two output sets; sky or output tiles per batched pass             */
+  uint32_t *d_fvis_v = nullptr, *d_fvis = nullptr, *d_fvis2 = nullptr;
+  int64_t btpp = 0;
   int32_t* d_rshist[2] = {};  /* radix-sort digit tables per stream (Viss, grouping)   */
   int64_t rshist_cap = 0;
   /* per-sky segment schedules (vw_set_sky_schedules): the batched Viss of
@@ -547,6 +550,10 @@ ReconShape recon_shape(int64_t npts, int64_t nq = INT64_MAX) {
   return r;
 }
 
+int64_t class_budget(const Ctx* c) {
+  return c->cfg.class_budget_bytes > 0 ? c->cfg.class_budget_bytes : (int64_t)2 << 30;
+}
+
 /* output tiles per recon pass: as many as the class scratch holds */
 int64_t recon_pass_tiles(const Ctx* c, int64_t ntile_all, int64_t kind_w) {
   return std::max<int64_t>(1, std::min<int64_t>(ntile_all, c->cls_cap / kind_w));
@@ -674,6 +681,15 @@ int join_recon(Ctx* c) {
 int create_batch(Ctx* c) {
   int rc;
   const int64_t npix_pad = c->ntile * c->TP;
+  /* tiles per pass: as many as hold their occlusion bits (a bit per (point,
+   * antenna frame)) in the class budget */
+  const int64_t fbytes = c->TP / 8 * c->nfr_pad;
+  c->btpp = std::max<int64_t>(1, std::min(std::max(c->ntile, c->ngt), class_budget(c) / fbytes));
+  for (int b = 0; b < 3; ++b) {
+    const int64_t nt = std::min(c->btpp, b == 2 ? c->ngt : c->ntile);
+    if (nt && (rc = dalloc(c, b == 0 ? &c->d_fvis_v : b == 1 ? &c->d_fvis : &c->d_fvis2, (size_t)(nt * fbytes / 4))))
+      return rc;
+  }
   if ((rc = dalloc(c, &c->d_skyf, (size_t)(c->nsky * c->npix))) ||
       (rc = dalloc(c, &c->d_skyh, (size_t)(npix_pad * c->nsky_pad))) ||
       (rc = dalloc(c, &c->d_skyl, (size_t)(npix_pad * c->nsky_pad))))
@@ -681,18 +697,17 @@ int create_batch(Ctx* c) {
   for (int k = 0; k < 4; ++k)
     if ((rc = dalloc(c, &c->d_gpk[k], (size_t)(c->nq_pad * c->nsky_pad)))) return rc;
   int64_t vch = 1;
-  const int64_t vlast = c->ntile - (c->ntile - 1) / c->vtpp * c->vtpp;
+  const int64_t vfull = std::min(c->btpp, c->ntile), vlast = c->ntile - (c->ntile - 1) / vfull * vfull;
   for (int k = 0; k < c->segs; ++k)
-    for (int64_t nt : {c->vtpp, vlast})
+    for (int64_t nt : {vfull, vlast})
       for (int64_t tg : VW_BATCH_TARGETS) vch = std::max(vch, vissb_shape(c, (int64_t)c->seg_tlen[k] * c->P, nt, tg).nchunk);
   c->bpart_cap = vch * c->nsky_pad * c->nh_pad;
   if ((rc = dalloc(c, &c->d_bpart, (size_t)c->bpart_cap))) return rc;
-  const int64_t kind_w = c->nq_pad;
   int64_t rp = 1, wp = 1;
   for (int img = 0; img < 2; ++img) {
-    const int64_t npts = img ? c->ngp : c->npix, nta = img ? c->ngt : c->ntile;
+    const int64_t npts = img ? c->ngp : c->npix;
     if (npts <= 0) continue;
-    const int64_t pp = recon_pass_tiles(c, nta, kind_w) * c->TP;
+    const int64_t pp = c->btpp * c->TP;
     const int64_t last = npts - (npts - 1) / pp * pp;
     for (int64_t n : {std::min(npts, pp), last})
       for (int64_t tg : VW_BATCH_TARGETS) {
@@ -709,7 +724,7 @@ int create_batch(Ctx* c) {
         (rc = dalloc(c, &c->d_okey2[w], (size_t)n)) || (rc = dalloc(c, &c->d_order[w], (size_t)n)))
       return rc;
   }
-  if ((rc = dalloc(c, &c->d_orec, (size_t)c->nq_pad)) || (rc = dalloc(c, &c->d_oant, 10 * (size_t)c->nq_pad)) ||
+  if ((rc = dalloc(c, &c->d_orec, (size_t)c->nq_pad)) ||
       (rc = dalloc(c, &c->d_oia, (size_t)c->nq_pad)) || (rc = dalloc(c, &c->d_oib, (size_t)c->nq_pad)))
     return rc;
   {
@@ -813,8 +828,7 @@ int create_device(Ctx* c) {
   const size_t mh = (size_t)c->max_nh;
   const int64_t kind_w = c->generic ? c->nh_pad : c->nq_pad; /* recon class row width */
   const int64_t need = std::max<int64_t>(c->ntile * c->nh_pad, std::max<int64_t>(c->ntile, c->ngt) * kind_w);
-  const int64_t budget = c->cfg.class_budget_bytes > 0 ? c->cfg.class_budget_bytes : (int64_t)2 << 30;
-  c->cls_cap = std::min<int64_t>(need, budget);
+  c->cls_cap = std::min<int64_t>(need, class_budget(c));
   if (c->cls_cap < std::max(c->nh_pad, kind_w)) c->cls_cap = std::max(c->nh_pad, kind_w);
   c->cls_cap = (c->cls_cap + 3) / 4 * 4;
   c->vtpp = std::max<int64_t>(1, std::min<int64_t>(c->ntile, c->cls_cap / c->nh_pad));
@@ -935,21 +949,14 @@ void launch_classify(Ctx* c, const uint8_t* bits, int64_t nt, uint8_t* cls, hipS
     k_classify<false><<<nb, 256, 0, st>>>(bits, c->nfr_pad, nhb, c->d_rows, c->nh, c->nh_pad, (uint32_t*)cls, ts);
 }
 
-/* class table of a tile pass into the class scratch: cone bits per
- * (tile, antenna frame), then per (tile, half row) or (tile, group in the
- * batched recon's work order) */
-int enq_classes(Ctx* c, const double* cone, int64_t ntile_all, int64_t tile0, int64_t nt, bool groups,
-                uint8_t* bits, uint8_t* cls, hipStream_t st, uint64_t* ts = nullptr) {
+/* row classes of nt tiles from tile0 into cls ([nt][nh_pad] bytes) */
+int enq_classes(Ctx* c, const double* cone, int64_t ntile_all, int64_t tile0, int64_t nt, uint8_t* bits, uint8_t* cls,
+                hipStream_t st, uint64_t* ts = nullptr) {
   const int64_t nfr = (int64_t)c->tlen * c->A;
   if (c->nfr_pad <= VW_GCLS_LDS_MAX) {
     /* one block per tile makes the tile's cone bits in LDS: no bit table */
-    const size_t lds = (size_t)c->nfr_pad;
-    if (groups)
-      k_group_cls_tile<<<(unsigned)nt, 256, lds, st>>>(cone, ntile_all, tile0, c->d_ant8, nfr,
-                                                       c->d_oia, c->d_oib, c->d_info, c->nq_pad, (uint32_t*)cls);
-    else
-      k_classify_tile<<<(unsigned)nt, 256, lds, st>>>(cone, ntile_all, tile0, c->d_ant8, nfr, c->d_rows, c->nh,
-                                                      c->nh_pad, (uint32_t*)cls, ts);
+    k_classify_tile<<<(unsigned)nt, 256, (size_t)c->nfr_pad, st>>>(cone, ntile_all, tile0, c->d_ant8, nfr, c->d_rows,
+                                                                   c->nh, c->nh_pad, (uint32_t*)cls, ts);
     KC();
     return VW_OK;
   }
@@ -958,14 +965,19 @@ int enq_classes(Ctx* c, const double* cone, int64_t ntile_all, int64_t tile0, in
   k_ant_bits<<<blocks_for(nt * c->nfr_pad), 256, 0, st>>>(cone, ntile_all, tile0, nt, c->d_ant8, nfr, c->nfr_pad, bits,
                                                           ts);
   KC();
-  if (groups) {
-    const int nqb = (int)((c->nq_pad + VW_GCLS_BLOCK - 1) / VW_GCLS_BLOCK);
-    const unsigned nb = (unsigned)(nt * nqb);
-    /* frame rows here are longer than the LDS staging limit */
-    k_group_cls<false><<<nb, 256, 0, st>>>(bits, c->nfr_pad, nqb, c->d_oia, c->d_oib, c->d_info, c->nq_pad,
-                                           (uint32_t*)cls);
-  } else
-    launch_classify(c, bits, nt, cls, st, ts);
+  launch_classify(c, bits, nt, cls, st, ts);
+  KC();
+  return VW_OK;
+}
+
+/* occlusion bits of the points of nt tiles from tile0, of the sky or the lm
+ * grid, against the segment's antenna frames */
+int enq_frame_vis(Ctx* c, bool img, int64_t tile0, int64_t nt, uint32_t* out, hipStream_t st) {
+  const int64_t nfr = (int64_t)c->tlen * c->A, nblk = nt * (c->TP / 64);
+  const dim3 grid((unsigned)((nblk + 3) / 4), (unsigned)((nfr + 63) / 64));
+  k_frame_vis<<<grid, 256, 0, st>>>(img ? c->d_gl : c->d_l, img ? c->d_gm : c->d_m, img ? c->d_gn : c->d_n,
+                                    img ? c->ngp : c->npix, img ? c->d_gcone : c->d_cone, img ? c->ngt : c->ntile,
+                                    tile0, nblk, c->TP, c->d_ant8, nfr, c->nfr_pad, out);
   KC();
   return VW_OK;
 }
@@ -1086,18 +1098,18 @@ int enq_order(Ctx* c, int which) {
                                      c->d_oidx[which], n, 2);
 }
 
-/* one tile pass of the batched Viss: classes, the product kernel, the fold */
+/* one tile pass of the batched Viss: occlusion bits, the product kernel, the fold */
 int enq_viss_batch(Ctx* c, int64_t tile0, int64_t nt) {
   int rc;
-  if ((rc = enq_classes(c, c->d_cone, c->ntile, tile0, nt, false, c->d_bits_v, c->d_cls_v, c->st))) return rc;
+  if ((rc = enq_frame_vis(c, false, tile0, nt, c->d_fvis_v, c->st))) return rc;
   const VissBShape s = vissb_shape(c, c->nh, nt, c->vb_target, c->bpart_cap / (c->nsky_pad * c->nh_pad));
   if (s.nchunk * c->nsky_pad * c->nh_pad > c->bpart_cap) return c->fail(VW_ERR_RANGE, "internal: batch partial buffer too small");
   VissBArgs a{};
-  a.l = c->d_l; a.m = c->d_m; a.n = c->d_n; a.nm1 = c->d_nm1;
+  a.l = c->d_l; a.m = c->d_m; a.nm1 = c->d_nm1;
   a.skyh = (const uint4*)c->d_skyh; a.skyl = (const uint4*)c->d_skyl;
   a.npix = c->npix; a.nsky_pad = c->nsky_pad;
   a.tile0 = tile0; a.ntile = nt; a.TP = c->TP;
-  a.rows = c->d_rows; a.ant8 = c->d_ant8; a.cls = c->d_cls_v; a.perm = c->d_order[0];
+  a.rows = c->d_rows; a.fvis = c->d_fvis_v; a.nfr_pad = c->nfr_pad; a.perm = c->d_order[0];
   a.nh = c->nh; a.nh_pad = c->nh_pad;
   a.tpc = s.tpc; a.nchunk = s.nchunk; a.nrb = s.nrb; a.nrbw = s.nrbw;
   a.part = c->d_bpart;
@@ -1131,8 +1143,9 @@ int enq_viss(Ctx* c, bool count, bool fill = false) {
   int rc;
   if (c->batch) ev_begin(c, ST_VISS);
   uint64_t *first = nullptr, *last = nullptr;
-  for (int64_t tile0 = 0; tile0 < c->ntile; tile0 += c->vtpp) {
-    const int64_t nt = std::min(c->vtpp, c->ntile - tile0);
+  const int64_t tpp = c->batch ? c->btpp : c->vtpp;
+  for (int64_t tile0 = 0; tile0 < c->ntile; tile0 += tpp) {
+    const int64_t nt = std::min(tpp, c->ntile - tile0);
     double2* vh = fill && !c->batch && tile0 + nt == c->ntile ? c->d_vh : nullptr;
     uint64_t *tf = nullptr, *tl = nullptr; /* stamps of the pass's first and last launches */
     if (!c->batch) {
@@ -1151,7 +1164,7 @@ int enq_viss(Ctx* c, bool count, bool fill = false) {
     }
     VissShape s = viss_shape(c, c->nh, nt, count, c->nchunk_max);
     if (s.nchunk > c->nchunk_max) return c->fail(VW_ERR_RANGE, "internal: chunk buffer too small");
-    if ((rc = enq_classes(c, c->d_cone, c->ntile, tile0, nt, false, c->d_bits_v, c->d_cls_v, c->st, tf))) return rc;
+    if ((rc = enq_classes(c, c->d_cone, c->ntile, tile0, nt, c->d_bits_v, c->d_cls_v, c->st, tf))) return rc;
     VissArgs a{};
     a.tab = c->d_tab;
     a.l = c->d_l; a.m = c->d_m; a.n = c->d_n; a.nm1 = c->d_nm1; a.B = c->d_B; a.Bf = c->d_Bf;
@@ -1273,9 +1286,8 @@ int enq_group(Ctx* c, bool keys_done, uint64_t** ts_out) {
     int rc;
     ev_begin(c, ST_GROUP, c->stB);
     if ((rc = enq_order(c, 1))) return rc;
-    k_group_order_recs<<<blocks_for(c->nq_pad), 256, 0, c->stB>>>(c->d_order[1], c->gs.rec, c->gs.ant, c->gs.gia,
-                                                                  c->gs.gib, c->nq_pad, c->d_orec, c->d_oant,
-                                                                  c->d_oia, c->d_oib);
+    k_group_order_recs<<<blocks_for(c->nq_pad), 256, 0, c->stB>>>(c->d_order[1], c->gs.rec, c->gs.gia, c->gs.gib,
+                                                                  c->nq_pad, c->d_orec, c->d_oia, c->d_oib);
     KC();
     k_group_pack<<<blocks_for(c->nq_pad * c->nsky_pad), 256, 0, c->stB>>>(
         c->d_goff, c->d_idx_sorted, c->d_vh, c->nh, c->P, full ? 1 : 0, c->cfg.blockage, c->cfg.occ_mode, c->d_info,
@@ -1292,23 +1304,20 @@ void launch_recon(const ReconArgs& a, hipStream_t st) {
   k_recon<RECON_PPL, MIXED, KIND><<<(unsigned)(a.sets.s[0].nblk + a.sets.s[1].nblk), 256, 0, st>>>(a);
 }
 
-/* batched recon of one output set: per tile pass the (tile, group) classes,
+/* batched recon of one output set: per tile pass the occlusion bits,
  * the product kernel and the fold into the per-sky accumulators */
 int enq_recon_set_batch(Ctx* c, bool img) {
   hipStream_t st = img ? c->st2 : c->stB;
-  uint8_t* cls = img ? c->d_cls2 : c->d_cls;
-  uint8_t* bits = img ? c->d_bits2 : c->d_bits;
+  uint32_t* fvis = img ? c->d_fvis2 : c->d_fvis;
   const bool rep = c->cfg.blockage != 0;
   const int64_t npts_all = img ? c->ngp : c->npix;
   const int64_t ntile_all = img ? c->ngt : c->ntile;
-  const double* cone = img ? c->d_gcone : c->d_cone;
-  const int64_t otpp = recon_pass_tiles(c, ntile_all, c->nq_pad);
-  for (int64_t tile0 = 0; tile0 < ntile_all; tile0 += otpp) {
-    const int64_t nt = std::min(otpp, ntile_all - tile0);
+  for (int64_t tile0 = 0; tile0 < ntile_all; tile0 += c->btpp) {
+    const int64_t nt = std::min(c->btpp, ntile_all - tile0);
     const int64_t pt0 = tile0 * c->TP;
     const int64_t np = std::min(nt * c->TP, npts_all - pt0);
     if (rep) {
-      int rc = enq_classes(c, cone, ntile_all, tile0, nt, true, bits, cls, st);
+      int rc = enq_frame_vis(c, img, tile0, nt, fvis, st);
       if (rc) return rc;
     }
     const ReconBShape s = reconb_shape(c, np, c->rb_target);
@@ -1318,9 +1327,9 @@ int enq_recon_set_batch(Ctx* c, bool img) {
     a.l = img ? c->d_gl : c->d_l;
     a.m = img ? c->d_gm : c->d_m;
     a.n = img ? c->d_gn : c->d_n;
-    a.pt0 = pt0; a.npts = np; a.TP = c->TP;
-    a.gcls = cls; a.nq_pad = c->nq_pad; a.gperm = c->d_order[1]; a.orec = c->d_orec; a.oant = c->d_oant;
-    a.rec = c->gs.rec; a.gant = c->gs.ant; a.info = c->d_info;
+    a.pt0 = pt0; a.npts = np;
+    a.fvis = fvis; a.nfr_pad = c->nfr_pad; a.gperm = c->d_order[1]; a.orec = c->d_orec;
+    a.oia = c->d_oia; a.oib = c->d_oib; a.info = c->d_info;
     a.vrh = (const uint4*)c->d_gpk[0]; a.vrl = (const uint4*)c->d_gpk[1];
     a.vih = (const uint4*)c->d_gpk[2]; a.vil = (const uint4*)c->d_gpk[3];
     a.nsky_pad = c->nsky_pad;
@@ -1402,7 +1411,7 @@ int enq_recon_one(Ctx* c, double* const (&acc)[2], uint32_t* const (&wacc)[2], c
     } else if (kind == VW_KIND_GENERIC) {
       for (int i = 0; i < 2; ++i) {
         const ReconSet& S = a.sets.s[i];
-        if (S.nt && (rc = enq_classes(c, S.cone, S.ntile, S.tile0, S.nt, false, bits[i], (uint8_t*)S.cls, c->stB, tm)))
+        if (S.nt && (rc = enq_classes(c, S.cone, S.ntile, S.tile0, S.nt, bits[i], (uint8_t*)S.cls, c->stB, tm)))
           return rc;
       }
     }
@@ -1961,7 +1970,7 @@ VW_API int vw_viss_adjoint(void* p, const vw_c128* res, double* g) {
   HC(hipMemcpyAsync(c->d_adj_res, res, sizeof(vw_c128) * c->nh, hipMemcpyHostToDevice, c->st));
   for (int64_t tile0 = 0; tile0 < c->ntile; tile0 += c->vtpp) {
     const int64_t nt = std::min(c->vtpp, c->ntile - tile0);
-    if ((rc = enq_classes(c, c->d_cone, c->ntile, tile0, nt, false, c->d_bits_v, c->d_cls_v, c->st))) return rc;
+    if ((rc = enq_classes(c, c->d_cone, c->ntile, tile0, nt, c->d_bits_v, c->d_cls_v, c->st))) return rc;
     VissAdjArgs a{};
     a.tab = c->d_tab;
     a.l = c->d_l; a.m = c->d_m; a.n = c->d_n; a.nm1 = c->d_nm1; a.npix = c->npix;

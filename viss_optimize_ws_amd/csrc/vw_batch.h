@@ -135,12 +135,11 @@ __global__ void k_row_keys(const RowRec* __restrict__ rows, const double* __rest
   keys[i] = i < nh ? vw_pair_key(ant8, rows[i].ia, rows[i].ib) : 4096;
   idx[i] = (int32_t)i;
 }
-/* cell centres, representative antenna frames and their frame indices in
- * the recon's work order */
+/* cell centres and the representatives' antenna-frame indices in the recon's
+ * work order */
 __global__ void k_group_order_recs(const int32_t* __restrict__ order, const GRec* __restrict__ rec,
-                                   const double* __restrict__ gant, const int32_t* __restrict__ gia,
-                                   const int32_t* __restrict__ gib, int64_t n, double2* __restrict__ orec,
-                                   double* __restrict__ oant, int32_t* __restrict__ oia, int32_t* __restrict__ oib) {
+                                   const int32_t* __restrict__ gia, const int32_t* __restrict__ gib, int64_t n,
+                                   double2* __restrict__ orec, int32_t* __restrict__ oia, int32_t* __restrict__ oib) {
   int64_t j = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (j >= n) return;
   const int64_t q = order[j];
@@ -148,8 +147,6 @@ __global__ void k_group_order_recs(const int32_t* __restrict__ order, const GRec
   orec[j] = make_double2(g.ugu, g.vgu);
   oia[j] = gia[q];
   oib[j] = gib[q];
-#pragma unroll
-  for (int f = 0; f < 10; ++f) oant[j * 10 + f] = gant[q * 10 + f];
 }
 __global__ void k_group_keys(const int32_t* __restrict__ gia, const int32_t* __restrict__ gib,
                              const double* __restrict__ ant8, const DevInfo* __restrict__ info, int64_t n,
@@ -161,16 +158,78 @@ __global__ void k_group_keys(const int32_t* __restrict__ gia, const int32_t* __r
 }
 
 /* ------------------------------------------------------------------ */
+/* occlusion bits                                                       */
+/* ------------------------------------------------------------------ */
+
+/* Which points each antenna frame sees, one word per (32-point block of the
+ * pass, frame): out[block][nfr_pad], bit j = point 32 block + j.  A row's or a
+ * group's mask over 32 points is the AND of its two frames' words, so the
+ * occlusion test runs once per (point, frame) instead of twice per masked term
+ * (an epoch's A frames serve A (A - 1) / 2 rows), and the term loops of the
+ * products hold no test.  A frame that the tile's cone finds all visible or
+ * all hidden needs none at all; bits are the per-point FP64 test's otherwise,
+ * so a mask equals the pair class with its per-point tests.
+ * A wave owns 64 points and 64 frames: lane f holds frame f's position and
+ * words, the partly visible frames are broadcast one by one; 50 us for 196,608
+ * points x 2,080 frames.  64 skies at Nside 128, 16 antennas, 205 epochs and a
+ * 256^2 image, against class bytes with the FP64 test in the term loops (a
+ * divergent branch per masked term in the recon): k_reconb 22.3 -> 16.3 ms and
+ * k_vissb 7.4 -> 6.5 ms of overlapped kernel time, the call 36.8 -> 33.8 ms,
+ * results equal bit for bit. */
+__global__ __launch_bounds__(256) void k_frame_vis(const double* __restrict__ l, const double* __restrict__ m,
+                                                   const double* __restrict__ n, int64_t npts,
+                                                   const double* __restrict__ cone, int64_t ntile, int64_t tile0,
+                                                   int64_t nblk, int64_t TP, const double* __restrict__ ant8,
+                                                   int64_t nfr, int64_t nfr_pad, uint32_t* __restrict__ out) {
+  const int lane = threadIdx.x & 63;
+  const int64_t b = (int64_t)blockIdx.x * 4 + vw_rfl((int)(threadIdx.x >> 6));
+  if (b >= nblk) return;
+  const int64_t t = tile0 + b * 64 / TP;
+  const int64_t p = tile0 * TP + b * 64 + lane;
+  const bool ok = p < npts;
+  const int64_t pp = ok ? p : npts - 1;
+  const double pl = l[pp], pm = m[pp], pn = n[pp];
+  const int64_t f = (int64_t)blockIdx.y * 64 + lane;
+  const double* q = ant8 + (f < nfr ? f : nfr - 1) * 8;
+  const double x = q[0], y = q[1], z = q[2], in = q[3], cp = q[7];
+  const int cb = vw_cone_bits(q[4], q[5], q[6], cone[t], cone[ntile + t], cone[2 * ntile + t], cone[3 * ntile + t],
+                              cone[4 * ntile + t], cp);
+  uint32_t lo = !(cb & 2) && (cb & 1) ? 0xffffffffu : 0u, hi = lo;
+  uint64_t some = __ballot(f < nfr && !(cb & 3));
+  while (some) {
+    const int j = __builtin_ctzll(some);
+    some &= some - 1;
+    auto at = [j](double v) {
+      const uint64_t w = __builtin_bit_cast(uint64_t, v);
+      const uint32_t a = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)w, j);
+      const uint32_t c = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(w >> 32), j);
+      return __builtin_bit_cast(double, (uint64_t)c << 32 | a);
+    };
+    const uint64_t v = __ballot(ok && vw_visible(pl, pm, pn, at(x), at(y), at(z), at(in), at(cp)));
+    lo = lane == j ? (uint32_t)v : lo;
+    hi = lane == j ? (uint32_t)(v >> 32) : hi;
+  }
+  out[2 * b * nfr_pad + f] = lo;
+  out[(2 * b + 1) * nfr_pad + f] = hi;
+}
+
+/* all ones where bit `bit` of x is set, else zero */
+__device__ __forceinline__ int vw_bit_mask(uint32_t x, int bit) { return __builtin_amdgcn_sbfe((int)x, bit, 1); }
+__device__ __forceinline__ float vw_and_f32(float x, int mask) {
+  return __builtin_bit_cast(float, __builtin_bit_cast(int, x) & mask);
+}
+
+/* ------------------------------------------------------------------ */
 /* Viss                                                                 */
 /* ------------------------------------------------------------------ */
 struct VissBArgs {
-  const double *l, *m, *n, *nm1;
+  const double *l, *m, *nm1;
   const uint4 *skyh, *skyl; /* packed sky, 16-byte units                        */
   int64_t npix, nsky_pad;
   int64_t tile0, ntile, TP;  /* tiles of this pass                              */
   const RowRec* rows;
-  const double* ant8;
-  const uint8_t* cls;        /* [ntile][nh_pad] pass-relative class bytes         */
+  const uint32_t* fvis;      /* [32-pixel block of the pass][nfr_pad] occlusion bits */
+  int64_t nfr_pad;
   const int32_t* perm;       /* work order: block row j is half row perm[j]       */
   int64_t nh, nh_pad;
   int64_t tpc, nchunk, nrb, nrbw; /* tiles per chunk, chunks, 16-row blocks, blocks of 4 */
@@ -219,13 +278,14 @@ __device__ __forceinline__ vw_bf16x8 vw_lds_bf16x8(const __bf16* buf, int row, i
 
 /* one wave: 16 half rows x (16 NB) skies over the tiles of one chunk; a
  * workgroup is four waves (64 consecutive rows) on the same pixels.  Per
- * k-step of 32 pixels the workgroup stages the sky operand, the pixels' l,
- * m, n - 1, n and the 64 rows' class bytes on the step's tile through
- * double-buffered LDS.  Every step issues the same global loads, for the
- * next step, unconditionally (indices clamped in range), and waits for them
- * only before their LDS stores at its end: a load waited for right after it
- * is issued would also wait for the loads in flight before it (the vector
- * memory counter is in order), exposing their latency. */
+ * k-step of 32 pixels the workgroup stages the sky operand and the pixels' l,
+ * m, n - 1 through double-buffered LDS; a lane's row takes its mask over the
+ * step's pixels from its two frames' words of the occlusion bits.  Every step
+ * issues the same global loads, for the next step, unconditionally (indices
+ * clamped in range), and waits for them only before their LDS stores at its
+ * end: a load waited for right after it is issued would also wait for the
+ * loads in flight before it (the vector memory counter is in order), exposing
+ * their latency. */
 #ifndef VW_VISSB_WAVES
 #define VW_VISSB_WAVES 3
 #endif
@@ -233,9 +293,7 @@ template <int NB>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(VW_VISSB_WAVES))) void k_vissb(VissBArgs a) {
   using Stage = VwStage<2, NB>;
   __shared__ __attribute__((aligned(16))) __bf16 bsh[2][Stage::ROWS * VW_LROW];
-  __shared__ double px[2][4][32]; /* l, m, n - 1, n of a k-step's pixels */
-  __shared__ uint8_t pcls[2][64]; /* class bytes of the 64 rows on a k-step's tile */
-  __shared__ double frs[10][64];  /* the 64 rows' antenna frames (mixed-tile masks) */
+  __shared__ double px[2][3][32]; /* l, m, n - 1 of a k-step's pixels */
   const int64_t vb = vw_xcd_block(blockIdx.x, gridDim.x);
   const int64_t rbw = vb % a.nrbw;
   const int64_t rest = vb / a.nrbw;
@@ -245,20 +303,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(VW_VISSB_WA
   const int r = lane & 15, g = lane >> 4;
   const int64_t rb = rbw * 4 + wave;
   const bool wave_on = rb < a.nrb; /* uniform; every wave still joins the barriers */
-  const int64_t jr = rb * 16 + r;  /* block row; < nh_pad: nrb * 16 <= nh_pad */
+  const int64_t jr = rb * 16 + r;  /* block row */
   /* the sorted order puts the padding rows (index >= nh) last */
-  const int64_t h = jr < a.nh ? a.perm[jr] : jr;
-  const int64_t hc = h < a.nh ? h : a.nh - 1;
-  const RowRec rec = a.rows[hc];
-  /* the rows' antenna frames (per-pixel masks on mixed tiles), held in LDS
-   * rather than in 20 registers per lane: read only on mixed tiles */
-  if (g == 0) {
-    const double* qa = a.ant8 + (int64_t)rec.ia * 8;
-    const double* qb = a.ant8 + (int64_t)rec.ib * 8;
-    const int w_ = wave * 16 + r;
-    frs[0][w_] = qa[0]; frs[1][w_] = qa[1]; frs[2][w_] = qa[2]; frs[3][w_] = qa[3]; frs[4][w_] = qa[7];
-    frs[5][w_] = qb[0]; frs[6][w_] = qb[1]; frs[7][w_] = qb[2]; frs[8][w_] = qb[3]; frs[9][w_] = qb[7];
-  }
+  const bool row_on = jr < a.nh;
+  const RowRec rec = a.rows[a.perm[row_on ? jr : 0]];
+  const uint32_t rmask = row_on ? 0xffffffffu : 0u;
   const int64_t t0 = a.tile0 + chunk * a.tpc;
   const int64_t tend = a.tile0 + a.ntile;
   const int64_t t1 = (t0 + a.tpc < tend) ? t0 + a.tpc : tend;
@@ -268,26 +317,24 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(VW_VISSB_WA
   const int64_t row0 = sg * 16 * NB;
 
   Stage stg;
-  /* thread t: coordinate (t / 32) % 4 of pixel t % 32 of a step (threads
-   * 128-255 repeat 0-127, only the first store); lane (r, g): its row's
-   * class byte (only g = 0 stores) */
-  const int xc_ = (int)((threadIdx.x >> 5) & 3);
-  const double* xsrc = xc_ == 0 ? a.l : (xc_ == 1 ? a.m : (xc_ == 2 ? a.nm1 : a.n));
+  /* thread t < 96: coordinate t / 32 of pixel t % 32 of a step (the others
+   * repeat a load, unstored) */
+  const int xc_ = (int)(threadIdx.x >> 5);
+  const double* xsrc = xc_ == 0 ? a.l : (xc_ == 1 ? a.m : a.nm1);
+  const uint32_t* fv = a.fvis + (kb0 - (a.tile0 << ksh)) * a.nfr_pad;
   double xp;
-  int xcl;
-#define VW_X_LOAD(k_)                                                                   \
-  do {                                                                                  \
-    const int64_t p_ = ((kb0 + (k_)) << 5) + (threadIdx.x & 31);                        \
-    const double v_ = xsrc[p_ < a.npix ? p_ : a.npix - 1];                              \
-    xp = p_ < a.npix ? v_ : 0.0;                                                        \
-    /* rows past nh carry the hidden class in the table */                             \
-    const int c_ = (int)a.cls[(((kb0 + (k_)) >> ksh) - a.tile0) * a.nh_pad + h];       \
-    xcl = wave_on ? c_ : VW_CLS_HIDDEN;                                                 \
+  uint32_t xa, xb; /* the next step's words of the row's two frames */
+#define VW_X_LOAD(k_)                                             \
+  do {                                                            \
+    const int64_t p_ = ((kb0 + (k_)) << 5) + (threadIdx.x & 31);  \
+    const double v_ = xsrc[p_ < a.npix ? p_ : a.npix - 1];        \
+    xp = p_ < a.npix ? v_ : 0.0;                                  \
+    xa = fv[(k_) * a.nfr_pad + rec.ia];                           \
+    xb = fv[(k_) * a.nfr_pad + rec.ib];                           \
   } while (0)
-#define VW_X_STORE(b_)                                           \
-  do {                                                           \
-    if (threadIdx.x < 128) px[b_][xc_][threadIdx.x & 31] = xp;   \
-    if (g == 0) pcls[b_][wave * 16 + r] = (uint8_t)xcl;          \
+#define VW_X_STORE(b_)                                          \
+  do {                                                          \
+    if (threadIdx.x < 96) px[b_][xc_][threadIdx.x & 31] = xp;   \
   } while (0)
 
   vw_f32x4b accR[NB], accI[NB], sumR[NB], sumI[NB];
@@ -306,51 +353,34 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(VW_VISSB_WA
   stg.store(bsh[0]);
   __syncthreads();
 
+  bool dirty = false; /* uniform: the block's accumulators hold products */
   for (int64_t k = 0; k < K; ++k) {
     const int buf = (int)(k & 1);
     const int64_t kn = k + 1 < K ? k + 1 : k; /* the last step reloads itself */
+    const uint32_t mw = xa & xb & rmask;      /* bit kk: pixel kk of the step is seen */
     stg.load(a.skyh, a.skyl, nullptr, nullptr, kb0 + kn, a.nsky_pad, row0);
     VW_X_LOAD(kn);
-    const int cls = (int)pcls[buf][wave * 16 + r];
-    const bool act = __ballot(cls != VW_CLS_HIDDEN) != 0;
-    const bool any_mixed = __ballot(cls == VW_CLS_MIXED) != 0;
-    if (act) {
+    if (wave_on && __ballot(mw != 0) != 0) {
       const double* pl_ = px[buf][0];
       const double* pm_ = px[buf][1];
       const double* pz_ = px[buf][2];
-      const double* pn_ = px[buf][3];
       float cv[8], sv[8];
-      /* two forms of the step, chosen per wave: without mixed rows a lane's
-       * mask is its row's class alone (no per-term branch); with them every
-       * lane evaluates both antennas' predicates, branch-free */
-#define VW_PHASOR(MASKED_)                                                                              \
-  do {                                                                                                  \
-    _Pragma("unroll") for (int i = 0; i < 8; ++i) {                                                     \
-      const int kk = g * 8 + i;                                                                         \
-      const double pl = pl_[kk], pm = pm_[kk], pz = pz_[kk];                                            \
-      const double x = vw_viss_phase(rec.u, rec.v, rec.w, pl, pm, pz);                                  \
-      const float f = (float)__builtin_amdgcn_fract(x);                                                 \
-      const float sn = __builtin_amdgcn_sinf(f), cs = __builtin_amdgcn_cosf(f);                         \
-      bool on = cls == VW_CLS_VISIBLE;                                                                  \
-      if (MASKED_) {                                                                                    \
-        const double pn = pn_[kk];                                                                      \
-        const int va = vw_visible(pl, pm, pn, fa[0], fa[1], fa[2], fa[3], fa[4]);                       \
-        const int vb = vw_visible(pl, pm, pn, fb[0], fb[1], fb[2], fb[3], fb[4]);                       \
-        on = on | ((cls == VW_CLS_MIXED) & ((va & vb) != 0));                                           \
-      }                                                                                                 \
-      cv[i] = on ? cs : 0.0f;                                                                           \
-      sv[i] = on ? sn : 0.0f;                                                                           \
-    }                                                                                                   \
+      /* two forms of the step, chosen per wave: with and without masks */
+#define VW_PHASOR(MASKED_)                                                  \
+  do {                                                                      \
+    _Pragma("unroll") for (int i = 0; i < 8; ++i) {                         \
+      const int kk = g * 8 + i;                                             \
+      const double x = vw_viss_phase(rec.u, rec.v, rec.w, pl_[kk], pm_[kk], pz_[kk]); \
+      const float f = (float)__builtin_amdgcn_fract(x);                     \
+      const float sn = __builtin_amdgcn_sinf(f), cs = __builtin_amdgcn_cosf(f); \
+      const int on = MASKED_ ? vw_bit_mask(m8, i) : -1;                     \
+      cv[i] = MASKED_ ? vw_and_f32(cs, on) : cs;                            \
+      sv[i] = MASKED_ ? vw_and_f32(sn, on) : sn;                            \
+    }                                                                       \
   } while (0)
-      if (any_mixed) {
-        const int w_ = wave * 16 + r;
-        const double fa[5] = {frs[0][w_], frs[1][w_], frs[2][w_], frs[3][w_], frs[4][w_]};
-        const double fb[5] = {frs[5][w_], frs[6][w_], frs[7][w_], frs[8][w_], frs[9][w_]};
-        VW_PHASOR(true);
-      } else {
-        const double fa[5] = {}, fb[5] = {};
-        VW_PHASOR(false);
-      }
+      const uint32_t m8 = mw >> (8 * g);
+      if (__ballot(mw != 0xffffffffu)) VW_PHASOR(true);
+      else VW_PHASOR(false);
 #undef VW_PHASOR
       vw_bf16x8 ach, acl, ash, asl;
       vw_split8(cv, ach, acl);
@@ -363,20 +393,21 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(VW_VISSB_WA
         accR[nb] = vw_mac3(ach, acl, bh, bl, accR[nb]);
         accI[nb] = vw_mac3(ash, asl, bh, bl, accI[nb]);
       }
-      if ((k & 7) == 7) {
-        /* blocked sums: the products of 256 pixels accumulate in the matrix
-         * core's FP32 accumulators, which are then added to FP32 block sums
-         * (folded across chunks in FP64): error ~ (256 + K / 256) ulp
-         * rather than K ulp.  A tile's class is the same on all its steps,
-         * so act holds on the whole block */
+      dirty = true;
+    }
+    if ((k & 7) == 7 && dirty) {
+      /* blocked sums: the products of 256 pixels accumulate in the matrix
+       * core's FP32 accumulators, which are then added to FP32 block sums
+       * (folded across chunks in FP64): error ~ (256 + K / 256) ulp
+       * rather than K ulp */
 #pragma unroll
-        for (int nb = 0; nb < NB; ++nb) {
-          sumR[nb] += accR[nb];
-          sumI[nb] += accI[nb];
-          accR[nb] = vw_f32x4b{0.f, 0.f, 0.f, 0.f};
-          accI[nb] = vw_f32x4b{0.f, 0.f, 0.f, 0.f};
-        }
+      for (int nb = 0; nb < NB; ++nb) {
+        sumR[nb] += accR[nb];
+        sumI[nb] += accI[nb];
+        accR[nb] = vw_f32x4b{0.f, 0.f, 0.f, 0.f};
+        accI[nb] = vw_f32x4b{0.f, 0.f, 0.f, 0.f};
       }
+      dirty = false;
     }
     /* buffers of step k - 1: every wave passed the barrier after reading
      * them (the last step writes its own reload there, unread) */
@@ -489,18 +520,16 @@ __global__ void k_group_pack(const int32_t* __restrict__ goff, const int32_t* __
 
 struct ReconBArgs {
   const double *l, *m, *n;
-  int64_t pt0, npts, TP;      /* points [pt0, pt0 + npts) of this pass            */
-  const uint8_t* gcls;        /* [tiles of the pass][nq_pad] classes in work order  */
+  int64_t pt0, npts;          /* points [pt0, pt0 + npts) of this pass            */
+  const uint32_t* fvis;       /* [32-point block of the pass][nfr_pad] occlusion bits */
+  int64_t nfr_pad;
   const int32_t* gperm;       /* work order: position j is group gperm[j]          */
   const double2* orec;        /* (ugu, vgu) in work order                          */
-  const double* oant;         /* [position][10] representative frames, work order  */
-  int64_t nq_pad;
-  const GRec* rec;            /* cell centres (wavelengths)                        */
-  const double* gant;         /* [q][10] representative antenna frames             */
+  const int32_t *oia, *oib;   /* the representative's antenna frames, work order   */
   const DevInfo* info;
   const uint4 *vrh, *vrl, *vih, *vil; /* packed group visibilities, 16-byte units */
   int64_t nsky_pad;
-  int rep;                    /* 1: representative classes; 0: every group counts  */
+  int rep;                    /* 1: the representative's mask; 0: every group counts */
   int64_t nchunk, pblk, pbw;  /* group ranges, 16-point blocks, blocks of 4        */
   double* part;               /* [nchunk][nsky_pad][pstride]                       */
   uint32_t* wpart;            /* [nchunk][pstride]                                 */
@@ -509,9 +538,12 @@ struct ReconBArgs {
 
 /* one wave: 16 output points x (16 NB) skies over one range of groups; a
  * workgroup is four waves (64 consecutive points of one output tile).  Per
- * k-step of 32 groups the workgroup stages the packed group visibilities,
- * the groups' cell centres and their class bytes for the tile through
- * double-buffered LDS. */
+ * k-step of 32 groups the workgroup stages the packed group visibilities, the
+ * groups' cell centres and, per wave, the groups' masks over its 16 points
+ * through double-buffered LDS.  A mask is the AND of two words of the
+ * occlusion bits; the words are gathered one step ahead, their frame indices
+ * two.  Masks are zero for positions out of range and for the key-0 group, so
+ * they are all the term loop asks. */
 #ifndef VW_RECONB_WAVES
 #define VW_RECONB_WAVES 3
 #endif
@@ -519,10 +551,8 @@ template <int NB>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(VW_RECONB_WAVES))) void k_reconb(ReconBArgs a) {
   using Stage = VwStage<4, NB>;
   __shared__ __attribute__((aligned(16))) __bf16 bsh[2][Stage::ROWS * VW_LROW];
-  __shared__ double2 grec[2][32];                      /* (ugu, vgu)      */
-  __shared__ __attribute__((aligned(16))) int32_t gq[2][32]; /* group index */
-  __shared__ double gfr[2][320];                       /* frames, 10 per position */
-  __shared__ __attribute__((aligned(16))) uint8_t gcl[2][32]; /* classes */
+  __shared__ double2 grec[2][32]; /* (ugu, vgu) */
+  __shared__ __attribute__((aligned(16))) uint16_t gm[2][4][32]; /* masks: bit r = point r of the wave */
   const int64_t vb = vw_xcd_block(blockIdx.x, gridDim.x);
   const int64_t pbw = vb % a.pbw;
   const int64_t rest = vb / a.pbw;
@@ -533,7 +563,6 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(VW_RECONB_W
   const int64_t pb = pbw * 4 + wave;
   const bool wave_on = pb < a.pblk;
   const int64_t pbase = pb * 16;          /* pass-relative */
-  const int64_t tile = (pbw * 64) / a.TP; /* the workgroup's 64 points lie in one tile */
   const int64_t p = pbase + r;
   const bool okp = wave_on && p < a.npts;
   const int64_t pp = a.pt0 + (okp ? p : 0);
@@ -551,45 +580,46 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(VW_RECONB_W
   const int64_t row0 = sg * 16 * NB;
 
   Stage stg;
-  /* threads 0-31: the group at one position of the k-step and its cell
-   * centre (ugu, vgu); 32-33: 16 class bytes of the workgroup's tile; the
-   * records and the class table are laid out in work order */
+  /* wave 0, threads 0-31: the cell centre (ugu, vgu) of one position of the
+   * k-step; wave 1: lane (b, j) the mask of position j over the workgroup's
+   * 32-point block b */
+  const int xj = lane & 31, xb = lane >> 5;
+  const uint32_t* fv = a.fvis + (pbw * 2 + xb) * a.nfr_pad;
   double2 xr = make_double2(0.0, 0.0);
-  double xf0 = 0.0, xf1 = 0.0; /* frame doubles t and t + 256 of the k-step (t + 256 < 320) */
-  int32_t xq = 0;
-  vw_u32x4 xc = {0x01010101u, 0x01010101u, 0x01010101u, 0x01010101u};
-#define VW_X_LOAD(k_)                                                                    \
-  do {                                                                                   \
-    const int t_ = (int)threadIdx.x;                                                     \
-    const int64_t j0_ = qa + 32 * (k_);                                                  \
-    if (t_ < 32) {                                                                       \
-      /* j0 + 32 <= nq_pad: j0 < qe <= nq_pad and both are multiples of 32 */            \
-      xq = a.gperm[j0_ + t_];                                                            \
-      xr = a.orec[j0_ + t_];                                                             \
-    } else if (t_ < 34 && a.rep) {                                                       \
-      /* the lane's offset is formed here each step (opaque thread index):     \
-       * held across the loop it was spilled at this kernel's register budget */ \
-      int tc_ = t_ - 32;                                                                 \
-      __asm__ volatile("" : "+v"(tc_));                                                  \
-      xc = *(const vw_u32x4*)(a.gcls + tile * a.nq_pad + j0_ + 16 * tc_);                \
-    }                                                                                    \
-    if (a.rep) {                                                                         \
-      xf0 = a.oant[j0_ * 10 + t_];                                                       \
-      if (t_ < 64) xf1 = a.oant[j0_ * 10 + 256 + t_];                                    \
-    }                                                                                    \
+  int32_t xia = 0, xib = 0; /* frames of the step after the staged one; < 0: no group */
+  uint32_t xm0 = 0, xm1 = 0;
+#define VW_X_INDEX(k_)                                         \
+  do {                                                         \
+    if (wave == 1) {                                           \
+      const int64_t j_ = qa + 32 * (k_) + xj;                  \
+      const int64_t jc_ = j_ < qe ? j_ : qa;                   \
+      const bool in_ = j_ < qe && a.gperm[jc_] >= q0;          \
+      const int32_t ia_ = a.oia[jc_], ib_ = a.oib[jc_];        \
+      xia = in_ ? ia_ : -1;                                    \
+      xib = ib_;                                               \
+    }                                                          \
+  } while (0)
+#define VW_X_LOAD(k_)                                                       \
+  do {                                                                      \
+    if (wave == 0) {                                                        \
+      /* qa + 32 k + 32 <= nq_pad: both are multiples of 32 */              \
+      if (lane < 32) xr = a.orec[qa + 32 * (k_) + lane];                    \
+    } else if (wave == 1) {                                                 \
+      xm0 = xm1 = xia >= 0 ? 0xffffffffu : 0u;                              \
+      if (a.rep && xia >= 0) {                                              \
+        xm0 = fv[xia];                                                      \
+        xm1 = fv[xib];                                                      \
+      }                                                                     \
+    }                                                                       \
   } while (0)
 #define VW_X_STORE(b_)                                        \
   do {                                                        \
-    const int t_ = (int)threadIdx.x;                          \
-    if (t_ < 32) {                                            \
-      grec[b_][t_] = xr;                                      \
-      gq[b_][t_] = xq;                                        \
-    } else if (t_ < 34) {                                     \
-      *(vw_u32x4*)(&gcl[b_][16 * (t_ - 32)]) = xc;            \
-    }                                                         \
-    if (a.rep) {                                              \
-      gfr[b_][t_] = xf0;                                      \
-      if (t_ < 64) gfr[b_][256 + t_] = xf1;                   \
+    if (wave == 0) {                                          \
+      if (lane < 32) grec[b_][lane] = xr;                     \
+    } else if (wave == 1) {                                   \
+      const uint32_t m_ = xm0 & xm1;                          \
+      gm[b_][2 * xb][xj] = (uint16_t)m_;                      \
+      gm[b_][2 * xb + 1][xj] = (uint16_t)(m_ >> 16);          \
     }                                                         \
   } while (0)
   vw_f32x4b acc[NB];
@@ -603,8 +633,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(VW_RECONB_W
   uint32_t cnt = 0;
 
   if (K > 0) {
+    VW_X_INDEX(0);
     stg.load(a.vrh, a.vrl, a.vih, a.vil, qa >> 5, a.nsky_pad, row0);
     VW_X_LOAD(0);
+    VW_X_INDEX(1);
     stg.store(bsh[0]);
     VW_X_STORE(0);
   }
@@ -615,23 +647,15 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(VW_RECONB_W
     if (more) {
       stg.load(a.vrh, a.vrl, a.vih, a.vil, (qa >> 5) + k + 1, a.nsky_pad, row0);
       VW_X_LOAD(k + 1);
+      VW_X_INDEX(k + 2);
     }
-    /* positions of the lane: 8 g .. 8 g + 7 of the k-step */
-    const int64_t jk = qa + 32 * k + g * 8;
-    const uint64_t cw = *(const uint64_t*)(&gcl[buf][g * 8]);
-    const vw_u32x4 q03 = *(const vw_u32x4*)(&gq[buf][g * 8]), q47 = *(const vw_u32x4*)(&gq[buf][g * 8 + 4]);
-    /* a k-step whose groups are all hidden from this tile adds nothing; one
-     * whose groups are all in range, visible and of nonzero key needs no
-     * per-term mask.  Lane l < 32 tests position l of the step, so that the
-     * two step flags cost one test per lane and two ballots */
-    const int lt = lane & 31;
-    const int cl_ = (int)gcl[buf][lt];
-    const bool in_ = qa + 32 * k + lt < qe;
-    const bool live1 = lane < 32 && in_ && cl_ != VW_CLS_HIDDEN;
-    const bool bad1 = lane < 32 && !(in_ && cl_ == VW_CLS_VISIBLE && (int64_t)gq[buf][lt] >= q0);
-    if (wave_on && __ballot(live1) != 0) {
+    /* masks of the lane's positions 8 g .. 8 g + 7; a k-step that no point of
+     * the wave sees adds nothing, one that all see needs no masks */
+    const vw_u32x4 mw = *(const vw_u32x4*)(&gm[buf][wave][g * 8]);
+    const uint32_t ml = gm[buf][wave][lane & 31];
+    if (wave_on && __ballot(ml != 0) != 0) {
       float cv[8], sv[8];
-      if (__ballot(bad1) == 0) {
+      if (__ballot(ml != 0xffffu) == 0) {
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
           const double2 u = grec[buf][g * 8 + i];
@@ -644,21 +668,13 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(VW_RECONB_W
       } else {
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
-          const int64_t q = (int32_t)(i < 4 ? q03[i & 3] : q47[i & 3]);
-          const int cls = (int)((cw >> (8 * i)) & 0xffu);
-          bool on = jk + i < qe && q >= q0 && cls != VW_CLS_HIDDEN;
-          if (on && cls == VW_CLS_MIXED) {
-            const double* d = &gfr[buf][(g * 8 + i) * 10];
-            on = vw_visible(pl, pm, pn, d[0], d[1], d[2], d[3], d[4]) &&
-                 vw_visible(pl, pm, pn, d[5], d[6], d[7], d[8], d[9]);
-          }
+          const int on = vw_bit_mask(mw[i >> 1] >> r, 16 * (i & 1));
           const double2 u = grec[buf][g * 8 + i];
           const double x = vw_recon_phase(u.x, u.y, lp, mp);
           const float f = (float)__builtin_amdgcn_fract(x);
-          const float sn = __builtin_amdgcn_sinf(f), cs = __builtin_amdgcn_cosf(f);
-          cv[i] = on ? cs : 0.0f;
-          sv[i] = on ? -sn : 0.0f;
-          cnt += on ? 1u : 0u;
+          cv[i] = vw_and_f32(__builtin_amdgcn_cosf(f), on);
+          sv[i] = vw_and_f32(-__builtin_amdgcn_sinf(f), on);
+          cnt -= (uint32_t)on;
         }
       }
       vw_bf16x8 ach, acl, ash, asl;
@@ -688,6 +704,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(VW_RECONB_W
     }
     __syncthreads();
   }
+#undef VW_X_INDEX
 #undef VW_X_LOAD
 #undef VW_X_STORE
   if (!wave_on) return;

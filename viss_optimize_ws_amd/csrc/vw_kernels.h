@@ -324,7 +324,7 @@ __device__ __forceinline__ void vw_tile_bits_lds(uint8_t* sb, const double* __re
  * word.  The rows' frame indices pass through LDS (loaded with consecutive
  * lanes on consecutive records, read back four rows a thread), beside the
  * tile's row of cone bits staged in LDS (STAGE; nfr_pad bytes of dynamic
- * LDS) or, for longer rows, gathered from global memory, as k_group_cls. */
+ * LDS) or, for longer rows, gathered from global memory. */
 #define VW_GCLS_BLOCK 1024
 template <bool STAGE>
 __global__ __launch_bounds__(256) void k_classify(const uint8_t* __restrict__ bits, int64_t nfr_pad, int nhb,
@@ -1639,85 +1639,6 @@ __global__ void k_group_data(const int64_t* __restrict__ gkeys, const int32_t* _
   vw_frame32(qa, g.ant32 + q * 8);
   vw_frame32(qb, g.ant32 + q * 8 + 4);
   vw_ts_end(ts);
-}
-
-/* class of (output tile, group) from the representative's antennas, for the
- * batched recon: entry j of a tile's row pairs frames ia[j] and ib[j] (in the
- * work order, which puts the groups past nuniq last: entries j >= nuniq are
- * hidden).  A
- * block covers VW_GCLS_BLOCK entries of one tile's row, four a thread
- * written as one class word (byte e = entry 4 i + e).  Each thread issues
- * its index loads first, then the block stages that tile's frame row of
- * cone bits in LDS (STAGE; nfr_pad bytes of dynamic LDS; longer rows are
- * gathered from global memory), so the loads overlap.  Blocks that start
- * past the 64-entry block holding entry nuniq - 1 write nothing: the recon
- * kernel reads the classes of entries below nuniq only, in aligned blocks of
- * 32. */
-template <bool STAGE>
-__global__ __launch_bounds__(256) void k_group_cls(const uint8_t* __restrict__ bits, int64_t nfr_pad, int nqb,
-                                                   const int32_t* __restrict__ ia, const int32_t* __restrict__ ib,
-                                                   const DevInfo* __restrict__ info, int64_t nq_pad,
-                                                   uint32_t* __restrict__ gcls) {
-  extern __shared__ uint4 sbits[];
-  static_assert(VW_GCLS_BLOCK == 4 * 256, "four entries a thread");
-  const uint32_t tr = blockIdx.x / (uint32_t)nqb, qc = blockIdx.x - tr * (uint32_t)nqb;
-  const int64_t j00 = (int64_t)qc * VW_GCLS_BLOCK;
-  const int64_t nu = info->nuniq;
-  if (j00 >= (nu + 63) / 64 * 64) return;
-  const uint8_t* row = bits + (int64_t)tr * nfr_pad;
-  const int64_t j0 = j00 + 4 * threadIdx.x;
-  const bool live = j0 < nq_pad; /* nq_pad is a multiple of 64: whole words only */
-  const int64_t jl = live ? j0 : 0;
-  /* indices past nuniq are not frames: gather frame 0 for them instead */
-  const int4 a4 = *(const int4*)(ia + jl), b4 = *(const int4*)(ib + jl);
-  const int av[4] = {a4.x, a4.y, a4.z, a4.w}, bv[4] = {b4.x, b4.y, b4.z, b4.w};
-  if (STAGE) {
-    /* nfr_pad is a multiple of 64 and the row starts 64-byte aligned */
-    for (int64_t i = threadIdx.x; i < nfr_pad / 16; i += 256) sbits[i] = ((const uint4*)row)[i];
-    __syncthreads();
-  }
-  const uint8_t* b = STAGE ? (const uint8_t*)sbits : row;
-  uint32_t w = 0;
-#pragma unroll
-  for (int e = 0; e < 4; ++e) {
-    const bool grp = jl + e < nu;
-    const uint32_t cls = (uint32_t)vw_pair_class(b[grp ? av[e] : 0], b[grp ? bv[e] : 0]);
-    w |= (grp ? cls : (uint32_t)VW_CLS_HIDDEN) << (8 * e);
-  }
-  if (live) gcls[((int64_t)tr * nq_pad + j0) >> 2] = w;
-}
-
-/* k_group_cls with the cone bits made in place: one block per tile of the
- * pass computes the tile's frame bits into LDS (nfr bytes of dynamic LDS),
- * then writes the class words of entries below nuniq rounded up to 64 (the
- * entries the recon kernels read), VW_GCLS_BLOCK at a time */
-__global__ __launch_bounds__(256) void k_group_cls_tile(const double* __restrict__ cone, int64_t ntile,
-                                                        int64_t tile0, const double* __restrict__ ant8, int64_t nfr,
-                                                        const int32_t* __restrict__ ia,
-                                                        const int32_t* __restrict__ ib,
-                                                        const DevInfo* __restrict__ info, int64_t nq_pad,
-                                                        uint32_t* __restrict__ gcls) {
-  extern __shared__ uint4 sbits[];
-  const int64_t tr = blockIdx.x;
-  const int64_t nu = info->nuniq;
-  const int64_t qend = (nu + 63) / 64 * 64 < nq_pad ? (nu + 63) / 64 * 64 : nq_pad;
-  if (qend == 0) return;
-  uint8_t* sb = (uint8_t*)sbits;
-  vw_tile_bits_lds(sb, cone, ntile, tile0 + tr, ant8, nfr);
-  __syncthreads();
-  for (int64_t j0 = 4 * threadIdx.x; j0 < qend; j0 += VW_GCLS_BLOCK) {
-    /* indices past nuniq are not frames: frame 0 stands in for them */
-    const int4 a4 = *(const int4*)(ia + j0), b4 = *(const int4*)(ib + j0);
-    const int av[4] = {a4.x, a4.y, a4.z, a4.w}, bv[4] = {b4.x, b4.y, b4.z, b4.w};
-    uint32_t w = 0;
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      const bool grp = j0 + e < nu;
-      const uint32_t cls = (uint32_t)vw_pair_class(sb[grp ? av[e] : 0], sb[grp ? bv[e] : 0]);
-      w |= (grp ? cls : (uint32_t)VW_CLS_HIDDEN) << (8 * e);
-    }
-    gcls[(tr * nq_pad + j0) >> 2] = w;
-  }
 }
 
 /* The output sets of one recon launch (HEALPix map, lm image, one tile pass of
