@@ -21,6 +21,7 @@
 #include "vw_batch.h"
 #include "vw_kernels.h"
 #include "vw_shared.h"
+#include "vw_xfer.h"
 
 #define VW_API extern "C" __attribute__((visibility("default")))
 
@@ -37,6 +38,7 @@ enum Stage { ST_GEN = 0, ST_VISS, ST_CONJ, ST_GROUP, ST_RECON, ST_FIN, ST_VISSK,
 struct Ctx {
   vw_config cfg{};
   std::string err;
+  VwXfer xfer; /* results into the caller's memory */
   /* plan */
   int64_t nside = 0, npix = 0, TP = 256, ntile = 0;
   int A = 0, P = 0, T = 0, segs = 0, max_tlen = 0;
@@ -909,6 +911,7 @@ int create_device(Ctx* c) {
       return rc;
   }
   if (c->batch && (rc = create_batch(c))) return rc;
+  c->xfer.reserve(sizeof(double) * (size_t)(c->nsky * (c->npix + (int64_t)c->cfg.img_n * c->cfg.img_n)));
   if ((rc = enq_reset_fill(c))) return rc;
   if ((rc = upload_day(c))) return rc;
   HC(hipStreamSynchronize(c->st));
@@ -1761,7 +1764,8 @@ VW_API int vw_viss_half(void* p, vw_c128* out) {
   if (!c) return VW_ERR_ARG;
   int rc = enq_viss(c, false);
   if (rc) return rc;
-  if (out) HC(hipMemcpyAsync(out, c->d_vraw, sizeof(vw_c128) * c->nh * c->nsky, hipMemcpyDeviceToHost, c->st));
+  const VwXfer::Seg o = {out, c->d_vraw, sizeof(vw_c128) * c->nh * c->nsky};
+  if (out) HC(c->xfer.out(&o, 1, c->st));
   return sync(c);
 }
 
@@ -1770,8 +1774,9 @@ VW_API int vw_conj_fill(void* p, vw_c128* oh, vw_c128* of) {
   if (!c) return VW_ERR_ARG;
   int rc = enq_conj(c);
   if (rc) return rc;
-  if (oh) HC(hipMemcpyAsync(oh, c->d_vh, sizeof(vw_c128) * c->nh * c->nsky, hipMemcpyDeviceToHost, c->st));
-  if (of) HC(hipMemcpyAsync(of, c->d_vfull, sizeof(vw_c128) * 2 * c->nh * c->nsky, hipMemcpyDeviceToHost, c->st));
+  const size_t nb = sizeof(vw_c128) * c->nh * c->nsky;
+  const VwXfer::Seg o[2] = {{oh, c->d_vh, oh ? nb : 0}, {of, c->d_vfull, of ? 2 * nb : 0}};
+  HC(c->xfer.out(o, 2, c->st));
   return sync(c);
 }
 
@@ -1855,24 +1860,21 @@ VW_API int vw_finalize(void* p, double* C, uint32_t* W, double* img, uint32_t* W
     KC();
     add_bracket(c, ST_FIN, ts, ts);
   }
-  if (C) {
-    if (c->cfg.healpix_out)
-      HC(hipMemcpyAsync(C, c->d_out, sizeof(double) * c->npix * c->nsky, hipMemcpyDeviceToHost, c->st));
-    else std::memset(C, 0, sizeof(double) * c->npix * c->nsky);
-  }
   const int64_t nw = c->sky_sched ? c->nsky : 1; /* weight maps */
-  if (W) {
-    if (c->cfg.healpix_out)
-      HC(hipMemcpyAsync(W, c->sky_sched ? c->d_Wsky : c->d_wout, sizeof(uint32_t) * c->npix * nw,
-                        hipMemcpyDeviceToHost, c->st));
-    else std::memset(W, 0, sizeof(uint32_t) * c->npix * nw);
+  VwXfer::Seg o[4];
+  int no = 0;
+  if (c->cfg.healpix_out) {
+    if (C) o[no++] = {C, c->d_out, sizeof(double) * c->npix * c->nsky};
+    if (W) o[no++] = {W, c->sky_sched ? c->d_Wsky : c->d_wout, sizeof(uint32_t) * c->npix * nw};
+  } else {
+    if (C) std::memset(C, 0, sizeof(double) * c->npix * c->nsky);
+    if (W) std::memset(W, 0, sizeof(uint32_t) * c->npix * nw);
   }
   if (c->ngp) {
-    if (img) HC(hipMemcpyAsync(img, c->d_iout, sizeof(double) * NN * c->nsky, hipMemcpyDeviceToHost, c->st));
-    if (Wimg)
-      HC(hipMemcpyAsync(Wimg, c->sky_sched ? c->d_iwout_sky : c->d_iwout, sizeof(uint32_t) * NN * nw,
-                        hipMemcpyDeviceToHost, c->st));
+    if (img) o[no++] = {img, c->d_iout, sizeof(double) * NN * c->nsky};
+    if (Wimg) o[no++] = {Wimg, c->sky_sched ? c->d_iwout_sky : c->d_iwout, sizeof(uint32_t) * NN * nw};
   }
+  HC(c->xfer.out(o, no, c->st));
   return sync(c);
 }
 
@@ -1889,10 +1891,11 @@ VW_API int vw_get_accumulators(void* p, double* C, uint32_t* W, double* G, uint3
   if (!c) return VW_ERR_ARG;
   if (c->sky_sched) return c->fail(VW_ERR_STATE, "accumulators of per-sky schedules are not exported");
   if (int rj = join_recon(c)) return rj;
-  if (C) HC(hipMemcpyAsync(C, c->d_Cacc, sizeof(double) * c->npix * c->nsky, hipMemcpyDeviceToHost, c->st));
-  if (W) HC(hipMemcpyAsync(W, c->d_Wacc, sizeof(uint32_t) * c->npix, hipMemcpyDeviceToHost, c->st));
-  if (c->ngp && G) HC(hipMemcpyAsync(G, c->d_Gacc, sizeof(double) * c->ngp * c->nsky, hipMemcpyDeviceToHost, c->st));
-  if (c->ngp && GW) HC(hipMemcpyAsync(GW, c->d_GWacc, sizeof(uint32_t) * c->ngp, hipMemcpyDeviceToHost, c->st));
+  const VwXfer::Seg o[4] = {{C, c->d_Cacc, C ? sizeof(double) * c->npix * c->nsky : 0},
+                            {W, c->d_Wacc, W ? sizeof(uint32_t) * c->npix : 0},
+                            {G, c->d_Gacc, G ? sizeof(double) * c->ngp * c->nsky : 0},
+                            {GW, c->d_GWacc, GW ? sizeof(uint32_t) * c->ngp : 0}};
+  HC(c->xfer.out(o, 4, c->st));
   if (wtotal)
     HC(hipMemcpyAsync(wtotal, (char*)c->d_info + offsetof(DevInfo, wtotal), sizeof(int64_t), hipMemcpyDeviceToHost,
                       c->st));
@@ -1992,7 +1995,8 @@ VW_API int vw_viss_adjoint(void* p, const vw_c128* res, double* g) {
                                                        c->d_adj_out);
     KC();
   }
-  HC(hipMemcpyAsync(g, c->d_adj_out, sizeof(double) * c->npix, hipMemcpyDeviceToHost, c->st));
+  const VwXfer::Seg og = {g, c->d_adj_out, sizeof(double) * c->npix};
+  HC(c->xfer.out(&og, 1, c->st));
   return sync(c);
 }
 

@@ -26,6 +26,7 @@
 
 #include "../../include/vissws.h"
 #include "../../include/vw_unet.h"
+#include "vw_xfer.h"
 
 #define VW_API extern "C" __attribute__((visibility("default")))
 
@@ -1018,6 +1019,9 @@ struct Net {
   int32_t* idx = nullptr;
   int64_t idx_cap = 0;
   double train_ms = 0.0;
+  VwXfer xfer;             /* predictions into the caller's memory */
+  float* stage = nullptr;  /* FP32 images of a batch on their way in or out */
+  int64_t stage_cap = 0;
   float* scratch_dev = nullptr; /* this device's address of scratch (vw_unet_predict_noalloc) */
 
   int fail(int code, const std::string& e) {
@@ -1349,32 +1353,25 @@ struct Ops {
     UC(hipGetLastError());
     return VW_OK;
   }
-  /* host FP32 -> tensor t of the storage type, through a staging buffer:
-   * allocated per call, or the caller's (staging, no allocation) */
-  static int upload(Net* c, const float* host, int t, int n, bool grad = false, float* staging = nullptr) {
+  /* host FP32 -> tensor t of the storage type through the device staging
+   * buffer.  Stream-ordered only: host stays in use until the stream is waited
+   * for */
+  static int upload(Net* c, const float* host, int t, int n, float* staging, bool grad = false) {
     const int64_t ne = n * c->elems(t);
-    float* tmp = staging;
-    if (!tmp) UC(hipMalloc(&tmp, sizeof(float) * ne));
-    hipError_t e = hipMemcpyAsync(tmp, host, sizeof(float) * ne, hipMemcpyHostToDevice, c->st);
-    if (e == hipSuccess) {
-      k_from_f32<T><<<nblk(ne), 256, 0, c->st>>>(tmp, (T*)(grad ? c->d[t] : c->a[t]), ne);
-      e = hipGetLastError();
-    }
-    if (e == hipSuccess) e = hipStreamSynchronize(c->st);
-    if (!staging) (void)hipFree(tmp);
-    if (e != hipSuccess) return c->fail(VW_ERR_DEVICE, std::string("upload: ") + hipGetErrorString(e));
+    UC(hipMemcpyAsync(staging, host, sizeof(float) * ne, hipMemcpyHostToDevice, c->st));
+    k_from_f32<T><<<nblk(ne), 256, 0, c->st>>>(staging, (T*)(grad ? c->d[t] : c->a[t]), ne);
+    UC(hipGetLastError());
     return VW_OK;
   }
-  static int download(Net* c, int t, int n, float* host, float* staging = nullptr) {
+  /* tensor t into host memory, filled on return; xf null: a plain copy */
+  static int download(Net* c, int t, int n, float* host, float* staging, VwXfer* xf) {
     const int64_t ne = n * c->elems(t);
-    float* tmp = staging;
-    if (!tmp) UC(hipMalloc(&tmp, sizeof(float) * ne));
-    k_to_f32<T><<<nblk(ne), 256, 0, c->st>>>((const T*)c->a[t], tmp, ne);
-    hipError_t e = hipGetLastError();
-    if (e == hipSuccess) e = hipMemcpyAsync(host, tmp, sizeof(float) * ne, hipMemcpyDeviceToHost, c->st);
-    if (e == hipSuccess) e = hipStreamSynchronize(c->st);
-    if (!staging) (void)hipFree(tmp);
-    if (e != hipSuccess) return c->fail(VW_ERR_DEVICE, std::string("download: ") + hipGetErrorString(e));
+    k_to_f32<T><<<nblk(ne), 256, 0, c->st>>>((const T*)c->a[t], staging, ne);
+    UC(hipGetLastError());
+    const VwXfer::Seg o = {host, staging, sizeof(float) * ne};
+    if (xf) UC(xf->out(&o, 1, c->st));
+    else UC(hipMemcpyAsync(o.host, o.dev, o.bytes, hipMemcpyDeviceToHost, c->st));
+    UC(hipStreamSynchronize(c->st));
     return VW_OK;
   }
   static int gather(Net* c, const int32_t* idx, int n) {
@@ -1543,6 +1540,7 @@ VW_API void vw_unet_destroy(void* p) {
   if (!c) return;
   if (c->st) (void)hipStreamSynchronize(c->st);
   for (void* q : c->allocs) (void)hipFree(q);
+  if (c->stage) (void)hipFree(c->stage);
   if (c->X) (void)hipFree(c->X);
   if (c->Y) (void)hipFree(c->Y);
   if (c->idx) (void)hipFree(c->idx);
@@ -1570,6 +1568,26 @@ VW_API int vw_unet_set_params(void* p, const float* in) {
 }
 
 namespace {
+/* device staging for n images, kept by the network (an allocation and a free,
+ * which waits for the device, per direction and call were a third of a
+ * five-image prediction) */
+int ensure_stage(Net* c, int n) {
+  const int64_t ne = (int64_t)n * c->N * c->N;
+  if (ne <= c->stage_cap) return VW_OK;
+  if (c->stage) (void)hipFree(c->stage);
+  c->stage = nullptr;
+  c->stage_cap = 0;
+  UC(hipMalloc(&c->stage, sizeof(float) * ne));
+  c->stage_cap = ne;
+  return VW_OK;
+}
+
+/* the caller's buffers are free on return, also after an error */
+int settled(Net* c, int rc) {
+  if (rc) (void)hipStreamSynchronize(c->st);
+  return rc;
+}
+
 int ensure_loss(Net* c, int64_t n) {
   if (n <= c->loss_cap) return VW_OK;
   if (c->loss) (void)hipFree(c->loss);
@@ -1586,16 +1604,16 @@ VW_API int vw_unet_loss_grad(void* p, const float* X, const float* Y, int32_t n,
   if (!c || !X || !Y) return VW_ERR_ARG;
   if (n < 1 || n > c->BM) return c->fail(VW_ERR_ARG, "n must be in [1, batch_max]");
   int rc;
-  if ((rc = ensure_loss(c, 1))) return rc;
+  if ((rc = ensure_loss(c, 1)) || (rc = ensure_stage(c, n))) return rc;
   rc = dispatch(c, [&](auto ops) {
     using O = decltype(ops);
     int r;
-    if ((r = O::upload(c, X, Net::X0, n)) || (r = O::upload(c, Y, Net::YT, n)) || (r = O::forward(c, n)) ||
+    if ((r = O::upload(c, X, Net::X0, n, c->stage)) || (r = O::upload(c, Y, Net::YT, n, c->stage)) || (r = O::forward(c, n)) ||
         (r = O::backward(c, n, 0)))
       return r;
     return VW_OK;
   });
-  if (rc) return rc;
+  if (rc) return settled(c, rc);
   UC(hipStreamSynchronize(c->st));
   if (loss) UC(hipMemcpy(loss, c->loss, sizeof(double), hipMemcpyDeviceToHost));
   if (grad) {
@@ -1715,16 +1733,19 @@ VW_API int vw_unet_predict(void* p, const float* X, int32_t n, float* out) {
   Net* c = as_net(p);
   if (!c || !X || !out || n < 0) return VW_ERR_ARG;
   const int64_t HH = (int64_t)c->N * c->N;
+  if (int rs = ensure_stage(c, std::min<int32_t>(c->BM, n))) return rs;
+  c->xfer.reserve(sizeof(float) * (size_t)(std::min<int32_t>(c->BM, n) * HH));
   for (int32_t b0 = 0; b0 < n; b0 += c->BM) {
     const int k = std::min(c->BM, n - b0);
     int rc = dispatch(c, [&](auto ops) {
       using O = decltype(ops);
       int r;
-      if ((r = O::upload(c, X + b0 * HH, Net::X0, k)) || (r = O::forward(c, k)) || (r = O::download(c, Net::OUT, k, out + b0 * HH)))
+      if ((r = O::upload(c, X + b0 * HH, Net::X0, k, c->stage)) || (r = O::forward(c, k)) ||
+          (r = O::download(c, Net::OUT, k, out + b0 * HH, c->stage, &c->xfer)))
         return r;
       return VW_OK;
     });
-    if (rc) return rc;
+    if (rc) return settled(c, rc);
   }
   return VW_OK;
 }
@@ -1749,12 +1770,12 @@ VW_API int vw_unet_predict_noalloc(void* p, const float* X, int32_t n, float* ou
     int rc = dispatch(c, [&](auto ops) {
       using O = decltype(ops);
       int r;
-      if ((r = O::upload(c, X + b0 * HH, Net::X0, k, false, c->scratch_dev)) || (r = O::forward(c, k)) ||
-          (r = O::download(c, Net::OUT, k, out + b0 * HH, c->scratch_dev)))
+      if ((r = O::upload(c, X + b0 * HH, Net::X0, k, c->scratch_dev)) || (r = O::forward(c, k)) ||
+          (r = O::download(c, Net::OUT, k, out + b0 * HH, c->scratch_dev, nullptr)))
         return r;
       return VW_OK;
     });
-    if (rc) return rc;
+    if (rc) return settled(c, rc);
   }
   return VW_OK;
 }
