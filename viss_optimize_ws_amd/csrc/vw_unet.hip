@@ -176,35 +176,53 @@ __global__ __launch_bounds__(256) void k_conv3_mfma(const _Float16* __restrict__
         if (tap < 9 && ob + r < cout) aw[ks] = *(const vw_h8*)(Wk + ((int64_t)(ob + r) * K + tap * cin + c0 + ci0));
       }
     }
-    __syncthreads();
     if (VS && H % 8 == 0) {
-      /* interior columns: a lane takes a channel pair and 8 pixels of one row
+      /* every load of the tile is issued before the first is stored: one
+       * memory latency a chunk instead of one per loop trip (5 or 8).
+       * interior columns: a lane takes a channel pair and 8 pixels of one row
        * (two aligned 16-byte loads) and writes each pixel's pair as one dword;
        * lanes run over the pairs first, so a write phase covers consecutive
        * dwords */
-      const int npair = cb >> 1;
-      for (int idx = threadIdx.x; idx < npair * 36; idx += 256) {
-        const int cp = idx % npair, rest = idx / npair, yy = rest >> 1, hx = rest & 1;
-        const int gy = ty0 + yy - 1, gx = tx0 + 8 * hx;
-        vw_h8 v0 = {}, v1 = {};
-        if (gy >= 0 && gy < H && gx < H) {
-          const _Float16* s0 = in + ((int64_t)n * cin + c0 + 2 * cp) * HH + (int64_t)gy * H + gx;
-          v0 = *(const vw_h8*)s0;
-          v1 = *(const vw_h8*)(s0 + HH);
-        }
-        _Float16* d = tile + (yy * 18 + 1 + 8 * hx) * LR + 2 * cp;
+      constexpr int NP = CB / 2, NI = (NP * 36 + 255) / 256, NH = (CB * 36 + 255) / 256;
+      const _Float16* src = in + ((int64_t)n * cin + c0) * HH; /* CB planes: offsets below fit 32 bits */
+      vw_h8 v0[NI], v1[NI];
+      _Float16 hv[NH]; /* halo columns tx0 - 1 and tx0 + 16 */
 #pragma unroll
-        for (int i = 0; i < 8; ++i) *(vw_h2*)(d + i * LR) = vw_h2{v0[i], v1[i]};
+      for (int e = 0; e < NI; ++e) {
+        const int idx = threadIdx.x + 256 * e;
+        const int cp = idx % NP, rest = idx / NP, gy = ty0 + (rest >> 1) - 1, gx = tx0 + 8 * (rest & 1);
+        const bool on = idx < NP * 36 && gy >= 0 && gy < H && gx < H;
+        const int off = on ? 2 * cp * (int)HH + gy * H + gx : 0;
+        v0[e] = *(const vw_h8*)(src + off);
+        v1[e] = *(const vw_h8*)(src + off + (int)HH);
+        if (!on) v0[e] = v1[e] = vw_h8{};
       }
-      /* halo columns tx0 - 1 and tx0 + 16 */
-      for (int idx = threadIdx.x; idx < cb * 36; idx += 256) {
-        const int c = idx % cb, rest = idx / cb, yy = rest >> 1, side = rest & 1;
-        const int gy = ty0 + yy - 1, gx = side ? tx0 + 16 : tx0 - 1;
-        _Float16 v = (_Float16)0.f;
-        if (gy >= 0 && gy < H && gx >= 0 && gx < H) v = in[((int64_t)n * cin + c0 + c) * HH + (int64_t)gy * H + gx];
-        tile[(yy * 18 + (side ? 17 : 0)) * LR + c] = v;
+#pragma unroll
+      for (int e = 0; e < NH; ++e) {
+        const int idx = threadIdx.x + 256 * e;
+        const int c = idx % CB, rest = idx / CB, gy = ty0 + (rest >> 1) - 1, gx = rest & 1 ? tx0 + 16 : tx0 - 1;
+        const bool on = idx < CB * 36 && gy >= 0 && gy < H && gx >= 0 && gx < H;
+        const _Float16 v = src[on ? c * (int)HH + gy * H + gx : 0];
+        hv[e] = on ? v : (_Float16)0.f;
+      }
+      __syncthreads(); /* the last chunk's reads of the tile are done */
+#pragma unroll
+      for (int e = 0; e < NI; ++e) {
+        const int idx = threadIdx.x + 256 * e;
+        const int cp = idx % NP, rest = idx / NP;
+        _Float16* d = tile + ((rest >> 1) * 18 + 1 + 8 * (rest & 1)) * LR + 2 * cp;
+        if (idx < NP * 36)
+#pragma unroll
+          for (int i = 0; i < 8; ++i) *(vw_h2*)(d + i * LR) = vw_h2{v0[e][i], v1[e][i]};
+      }
+#pragma unroll
+      for (int e = 0; e < NH; ++e) {
+        const int idx = threadIdx.x + 256 * e;
+        const int c = idx % CB, rest = idx / CB;
+        if (idx < CB * 36) tile[((rest >> 1) * 18 + (rest & 1 ? 17 : 0)) * LR + c] = hv[e];
       }
     } else {
+      __syncthreads();
       for (int idx = threadIdx.x; idx < 324 * cb; idx += 256) {
         const int c = idx / 324, q = idx - c * 324, yy = q / 18, xx = q - yy * 18;
         const int gy = ty0 + yy - 1, gx = tx0 + xx - 1;
