@@ -52,6 +52,11 @@ struct Ctx {
   int64_t ngp = 0, ngt = 0;
   std::vector<int64_t> gidx;
   int64_t max_nh = 0, nh_pad = 0, nchunk_max = 1;
+  /* a whole step's launches: runs (first, count) of the schedule's segments, and
+   * the epochs of the longest (the buffers'; max_tlen is the longest segment) */
+  std::vector<std::pair<int, int>> runs;
+  int buf_tlen = 0;
+  VwMerge mg{}; /* the segments in the segment buffers */
   /* device */
   hipStream_t st = nullptr;
   /* streams: st carries the segment geometry, Viss and conjugate fill; stB
@@ -313,6 +318,86 @@ bool fact_auto_plain(const vw_config* cfg, double lambda) {
 }
 
 /* ---------------- plan ---------------- */
+int64_t class_budget(const Ctx* c) {
+  return c->cfg.class_budget_bytes > 0 ? c->cfg.class_budget_bytes : (int64_t)2 << 30;
+}
+
+int run_tlen(const Ctx* c, int r) {
+  int t = 0;
+  for (int k = 0; k < c->runs[r].second; ++k) t += c->seg_tlen[c->runs[r].first + k];
+  return t;
+}
+
+/* the groups' positions of count segments from first, and their rows */
+VwMerge merge_of(const Ctx* c, const int32_t* tlen, int count) {
+  const int mul = c->cfg.recon_mode == VW_RECON_FULL ? 2 : 1;
+  VwMerge m{};
+  m.n = count;
+  for (int k = 0; k < count; ++k) {
+    const int nh = tlen[k] * c->P;
+    m.row0[k + 1] = m.row0[k] + nh;
+    /* a lone segment's positions are its rows */
+    m.base[k + 1] = count > 1 ? m.base[k] + (mul * nh + 64) / 64 * 64 : mul * nh;
+  }
+  return m;
+}
+
+void size_buffers(Ctx* c) {
+  c->buf_tlen = c->max_tlen;
+  int64_t nq = 2 * (int64_t)c->max_tlen * c->P;
+  for (int r = 0; r < (int)c->runs.size(); ++r) {
+    c->buf_tlen = std::max(c->buf_tlen, run_tlen(c, r));
+    if (c->runs[r].second > 1) {
+      const VwMerge m = merge_of(c, &c->seg_tlen[c->runs[r].first], c->runs[r].second);
+      nq = std::max<int64_t>(nq, m.base[m.n]);
+    }
+  }
+  c->max_nh = (int64_t)c->buf_tlen * c->P;
+  c->nh_pad = (c->max_nh + 63) / 64 * 64;
+  c->nq_pad = (std::max(nq, 2 * c->max_nh) + 63) / 64 * 64;
+}
+
+/* A short segment's kernels take a few microseconds each, and a whole step was
+ * bound by the host enqueueing nine of them, and the stream waits, for every
+ * segment (70 us a segment, 290 of a 350 us run of four at Nside 32, 8 antennas).
+ * Consecutive short segments of a one-sky step share their launches: one
+ * geometry and Viss over all their rows, a workgroup each for the grouping, and
+ * recon ranges that each lie in one segment: that run 350 -> 280 us, the call 497
+ * -> 405; three ragged segments of 715 rows 705 -> 661.  Short: the groups fit
+ * k_group_one; runs end at VW_MERGE_ROWS rows, from where a launch fills the chip by itself
+ * and the overlap of one run's recon with the next one's Viss is worth more.
+ * The schedule's last segment stays alone: its rows and groups are what the
+ * stage calls find after a step. */
+#define VW_MERGE_ROWS 4096
+void plan_runs(Ctx* c) {
+  const bool may = !c->batch && !c->generic && c->cfg.blockage;
+  const int mul = c->cfg.recon_mode == VW_RECON_FULL ? 2 : 1;
+  c->runs.clear();
+  int64_t rows = 0;
+  for (int k = 0; k < c->segs; ++k) {
+    const int64_t nr = (int64_t)mul * c->seg_tlen[k] * c->P;
+    const bool short_ = may && nr <= VW_GROUP_ONE_MAX && k + 1 < c->segs;
+    const bool joins = short_ && rows > 0 && rows + nr <= VW_MERGE_ROWS && c->runs.back().second < VW_MERGE_MAX &&
+                       c->seg_t0[k] == c->seg_t0[k - 1] + c->seg_tlen[k - 1];
+    if (joins) {
+      ++c->runs.back().second;
+      rows += nr;
+    } else {
+      c->runs.push_back({k, 1});
+      rows = short_ ? nr : 0;
+    }
+  }
+  size_buffers(c);
+  /* with a class budget that would cut the longer rows into tile passes the
+   * segments stay alone */
+  const int64_t tiles = std::max(c->ntile, c->ngt);
+  if (tiles * std::max(c->nh_pad, c->nq_pad) > class_budget(c)) {
+    c->runs.clear();
+    for (int k = 0; k < c->segs; ++k) c->runs.push_back({k, 1});
+    size_buffers(c);
+  }
+}
+
 int make_plan(Ctx* c, const vw_config* cfg) {
   c->cfg = *cfg;
   c->cfg.seg_tlen = nullptr;
@@ -417,9 +502,7 @@ int make_plan(Ctx* c, const vw_config* cfg) {
   }
   c->ngp = (int64_t)c->gidx.size();
   c->ngt = (c->ngp + c->TP - 1) / c->TP;
-  c->max_nh = (int64_t)c->max_tlen * c->P;
-  c->nh_pad = (c->max_nh + 63) / 64 * 64;
-  c->nq_pad = (2 * c->max_nh + 63) / 64 * 64;
+  size_buffers(c);
   /* occ_mode 1 and 2 read one member per group: the representative kernel,
    * with the finite-value filter of the member sets except for the uv-mirror
    * occ_mode 2 form (recon_seg_blockage_half_rep); occ_mode 0 averages every
@@ -439,6 +522,7 @@ int make_plan(Ctx* c, const vw_config* cfg) {
     c->nsg = (b16 + c->nbw - 1) / c->nbw;
     c->nsky_pad = c->nsg * c->nbw * 16;
   }
+  plan_runs(c);
   if (c->max_nh > (int64_t)INT32_MAX / 4) return c->fail(VW_ERR_RANGE, "segment too long for 32-bit row indices");
   return VW_OK;
 }
@@ -550,10 +634,6 @@ ReconShape recon_shape(int64_t npts, int64_t nq = INT64_MAX) {
    * 32, 28 of them with work) */
   r.nchunk = std::min(r.nchunk, std::max<int64_t>(1, nq / 16 + (nq % 16 != 0)));
   return r;
-}
-
-int64_t class_budget(const Ctx* c) {
-  return c->cfg.class_budget_bytes > 0 ? c->cfg.class_budget_bytes : (int64_t)2 << 30;
 }
 
 /* output tiles per recon pass: as many as the class scratch holds */
@@ -755,7 +835,7 @@ int enq_reset_fill(Ctx* c) {
   add(c->d_Wacc, c->npix);
   add(c->d_Gacc, 2 * c->ngp * c->nsky);
   add(c->d_GWacc, c->ngp);
-  add(c->d_info, (int64_t)(sizeof(DevInfo) / 4));
+  add(c->d_info, (int64_t)(VW_MERGE_MAX * sizeof(DevInfo) / 4));
   if (c->sky_sched) {
     add(c->d_Wsky, c->npix * c->nsky);
     add(c->d_GWsky, c->ngp * c->nsky);
@@ -837,26 +917,28 @@ int create_device(Ctx* c) {
   /* partial buffers fit the largest pass shape: a full pass and the last one */
   int64_t nch = 1;
   const int64_t vlast = c->ntile - (c->ntile - 1) / c->vtpp * c->vtpp;
-  for (int k = 0; k < c->segs; ++k)
-    for (int64_t nt : {c->vtpp, vlast}) nch = std::max(nch, viss_shape(c, (int64_t)c->seg_tlen[k] * c->P, nt).nchunk);
+  std::vector<int> tlens(c->seg_tlen.begin(), c->seg_tlen.end());
+  for (int r = 0; r < (int)c->runs.size(); ++r) tlens.push_back(run_tlen(c, r));
+  for (int tl : tlens)
+    for (int64_t nt : {c->vtpp, vlast}) nch = std::max(nch, viss_shape(c, (int64_t)tl * c->P, nt).nchunk);
   c->nchunk_max = nch;
   if (c->vfact) {
     int64_t fp = 1;
-    for (int k = 0; k < c->segs; ++k)
+    for (int tl : tlens)
       for (int64_t nt : {c->vtpp, vlast})
-        fp = std::max(fp, (int64_t)c->seg_tlen[k] * viss_fshape(c, c->seg_tlen[k], nt).nchunk *
+        fp = std::max(fp, (int64_t)tl * viss_fshape(c, tl, nt).nchunk *
                               vissf_blocks(vissf_groups(c->A)) * 256);
     c->fpart_cap = fp;
-    if ((rc = dalloc(c, &c->d_fpart, (size_t)fp)) || (rc = dalloc(c, &c->d_aph, (size_t)c->max_tlen * c->A)) ||
-        (rc = dalloc(c, &c->d_aphl, (size_t)c->max_tlen * c->A)) ||
-        (rc = dalloc(c, &c->d_fesum, (size_t)c->max_tlen * vissf_blocks(vissf_groups(c->A)) * 256)))
+    if ((rc = dalloc(c, &c->d_fpart, (size_t)fp)) || (rc = dalloc(c, &c->d_aph, (size_t)c->buf_tlen * c->A)) ||
+        (rc = dalloc(c, &c->d_aphl, (size_t)c->buf_tlen * c->A)) ||
+        (rc = dalloc(c, &c->d_fesum, (size_t)c->buf_tlen * vissf_blocks(vissf_groups(c->A)) * 256)))
       return rc;
   }
   for (int b = 0; b < 2; ++b) {
     Ctx::SegSet& g = c->seg[b];
     const size_t msk = mh * (size_t)c->nsky; /* batched: [nsky][nh] */
     if ((rc = dalloc(c, &g.rows, mh)) || (rc = dalloc(c, &g.rowt, (size_t)c->nh_pad)) ||
-        (rc = dalloc(c, &g.ant8, 8 * (size_t)c->max_tlen * c->A)) || (rc = dalloc(c, &g.vraw, msk)) ||
+        (rc = dalloc(c, &g.ant8, 8 * (size_t)c->buf_tlen * c->A)) || (rc = dalloc(c, &g.vraw, msk)) ||
         (rc = dalloc(c, &g.vh, msk)) || (rc = dalloc(c, &g.vfull, 2 * msk)))
       return rc;
   }
@@ -864,9 +946,9 @@ int create_device(Ctx* c) {
   if ((rc = dalloc(c, &c->d_cls, (size_t)c->cls_cap)) || (rc = dalloc(c, &c->d_cls_v, (size_t)c->cls_cap)) ||
       (rc = dalloc(c, &c->d_part, (size_t)nch * c->nh_pad)) ||
       (rc = dalloc(c, &c->d_keys, 2 * mh)) || (rc = dalloc(c, &c->d_keys_sorted, 2 * mh)) ||
-      (rc = dalloc(c, &c->d_gkeys, 2 * mh + 1)) || (rc = dalloc(c, &c->d_idx_sorted, 2 * mh)) ||
-      (rc = dalloc(c, &c->d_goff, 2 * mh + 2)) || (rc = dalloc(c, &c->d_rank, 2 * mh)) ||
-      (rc = dalloc(c, &c->d_info, 1)) || (rc = dalloc(c, &c->d_sums, 5 * 256)) ||
+      (rc = dalloc(c, &c->d_gkeys, (size_t)c->nq_pad + 1)) || (rc = dalloc(c, &c->d_idx_sorted, (size_t)c->nq_pad)) ||
+      (rc = dalloc(c, &c->d_goff, (size_t)c->nq_pad + 2)) || (rc = dalloc(c, &c->d_rank, 2 * mh)) ||
+      (rc = dalloc(c, &c->d_info, VW_MERGE_MAX)) || (rc = dalloc(c, &c->d_sums, 5 * 256)) ||
       (rc = dalloc(c, &c->d_out, (size_t)c->npix * c->nsky)) || (rc = dalloc(c, &c->d_wout, (size_t)c->npix)) ||
       (rc = dalloc(c, &c->d_iout, (size_t)std::max<int64_t>(1, (int64_t)c->cfg.img_n * c->cfg.img_n) * c->nsky)) ||
       (rc = dalloc(c, &c->d_iwout, (size_t)std::max<int64_t>(1, (int64_t)c->cfg.img_n * c->cfg.img_n))))
@@ -883,7 +965,7 @@ int create_device(Ctx* c) {
       if (npts <= 0) continue;
       const int64_t pp = recon_pass_tiles(c, nta, kind_w) * c->TP;
       const int64_t last = npts - (npts - 1) / pp * pp;
-      for (int64_t n : {std::min(npts, pp), last}) rp = std::max(rp, recon_shape(n).nchunk * n);
+      for (int64_t n : {std::min(npts, pp), last}) rp = std::max(rp, (recon_shape(n).nchunk + VW_MERGE_MAX) * n);
     }
     c->rpart_cap = rp;
     if ((rc = dalloc(c, &c->d_rpart, (size_t)rp)) || (rc = dalloc(c, &c->d_rwpart, (size_t)rp))) return rc;
@@ -900,7 +982,7 @@ int create_device(Ctx* c) {
       c->rshist_cap = 256 * ((2 * c->max_nh + VW_RS_BLOCK - 1) / VW_RS_BLOCK);
       if ((rc = dalloc(c, &c->d_rshist[1], (size_t)c->rshist_cap + 256))) return rc; /* + digit totals */
     }
-    c->nfr_pad = ((int64_t)c->max_tlen * c->A + 63) / 64 * 64;
+    c->nfr_pad = ((int64_t)c->buf_tlen * c->A + 63) / 64 * 64;
     c->bits_cap = maxnt * c->nfr_pad;
     if ((rc = dalloc(c, &c->d_bits, (size_t)c->bits_cap)) || (rc = dalloc(c, &c->d_bits_v, (size_t)c->bits_cap)))
       return rc;
@@ -919,9 +1001,9 @@ int create_device(Ctx* c) {
 }
 
 /* ---------------- stages (enqueue only) ---------------- */
-int enq_gen(Ctx* c, int t0, int tlen) {
-  if (t0 < 0 || tlen <= 0 || tlen > c->max_tlen || (int64_t)t0 + tlen > c->T)
-    return c->fail(VW_ERR_ARG, "segment [t0, t0+tlen) out of range");
+/* epochs [t0, t0 + tlen) into the segment buffers, as the segments mg */
+int enq_gen_rows(Ctx* c, int t0, int tlen, const VwMerge& mg) {
+  c->mg = mg;
   c->t0 = t0;
   c->tlen = tlen;
   c->nh = (int64_t)tlen * c->P;
@@ -939,6 +1021,13 @@ int enq_gen(Ctx* c, int t0, int tlen) {
   c->have_seg = true;
   c->have_viss = c->have_conj = c->have_groups = false;
   return VW_OK;
+}
+
+int enq_gen(Ctx* c, int t0, int tlen) {
+  if (t0 < 0 || tlen <= 0 || tlen > c->max_tlen || (int64_t)t0 + tlen > c->T)
+    return c->fail(VW_ERR_ARG, "segment [t0, t0+tlen) out of range");
+  const int32_t tl = tlen;
+  return enq_gen_rows(c, t0, tlen, merge_of(c, &tl, 1));
 }
 
 /* row classes of nt tiles into cls ([nt][nh_pad] bytes) from their cone bits */
@@ -991,7 +1080,7 @@ int enq_group_masks(Ctx* c, const ReconSets& sets, uint8_t* const* bits, uint64_
   const int64_t nfr = (int64_t)c->tlen * c->A;
   const unsigned nb = (unsigned)(sets.s[0].nt + sets.s[1].nt);
   if (c->nfr_pad <= VW_GCLS_LDS_MAX) {
-    k_group_mask<true><<<nb, 256, (size_t)c->nfr_pad, c->stB>>>(sets, c->d_ant8, nfr, c->nfr_pad, c->gs.gia, c->gs.gib,
+    k_group_mask<true><<<nb, 256, (size_t)c->nfr_pad, c->stB>>>(c->mg, sets, c->d_ant8, nfr, c->nfr_pad, c->gs.gia, c->gs.gib,
                                                                  c->d_info, c->nq_pad, ts);
     KC();
     return VW_OK;
@@ -1004,7 +1093,7 @@ int enq_group_masks(Ctx* c, const ReconSets& sets, uint8_t* const* bits, uint64_
                                                                   c->nfr_pad, bits[i], nullptr);
     KC();
   }
-  k_group_mask<false><<<nb, 256, 0, c->stB>>>(sets, c->d_ant8, nfr, c->nfr_pad, c->gs.gia, c->gs.gib, c->d_info,
+  k_group_mask<false><<<nb, 256, 0, c->stB>>>(c->mg, sets, c->d_ant8, nfr, c->nfr_pad, c->gs.gia, c->gs.gib, c->d_info,
                                               c->nq_pad, ts);
   KC();
   return VW_OK;
@@ -1229,6 +1318,14 @@ int enq_conj(Ctx* c) {
 int enq_group_keys(Ctx* c) {
   bool full = c->cfg.recon_mode == VW_RECON_FULL;
   int64_t nr = full ? 2 * c->nh : c->nh;
+  if (c->mg.n > 1 || nr <= VW_GROUP_ONE_MAX) {
+    uint64_t* ts = new_ts(c);
+    k_group_one<<<c->mg.n, 1024, 0, c->stB>>>(c->mg, c->d_rows, c->P, full ? 1 : 0, c->bl_max, c->lambda,
+                                              c->cfg.blockage, c->d_idx_sorted, c->d_gkeys, c->d_goff, c->d_info, ts);
+    KC();
+    add_bracket(c, ST_GROUP, ts, ts);
+    return VW_OK;
+  }
   const bool rsort = nr > VW_RANK_MAX;
   uint64_t *first = new_ts(c), *last = new_ts(c);
   k_segsums<<<4, 64, 0, c->stB>>>(c->d_rows, c->nh, c->P, c->d_sums, first);
@@ -1266,9 +1363,8 @@ int enq_group_keys(Ctx* c) {
  * antenna frames) of the current groups */
 int enq_group_data(Ctx* c, const double2* vh, uint64_t** ts_out = nullptr) {
   bool full = c->cfg.recon_mode == VW_RECON_FULL;
-  int64_t nr = full ? 2 * c->nh : c->nh;
   uint64_t* ts = new_ts(c);
-  k_group_data<<<blocks_for(nr), 256, 0, c->stB>>>(c->d_gkeys, c->d_goff, c->d_idx_sorted, vh, c->d_rows,
+  k_group_data<<<blocks_for(c->mg.base[c->mg.n]), 256, 0, c->stB>>>(c->mg, c->d_gkeys, c->d_goff, c->d_idx_sorted, vh, c->d_rows,
                                                   c->d_ant8, c->P, full ? 1 : 0, c->cfg.blockage, c->cfg.occ_mode,
                                                   c->cfg.precision == VW_PREC_PLAIN && c->generic ? VW_TAB_SCALE : 1.0,
                                                   c->d_info,
@@ -1394,7 +1490,17 @@ int enq_recon_one(Ctx* c, double* const (&acc)[2], uint32_t* const (&wacc)[2], c
       S.npts = std::min(S.nt * c->TP, (i ? c->ngp : c->npix) - S.pt0);
       S.cls = (uint32_t*)(i ? c->d_cls2 : c->d_cls);
       S.bits = bits[i];
-      const ReconShape rs = recon_shape(S.npts, full ? 2 * c->nh : c->nh);
+      const int64_t nr = full ? 2 * c->nh : c->nh;
+      ReconShape rs = recon_shape(S.npts, nr);
+      if (c->mg.n == 1) {
+        S.cst[1] = (int)rs.nchunk;
+      } else { /* by the segments' rows, at least 16 groups a range */
+        for (int k = 0; k < c->mg.n; ++k) {
+          const int64_t rk = (int64_t)(c->mg.row0[k + 1] - c->mg.row0[k]) * (full ? 2 : 1);
+          S.cst[k + 1] = S.cst[k] + (int)std::max<int64_t>(1, std::min((rk + 15) / 16, rs.nchunk * rk / nr));
+        }
+        rs.nchunk = S.cst[c->mg.n];
+      }
       if (rs.nchunk * S.npts > c->rpart_cap) return c->fail(VW_ERR_RANGE, "internal: recon partial buffer too small");
       S.nchunk = rs.nchunk;
       S.pwaves = rs.pwaves;
@@ -1418,6 +1524,7 @@ int enq_recon_one(Ctx* c, double* const (&acc)[2], uint32_t* const (&wacc)[2], c
           return rc;
       }
     }
+    a.mg = c->mg;
     a.tab = c->d_tab;
     a.TP = c->TP;
     a.nq_pad = c->nq_pad;
@@ -1497,8 +1604,9 @@ int enq_recon(Ctx* c, bool keys_done = false) {
 int enq_step(Ctx* c) {
   int rc;
   if (!c->sky_sched) {
-    for (int s = 0; s < c->segs; ++s) {
-      if ((rc = enq_gen(c, c->seg_t0[s], c->seg_tlen[s]))) return rc;
+    for (int r = 0; r < (int)c->runs.size(); ++r) {
+      const int s = c->runs[r].first;
+      if ((rc = enq_gen_rows(c, c->seg_t0[s], run_tlen(c, r), merge_of(c, &c->seg_tlen[s], c->runs[r].second)))) return rc;
       /* the groups' keys and order need the rows only: beside the Viss */
       HC(hipEventRecord(c->ev_gen, c->st));
       HC(hipStreamWaitEvent(c->stB, c->ev_gen, 0));

@@ -49,6 +49,16 @@ struct DevInfo {
   int32_t pad;
 };
 
+/* The segments that a launch of the one-sky step covers: one, or a run of short
+ * ones.  Segment s has half rows [row0[s], row0[s + 1]) of the segment buffers
+ * and its groups at positions base[s] + q, base a multiple of 64 with room for
+ * one entry more than the segment has rows; its DevInfo is entry s. */
+#define VW_MERGE_MAX 16
+struct VwMerge {
+  int n;
+  int row0[VW_MERGE_MAX + 1], base[VW_MERGE_MAX + 1];
+};
+
 #define VW_FULLMASK 0xffffffffffffffffULL
 
 __device__ __forceinline__ int vw_rfl(int x) { return __builtin_amdgcn_readfirstlane(x); }
@@ -1356,10 +1366,8 @@ __device__ __forceinline__ int vw_polar_ok(const vw_segparams& sp) {
  * one workgroup with a 64-bit division and a load waited for per row took 86 us
  * for 31,744 half rows. */
 #define VW_SEG_BATCH 16
-__global__ __launch_bounds__(64) void k_segsums(const RowRec* __restrict__ rows, int64_t nh, int P,
-                                                double* __restrict__ sums, uint64_t* __restrict__ ts) {
-  vw_ts_begin(ts);
-  const int t = blockIdx.x * 64 + threadIdx.x;
+__device__ __forceinline__ void vw_segsum_partial(const RowRec* __restrict__ rows, int64_t nh, int P, int t,
+                                                  double* __restrict__ sums) {
   const int64_t n = 2 * nh;
   double a0 = 0.0, a1 = 0.0, a2 = 0.0, a3 = 0.0, a4 = 0.0;
   const int64_t gstep = (int64_t)(256 / (2 * P)) * P; /* full row i -> i + 256: epochs (as half rows) and pairs */
@@ -1387,6 +1395,11 @@ __global__ __launch_bounds__(64) void k_segsums(const RowRec* __restrict__ rows,
       }
   }
   sums[t] = a0; sums[256 + t] = a1; sums[512 + t] = a2; sums[768 + t] = a3; sums[1024 + t] = a4;
+}
+__global__ __launch_bounds__(64) void k_segsums(const RowRec* __restrict__ rows, int64_t nh, int P,
+                                                double* __restrict__ sums, uint64_t* __restrict__ ts) {
+  vw_ts_begin(ts);
+  vw_segsum_partial(rows, nh, P, blockIdx.x * 64 + threadIdx.x, sums);
 }
 
 /* mode row -> (half row, conjugate flag) */
@@ -1537,6 +1550,107 @@ __global__ __launch_bounds__(1024) void k_groups(const int64_t* __restrict__ ks,
   vw_ts_end(ts);
 }
 
+/* The whole grouping of short segments, one workgroup each: the w-plane sums and
+ * parameters as k_segsums and k_keys compute them, the rows' keys, their stable
+ * order (a bitonic sort of the distinct (key, row) pairs, one a thread, strides
+ * below 64 by lane exchange, the rest through LDS) and the runs.  For up to
+ * 1,024 rows; with four rows a thread, for 3,840, the one workgroup waited so
+ * long for a CU beside the recon kernel that a 16-segment run at Nside 128 took
+ * 9.3 instead of 9.0 ms. */
+#define VW_GROUP_ONE_MAX 1024
+__global__ __launch_bounds__(1024) void k_group_one(VwMerge mg, const RowRec* __restrict__ rows, int P, int full,
+                                                    double bl_max, double lambda, int blockage,
+                                                    int32_t* __restrict__ idx_sorted, int64_t* __restrict__ gkeys,
+                                                    int32_t* __restrict__ goff, DevInfo* __restrict__ info,
+                                                    uint64_t* __restrict__ ts) {
+  vw_ts_begin(ts);
+  constexpr int N = 1024;
+  __shared__ double sums[5 * 256];
+  __shared__ vw_segparams ssp;
+  __shared__ int64_t sk[N];
+  __shared__ int32_t si[N];
+  __shared__ int32_t wtot[16];
+  const int t = threadIdx.x, lane = t & 63, wave = t >> 6, sg = blockIdx.x;
+  const int nh = mg.row0[sg + 1] - mg.row0[sg], nr = full ? 2 * nh : nh; /* <= VW_GROUP_ONE_MAX */
+  rows += mg.row0[sg];
+  idx_sorted += mg.base[sg];
+  gkeys += mg.base[sg];
+  goff += mg.base[sg];
+  info += sg;
+  if (t < 256) vw_segsum_partial(rows, nh, P, t, sums);
+  __syncthreads();
+  for (int st = 128; st > 0; st >>= 1) {
+    /* the five sums' trees side by side */
+    const int k = t >> 8, j = t & 255;
+    if (j < st) {
+      sums[256 * k + j] = sums[256 * k + j] + sums[256 * k + j + st];
+      if (k == 0) sums[1024 + j] = sums[1024 + j] + sums[1024 + j + st];
+    }
+    __syncthreads();
+  }
+  if (t == 0) {
+    vw_segparams_from_sums(sums[0], sums[256], sums[512], sums[768], sums[1024], bl_max, lambda, &ssp);
+    info->sp = ssp;
+    info->polar = vw_polar_ok(ssp);
+  }
+  __syncthreads();
+  const vw_segparams sp = ssp;
+  bool neg;
+  const int64_t h = vw_row_half(t < nr ? t : 0, P, full != 0, &neg);
+  const double sgn = neg ? -1.0 : 1.0;
+  const int64_t k0 = vw_grid_key(sgn * rows[h].u, sgn * rows[h].v, &sp, full ? 0 : 1);
+  int64_t key = t < nr ? k0 : INT64_MAX; /* keys are non-negative and below it */
+  int32_t idx = t;
+  for (int k = 2; k <= N; k <<= 1)
+    for (int j = k >> 1; j > 0; j >>= 1) {
+      int64_t kb;
+      int32_t ib;
+      if (j >= 64) {
+        __syncthreads();
+        sk[t] = key;
+        si[t] = idx;
+        __syncthreads();
+        kb = sk[t ^ j];
+        ib = si[t ^ j];
+      } else {
+        kb = __shfl_xor(key, j, 64);
+        ib = __shfl_xor(idx, j, 64);
+      }
+      const bool less = kb < key || (kb == key && ib < idx);
+      if (less == (((t & k) == 0) == ((t & j) == 0))) {
+        key = kb;
+        idx = ib;
+      }
+    }
+  __syncthreads();
+  sk[t] = key;
+  if (t < nr) idx_sorted[t] = idx;
+  __syncthreads();
+  const bool f = t < nr && (t == 0 || key != sk[t > 0 ? t - 1 : 0]);
+  const uint64_t b = __ballot(f);
+  if (lane == 0) wtot[wave] = __popcll(b);
+  __syncthreads();
+  int32_t before = 0, all = 0;
+#pragma unroll
+  for (int w = 0; w < 16; ++w) {
+    const int32_t x = wtot[w];
+    before += w < wave ? x : 0;
+    all += x;
+  }
+  if (f) {
+    const int32_t g = before + __popcll(b & ((1ull << lane) - 1));
+    gkeys[g] = key;
+    goff[g] = t;
+  }
+  if (t == 0) {
+    goff[all] = nr;
+    info->nuniq = all;
+    info->first_nz = (all > 0 && key == 0) ? 1 : 0;
+    if (!blockage) info->wtotal += all; /* blockage 0 takes one segment a launch */
+  }
+  vw_ts_end(ts);
+}
+
 /* Occlusion in FP32, exact where it decides.  d = s . u - cosphi with every
  * operand rounded to FP32 is within 4e-7 of the FP64 test's difference
  * (operands 2^-24 relative each, |s| = |u| = 1, three roundings of sums below
@@ -1578,14 +1692,21 @@ struct GroupSoA {
   int32_t *gia, *gib, *grep;
 };
 
-__global__ void k_group_data(const int64_t* __restrict__ gkeys, const int32_t* __restrict__ goff,
+__global__ void k_group_data(VwMerge mg, const int64_t* __restrict__ gkeys, const int32_t* __restrict__ goff,
                              const int32_t* __restrict__ idx_sorted, const double2* __restrict__ vh,
                              const RowRec* __restrict__ rows, const double* __restrict__ ant8, int P, int full,
                              int blockage, int occ_mode, double uv_scale,
                              const DevInfo* __restrict__ info, GroupSoA g, uint64_t* __restrict__ ts) {
   vw_ts_begin(ts);
   int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (q >= info->nuniq) {
+  int base = 0, row0 = 0;
+  for (int k = 1; k < mg.n; ++k)
+    if (q >= mg.base[k]) {
+      base = mg.base[k];
+      row0 = mg.row0[k];
+      ++info;
+    }
+  if (q - base >= info->nuniq) {
     vw_ts_end(ts); /* the grid covers the rows: the last workgroup often holds no group */
     return;
   }
@@ -1594,6 +1715,9 @@ __global__ void k_group_data(const int64_t* __restrict__ gkeys, const int32_t* _
   int32_t s0 = goff[q], s1 = goff[q + 1];
   double ugu = 0.0, vgu = 0.0;
   if (key != 0) vw_key_uv(key, &sp, &ugu, &vgu);
+  idx_sorted += base;
+  rows += row0;
+  vh += row0;
   bool neg;
   /* the one member a single-representative rule reads: occ_mode 1 the
    * first of the sorted run, occ_mode 2 the median (viss_recon_kernel.cuh:
@@ -1654,6 +1778,7 @@ struct ReconSet {
                        * kinds), [nt][nh_pad] row class bytes (generic kind)     */
   const uint8_t* bits; /* [nt][nfr_pad] cone bits (long frame rows)               */
   int64_t nchunk;     /* group ranges per point block                            */
+  int cst[VW_MERGE_MAX + 1]; /* of them, segment s has [cst[s], cst[s + 1])      */
   int64_t pwaves;     /* point blocks (waves) per group range                    */
   int64_t nblk;       /* workgroups of the recon kernel                          */
   double* part;       /* [nchunk][npts]                                          */
@@ -1675,7 +1800,7 @@ struct ReconSets {
  * before the gathers), and writes the masks of ballots.  Words of entries
  * below nuniq rounded up to 64 are written: the recon reads no others. */
 template <bool TILE>
-__global__ __launch_bounds__(256) void k_group_mask(ReconSets sets, const double* __restrict__ ant8, int64_t nfr,
+__global__ __launch_bounds__(256) void k_group_mask(VwMerge mg, ReconSets sets, const double* __restrict__ ant8, int64_t nfr,
                                                     int64_t nfr_pad, const int32_t* __restrict__ ia,
                                                     const int32_t* __restrict__ ib, const DevInfo* __restrict__ info,
                                                     int64_t nq_pad, uint64_t* __restrict__ ts) {
@@ -1684,8 +1809,6 @@ __global__ __launch_bounds__(256) void k_group_mask(ReconSets sets, const double
   const int si = (int)blockIdx.x >= (int)sets.s[0].nt;
   const ReconSet& S = sets.s[si];
   const int64_t tr = blockIdx.x - (si ? sets.s[0].nt : 0);
-  const int nu = vw_rfl((int)info->nuniq), q0 = vw_rfl((int)info->first_nz);
-  const int qend = (nu + 63) / 64 * 64; /* <= nq_pad, a multiple of 64 */
   const uint8_t* b = TILE ? (const uint8_t*)sbits : S.bits + tr * nfr_pad;
   if (TILE) {
     vw_tile_bits_lds((uint8_t*)sbits, S.cone, S.ntile, S.tile0 + tr, ant8, nfr);
@@ -1693,24 +1816,28 @@ __global__ __launch_bounds__(256) void k_group_mask(ReconSets sets, const double
   }
   const int wave = vw_rfl((int)(threadIdx.x >> 6)), lane = threadIdx.x & 63;
   uint32_t* out = S.cls + tr * (nq_pad >> 4);
-  for (int j0 = 256 * wave; j0 < qend; j0 += 1024) {
-    int av[4], bv[4];
+  for (int sg = 0; sg < mg.n; ++sg) {
+    const int base = mg.base[sg], nu = base + vw_rfl((int)info[sg].nuniq), q0 = base + vw_rfl((int)info[sg].first_nz);
+    const int qend = (nu + 63) / 64 * 64; /* <= nq_pad, a multiple of 64 */
+    for (int j0 = base + 256 * wave; j0 < qend; j0 += 1024) {
+      int av[4], bv[4];
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      const int q = j0 + 64 * e + lane;
-      /* indices past nuniq are not frames: frame 0 stands in for them */
-      av[e] = q < nu ? ia[q] : 0;
-      bv[e] = q < nu ? ib[q] : 0;
-    }
+      for (int e = 0; e < 4; ++e) {
+        const int q = j0 + 64 * e + lane;
+        /* indices past nuniq are not frames: frame 0 stands in for them */
+        av[e] = q < nu ? ia[q] : 0;
+        bv[e] = q < nu ? ib[q] : 0;
+      }
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      const int q = j0 + 64 * e + lane;
-      const bool in = q >= q0 && q < nu;
-      const int c = vw_pair_class(b[av[e]], b[bv[e]]);
-      const uint64_t v = __ballot(in && c == VW_CLS_VISIBLE), m = __ballot(in && c == VW_CLS_MIXED);
-      if (lane < 4 && j0 + 64 * e < qend)
-        out[((j0 + 64 * e) >> 4) + lane] =
-            (uint32_t)((v >> (16 * lane)) & 0xffffu) | ((uint32_t)((m >> (16 * lane)) & 0xffffu) << 16);
+      for (int e = 0; e < 4; ++e) {
+        const int q = j0 + 64 * e + lane;
+        const bool in = q >= q0 && q < nu;
+        const int c = vw_pair_class(b[av[e]], b[bv[e]]);
+        const uint64_t v = __ballot(in && c == VW_CLS_VISIBLE), m = __ballot(in && c == VW_CLS_MIXED);
+        if (lane < 4 && j0 + 64 * e < qend)
+          out[((j0 + 64 * e) >> 4) + lane] =
+              (uint32_t)((v >> (16 * lane)) & 0xffffu) | ((uint32_t)((m >> (16 * lane)) & 0xffffu) << 16);
+      }
     }
   }
   vw_ts_end(ts);
@@ -1720,6 +1847,7 @@ __global__ __launch_bounds__(256) void k_group_mask(ReconSets sets, const double
 /* reconstruction                                                       */
 /* ------------------------------------------------------------------ */
 struct ReconArgs {
+  VwMerge mg;
   const double2* tab;  /* the sine table (plain), built once per context */
   ReconSets sets;
   int64_t TP, nq_pad, nh_pad;
@@ -1914,16 +2042,20 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(
   if (chunk >= S.nchunk) return;
   const int64_t pbase = pw * 64 * PPL; /* pass-relative */
   const int64_t tile = pbase / a.TP;   /* pass-relative tile (class tables are per pass) */
-  const vw_segparams sp = a.info->sp;
-  /* group counts fit 32 bits; uniform values keep the range tests scalar */
-  const int64_t nu = vw_rfl((int)a.info->nuniq);
-  const int64_t q0 = vw_rfl((int)a.info->first_nz);
-  const bool polar = vw_rfl(a.info->polar) != 0;
+  int sg = 0; /* the chunk's segment */
+  while (sg + 1 < a.mg.n && (int)chunk >= S.cst[sg + 1]) ++sg;
+  const DevInfo* info = a.info + sg;
+  const vw_segparams sp = info->sp;
+  /* group positions fit 32 bits; uniform values keep the range tests scalar */
+  const int64_t nu = a.mg.base[sg] + vw_rfl((int)info->nuniq);
+  const int64_t q0 = a.mg.base[sg] + vw_rfl((int)info->first_nz);
+  const bool polar = vw_rfl(info->polar) != 0;
   /* group range of this chunk, aligned to 16 groups */
   const int64_t base = q0 & ~(int64_t)15;
-  const int64_t span = ((nu - base) + S.nchunk - 1) / S.nchunk;
+  const int64_t nch = S.cst[sg + 1] - S.cst[sg];
+  const int64_t span = ((nu - base) + nch - 1) / nch;
   const int64_t spanA = (span + 15) & ~(int64_t)15;
-  const int64_t qa_ = vw_rfl((int)(base + chunk * spanA));
+  const int64_t qa_ = vw_rfl((int)(base + (chunk - S.cst[sg]) * spanA));
   const int64_t qb_ = vw_rfl((int)(qa_ + spanA < nu ? qa_ + spanA : nu));
 
   double pl[PPL], pm[PPL], pn[PPL], lp[PPL], mp[PPL];

@@ -114,13 +114,14 @@ class VwXfer {
 
  private:
   /* Measured into fresh pages, plain copy against this, us: 134 MB 12,500 3,420;
-   * 22 MB 2,160 700; 9.4 MB 1,010 430.  Results of a few MB are gained only into
-   * fresh pages (2.1 MB 473 270) and lost into warm ones (the 1.7 MB of an
-   * ordinary training pair: the call 712 -> 814), so they stay plain.  2 MiB chunks keep the copies' launch and event
+   * 22 MB 2,160 700; 9.4 MB 1,010 430.  Results of a few MB gain only into fresh
+   * pages (2.1 MB 473 270), not into a program's recycled arrays (5.5 MB of Nside
+   * 128 maps 464 461; with the 1.7 MB of an ordinary training pair the call went
+   * from 712 to 814), so they stay plain.  2 MiB chunks keep the copies' launch and event
    * (20 us together, 9.9 ms for 134 MB in 256 KiB chunks) below their 40 us;
    * the smallest results take smaller ones so that four threads share them.
    * 7 or 11 helpers measured the same. */
-  static constexpr size_t kPlain = 4 << 20, kChunkMin = 256 << 10, kChunkMax = 2 << 20, kRing = 32 << 20;
+  static constexpr size_t kPlain = 8 << 20, kChunkMin = 256 << 10, kChunkMax = 2 << 20, kRing = 32 << 20;
   static constexpr int kSlots = 64, kSegs = 8, kThreads = 3;
 
   char* ring_ = nullptr;
