@@ -148,7 +148,7 @@ struct Ctx {
   /* occlusion bits [32-point block of a pass][nfr_pad] of the Viss and of the
    * recon's two output sets; sky or output tiles per batched pass             */
   uint32_t *d_fvis_v = nullptr, *d_fvis = nullptr, *d_fvis2 = nullptr;
-  int64_t btpp = 0;
+  int64_t ftpp = 0; /* 0: a form that takes no occlusion bits */
   int32_t* d_rshist[2] = {};  /* radix-sort digit tables per stream (Viss, grouping)   */
   int64_t rshist_cap = 0;
   /* per-sky segment schedules (vw_set_sky_schedules): the batched Viss of
@@ -638,7 +638,8 @@ ReconShape recon_shape(int64_t npts, int64_t nq = INT64_MAX) {
 
 /* output tiles per recon pass: as many as the class scratch holds */
 int64_t recon_pass_tiles(const Ctx* c, int64_t ntile_all, int64_t kind_w) {
-  return std::max<int64_t>(1, std::min<int64_t>(ntile_all, c->cls_cap / kind_w));
+  const int64_t most = c->ftpp ? std::min(c->ftpp, ntile_all) : ntile_all;
+  return std::max<int64_t>(1, std::min<int64_t>(most, c->cls_cap / kind_w));
 }
 
 /* batched launch shapes.  Viss: a wave is 16 half rows x 16 nbw skies over a
@@ -763,15 +764,7 @@ int join_recon(Ctx* c) {
 int create_batch(Ctx* c) {
   int rc;
   const int64_t npix_pad = c->ntile * c->TP;
-  /* tiles per pass: as many as hold their occlusion bits (a bit per (point,
-   * antenna frame)) in the class budget */
-  const int64_t fbytes = c->TP / 8 * c->nfr_pad;
-  c->btpp = std::max<int64_t>(1, std::min(std::max(c->ntile, c->ngt), class_budget(c) / fbytes));
-  for (int b = 0; b < 3; ++b) {
-    const int64_t nt = std::min(c->btpp, b == 2 ? c->ngt : c->ntile);
-    if (nt && (rc = dalloc(c, b == 0 ? &c->d_fvis_v : b == 1 ? &c->d_fvis : &c->d_fvis2, (size_t)(nt * fbytes / 4))))
-      return rc;
-  }
+  if ((rc = dalloc(c, &c->d_fvis_v, (size_t)(std::min(c->ftpp, c->ntile) * c->TP / 32 * c->nfr_pad)))) return rc;
   if ((rc = dalloc(c, &c->d_skyf, (size_t)(c->nsky * c->npix))) ||
       (rc = dalloc(c, &c->d_skyh, (size_t)(npix_pad * c->nsky_pad))) ||
       (rc = dalloc(c, &c->d_skyl, (size_t)(npix_pad * c->nsky_pad))))
@@ -779,7 +772,7 @@ int create_batch(Ctx* c) {
   for (int k = 0; k < 4; ++k)
     if ((rc = dalloc(c, &c->d_gpk[k], (size_t)(c->nq_pad * c->nsky_pad)))) return rc;
   int64_t vch = 1;
-  const int64_t vfull = std::min(c->btpp, c->ntile), vlast = c->ntile - (c->ntile - 1) / vfull * vfull;
+  const int64_t vfull = std::min(c->ftpp, c->ntile), vlast = c->ntile - (c->ntile - 1) / vfull * vfull;
   for (int k = 0; k < c->segs; ++k)
     for (int64_t nt : {vfull, vlast})
       for (int64_t tg : VW_BATCH_TARGETS) vch = std::max(vch, vissb_shape(c, (int64_t)c->seg_tlen[k] * c->P, nt, tg).nchunk);
@@ -789,7 +782,7 @@ int create_batch(Ctx* c) {
   for (int img = 0; img < 2; ++img) {
     const int64_t npts = img ? c->ngp : c->npix;
     if (npts <= 0) continue;
-    const int64_t pp = c->btpp * c->TP;
+    const int64_t pp = c->ftpp * c->TP;
     const int64_t last = npts - (npts - 1) / pp * pp;
     for (int64_t n : {std::min(npts, pp), last})
       for (int64_t tg : VW_BATCH_TARGETS) {
@@ -914,6 +907,16 @@ int create_device(Ctx* c) {
   if (c->cls_cap < std::max(c->nh_pad, kind_w)) c->cls_cap = std::max(c->nh_pad, kind_w);
   c->cls_cap = (c->cls_cap + 3) / 4 * 4;
   c->vtpp = std::max<int64_t>(1, std::min<int64_t>(c->ntile, c->cls_cap / c->nh_pad));
+  /* tiles per recon (and batched Viss) pass whose occlusion bits, a bit per
+   * (point, antenna frame), the class budget holds */
+  c->nfr_pad = ((int64_t)c->buf_tlen * c->A + 63) / 64 * 64;
+  if (c->batch || (c->cfg.precision == VW_PREC_MIXED && c->cfg.blockage && !c->generic)) {
+    c->ftpp = std::max<int64_t>(1, std::min(std::max(c->ntile, c->ngt), class_budget(c) / (c->TP / 8 * c->nfr_pad)));
+    for (int img = 0; img < 2; ++img) {
+      const int64_t nt = std::min(c->ftpp, img ? c->ngt : c->ntile);
+      if (nt && (rc = dalloc(c, img ? &c->d_fvis2 : &c->d_fvis, (size_t)(nt * c->TP / 32 * c->nfr_pad)))) return rc;
+    }
+  }
   /* partial buffers fit the largest pass shape: a full pass and the last one */
   int64_t nch = 1;
   const int64_t vlast = c->ntile - (c->ntile - 1) / c->vtpp * c->vtpp;
@@ -956,7 +959,8 @@ int create_device(Ctx* c) {
   {
     const size_t nq = (size_t)c->nq_pad;
     GroupSoA& g = c->gs;
-    if ((rc = dalloc(c, &g.rec, nq)) || (rc = dalloc(c, &g.v, nq)) || (rc = dalloc(c, &g.ant, 10 * nq)) || (rc = dalloc(c, &g.ant32, 8 * nq)) ||
+    if ((rc = dalloc(c, &g.rec, nq)) || (rc = dalloc(c, &g.v, nq)) ||
+        (c->cfg.precision == VW_PREC_PLAIN && ((rc = dalloc(c, &g.ant, 10 * nq)) || (rc = dalloc(c, &g.ant32, 8 * nq)))) ||
         (rc = dalloc(c, &g.gia, nq)) || (rc = dalloc(c, &g.gib, nq)) || (rc = dalloc(c, &g.grep, nq)))
       return rc;
     int64_t rp = 1;
@@ -982,7 +986,6 @@ int create_device(Ctx* c) {
       c->rshist_cap = 256 * ((2 * c->max_nh + VW_RS_BLOCK - 1) / VW_RS_BLOCK);
       if ((rc = dalloc(c, &c->d_rshist[1], (size_t)c->rshist_cap + 256))) return rc; /* + digit totals */
     }
-    c->nfr_pad = ((int64_t)c->buf_tlen * c->A + 63) / 64 * 64;
     c->bits_cap = maxnt * c->nfr_pad;
     if ((rc = dalloc(c, &c->d_bits, (size_t)c->bits_cap)) || (rc = dalloc(c, &c->d_bits_v, (size_t)c->bits_cap)))
       return rc;
@@ -1074,18 +1077,12 @@ int enq_frame_vis(Ctx* c, bool img, int64_t tile0, int64_t nt, uint32_t* out, hi
   return VW_OK;
 }
 
-/* the one-sky recon's group masks of a pass ([nt][nq_pad / 16] words per output
+/* the one-sky recon's group masks of a pass ([nt][nq_pad / 16] 64-bit words per output
  * set) into the sets' class scratch */
 int enq_group_masks(Ctx* c, const ReconSets& sets, uint8_t* const* bits, uint64_t* ts) {
-  const int64_t nfr = (int64_t)c->tlen * c->A;
-  const unsigned nb = (unsigned)(sets.s[0].nt + sets.s[1].nt);
-  if (c->nfr_pad <= VW_GCLS_LDS_MAX) {
-    k_group_mask<true><<<nb, 256, (size_t)c->nfr_pad, c->stB>>>(c->mg, sets, c->d_ant8, nfr, c->nfr_pad, c->gs.gia, c->gs.gib,
-                                                                 c->d_info, c->nq_pad, ts);
-    KC();
-    return VW_OK;
-  }
-  for (int i = 0; i < 2; ++i) {
+  const int64_t nfr = (int64_t)c->tlen * c->A, nt = sets.s[0].nt + sets.s[1].nt;
+  const bool tile = c->nfr_pad <= VW_GCLS_LDS_MAX, mixed = c->cfg.precision == VW_PREC_MIXED;
+  for (int i = 0; i < 2 && !tile; ++i) {
     const ReconSet& S = sets.s[i];
     if (!S.nt) continue;
     if (S.nt * c->nfr_pad > c->bits_cap) return c->fail(VW_ERR_RANGE, "internal: cone bit buffer too small");
@@ -1093,8 +1090,13 @@ int enq_group_masks(Ctx* c, const ReconSets& sets, uint8_t* const* bits, uint64_
                                                                   c->nfr_pad, bits[i], nullptr);
     KC();
   }
-  k_group_mask<false><<<nb, 256, 0, c->stB>>>(c->mg, sets, c->d_ant8, nfr, c->nfr_pad, c->gs.gia, c->gs.gib, c->d_info,
-                                              c->nq_pad, ts);
+  const unsigned nb = (unsigned)nt;
+#define VW_GM(TILE_, BITS_)                                                                                       \
+  k_group_mask<TILE_, BITS_><<<nb, 256, TILE_ ? (size_t)c->nfr_pad : 0, c->stB>>>(                                 \
+      c->mg, sets, c->d_ant8, nfr, c->nfr_pad, c->TP, c->gs.gia, c->gs.gib, c->d_info, c->nq_pad, ts)
+  if (tile) mixed ? VW_GM(true, true) : VW_GM(true, false);
+  else mixed ? VW_GM(false, true) : VW_GM(false, false);
+#undef VW_GM
   KC();
   return VW_OK;
 }
@@ -1235,7 +1237,7 @@ int enq_viss(Ctx* c, bool count, bool fill = false) {
   int rc;
   if (c->batch) ev_begin(c, ST_VISS);
   uint64_t *first = nullptr, *last = nullptr;
-  const int64_t tpp = c->batch ? c->btpp : c->vtpp;
+  const int64_t tpp = c->batch ? c->ftpp : c->vtpp;
   for (int64_t tile0 = 0; tile0 < c->ntile; tile0 += tpp) {
     const int64_t nt = std::min(tpp, c->ntile - tile0);
     double2* vh = fill && !c->batch && tile0 + nt == c->ntile ? c->d_vh : nullptr;
@@ -1364,11 +1366,9 @@ int enq_group_keys(Ctx* c) {
 int enq_group_data(Ctx* c, const double2* vh, uint64_t** ts_out = nullptr) {
   bool full = c->cfg.recon_mode == VW_RECON_FULL;
   uint64_t* ts = new_ts(c);
-  k_group_data<<<blocks_for(c->mg.base[c->mg.n]), 256, 0, c->stB>>>(c->mg, c->d_gkeys, c->d_goff, c->d_idx_sorted, vh, c->d_rows,
-                                                  c->d_ant8, c->P, full ? 1 : 0, c->cfg.blockage, c->cfg.occ_mode,
-                                                  c->cfg.precision == VW_PREC_PLAIN && c->generic ? VW_TAB_SCALE : 1.0,
-                                                  c->d_info,
-                                                  c->gs, ts);
+  k_group_data<<<blocks_for(c->mg.base[c->mg.n]), 256, 0, c->stB>>>(
+      c->mg, c->d_gkeys, c->d_goff, c->d_idx_sorted, vh, c->d_rows, c->d_ant8, c->P, full ? 1 : 0, c->cfg.blockage,
+      c->cfg.occ_mode, c->cfg.precision == VW_PREC_PLAIN && c->generic ? VW_TAB_SCALE : 1.0, c->d_info, c->gs, ts);
   KC();
   add_bracket(c, ST_GROUP, ts, ts);
   if (ts_out) *ts_out = ts;
@@ -1411,8 +1411,8 @@ int enq_recon_set_batch(Ctx* c, bool img) {
   const bool rep = c->cfg.blockage != 0;
   const int64_t npts_all = img ? c->ngp : c->npix;
   const int64_t ntile_all = img ? c->ngt : c->ntile;
-  for (int64_t tile0 = 0; tile0 < ntile_all; tile0 += c->btpp) {
-    const int64_t nt = std::min(c->btpp, ntile_all - tile0);
+  for (int64_t tile0 = 0; tile0 < ntile_all; tile0 += c->ftpp) {
+    const int64_t nt = std::min(c->ftpp, ntile_all - tile0);
     const int64_t pt0 = tile0 * c->TP;
     const int64_t np = std::min(nt * c->TP, npts_all - pt0);
     if (rep) {
@@ -1488,8 +1488,9 @@ int enq_recon_one(Ctx* c, double* const (&acc)[2], uint32_t* const (&wacc)[2], c
       S.cone = i ? c->d_gcone : c->d_cone;
       S.pt0 = S.tile0 * c->TP;
       S.npts = std::min(S.nt * c->TP, (i ? c->ngp : c->npix) - S.pt0);
-      S.cls = (uint32_t*)(i ? c->d_cls2 : c->d_cls);
+      S.cls = (uint64_t*)(i ? c->d_cls2 : c->d_cls);
       S.bits = bits[i];
+      S.fvis = (uint64_t*)(i ? c->d_fvis2 : c->d_fvis);
       const int64_t nr = full ? 2 * c->nh : c->nh;
       ReconShape rs = recon_shape(S.npts, nr);
       if (c->mg.n == 1) {
@@ -1529,6 +1530,7 @@ int enq_recon_one(Ctx* c, double* const (&acc)[2], uint32_t* const (&wacc)[2], c
     a.TP = c->TP;
     a.nq_pad = c->nq_pad;
     a.nh_pad = c->nh_pad;
+    a.nfr_pad = c->nfr_pad;
     a.g = c->gs;
     a.goff = c->d_goff;
     a.idx_sorted = c->d_idx_sorted;

@@ -169,8 +169,7 @@ __global__ void k_group_keys(const int32_t* __restrict__ gia, const int32_t* __r
  * products hold no test.  A frame that the tile's cone finds all visible or
  * all hidden needs none at all; bits are the per-point FP64 test's otherwise,
  * so a mask equals the pair class with its per-point tests.
- * A wave owns 64 points and 64 frames: lane f holds frame f's position and
- * words, the partly visible frames are broadcast one by one; 50 us for 196,608
+ * A wave owns 64 points and 64 frames (vw_frame_words); 50 us for 196,608
  * points x 2,080 frames.  64 skies at Nside 128, 16 antennas, 205 epochs and a
  * 256^2 image, against class bytes with the FP64 test in the term loops (a
  * divergent branch per masked term in the recon): k_reconb 22.3 -> 16.3 ms and
@@ -191,26 +190,11 @@ __global__ __launch_bounds__(256) void k_frame_vis(const double* __restrict__ l,
   const double pl = l[pp], pm = m[pp], pn = n[pp];
   const int64_t f = (int64_t)blockIdx.y * 64 + lane;
   const double* q = ant8 + (f < nfr ? f : nfr - 1) * 8;
-  const double x = q[0], y = q[1], z = q[2], in = q[3], cp = q[7];
   const int cb = vw_cone_bits(q[4], q[5], q[6], cone[t], cone[ntile + t], cone[2 * ntile + t], cone[3 * ntile + t],
-                              cone[4 * ntile + t], cp);
-  uint32_t lo = !(cb & 2) && (cb & 1) ? 0xffffffffu : 0u, hi = lo;
-  uint64_t some = __ballot(f < nfr && !(cb & 3));
-  while (some) {
-    const int j = __builtin_ctzll(some);
-    some &= some - 1;
-    auto at = [j](double v) {
-      const uint64_t w = __builtin_bit_cast(uint64_t, v);
-      const uint32_t a = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)w, j);
-      const uint32_t c = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(w >> 32), j);
-      return __builtin_bit_cast(double, (uint64_t)c << 32 | a);
-    };
-    const uint64_t v = __ballot(ok && vw_visible(pl, pm, pn, at(x), at(y), at(z), at(in), at(cp)));
-    lo = lane == j ? (uint32_t)v : lo;
-    hi = lane == j ? (uint32_t)(v >> 32) : hi;
-  }
-  out[2 * b * nfr_pad + f] = lo;
-  out[(2 * b + 1) * nfr_pad + f] = hi;
+                              cone[4 * ntile + t], q[7]);
+  const uint64_t w = vw_frame_words(ant8, f, nfr, cb, pl, pm, pn, ok);
+  out[2 * b * nfr_pad + f] = (uint32_t)w;
+  out[(2 * b + 1) * nfr_pad + f] = (uint32_t)(w >> 32);
 }
 
 /* all ones where bit `bit` of x is set, else zero */

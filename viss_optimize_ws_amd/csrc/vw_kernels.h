@@ -62,6 +62,9 @@ struct VwMerge {
 #define VW_FULLMASK 0xffffffffffffffffULL
 
 __device__ __forceinline__ int vw_rfl(int x) { return __builtin_amdgcn_readfirstlane(x); }
+__device__ __forceinline__ uint64_t vw_rfl64(uint64_t x) {
+  return (uint64_t)(uint32_t)vw_rfl((int)(x >> 32)) << 32 | (uint32_t)vw_rfl((int)x);
+}
 
 /* Stage timing: the small kernels around a stage's large one write the device's
  * real-time counter to two words of host memory, ts[0] as the first workgroup
@@ -1687,9 +1690,9 @@ struct GRec {
 struct GroupSoA {
   GRec* rec;    /* 32 B */
   double2* v;   /* the visibility as (re, im), for segments without polar terms */
-  double* ant;  /* [q][10]: representative's antenna frames a and b    */
-  float* ant32; /* [q][8]: their unit vectors and thresholds in FP32 (vw_frame32) */
-  int32_t *gia, *gib, *grep;
+  double* ant;  /* [q][10]: representative's antenna frames a and b (plain form; */
+  float* ant32; /* [q][8]: in FP32, vw_frame32; null in the mixed form)        */
+  int32_t *gia, *gib, *grep; /* the representative's frames' indices, its half row */
 };
 
 __global__ void k_group_data(VwMerge mg, const int64_t* __restrict__ gkeys, const int32_t* __restrict__ goff,
@@ -1755,13 +1758,15 @@ __global__ void k_group_data(VwMerge mg, const int64_t* __restrict__ gkeys, cons
   RowRec r = rows[hr];
   g.gia[q] = r.ia;
   g.gib[q] = r.ib;
-  const double* qa = ant8 + (int64_t)r.ia * 8;
-  const double* qb = ant8 + (int64_t)r.ib * 8;
-  double* d = g.ant + q * 10;
-  d[0] = qa[0]; d[1] = qa[1]; d[2] = qa[2]; d[3] = qa[3]; d[4] = qa[7];
-  d[5] = qb[0]; d[6] = qb[1]; d[7] = qb[2]; d[8] = qb[3]; d[9] = qb[7];
-  vw_frame32(qa, g.ant32 + q * 8);
-  vw_frame32(qb, g.ant32 + q * 8 + 4);
+  if (g.ant) {
+    const double* qa = ant8 + (int64_t)r.ia * 8;
+    const double* qb = ant8 + (int64_t)r.ib * 8;
+    double* d = g.ant + q * 10;
+    d[0] = qa[0]; d[1] = qa[1]; d[2] = qa[2]; d[3] = qa[3]; d[4] = qa[7];
+    d[5] = qb[0]; d[6] = qb[1]; d[7] = qb[2]; d[8] = qb[3]; d[9] = qb[7];
+    vw_frame32(qa, g.ant32 + q * 8);
+    vw_frame32(qb, g.ant32 + q * 8 + 4);
+  }
   vw_ts_end(ts);
 }
 
@@ -1774,9 +1779,10 @@ struct ReconSet {
   int64_t ntile;      /* tiles of the whole set                                  */
   int64_t tile0, nt;  /* tiles of this pass                                      */
   int64_t pt0, npts;  /* its points [pt0, pt0 + npts), pt0 = tile0 * TP          */
-  uint32_t* cls;      /* [nt][nq_pad / 16] mask words of 16 groups (representative
+  uint64_t* cls;      /* [nt][nq_pad / 16] mask words of 16 groups (representative
                        * kinds), [nt][nh_pad] row class bytes (generic kind)     */
   const uint8_t* bits; /* [nt][nfr_pad] cone bits (long frame rows)               */
+  uint64_t* fvis;     /* [nt][nfr_pad][TP / 64] points seen (representative kinds) */
   int64_t nchunk;     /* group ranges per point block                            */
   int cst[VW_MERGE_MAX + 1]; /* of them, segment s has [cst[s], cst[s + 1])      */
   int64_t pwaves;     /* point blocks (waves) per group range                    */
@@ -1790,18 +1796,115 @@ struct ReconSets {
   ReconSet s[2]; /* a set without tiles or blocks is absent */
 };
 
+/* Which of a wave's 64 points (lane: pl, pm, pn; ok) each of 64 antenna frames
+ * sees: lane f returns frame f0 + f's word, bit j = point j.  cb: the frame's
+ * cone bits on the points' tile, which decide it where they can; the partly
+ * visible frames are broadcast one by one for the FP64 test of every point. */
+__device__ __forceinline__ uint64_t vw_frame_words(const double* __restrict__ ant8, int64_t f, int64_t nfr, int cb,
+                                                   double pl, double pm, double pn, bool ok) {
+  const uint64_t all = ~0ull;
+  uint64_t word = !(cb & 2) && (cb & 1) ? all : 0ull;
+  uint64_t some = __ballot(f < nfr && !(cb & 3));
+  if (!some) return word;
+  const double* q = ant8 + (f < nfr ? f : nfr - 1) * 8;
+  const double x = q[0], y = q[1], z = q[2], in = q[3], cp = q[7];
+  const int lane = threadIdx.x & 63;
+  while (some) {
+    const int j = __builtin_ctzll(some);
+    some &= some - 1;
+    auto at = [j](double v) {
+      const uint64_t w = __builtin_bit_cast(uint64_t, v);
+      const uint32_t a = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)w, j);
+      const uint32_t c = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(w >> 32), j);
+      return __builtin_bit_cast(double, (uint64_t)c << 32 | a);
+    };
+    const uint64_t v = __ballot(ok && vw_visible(pl, pm, pn, at(x), at(y), at(z), at(in), at(cp)));
+    word = lane == j ? v : word;
+  }
+  return word;
+}
+
+/* Occlusion bits of the frames that a tile's cone leaves open (b: the tile's
+ * cone bits), for one block of 64 points, by one wave: fo[f * stride], bit j =
+ * point j is seen from frame f.  The wave gathers open frames in LDS and takes
+ * 64 at a time, a lane a frame, against the points in turn (LDS broadcasts).
+ * Broadcasting the frames one by one and writing the decided frames' words too
+ * took twice the time; points as scalar loads or lane by lane, a queue shared by
+ * the workgroup, and further workgroups for 256 frames each, which test the
+ * cones again, were no faster (337 us for 6,289 tiles x 2,048 frames). */
+__device__ __forceinline__ void vw_open_frames(const uint8_t* b, int64_t nfr, const double* __restrict__ ant8,
+                                               double pl, double pm, double pn, bool ok, double* pts /* [3][64] */,
+                                               int32_t* queue /* [128] */, uint64_t* __restrict__ fo, int stride) {
+  const int lane = threadIdx.x & 63;
+  const uint64_t okm = __ballot(ok);
+  auto settle = [] { /* the wave's LDS writes are seen by its reads, and its reads done before its writes */
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  };
+  settle();
+  pts[lane] = pl;
+  pts[64 + lane] = pm;
+  pts[128 + lane] = pn;
+  auto take = [&](int n) { /* the queue's first n <= 64 frames */
+    settle();
+    const int f = lane < n ? queue[lane] : -1;
+    const double* q = ant8 + (int64_t)(f < 0 ? 0 : f) * 8;
+    const double x = q[0], y = q[1], z = q[2], in = q[3], cp = q[7];
+    uint32_t w[2];
+#pragma unroll
+    for (int hf = 0; hf < 2; ++hf) {
+      uint32_t v = 0;
+#pragma unroll 8
+      for (int j = 0; j < 32; ++j) {
+        const int p = 32 * hf + j;
+        v |= (uint32_t)vw_visible(pts[p], pts[64 + p], pts[128 + p], x, y, z, in, cp) << j;
+      }
+      w[hf] = v;
+    }
+    if (f >= 0) fo[(int64_t)f * stride] = ((uint64_t)w[1] << 32 | w[0]) & okm;
+    settle();
+  };
+  int cnt = 0;
+  for (int64_t f0 = 0; f0 < nfr; f0 += 64) {
+    const int64_t f = f0 + lane;
+    const bool open = f < nfr && !(b[f] & 3);
+    const uint64_t m = __ballot(open);
+    if (open) queue[cnt + __popcll(m & ((1ull << lane) - 1))] = (int32_t)f;
+    cnt += __popcll(m);
+    if (cnt >= 64) {
+      take(64);
+      cnt -= 64;
+      const int32_t r = queue[64 + lane];
+      settle();
+      if (lane < cnt) queue[lane] = r;
+    }
+  }
+  if (cnt) take(cnt);
+}
+
 /* The one-sky recon's form of the same classes: per (tile, 16 groups) one
- * word, bit j = group j is visible from the whole tile, bit 16 + j = partly;
- * groups below first_nz (the key-0 group) and past nuniq have neither bit, so
- * the recon walks set bits and needs no range test.  TILE: one block per tile
+ * 64-bit word, bit j = group j is visible from the whole tile, bits 16 + j and
+ * 32 + j = it is partly, with its first, its second antenna's frame left open
+ * by the tile's cone; hidden groups, groups below first_nz (the key-0 group) and
+ * past nuniq have none of them, so the recon walks set bits and needs no range
+ * test.  TILE: one block per tile
  * makes the tile's cone bits in LDS (frame rows up to VW_GCLS_LDS_MAX bytes);
  * else they come from the bit table of the pass.  A wave takes 4 x 64 groups
  * at a time, a lane one group of each 64 (coalesced index loads, all issued
  * before the gathers), and writes the masks of ballots.  Words of entries
- * below nuniq rounded up to 64 are written: the recon reads no others. */
-template <bool TILE>
+ * below nuniq rounded up to 64 are written: the recon reads no others.
+ * BITS (mixed form): the block also writes the open frames' occlusion bits
+ * (vw_open_frames), whose AND over a partly visible group's open frames is its
+ * mask; the recon loads the words as scalars.  Testing both antennas of every
+ * (point, group) in FP32, with an FP64 fallback, as the plain form does, cost it
+ * as much as two terms and 26 registers (5 instead of 8 waves a SIMD): two Nside
+ * 256 segments 24.3 -> 22.5 ms, the Nside 128 day 8.98 -> 8.56.  The plain form is
+ * bound by its FP64 terms and gained nothing (Nside 256 -2%, short segments and
+ * the lunar formation, with few groups a frame, +2 to 4%). */
+template <bool TILE, bool BITS>
 __global__ __launch_bounds__(256) void k_group_mask(VwMerge mg, ReconSets sets, const double* __restrict__ ant8, int64_t nfr,
-                                                    int64_t nfr_pad, const int32_t* __restrict__ ia,
+                                                    int64_t nfr_pad, int64_t TP, const int32_t* __restrict__ ia,
                                                     const int32_t* __restrict__ ib, const DevInfo* __restrict__ info,
                                                     int64_t nq_pad, uint64_t* __restrict__ ts) {
   vw_ts_begin(ts);
@@ -1815,7 +1918,19 @@ __global__ __launch_bounds__(256) void k_group_mask(VwMerge mg, ReconSets sets, 
     __syncthreads();
   }
   const int wave = vw_rfl((int)(threadIdx.x >> 6)), lane = threadIdx.x & 63;
-  uint32_t* out = S.cls + tr * (nq_pad >> 4);
+  if (BITS) {
+    __shared__ double spt[4][192];
+    __shared__ int32_t squeue[4][128];
+    const int nblk = (int)(TP / 64);
+    for (int blk = wave; blk < nblk; blk += 4) {
+      const int64_t p = tr * TP + 64 * blk + lane; /* pass-relative */
+      const bool ok = p < S.npts;
+      const int64_t pp = S.pt0 + (ok ? p : 0);
+      vw_open_frames(b, nfr, ant8, S.l[pp], S.m[pp], S.n[pp], ok, spt[wave], squeue[wave],
+                     S.fvis + tr * nfr_pad * nblk + blk, nblk);
+    }
+  }
+  uint64_t* out = S.cls + tr * (nq_pad >> 4);
   for (int sg = 0; sg < mg.n; ++sg) {
     const int base = mg.base[sg], nu = base + vw_rfl((int)info[sg].nuniq), q0 = base + vw_rfl((int)info[sg].first_nz);
     const int qend = (nu + 63) / 64 * 64; /* <= nq_pad, a multiple of 64 */
@@ -1832,11 +1947,15 @@ __global__ __launch_bounds__(256) void k_group_mask(VwMerge mg, ReconSets sets, 
       for (int e = 0; e < 4; ++e) {
         const int q = j0 + 64 * e + lane;
         const bool in = q >= q0 && q < nu;
-        const int c = vw_pair_class(b[av[e]], b[bv[e]]);
-        const uint64_t v = __ballot(in && c == VW_CLS_VISIBLE), m = __ballot(in && c == VW_CLS_MIXED);
-        if (lane < 4 && j0 + 64 * e < qend)
+        const int ba = b[av[e]], bb = b[bv[e]], c = vw_pair_class(ba, bb);
+        const uint64_t v = __ballot(in && c == VW_CLS_VISIBLE);
+        const uint64_t ma = __ballot(in && c == VW_CLS_MIXED && !(ba & 1));
+        const uint64_t mb = __ballot(in && c == VW_CLS_MIXED && !(bb & 1));
+        if (lane < 4 && j0 + 64 * e < qend) {
+          const int sh = 16 * lane;
           out[((j0 + 64 * e) >> 4) + lane] =
-              (uint32_t)((v >> (16 * lane)) & 0xffffu) | ((uint32_t)((m >> (16 * lane)) & 0xffffu) << 16);
+              ((v >> sh) & 0xffffu) | ((ma >> sh) & 0xffffu) << 16 | ((mb >> sh) & 0xffffu) << 32;
+        }
       }
     }
   }
@@ -1850,7 +1969,7 @@ struct ReconArgs {
   VwMerge mg;
   const double2* tab;  /* the sine table (plain), built once per context */
   ReconSets sets;
-  int64_t TP, nq_pad, nh_pad;
+  int64_t TP, nq_pad, nh_pad, nfr_pad;
   GroupSoA g;
   const int32_t* goff;
   const int32_t* idx_sorted;
@@ -2026,6 +2145,7 @@ template <int PPL, bool MIXED, int KIND>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(
     KIND == VW_KIND_GENERIC ? VW_RECON_WAVES_GENERIC : MIXED ? VW_RECON_WAVES_MIXED : VW_RECON_WAVES_PLAIN))) void k_recon(ReconArgs a) {
   constexpr bool TABLE = !MIXED && KIND == VW_KIND_GENERIC;
+  constexpr bool BITS = MIXED && VW_KIND_IS_REP(KIND); /* occlusion bits, see k_group_mask */
   __shared__ double2 tab[TABLE ? VW_TAB_N : 1];
   __shared__ double gring[4][2 * 64]; /* per wave: two blocks of 16 group records */
   if (TABLE) {
@@ -2059,7 +2179,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(
   const int64_t qb_ = vw_rfl((int)(qa_ + spanA < nu ? qa_ + spanA : nu));
 
   double pl[PPL], pm[PPL], pn[PPL], lp[PPL], mp[PPL];
-  float fl[PPL], fm[PPL], fn[PPL]; /* FP32 directions (partly visible tiles) */
+  float fl[PPL], fm[PPL], fn[PPL]; /* FP32 directions (partly visible groups, plain form) */
   bool ok[PPL];
 #pragma unroll
   for (int k = 0; k < PPL; ++k) {
@@ -2071,9 +2191,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(
     pn[k] = S.n[pp];
     lp[k] = fma(sp.fa, pn[k], pl[k]);
     mp[k] = fma(sp.fb, pn[k], pm[k]);
-    fl[k] = (float)pl[k];
-    fm[k] = (float)pm[k];
-    fn[k] = (float)pn[k];
+    if (!BITS) {
+      fl[k] = (float)pl[k];
+      fm[k] = (float)pm[k];
+      fn[k] = (float)pn[k];
+    }
   }
   ReconLane<PPL, MIXED> acc;
   uint32_t wl[PPL];
@@ -2097,27 +2219,45 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(
      * 64, so every block lies inside the records and the masks. */
     double* ring = gring[vw_rfl((int)(threadIdx.x >> 6))];
     const double* recd = (const double*)a.g.rec;
-    const uint32_t* mrow = VW_KIND_IS_REP(KIND) ? S.cls + tile * (a.nq_pad >> 4) : nullptr;
+    const uint64_t* mrow = VW_KIND_IS_REP(KIND) ? S.cls + tile * (a.nq_pad >> 4) : nullptr;
     double stage = (qa_ < qb_) ? recd[qa_ * 4 + lane] : 0.0;
-    uint32_t nmw = 0;
-    if (VW_KIND_IS_REP(KIND) && qa_ < qb_) nmw = (uint32_t)vw_rfl((int)mrow[qa_ >> 4]);
+    uint64_t nmw = 0;
+    if (VW_KIND_IS_REP(KIND) && qa_ < qb_) nmw = vw_rfl64(mrow[qa_ >> 4]);
+    /* lane j < 16: the frames of the block's group j; the words of the wave's
+     * points, 64 k points on for point k of a lane */
+    const int fw = (int)(a.TP / 64);
+    const uint64_t* fv = BITS ? S.fvis + tile * a.nfr_pad * fw + (pbase - tile * a.TP) / 64 : nullptr;
+    int32_t nia = 0, nib = 0;
+    if (BITS && qa_ < qb_) {
+      nia = a.g.gia[qa_ + (lane & 15)];
+      nib = a.g.gib[qa_ + (lane & 15)];
+    }
     int buf = 0;
     for (int q16 = (int)qa_; q16 < (int)qb_; q16 += 16, buf ^= 1) {
       ring[buf * 64 + lane] = stage;
       __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
       __builtin_amdgcn_wave_barrier();
       __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-      uint32_t mw = nmw;
+      uint64_t mw = nmw;
+      const int32_t cia = nia, cib = nib;
       if (q16 + 16 < (int)qb_) {
         stage = recd[(int64_t)(q16 + 16) * 4 + lane];
-        if (VW_KIND_IS_REP(KIND)) nmw = (uint32_t)vw_rfl((int)mrow[(q16 + 16) >> 4]);
+        if (VW_KIND_IS_REP(KIND)) {
+          nmw = vw_rfl64(mrow[(q16 + 16) >> 4]);
+          if (BITS) {
+            nia = a.g.gia[q16 + 16 + (lane & 15)];
+            nib = a.g.gib[q16 + 16 + (lane & 15)];
+          }
+        }
       }
       if (KIND == VW_KIND_AVG) { /* every group of nonzero key, no classes */
         const int lo = (int)q0 > q16 ? (int)q0 - q16 : 0, hi = (int)qb_ - q16 < 16 ? (int)qb_ - q16 : 16;
         mw = ((1u << hi) - 1u) & ~((1u << lo) - 1u);
       }
       const GRec* blk = (const GRec*)(ring + buf * 64);
-      uint32_t vis = mw & 0xffffu, part = mw >> 16;
+      uint32_t vis = (uint32_t)mw & 0xffffu;
+      const uint32_t opa = (uint32_t)(mw >> 16) & 0xffffu, opb = (uint32_t)(mw >> 32);
+      uint32_t part = opa | opb;
       if (KIND != VW_KIND_REP_FINITE) wu += (uint32_t)__builtin_popcount(vis);
       while (vis) {
         const int j = __builtin_ctz(vis);
@@ -2136,26 +2276,35 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(
           part &= part - 1;
           const GRec g = blk[j];
           if (KIND == VW_KIND_REP_FINITE && !isfinite(g.amp)) continue;
-          float fr[8];
-#pragma unroll
-          for (int e = 0; e < 8; ++e) fr[e] = a.g.ant32[(int64_t)(q16 + j) * 8 + e];
-          float vd[PPL], near_ = 4.f;
           bool use[PPL];
+          if constexpr (BITS) {
+            /* both frames' words, the one's twice where only it is open */
+            const int32_t fa = __builtin_amdgcn_readlane(cia, j), fb = __builtin_amdgcn_readlane(cib, j);
+            const uint64_t* va = fv + (int64_t)(opa >> j & 1 ? fa : fb) * fw;
+            const uint64_t* vb = fv + (int64_t)(opb >> j & 1 ? fb : fa) * fw;
 #pragma unroll
-          for (int k = 0; k < PPL; ++k) {
-            vd[k] = vw_vis32(fl[k], fm[k], fn[k], fr);
-            near_ = fminf(near_, fabsf(vd[k]));
-            use[k] = vd[k] > 0.f;
-          }
-          if (__ballot(near_ <= VW_VIS_EPS)) { /* a point on the horizon: the FP64 test */
-            const double* d = a.g.ant + (int64_t)(q16 + j) * 10;
+            for (int k = 0; k < PPL; ++k) use[k] = __builtin_amdgcn_inverse_ballot_w64(va[k] & vb[k]);
+          } else {
+            float fr[8];
+#pragma unroll
+            for (int e = 0; e < 8; ++e) fr[e] = a.g.ant32[(int64_t)(q16 + j) * 8 + e];
+            float vd[PPL], near_ = 4.f;
 #pragma unroll
             for (int k = 0; k < PPL; ++k) {
-              int ln = lane; /* opaque: the addresses are formed here, not kept in registers across the loop */
-              __asm__ volatile("" : "+v"(ln));
-              const int64_t pp = S.pt0 + (ok[k] ? pbase + ln + 64 * k : 0);
-              use[k] = vw_vis2<true>(ok[k], S.l[pp], S.m[pp], S.n[pp], d[0], d[1], d[2], d[3], d[4], d[5], d[6], d[7],
-                                     d[8], d[9]);
+              vd[k] = vw_vis32(fl[k], fm[k], fn[k], fr);
+              near_ = fminf(near_, fabsf(vd[k]));
+              use[k] = vd[k] > 0.f;
+            }
+            if (__ballot(near_ <= VW_VIS_EPS)) { /* a point on the horizon: the FP64 test */
+              const double* d = a.g.ant + (int64_t)(q16 + j) * 10;
+#pragma unroll
+              for (int k = 0; k < PPL; ++k) {
+                int ln = lane; /* opaque: the addresses are formed here, not kept in registers across the loop */
+                __asm__ volatile("" : "+v"(ln));
+                const int64_t pp = S.pt0 + (ok[k] ? pbase + ln + 64 * k : 0);
+                use[k] = vw_vis2<true>(ok[k], S.l[pp], S.m[pp], S.n[pp], d[0], d[1], d[2], d[3], d[4], d[5], d[6], d[7],
+                                       d[8], d[9]);
+              }
             }
           }
 #pragma unroll
@@ -2185,7 +2334,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(
         const int32_t pos = (np < 0) ? kk : posv[kk];
         bool ng;
         const int64_t h = vw_row_half(a.idx_sorted[pos], a.P, a.full != 0, &ng);
-        const int cls = vw_cls_lookup(S.cls, tile, a.nh_pad, h);
+        const int cls = vw_cls_lookup((const uint32_t*)S.cls, tile, a.nh_pad, h);
         if (cls == VW_CLS_HIDDEN) continue;
         bool mv[PPL];
         if (cls == VW_CLS_VISIBLE) {
