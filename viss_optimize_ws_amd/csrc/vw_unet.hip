@@ -124,10 +124,21 @@ __device__ __forceinline__ int64_t vu_xcd_block(int64_t b, int64_t nb) {
   return x * q + (x < r ? x : r) + i;
 }
 typedef _Float16 vw_h2 __attribute__((ext_vector_type(2)));
+/* The second output of a convolution, from the stored value and aux at its place:
+ * forward (RELU) the skip sum v + aux, in the data gradient v where the ReLU
+ * output aux is positive.  Written beside the first, they save the kernels that
+ * read it back (with the 8-wide output layer, four training steps at 256^2,
+ * batch 16, 5,549 -> 5,462 us). */
+template <bool RELU>
+__device__ __forceinline__ _Float16 vw_conv_second(_Float16 v, _Float16 aux) {
+  if (RELU) return (_Float16)((float)v + (float)aux);
+  return (float)aux > 0.f ? v : (_Float16)0.f;
+}
 template <bool RELU, int CB, bool PF, bool VS, int OCB>
 __global__ __launch_bounds__(256) void k_conv3_mfma(const _Float16* __restrict__ in, const _Float16* __restrict__ Wk,
                                                     const float* __restrict__ B, _Float16* __restrict__ out, int cin,
-                                                    int cout, int H, const _Float16* __restrict__ mask) {
+                                                    int cout, int H, const _Float16* __restrict__ mask,
+                                                    const _Float16* __restrict__ aux, _Float16* __restrict__ out2) {
   static_assert(CB == 16 || CB == 32, "channels per LDS chunk");
   constexpr int STEPS = CB == 32 ? 9 : 5;
   /* [y][x][ci], pixel rows of CB channels + 8 halves of padding (the 16
@@ -317,6 +328,12 @@ __global__ __launch_bounds__(256) void k_conv3_mfma(const _Float16* __restrict__
             if (!((float)mk[k] > 0.f)) v[k] = (_Float16)0.f;
         }
         *(vw_h8*)(out + oi) = v;
+        if (out2) {
+          const vw_h8 x = *(const vw_h8*)(aux + oi);
+#pragma unroll
+          for (int k = 0; k < 8; ++k) v[k] = vw_conv_second<RELU>(v[k], x[k]);
+          *(vw_h8*)(out2 + oi) = v;
+        }
       }
     }
     return;
@@ -336,6 +353,7 @@ __global__ __launch_bounds__(256) void k_conv3_mfma(const _Float16* __restrict__
         const int64_t oi = ((int64_t)n * cout + o) * HH + (int64_t)y * H + x;
         if (mask && !((float)mask[oi] > 0.f)) v = 0.f;
         out[oi] = (_Float16)v;
+        if (out2) out2[oi] = vw_conv_second<RELU>((_Float16)v, aux[oi]);
       }
     }
 }
@@ -789,25 +807,6 @@ __global__ void k_add(const T* __restrict__ a, const T* __restrict__ b, T* __res
  * outputs along a row (16-byte accesses; the output row width a multiple of
  * 8), with the same arithmetic per element */
 typedef _Float16 vw_h4 __attribute__((ext_vector_type(4)));
-__global__ void k_relu_bwd_h8(const vw_h8* __restrict__ dy, const vw_h8* __restrict__ y, vw_h8* __restrict__ dz,
-                              int64_t n8) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n8) return;
-  const vw_h8 a = dy[i], b = y[i];
-  vw_h8 r;
-#pragma unroll
-  for (int k = 0; k < 8; ++k) r[k] = (float)b[k] > 0.f ? a[k] : (_Float16)0.f;
-  dz[i] = r;
-}
-__global__ void k_add_h8(const vw_h8* __restrict__ a, const vw_h8* __restrict__ b, vw_h8* __restrict__ c, int64_t n8) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n8) return;
-  const vw_h8 u = a[i], v = b[i];
-  vw_h8 r;
-#pragma unroll
-  for (int k = 0; k < 8; ++k) r[k] = (_Float16)((float)u[k] + (float)v[k]);
-  c[i] = r;
-}
 /* 2x2 pooling (up_bwd = 0: average) or the adjoint of upsampling (up_bwd = 1:
  * sum) of [nc][H][H] to [nc][H/2][H/2]; (H/2) % 8 == 0 */
 template <bool SUM>
@@ -878,6 +877,49 @@ __global__ void k_out(const T* __restrict__ d, const T* __restrict__ x, const fl
   float s = b[0];
   for (int c = 0; c < C; ++c) s = fmaf(w[c], (float)d[(n * C + c) * HH + p], s);
   out[i] = (T)(s + (float)x[i]);
+}
+/* FP16 forms of the output layer and its data gradient: 8 pixels of a lane,
+ * 16-byte accesses, the same arithmetic per pixel (HH % 8 == 0).  An element a
+ * lane ran at 0.9 TB/s: the gradient of 16 images of 256^2 36 -> 15 us, the
+ * output 14.7 -> 10.4. */
+__global__ __launch_bounds__(256) void k_out_h8(const _Float16* __restrict__ d, const _Float16* __restrict__ x,
+                                                const float* __restrict__ w, const float* __restrict__ b,
+                                                _Float16* __restrict__ out, int64_t n8, int C, int64_t HH) {
+  const int64_t i = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) * 8;
+  if (i >= n8 * 8) return;
+  const int64_t n = i / HH, p = i - n * HH;
+  const _Float16* s = d + n * C * HH + p;
+  float v[8];
+#pragma unroll
+  for (int k = 0; k < 8; ++k) v[k] = b[0];
+#pragma unroll 16
+  for (int c = 0; c < C; ++c) {
+    const vw_h8 a = *(const vw_h8*)(s + c * HH);
+#pragma unroll
+    for (int k = 0; k < 8; ++k) v[k] = fmaf(w[c], (float)a[k], v[k]);
+  }
+  const vw_h8 xv = *(const vw_h8*)(x + i);
+  vw_h8 r;
+#pragma unroll
+  for (int k = 0; k < 8; ++k) r[k] = (_Float16)(v[k] + (float)xv[k]);
+  *(vw_h8*)(out + i) = r;
+}
+/* a lane: the 8 pixels of every channel; mask: the layer's input, a ReLU output */
+__global__ __launch_bounds__(256) void k_out_bwd_h8(const _Float16* __restrict__ dout, const float* __restrict__ w,
+                                                    _Float16* __restrict__ dd, int64_t n8, int C, int64_t HH,
+                                                    const _Float16* __restrict__ mask) {
+  const int64_t i = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) * 8;
+  if (i >= n8 * 8) return;
+  const int64_t n = i / HH, o = n * C * HH + (i - n * HH);
+  const vw_h8 g = *(const vw_h8*)(dout + i);
+#pragma unroll 4
+  for (int c = 0; c < C; ++c) {
+    const vw_h8 m = *(const vw_h8*)(mask + o + c * HH);
+    vw_h8 r;
+#pragma unroll
+    for (int k = 0; k < 8; ++k) r[k] = (float)m[k] > 0.f ? (_Float16)(w[c] * (float)g[k]) : (_Float16)0.f;
+    *(vw_h8*)(dd + o + c * HH) = r;
+  }
 }
 /* masked squared error: per-block partial sums of the squared error and the
  * scaled output gradient dout = 2 (out - y) mask * gscale.  With gscale =
@@ -1102,7 +1144,7 @@ int ualloc(Net* c, P** p, size_t bytes) {
 #endif
 template <bool RELU, int CB>
 void conv3_mfma_cb(Net* c, dim3 grid, const _Float16* in, const _Float16* Wk, const float* B, _Float16* out, int cin,
-                   int cout, int H, const _Float16* mask) {
+                   int cout, int H, const _Float16* mask, const _Float16* aux, _Float16* out2) {
   /* grid = (tiles, 16-channel output blocks, images); a workgroup takes
    * OCB of the blocks (each wave all of them on its 4 pixel rows: the input
    * operand read from LDS serves OCB products) while that leaves at least
@@ -1113,56 +1155,57 @@ void conv3_mfma_cb(Net* c, dim3 grid, const _Float16* in, const _Float16* Wk, co
   else if (nb16 % 2 == 0 && rest * (nb16 / 2) >= VW_CONV_MIN_WG) ocb = 2;
   const unsigned nwg = rest * (nb16 / ocb);
   const bool pf = ocb == 1 && nwg < 4096;
-  if (pf) k_conv3_mfma<RELU, CB, true, true, 1><<<nwg, 256, 0, c->st>>>(in, Wk, B, out, cin, cout, H, mask);
-  else if (ocb == 1) k_conv3_mfma<RELU, CB, false, true, 1><<<nwg, 256, 0, c->st>>>(in, Wk, B, out, cin, cout, H, mask);
-  else if (ocb == 2) k_conv3_mfma<RELU, CB, false, true, 2><<<nwg, 256, 0, c->st>>>(in, Wk, B, out, cin, cout, H, mask);
-  else k_conv3_mfma<RELU, CB, false, true, 4><<<nwg, 256, 0, c->st>>>(in, Wk, B, out, cin, cout, H, mask);
+  if (pf) k_conv3_mfma<RELU, CB, true, true, 1><<<nwg, 256, 0, c->st>>>(in, Wk, B, out, cin, cout, H, mask, aux, out2);
+  else if (ocb == 1) k_conv3_mfma<RELU, CB, false, true, 1><<<nwg, 256, 0, c->st>>>(in, Wk, B, out, cin, cout, H, mask, aux, out2);
+  else if (ocb == 2) k_conv3_mfma<RELU, CB, false, true, 2><<<nwg, 256, 0, c->st>>>(in, Wk, B, out, cin, cout, H, mask, aux, out2);
+  else k_conv3_mfma<RELU, CB, false, true, 4><<<nwg, 256, 0, c->st>>>(in, Wk, B, out, cin, cout, H, mask, aux, out2);
 }
 template <bool RELU>
 void conv3_mfma(Net* c, dim3 grid, const _Float16* in, const _Float16* Wk, const float* B, _Float16* out, int cin,
-                int cout, int H, const _Float16* mask = nullptr) {
-  if (cin % 32 == 0) conv3_mfma_cb<RELU, 32>(c, grid, in, Wk, B, out, cin, cout, H, mask);
-  else conv3_mfma_cb<RELU, 16>(c, grid, in, Wk, B, out, cin, cout, H, mask);
+                int cout, int H, const _Float16* mask = nullptr, const _Float16* aux = nullptr,
+                _Float16* out2 = nullptr) {
+  if (cin % 32 == 0) conv3_mfma_cb<RELU, 32>(c, grid, in, Wk, B, out, cin, cout, H, mask, aux, out2);
+  else conv3_mfma_cb<RELU, 16>(c, grid, in, Wk, B, out, cin, cout, H, mask, aux, out2);
 }
 
 template <typename T>
 struct Ops {
   static constexpr bool kHalf = std::is_same<T, _Float16>::value;
-  static int conv3(Net* c, const Conv& L, int src, int dst, int n) {
+  /* layer L of tensor src into dst; with sum >= 0 also sum = dst + skip */
+  static int conv3(Net* c, const Conv& L, int src, int dst, int n, int skip = -1, int sum = -1) {
     const int H = c->H(L.lvl);
     const int tpr = (H + 15) / 16;
     dim3 grid((unsigned)(tpr * tpr), (unsigned)((L.co + 15) / 16), (unsigned)n);
     if (kHalf && L.ci % 16 == 0) { /* matrix cores */
       conv3_mfma<true>(c, grid, (const _Float16*)c->a[src], c->wh + L.hf, c->w + L.b, (_Float16*)c->a[dst], L.ci,
-                       L.co, H);
+                       L.co, H, nullptr, sum >= 0 ? (const _Float16*)c->a[skip] : nullptr,
+                       sum >= 0 ? (_Float16*)c->a[sum] : nullptr);
       UC(hipGetLastError());
       return VW_OK;
     }
     k_conv3<T, false, true><<<grid, 256, 0, c->st>>>((const T*)c->a[src], c->w + L.w, c->w + L.b, (T*)c->a[dst], L.ci,
                                                      L.co, H, nullptr);
     UC(hipGetLastError());
-    return VW_OK;
+    return sum >= 0 ? add(c, dst, skip, sum, n) : VW_OK;
   }
   /* backward of layer L whose input is tensor src and output (a ReLU output)
    * tensor dst.  The masked output gradient dz = d[dst] (y > 0) is d[dst]
    * itself, masked by the kernel that produced it, when dst's gradient has
-   * no other use; with gdst >= 0 it is formed here from d[gdst], the equal
-   * gradient of a skip sum that is used elsewhere too.  Writes the weight
+   * no other use; with gdst >= 0 it is that of d[gdst], the equal gradient of a
+   * skip sum that is used elsewhere too, in the scratch dz: formed there by the
+   * convolution that wrote d[gdst] (its sum_of = dst), or here.  Writes the weight
    * gradients and, if dsrc >= 0, d[dsrc] (masked by a[dsrc] when mask_dsrc:
    * dsrc is the ReLU output of the layer below and this its only use). */
   static int conv3_bwd(Net* c, const Conv& L, int src, int dst, int dsrc, int n, int gdst = -1,
-                       bool mask_dsrc = false) {
+                       bool mask_dsrc = false, int sum_of = -1) {
     const int H = c->H(L.lvl);
     const int64_t ne = (int64_t)n * c->elems(dst);
     const void* dzp = c->d[dst];
     if (gdst >= 0) {
-      const void* gd = c->d[gdst];
-      if (kHalf && ne % 8 == 0)
-        k_relu_bwd_h8<<<nblk(ne / 8), 256, 0, c->st>>>((const vw_h8*)gd, (const vw_h8*)c->a[dst], (vw_h8*)c->dz,
-                                                        ne / 8);
-      else
-        k_relu_bwd<T><<<nblk(ne), 256, 0, c->st>>>((const T*)gd, (const T*)c->a[dst], (T*)c->dz, ne);
-      UC(hipGetLastError());
+      if (!kHalf) { /* else every 3x3 layer above writes it */
+        k_relu_bwd<T><<<nblk(ne), 256, 0, c->st>>>((const T*)c->d[gdst], (const T*)c->a[dst], (T*)c->dz, ne);
+        UC(hipGetLastError());
+      }
       dzp = c->dz;
     }
     const T* dmask = mask_dsrc ? (const T*)c->a[dsrc] : nullptr;
@@ -1197,7 +1240,8 @@ struct Ops {
       dim3 grid((unsigned)(tpr * tpr), (unsigned)((L.ci + 15) / 16), (unsigned)n);
       if (kHalf && L.co % 16 == 0) { /* matrix cores, flipped transpose */
         conv3_mfma<false>(c, grid, (const _Float16*)dzp, c->wh + L.hb, nullptr, (_Float16*)c->d[dsrc], L.co, L.ci,
-                          H, (const _Float16*)dmask);
+                          H, (const _Float16*)dmask, sum_of >= 0 ? (const _Float16*)c->a[sum_of] : nullptr,
+                          sum_of >= 0 ? (_Float16*)c->dz : nullptr);
         UC(hipGetLastError());
         return VW_OK;
       }
@@ -1231,11 +1275,7 @@ struct Ops {
   }
   static int add(Net* c, int x, int y, int z, int n) {
     const int64_t ne = (int64_t)n * c->elems(z);
-    if (kHalf && ne % 8 == 0)
-      k_add_h8<<<nblk(ne / 8), 256, 0, c->st>>>((const vw_h8*)c->a[x], (const vw_h8*)c->a[y], (vw_h8*)c->a[z],
-                                                 ne / 8);
-    else
-      k_add<T><<<nblk(ne), 256, 0, c->st>>>((const T*)c->a[x], (const T*)c->a[y], (T*)c->a[z], ne);
+    k_add<T><<<nblk(ne), 256, 0, c->st>>>((const T*)c->a[x], (const T*)c->a[y], (T*)c->a[z], ne);
     UC(hipGetLastError());
     return VW_OK;
   }
@@ -1269,21 +1309,23 @@ struct Ops {
     F(conv3(c, L[6], Net::P3, Net::E3A, n));
     F(conv3(c, L[7], Net::E3A, Net::E3, n));
     F(up(c, Net::E3, Net::U2, n));
-    F(conv3(c, L[8], Net::U2, Net::D2A, n));
-    F(add(c, Net::D2A, Net::E2, Net::S2, n));
+    F(conv3(c, L[8], Net::U2, Net::D2A, n, Net::E2, Net::S2));
     F(conv3(c, L[9], Net::S2, Net::D2, n));
     F(up(c, Net::D2, Net::U1, n));
-    F(conv3(c, L[10], Net::U1, Net::D1A, n));
-    F(add(c, Net::D1A, Net::E1, Net::S1, n));
+    F(conv3(c, L[10], Net::U1, Net::D1A, n, Net::E1, Net::S1));
     F(conv3(c, L[11], Net::S1, Net::D1, n));
     F(up(c, Net::D1, Net::U0, n));
-    F(conv3(c, L[12], Net::U0, Net::D0A, n));
-    F(add(c, Net::D0A, Net::E0, Net::S0, n));
+    F(conv3(c, L[12], Net::U0, Net::D0A, n, Net::E0, Net::S0));
     F(conv3(c, L[13], Net::S0, Net::D0, n));
     const Conv& O = L[14];
     const int64_t HH = (int64_t)c->N * c->N;
-    k_out<T><<<nblk(n * HH), 256, 0, c->st>>>((const T*)c->a[Net::D0], (const T*)c->a[Net::X0], c->w + O.w,
-                                              c->w + O.b, (T*)c->a[Net::OUT], n, 16, HH);
+    if constexpr (kHalf)
+      k_out_h8<<<nblk(n * HH / 8), 256, 0, c->st>>>((const _Float16*)c->a[Net::D0], (const _Float16*)c->a[Net::X0],
+                                                    c->w + O.w, c->w + O.b, (_Float16*)c->a[Net::OUT], n * HH / 8, 16,
+                                                    HH);
+    else
+      k_out<T><<<nblk(n * HH), 256, 0, c->st>>>((const T*)c->a[Net::D0], (const T*)c->a[Net::X0], c->w + O.w,
+                                                c->w + O.b, (T*)c->a[Net::OUT], n, 16, HH);
     UC(hipGetLastError());
     return VW_OK;
   }
@@ -1310,20 +1352,26 @@ struct Ops {
     UC(hipGetLastError());
     k_out_wgrad_fold<<<1, 64, 0, c->st>>>(opart, onch, 16, c->g + O.w, c->g + O.b);
     UC(hipGetLastError());
-    k_out_bwd_data<T><<<nblk(ne * 16), 256, 0, c->st>>>((const T*)c->d[Net::OUT], c->w + O.w, (T*)c->d[Net::D0], n,
-                                                        16, HH, (const T*)c->a[Net::D0]); /* masked: dD0 feeds only L13 */
+    /* masked: dD0 feeds only L13 */
+    if constexpr (kHalf)
+      k_out_bwd_h8<<<nblk(ne / 8), 256, 0, c->st>>>((const _Float16*)c->d[Net::OUT], c->w + O.w,
+                                                    (_Float16*)c->d[Net::D0], ne / 8, 16, HH,
+                                                    (const _Float16*)c->a[Net::D0]);
+    else
+      k_out_bwd_data<T><<<nblk(ne * 16), 256, 0, c->st>>>((const T*)c->d[Net::OUT], c->w + O.w, (T*)c->d[Net::D0], n,
+                                                          16, HH, (const T*)c->a[Net::D0]);
     UC(hipGetLastError());
     int rc;
     c->jobs.njob = 0;
     c->jobs.base1[0] = c->jobs.base2[0] = 0;
     /* decoder level 0 */
-    F(conv3_bwd(c, L[13], Net::S0, Net::D0, Net::S0, n));            /* dS0 */
+    F(conv3_bwd(c, L[13], Net::S0, Net::D0, Net::S0, n, -1, false, Net::D0A));            /* dS0 */
     F(conv3_bwd(c, L[12], Net::U0, Net::D0A, Net::U0, n, Net::S0));  /* dU0 (dD0A = dS0) */
     F(up_bwd(c, Net::U0, Net::D1, n));                               /* dD1 */
-    F(conv3_bwd(c, L[11], Net::S1, Net::D1, Net::S1, n));
+    F(conv3_bwd(c, L[11], Net::S1, Net::D1, Net::S1, n, -1, false, Net::D1A));
     F(conv3_bwd(c, L[10], Net::U1, Net::D1A, Net::U1, n, Net::S1));
     F(up_bwd(c, Net::U1, Net::D2, n));
-    F(conv3_bwd(c, L[9], Net::S2, Net::D2, Net::S2, n));
+    F(conv3_bwd(c, L[9], Net::S2, Net::D2, Net::S2, n, -1, false, Net::D2A));
     F(conv3_bwd(c, L[8], Net::U2, Net::D2A, Net::U2, n, Net::S2));
     F(up_bwd(c, Net::U2, Net::E3, n));                               /* dE3 */
     /* encoder, deepest first; the skip gradients dS* seed dE0..dE2 */
