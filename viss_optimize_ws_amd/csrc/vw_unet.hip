@@ -124,6 +124,37 @@ __device__ __forceinline__ int64_t vu_xcd_block(int64_t b, int64_t nb) {
   return x * q + (x < r ? x : r) + i;
 }
 typedef _Float16 vw_h2 __attribute__((ext_vector_type(2)));
+/* 8 pixels of a row, `left` of which are in the image (zeros past them).  ALIGNED
+ * (H % 8 == 0): whole, on 16 bytes; else on any element, the row's tail one by
+ * one: staged and stored an element a lane, with a division each, four training
+ * steps of 14 images of 248^2 took 19.6 ms (now 18.1, of which most is their
+ * weight gradients), 11 of 104^2 13.8 (12.3). */
+template <bool ALIGNED>
+__device__ __forceinline__ vw_h8 vw_ld8(const _Float16* p, int left) {
+  vw_h8 v = {};
+  if (ALIGNED) return *(const vw_h8*)p;
+  if (left >= 8) {
+    __builtin_memcpy(&v, p, 16);
+  } else {
+#pragma unroll
+    for (int i = 0; i < 7; ++i)
+      if (i < left) v[i] = p[i];
+  }
+  return v;
+}
+template <bool ALIGNED>
+__device__ __forceinline__ void vw_st8(_Float16* p, vw_h8 v, int left) {
+  if (ALIGNED) {
+    *(vw_h8*)p = v;
+  } else if (left >= 8) {
+    __builtin_memcpy(p, &v, 16);
+  } else {
+#pragma unroll
+    for (int i = 0; i < 7; ++i)
+      if (i < left) p[i] = v[i];
+  }
+}
+
 /* The second output of a convolution, from the stored value and aux at its place:
  * forward (RELU) the skip sum v + aux, in the data gradient v where the ReLU
  * output aux is positive.  Written beside the first, they save the kernels that
@@ -135,7 +166,7 @@ __device__ __forceinline__ _Float16 vw_conv_second(_Float16 v, _Float16 aux) {
   return (float)aux > 0.f ? v : (_Float16)0.f;
 }
 template <bool RELU, int CB, bool PF, bool VS, int OCB>
-__global__ __launch_bounds__(256) void k_conv3_mfma(const _Float16* __restrict__ in, const _Float16* __restrict__ Wk,
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(OCB == 4 ? 2 : 3))) void k_conv3_mfma(const _Float16* __restrict__ in, const _Float16* __restrict__ Wk,
                                                     const float* __restrict__ B, _Float16* __restrict__ out, int cin,
                                                     int cout, int H, const _Float16* __restrict__ mask,
                                                     const _Float16* __restrict__ aux, _Float16* __restrict__ out2) {
@@ -174,9 +205,7 @@ __global__ __launch_bounds__(256) void k_conv3_mfma(const _Float16* __restrict__
      * 16-channel chunks, (tap, 16 channels) for lanes g < 2 and the next tap
      * for g >= 2); with PF all of them are issued before the staging loads so
      * their latency overlaps it (for launches too small to hide it by
-     * occupancy: PF costs registers), without PF one per k-step.  VS stages
-     * the tile with 16-byte loads of channel pairs (the element-wise form is
-     * kept for H % 8 != 0). */
+     * occupancy: PF costs registers), without PF one per k-step. */
     vw_h8 aw[PF ? STEPS : 1];
     if constexpr (PF) {
 #pragma unroll
@@ -187,7 +216,7 @@ __global__ __launch_bounds__(256) void k_conv3_mfma(const _Float16* __restrict__
         if (tap < 9 && ob + r < cout) aw[ks] = *(const vw_h8*)(Wk + ((int64_t)(ob + r) * K + tap * cin + c0 + ci0));
       }
     }
-    if (VS && H % 8 == 0) {
+    {
       /* every load of the tile is issued before the first is stored: one
        * memory latency a chunk instead of one per loop trip (5 or 8).
        * interior columns: a lane takes a channel pair and 8 pixels of one row
@@ -204,8 +233,8 @@ __global__ __launch_bounds__(256) void k_conv3_mfma(const _Float16* __restrict__
         const int cp = idx % NP, rest = idx / NP, gy = ty0 + (rest >> 1) - 1, gx = tx0 + 8 * (rest & 1);
         const bool on = idx < NP * 36 && gy >= 0 && gy < H && gx < H;
         const int off = on ? 2 * cp * (int)HH + gy * H + gx : 0;
-        v0[e] = *(const vw_h8*)(src + off);
-        v1[e] = *(const vw_h8*)(src + off + (int)HH);
+        v0[e] = vw_ld8<VS>(src + off, on ? H - gx : 0);
+        v1[e] = vw_ld8<VS>(src + off + (int)HH, on ? H - gx : 0);
         if (!on) v0[e] = v1[e] = vw_h8{};
       }
 #pragma unroll
@@ -231,15 +260,6 @@ __global__ __launch_bounds__(256) void k_conv3_mfma(const _Float16* __restrict__
         const int idx = threadIdx.x + 256 * e;
         const int c = idx % CB, rest = idx / CB;
         if (idx < CB * 36) tile[((rest >> 1) * 18 + (rest & 1 ? 17 : 0)) * LR + c] = hv[e];
-      }
-    } else {
-      __syncthreads();
-      for (int idx = threadIdx.x; idx < 324 * cb; idx += 256) {
-        const int c = idx / 324, q = idx - c * 324, yy = q / 18, xx = q - yy * 18;
-        const int gy = ty0 + yy - 1, gx = tx0 + xx - 1;
-        _Float16 v = (_Float16)0.f;
-        if (gy >= 0 && gy < H && gx >= 0 && gx < H) v = in[((int64_t)n * cin + c0 + c) * HH + (int64_t)gy * H + gx];
-        tile[(yy * 18 + xx) * LR + c] = v;
       }
     }
     __syncthreads();
@@ -287,16 +307,18 @@ __global__ __launch_bounds__(256) void k_conv3_mfma(const _Float16* __restrict__
           if (tap < 9 && o < cout) av[b] = *(const vw_h8*)(Wk + ((int64_t)o * K + tap * cin + c0 + ci0));
         }
         VW_CONV_KSTEP(av);
+        /* a step's weights ahead at most: all nine cost a wave a SIMD */
+        __builtin_amdgcn_sched_barrier(0);
       }
     }
 #undef VW_CONV_KSTEP
   }
-  /* D[4 g + i][r]: output channel ob + 4 g + i, pixel (4 wave + j, r).  With
-   * VS (H % 8 == 0: whole 16-pixel rows) the tile goes through LDS as
+  /* D[4 g + i][r]: output channel ob + 4 g + i, pixel (4 wave + j, r).  The
+   * tile goes through LDS as
    * [16 channels][16 rows][16 + 8 pixels] halves and leaves as 16-byte
    * stores of 8 pixels (with 16-byte mask loads), instead of 2-byte stores
    * of 16 lanes per channel row. */
-  if (VS && H % 8 == 0) {
+  {
     _Float16* ob_ = tile;
 #pragma unroll
     for (int b = 0; b < OCB; ++b) {
@@ -322,40 +344,21 @@ __global__ __launch_bounds__(256) void k_conv3_mfma(const _Float16* __restrict__
         vw_h8 v = *(const vw_h8*)(ob_ + (oc * 16 + yy) * 24 + 8 * hx);
         const int64_t oi = ((int64_t)n * cout + o) * HH + (int64_t)y * H + x;
         if (mask) {
-          const vw_h8 mk = *(const vw_h8*)(mask + oi);
+          const vw_h8 mk = vw_ld8<VS>(mask + oi, H - x);
 #pragma unroll
           for (int k = 0; k < 8; ++k)
             if (!((float)mk[k] > 0.f)) v[k] = (_Float16)0.f;
         }
-        *(vw_h8*)(out + oi) = v;
+        vw_st8<VS>(out + oi, v, H - x);
         if (out2) {
-          const vw_h8 x = *(const vw_h8*)(aux + oi);
+          const vw_h8 a = vw_ld8<VS>(aux + oi, H - x);
 #pragma unroll
-          for (int k = 0; k < 8; ++k) v[k] = vw_conv_second<RELU>(v[k], x[k]);
-          *(vw_h8*)(out2 + oi) = v;
+          for (int k = 0; k < 8; ++k) v[k] = vw_conv_second<RELU>(v[k], a[k]);
+          vw_st8<VS>(out2 + oi, v, H - x);
         }
       }
     }
-    return;
   }
-#pragma unroll
-  for (int b = 0; b < OCB; ++b)
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int y = ty0 + 4 * wave + j, x = tx0 + r;
-      if (y >= H || x >= H) continue;
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int o = ob + 16 * b + 4 * g + i;
-        if (o >= cout) continue;
-        float v = acc[b][j][i] + (B ? B[o] : 0.f);
-        if (RELU) v = v > 0.f ? v : 0.f;
-        const int64_t oi = ((int64_t)n * cout + o) * HH + (int64_t)y * H + x;
-        if (mask && !((float)mask[oi] > 0.f)) v = 0.f;
-        out[oi] = (_Float16)v;
-        if (out2) out2[oi] = vw_conv_second<RELU>((_Float16)v, aux[oi]);
-      }
-    }
 }
 
 /* FP16 weight layouts for the matrix-core convolution, all 3x3 layers in
@@ -546,7 +549,9 @@ __global__ __launch_bounds__(256) void k_conv3_wgrad_t(const T* __restrict__ in,
  * above, at and below it; the six input rows a wave needs are each read once
  * and applied to every (row, ky) they serve.  Partials [chunk][co][ci][10] as
  * for k_conv3_wgrad_t.  Requires H % 8 == 0 and co_n % 16 == 0; input
- * channels past ci_n are staged as zeros (the first layer has one). */
+ * channels past ci_n are staged as zeros (the first layer has one).  (Other
+ * sides through the same kernel train three times as fast, but sum in another
+ * order than k_conv3_wgrad_t, which Adam's first steps amplify to 1e-3.) */
 #define VW_WGM_SX (3 * 18 * 4 * 16) /* input chunks [kx][18 rows][4][16 ci] */
 #define VW_WGM_SG (16 * 4 * 16)     /* gradient chunks [16 rows][4][16 co] */
 __global__ __launch_bounds__(256) void k_conv3_wgrad_mfma(const _Float16* __restrict__ in,
@@ -1155,10 +1160,14 @@ void conv3_mfma_cb(Net* c, dim3 grid, const _Float16* in, const _Float16* Wk, co
   else if (nb16 % 2 == 0 && rest * (nb16 / 2) >= VW_CONV_MIN_WG) ocb = 2;
   const unsigned nwg = rest * (nb16 / ocb);
   const bool pf = ocb == 1 && nwg < 4096;
-  if (pf) k_conv3_mfma<RELU, CB, true, true, 1><<<nwg, 256, 0, c->st>>>(in, Wk, B, out, cin, cout, H, mask, aux, out2);
-  else if (ocb == 1) k_conv3_mfma<RELU, CB, false, true, 1><<<nwg, 256, 0, c->st>>>(in, Wk, B, out, cin, cout, H, mask, aux, out2);
-  else if (ocb == 2) k_conv3_mfma<RELU, CB, false, true, 2><<<nwg, 256, 0, c->st>>>(in, Wk, B, out, cin, cout, H, mask, aux, out2);
-  else k_conv3_mfma<RELU, CB, false, true, 4><<<nwg, 256, 0, c->st>>>(in, Wk, B, out, cin, cout, H, mask, aux, out2);
+  const bool al = H % 8 == 0;
+#define VW_CONV(PF_, VS_, OCB_) \
+  k_conv3_mfma<RELU, CB, PF_, VS_, OCB_><<<nwg, 256, 0, c->st>>>(in, Wk, B, out, cin, cout, H, mask, aux, out2)
+  if (pf) al ? VW_CONV(true, true, 1) : VW_CONV(true, false, 1);
+  else if (ocb == 1) al ? VW_CONV(false, true, 1) : VW_CONV(false, false, 1);
+  else if (ocb == 2) al ? VW_CONV(false, true, 2) : VW_CONV(false, false, 2);
+  else al ? VW_CONV(false, true, 4) : VW_CONV(false, false, 4);
+#undef VW_CONV
 }
 template <bool RELU>
 void conv3_mfma(Net* c, dim3 grid, const _Float16* in, const _Float16* Wk, const float* B, _Float16* out, int cin,
