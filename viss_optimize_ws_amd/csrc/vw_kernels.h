@@ -45,7 +45,7 @@ struct DevInfo {
   int64_t nuniq;
   int64_t first_nz;
   int64_t wtotal;
-  int32_t polar; /* 1: the plain recon's polar terms may be used (vw_polar_ok) */
+  int32_t polar; /* the recon's polar terms may be used: bit 0 plain, bit 1 mixed (vw_polar_ok) */
   int32_t pad;
 };
 
@@ -1356,9 +1356,13 @@ __global__ void k_conj_fill(const double2* __restrict__ vraw, const RowRec* __re
  * umax (2 + |fa| + |fb|) turns.  Below 2^22 turns that is under 1e-9 of the
  * maps; it stays below for baselines of 14,000 km at 30 MHz.  Beyond it, and for
  * the unbounded slopes of rows that span no plane, the plain recon keeps the
- * (re, im) terms and their rounding. */
+ * (re, im) terms and their rounding.  So does the mixed recon beyond 2^25 turns,
+ * up to where the difference, 2^-28 turns, stays an eighth of the rounding of
+ * its FP32 fraction (one row at 1 MHz, phases of 2^39 turns: polar terms 3.3e-4
+ * of the map off, the others below 5e-6). */
 __device__ __forceinline__ int vw_polar_ok(const vw_segparams& sp) {
-  return (double)sp.half * sp.du * (2.0 + fabs(sp.fa) + fabs(sp.fb)) <= 4194304.0;
+  const double turns = (double)sp.half * sp.du * (2.0 + fabs(sp.fa) + fabs(sp.fb));
+  return (turns <= 4194304.0 ? 1 : 0) | (turns <= 33554432.0 ? 2 : 0);
 }
 
 /* The five sums of the w-plane fit over the full rows, in 256 strided partial
@@ -2106,13 +2110,17 @@ struct ReconLane {
       }
     }
   }
-  /* the (re, im) form of a group's terms, point after point (plain form,
-   * segments without polar terms) with the sine table in global memory; use ==
+  /* the (re, im) form of a group's terms, point after point (segments without
+   * polar terms), in the plain form with the sine table in global memory; use ==
    * nullptr: every point */
   __device__ __forceinline__ void add_one(const GRec& g, const double2& v, const bool* use, const double* lp,
                                           const double* mp, const double2* __restrict__ gtab) {
 #pragma unroll
     for (int k = 0; k < PPL; ++k) {
+      if (MIXED) {
+        f[k].term_ri(use == nullptr || use[k], g.ugu, g.vgu, (float)v.x, (float)v.y, lp[k], mp[k]);
+        continue;
+      }
       int ix;
       const double fr = vw_tab_split(vw_recon_phase(g.ugu, g.vgu, lp[k], mp[k]) * VW_TAB_SCALE, &ix);
       const double2 e = gtab[ix];
@@ -2169,7 +2177,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(
   /* group positions fit 32 bits; uniform values keep the range tests scalar */
   const int64_t nu = a.mg.base[sg] + vw_rfl((int)info->nuniq);
   const int64_t q0 = a.mg.base[sg] + vw_rfl((int)info->first_nz);
-  const bool polar = vw_rfl(info->polar) != 0;
+  const bool polar = (vw_rfl(info->polar) & (MIXED ? 2 : 1)) != 0;
   /* group range of this chunk, aligned to 16 groups */
   const int64_t base = q0 & ~(int64_t)15;
   const int64_t nch = S.cst[sg + 1] - S.cst[sg];
@@ -2232,89 +2240,96 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(
       nia = a.g.gia[qa_ + (lane & 15)];
       nib = a.g.gib[qa_ + (lane & 15)];
     }
-    int buf = 0;
-    for (int q16 = (int)qa_; q16 < (int)qb_; q16 += 16, buf ^= 1) {
-      ring[buf * 64 + lane] = stage;
-      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-      __builtin_amdgcn_wave_barrier();
-      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-      uint64_t mw = nmw;
-      const int32_t cia = nia, cib = nib;
-      if (q16 + 16 < (int)qb_) {
-        stage = recd[(int64_t)(q16 + 16) * 4 + lane];
-        if (VW_KIND_IS_REP(KIND)) {
-          nmw = vw_rfl64(mrow[(q16 + 16) >> 4]);
-          if (BITS) {
-            nia = a.g.gia[q16 + 16 + (lane & 15)];
-            nib = a.g.gib[q16 + 16 + (lane & 15)];
+    /* the walk, built with and without the polar terms: a choice per term cost
+     * the mixed form 3% (Nside 256, 32 antennas, 64 epochs: 7.28 -> 7.51 ms) */
+    auto walk = [&](auto polar_) {
+      constexpr bool POLAR = decltype(polar_)::value;
+      int buf = 0;
+      for (int q16 = (int)qa_; q16 < (int)qb_; q16 += 16, buf ^= 1) {
+        ring[buf * 64 + lane] = stage;
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        uint64_t mw = nmw;
+        const int32_t cia = nia, cib = nib;
+        if (q16 + 16 < (int)qb_) {
+          stage = recd[(int64_t)(q16 + 16) * 4 + lane];
+          if (VW_KIND_IS_REP(KIND)) {
+            nmw = vw_rfl64(mrow[(q16 + 16) >> 4]);
+            if (BITS) {
+              nia = a.g.gia[q16 + 16 + (lane & 15)];
+              nib = a.g.gib[q16 + 16 + (lane & 15)];
+            }
           }
         }
-      }
-      if (KIND == VW_KIND_AVG) { /* every group of nonzero key, no classes */
-        const int lo = (int)q0 > q16 ? (int)q0 - q16 : 0, hi = (int)qb_ - q16 < 16 ? (int)qb_ - q16 : 16;
-        mw = ((1u << hi) - 1u) & ~((1u << lo) - 1u);
-      }
-      const GRec* blk = (const GRec*)(ring + buf * 64);
-      uint32_t vis = (uint32_t)mw & 0xffffu;
-      const uint32_t opa = (uint32_t)(mw >> 16) & 0xffffu, opb = (uint32_t)(mw >> 32);
-      uint32_t part = opa | opb;
-      if (KIND != VW_KIND_REP_FINITE) wu += (uint32_t)__builtin_popcount(vis);
-      while (vis) {
-        const int j = __builtin_ctz(vis);
-        vis &= vis - 1;
-        const GRec g = blk[j];
-        if (KIND == VW_KIND_REP_FINITE) {
-          if (!isfinite(g.amp)) continue;
-          wu += 1;
+        if (KIND == VW_KIND_AVG) { /* every group of nonzero key, no classes */
+          const int lo = (int)q0 > q16 ? (int)q0 - q16 : 0, hi = (int)qb_ - q16 < 16 ? (int)qb_ - q16 : 16;
+          mw = ((1u << hi) - 1u) & ~((1u << lo) - 1u);
         }
-        if (MIXED || polar) acc.template add<false>(g, nullptr, lp, mp);
-        else acc.add_one(g, a.g.v[q16 + j], nullptr, lp, mp, a.tab);
-      }
-      if (VW_KIND_IS_REP(KIND)) {
-        while (part) {
-          const int j = __builtin_ctz(part);
-          part &= part - 1;
+        const GRec* blk = (const GRec*)(ring + buf * 64);
+        uint32_t vis = (uint32_t)mw & 0xffffu;
+        const uint32_t opa = (uint32_t)(mw >> 16) & 0xffffu, opb = (uint32_t)(mw >> 32);
+        uint32_t part = opa | opb;
+        if (KIND != VW_KIND_REP_FINITE) wu += (uint32_t)__builtin_popcount(vis);
+        while (vis) {
+          const int j = __builtin_ctz(vis);
+          vis &= vis - 1;
           const GRec g = blk[j];
-          if (KIND == VW_KIND_REP_FINITE && !isfinite(g.amp)) continue;
-          bool use[PPL];
-          if constexpr (BITS) {
-            /* both frames' words, the one's twice where only it is open */
-            const int32_t fa = __builtin_amdgcn_readlane(cia, j), fb = __builtin_amdgcn_readlane(cib, j);
-            const uint64_t* va = fv + (int64_t)(opa >> j & 1 ? fa : fb) * fw;
-            const uint64_t* vb = fv + (int64_t)(opb >> j & 1 ? fb : fa) * fw;
+          if (KIND == VW_KIND_REP_FINITE) {
+            if (!isfinite(g.amp)) continue;
+            wu += 1;
+          }
+          if (POLAR) acc.template add<false>(g, nullptr, lp, mp);
+          else acc.add_one(g, a.g.v[q16 + j], nullptr, lp, mp, a.tab);
+        }
+        if (VW_KIND_IS_REP(KIND)) {
+          while (part) {
+            const int j = __builtin_ctz(part);
+            part &= part - 1;
+            const GRec g = blk[j];
+            if (KIND == VW_KIND_REP_FINITE && !isfinite(g.amp)) continue;
+            bool use[PPL];
+            if constexpr (BITS) {
+              /* both frames' words, the one's twice where only it is open */
+              const int32_t fa = __builtin_amdgcn_readlane(cia, j), fb = __builtin_amdgcn_readlane(cib, j);
+              const uint64_t* va = fv + (int64_t)(opa >> j & 1 ? fa : fb) * fw;
+              const uint64_t* vb = fv + (int64_t)(opb >> j & 1 ? fb : fa) * fw;
 #pragma unroll
-            for (int k = 0; k < PPL; ++k) use[k] = __builtin_amdgcn_inverse_ballot_w64(va[k] & vb[k]);
-          } else {
-            float fr[8];
+              for (int k = 0; k < PPL; ++k) use[k] = __builtin_amdgcn_inverse_ballot_w64(va[k] & vb[k]);
+            } else {
+              float fr[8];
 #pragma unroll
-            for (int e = 0; e < 8; ++e) fr[e] = a.g.ant32[(int64_t)(q16 + j) * 8 + e];
-            float vd[PPL], near_ = 4.f;
-#pragma unroll
-            for (int k = 0; k < PPL; ++k) {
-              vd[k] = vw_vis32(fl[k], fm[k], fn[k], fr);
-              near_ = fminf(near_, fabsf(vd[k]));
-              use[k] = vd[k] > 0.f;
-            }
-            if (__ballot(near_ <= VW_VIS_EPS)) { /* a point on the horizon: the FP64 test */
-              const double* d = a.g.ant + (int64_t)(q16 + j) * 10;
+              for (int e = 0; e < 8; ++e) fr[e] = a.g.ant32[(int64_t)(q16 + j) * 8 + e];
+              float vd[PPL], near_ = 4.f;
 #pragma unroll
               for (int k = 0; k < PPL; ++k) {
-                int ln = lane; /* opaque: the addresses are formed here, not kept in registers across the loop */
-                __asm__ volatile("" : "+v"(ln));
-                const int64_t pp = S.pt0 + (ok[k] ? pbase + ln + 64 * k : 0);
-                use[k] = vw_vis2<true>(ok[k], S.l[pp], S.m[pp], S.n[pp], d[0], d[1], d[2], d[3], d[4], d[5], d[6], d[7],
-                                       d[8], d[9]);
+                vd[k] = vw_vis32(fl[k], fm[k], fn[k], fr);
+                near_ = fminf(near_, fabsf(vd[k]));
+                use[k] = vd[k] > 0.f;
+              }
+              if (__ballot(near_ <= VW_VIS_EPS)) { /* a point on the horizon: the FP64 test */
+                const double* d = a.g.ant + (int64_t)(q16 + j) * 10;
+#pragma unroll
+                for (int k = 0; k < PPL; ++k) {
+                  int ln = lane; /* opaque: the addresses are formed here, not kept in registers across the loop */
+                  __asm__ volatile("" : "+v"(ln));
+                  const int64_t pp = S.pt0 + (ok[k] ? pbase + ln + 64 * k : 0);
+                  use[k] = vw_vis2<true>(ok[k], S.l[pp], S.m[pp], S.n[pp], d[0], d[1], d[2], d[3], d[4], d[5], d[6],
+                                         d[7], d[8], d[9]);
+                }
               }
             }
-          }
 #pragma unroll
-          for (int k = 0; k < PPL; ++k) wl[k] += use[k] ? 1 : 0;
-          if (MIXED || polar) acc.template add<true>(g, use, lp, mp);
-          else acc.add_one(g, a.g.v[q16 + j], use, lp, mp, a.tab);
+            for (int k = 0; k < PPL; ++k) wl[k] += use[k] ? 1 : 0;
+            if (POLAR) acc.template add<true>(g, use, lp, mp);
+            else acc.add_one(g, a.g.v[q16 + j], use, lp, mp, a.tab);
+          }
         }
+        if (MIXED && buf) acc.fold(); /* every 32 groups */
       }
-      if (MIXED && buf) acc.fold(); /* every 32 groups */
-    }
+    };
+    if (polar) walk(std::true_type{});
+    else walk(std::false_type{});
   } else {
     /* generic representative sets (viss_recon_kernel.cuh:603-614, isfinite filter) */
     for (int64_t q = (qa_ > q0 ? qa_ : q0); q < qb_; ++q) {
