@@ -1077,6 +1077,29 @@ int enq_frame_vis(Ctx* c, bool img, int64_t tile0, int64_t nt, uint32_t* out, hi
   return VW_OK;
 }
 
+/* Workgroups a tile for the one-sky recon's masks: one where the tiles fill the
+ * chip, else so many that all of them come to VW_MASK_TARGET_WG, each with at
+ * least VW_MASK_MIN_FRAMES frames.  Each makes the tile's cone bits anew (frame
+ * rows that fit LDS), which the plain form, with no points to test here, would
+ * only pay for (lunar segment of 2,796 epochs at Nside 64: 0.88 -> 0.93 ms): it
+ * shares a tile's groups where the bits come from their table.  With one
+ * workgroup a tile throughout, mixed recons of few tiles and many frames waited for
+ * one wave's walk over the frames.  Mixed recon stage, ms, one workgroup against
+ * shared: lunar segments of 699 epochs at Nside 16, 64, 128 0.36 0.20, 0.43 0.32,
+ * 0.69 0.59, of 2,796 at Nside 64 1.27 0.85; 2 antennas and a 64^2 image, 16,384
+ * epochs at Nside 8 1.25 0.32, 60,000 at Nside 32 4.89 0.91, 400,000 at Nside 8
+ * 31.6 3.5, at Nside 128 138 36.8. */
+#ifndef VW_MASK_TARGET_WG
+#define VW_MASK_TARGET_WG 4096
+#endif
+#ifndef VW_MASK_MIN_FRAMES
+#define VW_MASK_MIN_FRAMES 512
+#endif
+int64_t group_mask_parts(int64_t nt, int64_t nfr, int64_t nr, bool mixed, bool tile) {
+  const int64_t most = mixed ? (nfr + VW_MASK_MIN_FRAMES - 1) / VW_MASK_MIN_FRAMES : tile ? 1 : (nr + 1023) / 1024;
+  return std::max<int64_t>(1, std::min<int64_t>(most, VW_MASK_TARGET_WG / nt));
+}
+
 /* the one-sky recon's group masks of a pass ([nt][nq_pad / 16] 64-bit words per output
  * set) into the sets' class scratch */
 int enq_group_masks(Ctx* c, const ReconSets& sets, uint8_t* const* bits, uint64_t* ts) {
@@ -1090,7 +1113,7 @@ int enq_group_masks(Ctx* c, const ReconSets& sets, uint8_t* const* bits, uint64_
                                                                   c->nfr_pad, bits[i], nullptr);
     KC();
   }
-  const unsigned nb = (unsigned)nt;
+  const unsigned nb = (unsigned)(nt * group_mask_parts(nt, nfr, c->mg.base[c->mg.n], mixed, tile));
 #define VW_GM(TILE_, BITS_)                                                                                       \
   k_group_mask<TILE_, BITS_><<<nb, 256, TILE_ ? (size_t)c->nfr_pad : 0, c->stB>>>(                                 \
       c->mg, sets, c->d_ant8, nfr, c->nfr_pad, c->TP, c->gs.gia, c->gs.gib, c->d_info, c->nq_pad, ts)

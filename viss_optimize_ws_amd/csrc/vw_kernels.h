@@ -1835,8 +1835,9 @@ __device__ __forceinline__ uint64_t vw_frame_words(const double* __restrict__ an
  * Broadcasting the frames one by one and writing the decided frames' words too
  * took twice the time; points as scalar loads or lane by lane, a queue shared by
  * the workgroup, and further workgroups for 256 frames each, which test the
- * cones again, were no faster (337 us for 6,289 tiles x 2,048 frames). */
-__device__ __forceinline__ void vw_open_frames(const uint8_t* b, int64_t nfr, const double* __restrict__ ant8,
+ * cones again, were no faster where the tiles fill the chip (337 us for 6,289
+ * tiles x 2,048 frames).  Frames [f0, f1). */
+__device__ __forceinline__ void vw_open_frames(const uint8_t* b, int64_t f0, int64_t f1, const double* __restrict__ ant8,
                                                double pl, double pm, double pn, bool ok, double* pts /* [3][64] */,
                                                int32_t* queue /* [128] */, uint64_t* __restrict__ fo, int stride) {
   const int lane = threadIdx.x & 63;
@@ -1870,9 +1871,9 @@ __device__ __forceinline__ void vw_open_frames(const uint8_t* b, int64_t nfr, co
     settle();
   };
   int cnt = 0;
-  for (int64_t f0 = 0; f0 < nfr; f0 += 64) {
+  for (; f0 < f1; f0 += 64) {
     const int64_t f = f0 + lane;
-    const bool open = f < nfr && !(b[f] & 3);
+    const bool open = f < f1 && !(b[f] & 3);
     const uint64_t m = __ballot(open);
     if (open) queue[cnt + __popcll(m & ((1ull << lane) - 1))] = (int32_t)f;
     cnt += __popcll(m);
@@ -1905,7 +1906,9 @@ __device__ __forceinline__ void vw_open_frames(const uint8_t* b, int64_t nfr, co
  * as much as two terms and 26 registers (5 instead of 8 waves a SIMD): two Nside
  * 256 segments 24.3 -> 22.5 ms, the Nside 128 day 8.98 -> 8.56.  The plain form is
  * bound by its FP64 terms and gained nothing (Nside 256 -2%, short segments and
- * the lunar formation, with few groups a frame, +2 to 4%). */
+ * the lunar formation, with few groups a frame, +2 to 4%).
+ * A tile's frames and groups are shared by gridDim.x / tiles workgroups
+ * (group_mask_parts). */
 template <bool TILE, bool BITS>
 __global__ __launch_bounds__(256) void k_group_mask(VwMerge mg, ReconSets sets, const double* __restrict__ ant8, int64_t nfr,
                                                     int64_t nfr_pad, int64_t TP, const int32_t* __restrict__ ia,
@@ -1913,9 +1916,11 @@ __global__ __launch_bounds__(256) void k_group_mask(VwMerge mg, ReconSets sets, 
                                                     int64_t nq_pad, uint64_t* __restrict__ ts) {
   vw_ts_begin(ts);
   extern __shared__ uint4 sbits[];
-  const int si = (int)blockIdx.x >= (int)sets.s[0].nt;
+  const uint32_t ntot = (uint32_t)(sets.s[0].nt + sets.s[1].nt);
+  const uint32_t parts = gridDim.x / ntot, part = blockIdx.x / ntot, blk_t = blockIdx.x - part * ntot;
+  const int si = (int)blk_t >= (int)sets.s[0].nt;
   const ReconSet& S = sets.s[si];
-  const int64_t tr = blockIdx.x - (si ? sets.s[0].nt : 0);
+  const int64_t tr = blk_t - (si ? sets.s[0].nt : 0);
   const uint8_t* b = TILE ? (const uint8_t*)sbits : S.bits + tr * nfr_pad;
   if (TILE) {
     vw_tile_bits_lds((uint8_t*)sbits, S.cone, S.ntile, S.tile0 + tr, ant8, nfr);
@@ -1926,11 +1931,12 @@ __global__ __launch_bounds__(256) void k_group_mask(VwMerge mg, ReconSets sets, 
     __shared__ double spt[4][192];
     __shared__ int32_t squeue[4][128];
     const int nblk = (int)(TP / 64);
+    const int64_t per = ((nfr + parts - 1) / parts + 63) / 64 * 64, f0 = part * per;
     for (int blk = wave; blk < nblk; blk += 4) {
       const int64_t p = tr * TP + 64 * blk + lane; /* pass-relative */
       const bool ok = p < S.npts;
       const int64_t pp = S.pt0 + (ok ? p : 0);
-      vw_open_frames(b, nfr, ant8, S.l[pp], S.m[pp], S.n[pp], ok, spt[wave], squeue[wave],
+      vw_open_frames(b, f0, f0 + per < nfr ? f0 + per : nfr, ant8, S.l[pp], S.m[pp], S.n[pp], ok, spt[wave], squeue[wave],
                      S.fvis + tr * nfr_pad * nblk + blk, nblk);
     }
   }
@@ -1938,7 +1944,7 @@ __global__ __launch_bounds__(256) void k_group_mask(VwMerge mg, ReconSets sets, 
   for (int sg = 0; sg < mg.n; ++sg) {
     const int base = mg.base[sg], nu = base + vw_rfl((int)info[sg].nuniq), q0 = base + vw_rfl((int)info[sg].first_nz);
     const int qend = (nu + 63) / 64 * 64; /* <= nq_pad, a multiple of 64 */
-    for (int j0 = base + 256 * wave; j0 < qend; j0 += 1024) {
+    for (int j0 = base + 256 * (wave + 4 * (int)part); j0 < qend; j0 += 1024 * (int)parts) {
       int av[4], bv[4];
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
