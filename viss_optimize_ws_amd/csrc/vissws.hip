@@ -366,18 +366,26 @@ void size_buffers(Ctx* c) {
  * -> 405; three ragged segments of 715 rows 705 -> 661.  Short: the groups fit
  * k_group_one; runs end at VW_MERGE_ROWS rows, from where a launch fills the chip by itself
  * and the overlap of one run's recon with the next one's Viss is worth more.
+ * No more segments a run than a recon has group ranges: each has a range of its
+ * own, with 12 bytes a point of partial sums, and where there are few ranges
+ * (5 at Nside 512, one from Nside 1024 on) the points alone fill the chip.
  * The schedule's last segment stays alone: its rows and groups are what the
  * stage calls find after a step. */
 #define VW_MERGE_ROWS 4096
+struct ReconShape {
+  int64_t pwaves, nchunk;
+};
+ReconShape recon_shape(int64_t npts, int64_t nq = INT64_MAX);
 void plan_runs(Ctx* c) {
   const bool may = !c->batch && !c->generic && c->cfg.blockage;
   const int mul = c->cfg.recon_mode == VW_RECON_FULL ? 2 : 1;
+  const int64_t most = std::min<int64_t>(VW_MERGE_MAX, recon_shape(std::max(c->npix, c->ngp)).nchunk);
   c->runs.clear();
   int64_t rows = 0;
   for (int k = 0; k < c->segs; ++k) {
     const int64_t nr = (int64_t)mul * c->seg_tlen[k] * c->P;
     const bool short_ = may && nr <= VW_GROUP_ONE_MAX && k + 1 < c->segs;
-    const bool joins = short_ && rows > 0 && rows + nr <= VW_MERGE_ROWS && c->runs.back().second < VW_MERGE_MAX &&
+    const bool joins = short_ && rows > 0 && rows + nr <= VW_MERGE_ROWS && c->runs.back().second < most &&
                        c->seg_t0[k] == c->seg_t0[k - 1] + c->seg_tlen[k - 1];
     if (joins) {
       ++c->runs.back().second;
@@ -616,10 +624,7 @@ VissFShape viss_fshape(const Ctx* c, int64_t tlen, int64_t nt, int64_t lim = 0) 
 #define VW_RECON_PPL 4
 #endif
 constexpr int RECON_PPL = VW_RECON_PPL;
-struct ReconShape {
-  int64_t pwaves, nchunk;
-};
-ReconShape recon_shape(int64_t npts, int64_t nq = INT64_MAX) {
+ReconShape recon_shape(int64_t npts, int64_t nq) {
   ReconShape r;
   r.pwaves = (npts + 64 * RECON_PPL - 1) / (64 * RECON_PPL);
   const int64_t target_waves = VW_RECON_TARGET_WAVES;
@@ -963,13 +968,14 @@ int create_device(Ctx* c) {
         (c->cfg.precision == VW_PREC_PLAIN && ((rc = dalloc(c, &g.ant, 10 * nq)) || (rc = dalloc(c, &g.ant32, 8 * nq)))) ||
         (rc = dalloc(c, &g.gia, nq)) || (rc = dalloc(c, &g.gib, nq)) || (rc = dalloc(c, &g.grep, nq)))
       return rc;
-    int64_t rp = 1;
+    int64_t rp = 1, most = 0; /* segments of the longest merged run, each with a range of its own at least */
+    for (const auto& r : c->runs) most = std::max<int64_t>(most, r.second > 1 ? r.second : 0);
     for (int img = 0; img < 2; ++img) {
       const int64_t npts = img ? c->ngp : c->npix, nta = img ? c->ngt : c->ntile;
       if (npts <= 0) continue;
       const int64_t pp = recon_pass_tiles(c, nta, kind_w) * c->TP;
       const int64_t last = npts - (npts - 1) / pp * pp;
-      for (int64_t n : {std::min(npts, pp), last}) rp = std::max(rp, (recon_shape(n).nchunk + VW_MERGE_MAX) * n);
+      for (int64_t n : {std::min(npts, pp), last}) rp = std::max(rp, (recon_shape(n).nchunk + most) * n);
     }
     c->rpart_cap = rp;
     if ((rc = dalloc(c, &c->d_rpart, (size_t)rp)) || (rc = dalloc(c, &c->d_rwpart, (size_t)rp))) return rc;
