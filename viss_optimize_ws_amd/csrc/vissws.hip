@@ -1075,10 +1075,10 @@ int enq_classes(Ctx* c, const double* cone, int64_t ntile_all, int64_t tile0, in
  * grid, against the segment's antenna frames */
 int enq_frame_vis(Ctx* c, bool img, int64_t tile0, int64_t nt, uint32_t* out, hipStream_t st) {
   const int64_t nfr = (int64_t)c->tlen * c->A, nblk = nt * (c->TP / 64);
-  const dim3 grid((unsigned)((nblk + 3) / 4), (unsigned)((nfr + 63) / 64));
-  k_frame_vis<<<grid, 256, 0, st>>>(img ? c->d_gl : c->d_l, img ? c->d_gm : c->d_m, img ? c->d_gn : c->d_n,
-                                    img ? c->ngp : c->npix, img ? c->d_gcone : c->d_cone, img ? c->ngt : c->ntile,
-                                    tile0, nblk, c->TP, c->d_ant8, nfr, c->nfr_pad, out);
+  const unsigned nb = (unsigned)((nblk + 3) / 4 * ((nfr + 63) / 64));
+  k_frame_vis<<<nb, 256, 0, st>>>(img ? c->d_gl : c->d_l, img ? c->d_gm : c->d_m, img ? c->d_gn : c->d_n,
+                                  img ? c->ngp : c->npix, img ? c->d_gcone : c->d_cone, img ? c->ngt : c->ntile, tile0,
+                                  nblk, c->TP, c->d_ant8, nfr, c->nfr_pad, out);
   KC();
   return VW_OK;
 }

@@ -174,21 +174,24 @@ __global__ void k_group_keys(const int32_t* __restrict__ gia, const int32_t* __r
  * 256^2 image, against class bytes with the FP64 test in the term loops (a
  * divergent branch per masked term in the recon): k_reconb 22.3 -> 16.3 ms and
  * k_vissb 7.4 -> 6.5 ms of overlapped kernel time, the call 36.8 -> 33.8 ms,
- * results equal bit for bit. */
+ * results equal bit for bit.
+ * A one-dimensional grid, point blocks fastest: a second dimension ends at 65,536
+ * workgroups, 4.2 million frames. */
 __global__ __launch_bounds__(256) void k_frame_vis(const double* __restrict__ l, const double* __restrict__ m,
                                                    const double* __restrict__ n, int64_t npts,
                                                    const double* __restrict__ cone, int64_t ntile, int64_t tile0,
                                                    int64_t nblk, int64_t TP, const double* __restrict__ ant8,
                                                    int64_t nfr, int64_t nfr_pad, uint32_t* __restrict__ out) {
   const int lane = threadIdx.x & 63;
-  const int64_t b = (int64_t)blockIdx.x * 4 + vw_rfl((int)(threadIdx.x >> 6));
+  const uint32_t npb = (uint32_t)((nblk + 3) / 4), fb = blockIdx.x / npb;
+  const int64_t b = (int64_t)(blockIdx.x - fb * npb) * 4 + vw_rfl((int)(threadIdx.x >> 6));
   if (b >= nblk) return;
   const int64_t t = tile0 + b * 64 / TP;
   const int64_t p = tile0 * TP + b * 64 + lane;
   const bool ok = p < npts;
   const int64_t pp = ok ? p : npts - 1;
   const double pl = l[pp], pm = m[pp], pn = n[pp];
-  const int64_t f = (int64_t)blockIdx.y * 64 + lane;
+  const int64_t f = (int64_t)fb * 64 + lane;
   const double* q = ant8 + (f < nfr ? f : nfr - 1) * 8;
   const int cb = vw_cone_bits(q[4], q[5], q[6], cone[t], cone[ntile + t], cone[2 * ntile + t], cone[3 * ntile + t],
                               cone[4 * ntile + t], q[7]);
