@@ -86,20 +86,29 @@ class VwXfer {
     issued_.store(0);
     err_.store(0);
     for (int s = 0; s < nslot_; ++s) slot_done_[s].store(-1);
-    const bool helped = start();
     hipError_t e = hipSuccess;
-    for (int64_t c = 0; c < nchunk_ && e == hipSuccess; ++c) {
+    int64_t c = 0;
+    auto issue = [&] {
+      const int s = (int)(c % nslot_);
+      const Seg g = chunk(c);
+      e = hipMemcpyAsync(ring_ + chunk_ * (size_t)s, g.dev, g.bytes, hipMemcpyDeviceToHost, st);
+      if (e == hipSuccess) e = hipEventRecord(ev_[s], st);
+      if (e == hipSuccess) issued_.store(++c, std::memory_order_release);
+    };
+    while (c < nslot_ && c < nchunk_ && e == hipSuccess) issue();
+    /* the kernels before the results may run for long: until the first chunk is
+     * there this thread waits alone, as for a plain copy, and no helper polls */
+    if (e == hipSuccess) e = hipEventSynchronize(ev_[0]);
+    const bool helped = e == hipSuccess && start();
+    while (c < nchunk_ && e == hipSuccess) {
       const int s = (int)(c % nslot_);
       /* the slot's last chunk has to be out: take a chunk on meanwhile */
-      while (c >= nslot_ && slot_done_[s].load(std::memory_order_acquire) != c - nslot_) {
+      while (slot_done_[s].load(std::memory_order_acquire) != c - nslot_) {
         int64_t k = next_.load();
         if (k < c && next_.compare_exchange_strong(k, k + 1)) finish(k);
         else pause();
       }
-      const Seg g = chunk(c);
-      e = hipMemcpyAsync(ring_ + chunk_ * (size_t)s, g.dev, g.bytes, hipMemcpyDeviceToHost, st);
-      if (e == hipSuccess) e = hipEventRecord(ev_[s], st);
-      if (e == hipSuccess) issued_.store(c + 1, std::memory_order_release);
+      issue();
     }
     if (e != hipSuccess) {
       err_.store(1);
