@@ -27,6 +27,7 @@
 #define VW_KERNELS_H
 
 #include <hip/hip_runtime.h>
+#include <float.h>
 #include <stdint.h>
 #include <type_traits>
 #include "vw_shared.h"
@@ -1703,7 +1704,7 @@ __global__ void k_group_data(VwMerge mg, const int64_t* __restrict__ gkeys, cons
                              const int32_t* __restrict__ idx_sorted, const double2* __restrict__ vh,
                              const RowRec* __restrict__ rows, const double* __restrict__ ant8, int P, int full,
                              int blockage, int occ_mode, double uv_scale,
-                             const DevInfo* __restrict__ info, GroupSoA g, uint64_t* __restrict__ ts) {
+                             DevInfo* __restrict__ info, GroupSoA g, uint64_t* __restrict__ ts) {
   vw_ts_begin(ts);
   int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   int base = 0, row0 = 0;
@@ -1752,9 +1753,14 @@ __global__ void k_group_data(VwMerge mg, const int64_t* __restrict__ gkeys, cons
   GRec gr;
   gr.ugu = ugu * uv_scale; /* 1024 for the plain generic kind's table sincos, else 1 (exact) */
   gr.vgu = vgu * uv_scale;
-  /* finite parts give a finite magnitude (the finite-value filter reads it);
-   * a part that is not finite makes every term NaN */
-  gr.amp = isfinite(vr) && isfinite(vi) ? fmin(hypot(vr, vi), 0x1.fffffffffffffp1020) : NAN;
+  /* finite parts give a finite magnitude, others none: the finite-value filter
+   * reads it.  A magnitude past what the polar terms hold (2 |V| from each of 32
+   * groups before a fold in FP64, |V| in FP32), or infinite parts, leave the
+   * segment to the (re, im) terms, which overflow where the sum of the parts does;
+   * a NaN is NaN in both */
+  const double mag = hypot(vr, vi);
+  gr.amp = isfinite(vr) && isfinite(vi) ? fmin(mag, DBL_MAX) : NAN;
+  if (!isnan(vr) && !isnan(vi) && !(mag <= FLT_MAX)) atomicAnd(&info->polar, mag < 0x1p1000 ? 1 : 0);
   gr.arg = atan2(vi, vr) * VW_INV_TWOPI;
   g.rec[q] = gr;
   g.v[q] = make_double2(vr, vi);
