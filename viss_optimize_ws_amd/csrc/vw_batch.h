@@ -167,8 +167,12 @@ __global__ void k_group_keys(const int32_t* __restrict__ gia, const int32_t* __r
  * occlusion test runs once per (point, frame) instead of twice per masked term
  * (an epoch's A frames serve A (A - 1) / 2 rows), and the term loops of the
  * products hold no test.  A frame that the tile's cone finds all visible or
- * all hidden needs none at all; bits are the per-point FP64 test's otherwise,
- * so a mask equals the pair class with its per-point tests.
+ * all hidden needs none at all; bits are the per-point FP64 test's otherwise.  A
+ * mask so equals the pair class with its per-point tests, but for a point at the
+ * far end of a cone whose rounded bound passes the frame by less than the point
+ * fails it (1e-15; bit 2 of vw_cone_bits): the class tests it for a pair whose
+ * other frame is partly visible, and passes it for one whose other frame is all
+ * visible; a frame has one word for both, and passes it here.
  * A wave owns 64 points and 64 frames (vw_frame_words); 50 us for 196,608
  * points x 2,080 frames.  64 skies at Nside 128, 16 antennas, 205 epochs and a
  * 256^2 image, against class bytes with the FP64 test in the term loops (a

@@ -1834,15 +1834,15 @@ __device__ __forceinline__ uint64_t vw_frame_words(const double* __restrict__ an
   return word;
 }
 
-/* Occlusion bits of the frames that a tile's cone leaves open (b: the tile's
- * cone bits), for one block of 64 points, by one wave: fo[f * stride], bit j =
- * point j is seen from frame f.  The wave gathers open frames in LDS and takes
- * 64 at a time, a lane a frame, against the points in turn (LDS broadcasts).
- * Broadcasting the frames one by one and writing the decided frames' words too
- * took twice the time; points as scalar loads or lane by lane, a queue shared by
- * the workgroup, and further workgroups for 256 frames each, which test the
- * cones again, were no faster where the tiles fill the chip (337 us for 6,289
- * tiles x 2,048 frames).  Frames [f0, f1). */
+/* Occlusion bits of the frames that a tile's cone leaves open, neither hidden nor
+ * visible by more than rounding (b: the tile's cone bits), for one block of 64
+ * points, by one wave: fo[f * stride], bit j = point j is seen from frame f.  The
+ * wave gathers open frames in LDS and takes 64 at a time, a lane a frame, against
+ * the points in turn (LDS broadcasts).  Broadcasting the frames one by one and
+ * writing the decided frames' words too took twice the time; points as scalar
+ * loads or lane by lane, a queue shared by the workgroup, and further workgroups
+ * for 256 frames each, which test the cones again, were no faster where the tiles
+ * fill the chip (337 us for 6,289 tiles x 2,048 frames).  Frames [f0, f1). */
 __device__ __forceinline__ void vw_open_frames(const uint8_t* b, int64_t f0, int64_t f1, const double* __restrict__ ant8,
                                                double pl, double pm, double pn, bool ok, double* pts /* [3][64] */,
                                                int32_t* queue /* [128] */, uint64_t* __restrict__ fo, int stride) {
@@ -1879,7 +1879,7 @@ __device__ __forceinline__ void vw_open_frames(const uint8_t* b, int64_t f0, int
   int cnt = 0;
   for (; f0 < f1; f0 += 64) {
     const int64_t f = f0 + lane;
-    const bool open = f < f1 && !(b[f] & 3);
+    const bool open = f < f1 && !(b[f] & 6);
     const uint64_t m = __ballot(open);
     if (open) queue[cnt + __popcll(m & ((1ull << lane) - 1))] = (int32_t)f;
     cnt += __popcll(m);
@@ -1897,9 +1897,9 @@ __device__ __forceinline__ void vw_open_frames(const uint8_t* b, int64_t f0, int
 /* The one-sky recon's form of the same classes: per (tile, 16 groups) one
  * 64-bit word, bit j = group j is visible from the whole tile, bits 16 + j and
  * 32 + j = it is partly, with its first, its second antenna's frame left open
- * by the tile's cone; hidden groups, groups below first_nz (the key-0 group) and
- * past nuniq have none of them, so the recon walks set bits and needs no range
- * test.  TILE: one block per tile
+ * by the tile's cone (not visible by more than rounding); hidden groups, groups
+ * below first_nz (the key-0 group) and past nuniq have none of them, so the recon
+ * walks set bits and needs no range test.  TILE: one block per tile
  * makes the tile's cone bits in LDS (frame rows up to VW_GCLS_LDS_MAX bytes);
  * else they come from the bit table of the pass.  A wave takes 4 x 64 groups
  * at a time, a lane one group of each 64 (coalesced index loads, all issued
@@ -1907,7 +1907,7 @@ __device__ __forceinline__ void vw_open_frames(const uint8_t* b, int64_t f0, int
  * below nuniq rounded up to 64 are written: the recon reads no others.
  * BITS (mixed form): the block also writes the open frames' occlusion bits
  * (vw_open_frames), whose AND over a partly visible group's open frames is its
- * mask; the recon loads the words as scalars.  Testing both antennas of every
+ * mask, the same as the two tests of each point; the recon loads the words as scalars.  Testing both antennas of every
  * (point, group) in FP32, with an FP64 fallback, as the plain form does, cost it
  * as much as two terms and 26 registers (5 instead of 8 waves a SIMD): two Nside
  * 256 segments 24.3 -> 22.5 ms, the Nside 128 day 8.98 -> 8.56.  The plain form is
@@ -1965,8 +1965,8 @@ __global__ __launch_bounds__(256) void k_group_mask(VwMerge mg, ReconSets sets, 
         const bool in = q >= q0 && q < nu;
         const int ba = b[av[e]], bb = b[bv[e]], c = vw_pair_class(ba, bb);
         const uint64_t v = __ballot(in && c == VW_CLS_VISIBLE);
-        const uint64_t ma = __ballot(in && c == VW_CLS_MIXED && !(ba & 1));
-        const uint64_t mb = __ballot(in && c == VW_CLS_MIXED && !(bb & 1));
+        const uint64_t ma = __ballot(in && c == VW_CLS_MIXED && !(ba & 4));
+        const uint64_t mb = __ballot(in && c == VW_CLS_MIXED && !(bb & 4));
         if (lane < 4 && j0 + 64 * e < qend) {
           const int sh = 16 * lane;
           out[((j0 + 64 * e) >> 4) + lane] =

@@ -296,7 +296,8 @@ VW_HD double vw_cosphi_from_altitude(double R, double h) {
   return -sqrt(fma(-q, q, 1.0));
 }
 
-/* One antenna against a tile cone: bit0 = all visible, bit1 = all hidden.
+/* One antenna against a tile cone: bit0 = all visible, bit1 = all hidden, bit2 =
+ * all visible whatever the rounding (VW_CONE_MARGIN).
  * classify_tile_cone (vissfast .cuh:91-98): with d = cos(delta) the angle to
  * the cone axis and A the cone half-angle, the extremes of s.u over the cone
  * are cos(delta + A) and cos(delta - A) while delta + A <= pi and A <= delta.
@@ -304,7 +305,12 @@ VW_HD double vw_cosphi_from_altitude(double R, double h) {
  * the reference formula is not conservative there (cones wider than a few
  * tens of degrees, e.g. 256-pixel tiles at Nside <= 8), so those two cases
  * clamp to -1 / +1.  For the small tiles of the production configurations
- * this is the reference's classification unchanged. */
+ * this is the reference's classification unchanged.
+ * bit0 is the bound as rounded, and a point at the far end of the cone can fail
+ * its own test where bit0 is set: sind and sinA are roots of differences, off by
+ * up to 3e-8 where they vanish, everything else by a few 1e-16.  With bit2 every
+ * point passes. */
+#define VW_CONE_MARGIN 1e-7
 VW_HD int vw_cone_bits(double ux, double uy, double uz, double cx, double cy, double cz,
                        double cosA, double sinA, double cosphi) {
   double d = vw_clamp1(vw_dot3(ux, uy, uz, cx, cy, cz));
@@ -312,7 +318,7 @@ VW_HD int vw_cone_bits(double ux, double uy, double uz, double cx, double cy, do
   double ss = sind * sinA;
   double lower = (cosA + d <= 0.0) ? -1.0 : fma(d, cosA, -ss);
   double upper = (cosA <= d) ? 1.0 : fma(d, cosA, ss);
-  return (lower >= cosphi ? 1 : 0) | (upper < cosphi ? 2 : 0);
+  return (lower >= cosphi ? 1 : 0) | (upper < cosphi ? 2 : 0) | (lower >= cosphi + VW_CONE_MARGIN ? 4 : 0);
 }
 
 /* Pair class from the two endpoint bit sets (vissfast .cuh:521-527). */
