@@ -142,7 +142,8 @@ typedef struct {
 } vw_geom_host;
 
 /* Device time of the last completed stage calls (ms): time stamps of the stages'
- * kernels, HIP events in batched contexts.  vw_run_all of one sky has no
+ * kernels, HIP events in batched contexts.  A kernel's time of a one-sky context
+ * may hold the tail of the small kernel before it.  vw_run_all of one sky has no
  * separate conjugate fill (conj_ms 0: part of viss_ms). */
 typedef struct {
   double gen_ms, viss_ms, conj_ms, group_ms, recon_ms, finalize_ms;

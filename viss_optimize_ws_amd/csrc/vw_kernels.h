@@ -69,8 +69,12 @@ __device__ __forceinline__ uint64_t vw_rfl64(uint64_t x) {
 
 /* Stage timing: the small kernels around a stage's large one write the device's
  * real-time counter to two words of host memory, ts[0] as the first workgroup
- * starts and ts[1] as the last one ends (ts may be null).  The large kernel's
- * time runs from the end of the kernel before it to the start of the one after.
+ * starts and ts[1] as the highest-numbered one ends (ts may be null).  The large
+ * kernel's time runs from the latter of the kernel before it to the start of the
+ * one after: all of the large kernel, and what the workgroups of the kernel before
+ * it still do after its highest-numbered one.  (A stamp of the large kernel's own
+ * start, a store before its loads, took the scalar loads of k_recon: 63 to 78
+ * registers, 8 to 6 waves.)
  * Events recorded around every stage cost a barrier packet and a call each: a
  * whole run at Nside 32 went from 716 to 527 us, a one-segment predict with
  * adjoint at Nside 64 from 1000 to 845 us. */
@@ -370,7 +374,6 @@ __global__ __launch_bounds__(256) void k_classify(const uint8_t* __restrict__ bi
   }
   __syncthreads();
   const int64_t h0 = hb + 4 * threadIdx.x;
-  vw_ts_end(ts);
   if (h0 >= nh_pad) return; /* nh_pad is a multiple of 64: whole words only */
   const int4 p0 = sab[2 * threadIdx.x], p1 = sab[2 * threadIdx.x + 1];
   const int av[4] = {p0.x, p0.z, p1.x, p1.z}, bv[4] = {p0.y, p0.w, p1.y, p1.w};
@@ -382,6 +385,7 @@ __global__ __launch_bounds__(256) void k_classify(const uint8_t* __restrict__ bi
     w |= (h0 + e < nh ? c : (uint32_t)VW_CLS_HIDDEN) << (8 * e);
   }
   cls[((int64_t)tr * nh_pad + h0) >> 2] = w;
+  vw_ts_end(ts); /* thread 0 of a workgroup has rows */
 }
 
 /* k_classify with the cone bits made in place: one block per tile of the
