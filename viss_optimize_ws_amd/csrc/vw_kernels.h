@@ -1701,7 +1701,7 @@ struct GroupSoA {
   double2* v;   /* the visibility as (re, im), for segments without polar terms */
   double* ant;  /* [q][10]: representative's antenna frames a and b (plain form; */
   float* ant32; /* [q][8]: in FP32, vw_frame32; null in the mixed form)        */
-  int32_t *gia, *gib, *grep; /* the representative's frames' indices, its half row */
+  int32_t *gia, *gib; /* the representative's frames' indices */
 };
 
 __global__ void k_group_data(VwMerge mg, const int64_t* __restrict__ gkeys, const int32_t* __restrict__ goff,
@@ -1768,7 +1768,6 @@ __global__ void k_group_data(VwMerge mg, const int64_t* __restrict__ gkeys, cons
   gr.arg = atan2(vi, vr) * VW_INV_TWOPI;
   g.rec[q] = gr;
   g.v[q] = make_double2(vr, vi);
-  g.grep[q] = (int32_t)hr;
   RowRec r = rows[hr];
   g.gia[q] = r.ia;
   g.gib[q] = r.ib;
