@@ -1,7 +1,7 @@
 /*
  * vissws.hip -- host orchestration and C-ABI of the gfx950 path
- * (include/vissws.h).  Three HIP streams per context, all at default
- * priority (geometry + Viss; grouping + HEALPix recon; lm-image recon); all
+ * (include/vissws.h).  Two HIP streams per context, all at default priority
+ * (geometry + Viss; grouping + recon), three in batched ones (lm-image recon); all
  * device memory is allocated once in vw_create and sized for the longest
  * segment, so the segment loop performs no allocation.  Stage functions
  * enqueue work; the public entry points synchronise before returning.
@@ -60,9 +60,10 @@ struct Ctx {
   /* device */
   hipStream_t st = nullptr;
   /* streams: st carries the segment geometry, Viss and conjugate fill; stB
-   * the grouping and HEALPix recon; st2 the lm-image recon.  The recon of
-   * segment s thus runs beside the Viss of segment s+1 (the segment
-   * buffers alternate between two sets) */
+   * the grouping and recon (a launch of the one-sky recon covers both output
+   * sets).  The recon of segment s thus runs beside the Viss of segment s+1 (the
+   * segment buffers alternate between two sets).  st2, of batched contexts alone:
+   * the lm-image recon beside the HEALPix one, between ev_fork and ev_join */
   hipStream_t stB = nullptr;
   hipStream_t st2 = nullptr;
   hipEvent_t ev_fork = nullptr, ev_join = nullptr, ev_conj = nullptr, ev_gen = nullptr;
@@ -854,11 +855,13 @@ int create_device(Ctx* c) {
   if (c->cfg.serial_stages) {
     c->st2 = c->stB = c->st; /* one stream: the stream waits below are no-ops */
   } else {
-    HC(hipStreamCreateWithFlags(&c->st2, hipStreamNonBlocking));
+    if (c->batch) HC(hipStreamCreateWithFlags(&c->st2, hipStreamNonBlocking));
     HC(hipStreamCreateWithFlags(&c->stB, hipStreamNonBlocking));
   }
-  HC(hipEventCreateWithFlags(&c->ev_fork, hipEventDisableTiming));
-  HC(hipEventCreateWithFlags(&c->ev_join, hipEventDisableTiming));
+  if (c->batch) {
+    HC(hipEventCreateWithFlags(&c->ev_fork, hipEventDisableTiming));
+    HC(hipEventCreateWithFlags(&c->ev_join, hipEventDisableTiming));
+  }
   HC(hipEventCreateWithFlags(&c->ev_conj, hipEventDisableTiming));
   HC(hipEventCreateWithFlags(&c->ev_gen, hipEventDisableTiming));
   for (int b = 0; b < 2; ++b) HC(hipEventCreateWithFlags(&c->ev_recon[b], hipEventDisableTiming));
@@ -966,7 +969,7 @@ int create_device(Ctx* c) {
     GroupSoA& g = c->gs;
     if ((rc = dalloc(c, &g.rec, nq)) || (rc = dalloc(c, &g.v, nq)) ||
         (c->cfg.precision == VW_PREC_PLAIN && ((rc = dalloc(c, &g.ant, 10 * nq)) || (rc = dalloc(c, &g.ant32, 8 * nq)))) ||
-        (rc = dalloc(c, &g.gia, nq)) || (rc = dalloc(c, &g.gib, nq)) || (rc = dalloc(c, &g.grep, nq)))
+        (rc = dalloc(c, &g.gia, nq)) || (rc = dalloc(c, &g.gib, nq)))
       return rc;
     int64_t rp = 1, most = 0; /* segments of the longest merged run, each with a range of its own at least */
     for (const auto& r : c->runs) most = std::max<int64_t>(most, r.second > 1 ? r.second : 0);
