@@ -42,8 +42,10 @@ extern "C" {
 #define VW_RECON_FULL 1   /* full uv grid  (main_recon_online.cu)         */
 
 /* Viss summation form (vw_config.viss_form) */
-#define VW_VISS_AUTO 0      /* per-row sums in the plain form; antenna-factorized in the mixed form
-                             * for n_ant <= 32                                                   */
+#define VW_VISS_AUTO 0      /* antenna-factorized in the mixed form for n_ant <= 32; in the plain form
+                             * for circular orbits with 13-16 or 22-32 antennas, baselines
+                             * (2 r_max) of up to 1.5e6 wavelengths and a finite sky; else per-row
+                             * sums                                                              */
 #define VW_VISS_ROWS 1      /* one phase / sin / cos term per (half row, pixel): the reference's
                              * phase rounding, bit for bit                                       */
 #define VW_VISS_ANT 2       /* antenna-factorized on the matrix cores in either form (n_ant <= 32);

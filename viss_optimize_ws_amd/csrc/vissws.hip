@@ -304,13 +304,14 @@ int sync(Ctx* c) {
  * factorized, ms: 12 antennas 0.298 0.309 / 0.490 0.579, 13 0.345 0.311 / 0.588
  * 0.583, 16 0.465 0.314 / 0.825 0.583; 20 0.691 0.734 / 1.234 1.403, 22 0.838
  * 0.741 / 1.512 1.410, 32 1.650 0.758 / 2.939 1.409.  So 13-16 and 22-32.
- * Both forms hold the same sums; each row's phase is rounded where the row form
- * rounds it, by up to 2^-53 of the longest baseline in turns several times
- * over.  At 4.7e5 turns (14,000 km at 10 MHz) that is 1.4e-10 of the
- * visibilities, at 1.4e6 (30 MHz) 4.7e-10; longer baselines keep the row form
- * and its rounding.  So do
- * skies that are not finite: a product with a masked weight would spread a NaN
- * to rows that do not see its pixel (enq_viss). */
+ * Both forms hold the same sums and are as far from the exact ones: their phases
+ * are rounded at different places, by 2^-53 of the baseline in turns a few times
+ * over.  The limit is one of agreement, not of accuracy: plain visibilities are
+ * held to 1e-9 of the row sums, and the forms differ by 1.4e-10 of the peak at
+ * 4.7e5 turns (14,000 km at 10 MHz) and by 4.7e-10 at 1.4e6 (30 MHz), so beyond
+ * about that the row form's roundings stay.  So do those of skies that are not
+ * finite: a product with a masked weight would spread a NaN to rows that do not
+ * see its pixel (enq_viss). */
 #define VW_FACT_MAX_TURNS 1.5e6
 bool fact_auto_plain(const vw_config* cfg, double lambda) {
   if (cfg->viss_form != VW_VISS_AUTO || cfg->precision != VW_PREC_PLAIN || cfg->geometry != VW_GEOM_CIRCULAR) return false;
@@ -430,7 +431,7 @@ int make_plan(Ctx* c, const vw_config* cfg) {
   c->P = c->A * (c->A - 1) / 2;
   /* automatic choice: the factorized form for the mixed precision (per
    * segment, Nside 128 / 16 antennas 0.16 against 0.30 ms, Nside 256 / 32
-   * antennas 3.0 against 7.0 ms); the plain form keeps the per-row phases */
+   * antennas 3.0 against 7.0 ms), for the plain one by fact_auto_plain */
   c->vfact = c->A <= 32 && (cfg->viss_form == VW_VISS_ANT || cfg->viss_form == VW_VISS_ANT_CHECK ||
                             (cfg->viss_form == VW_VISS_AUTO && cfg->precision == VW_PREC_MIXED));
   c->lambda = 3e8 / cfg->freq_hz;
