@@ -29,8 +29,9 @@ on a bounded sample.  Beside it on the same line:
     Viss and recon as BF16 hi/lo matrix-core products of on-the-fly phasor
     tiles against the sky / group-visibility matrix.
 Rooflines: kernel averages come from steps run with every stage on one stream
-(each kernel alone), HIP events recorded on the library's stream around each
-launch; `--legs` and `--serial` reproduce one leg for a rocprofv3 run.
+(each kernel alone), between device time stamps of the launches around it (HIP
+events in the batched form); `--legs` and `--serial` reproduce one leg for a
+rocprofv3 run.
 """
 import argparse
 import json
@@ -67,22 +68,23 @@ FP32_PEAK_TFLOPS = 157.3   # vector FP32: 32 lanes per SIMD (a wave64 FP32 FMA i
 BF16_PEAK_TFLOPS = 2500.0  # dense BF16 matrix cores
 FP64_INSTR_PEAK_T = FP64_PEAK_TFLOPS / 2  # FP64 lane-instructions per second (1e12)
 
+FP64_MATRIX_PEAK_TFLOPS = 78.6  # FP64 matrix cores: a 16x16x4 product (2,048 flops) in 64 cycles per SIMD
+
 # FP64 flops of one evaluated term in the plain forms as executed (fma = 2,
-# table index not counted).  Viss: phase u*l + v*m + w*(n-1) on operands
-# pre-scaled by 1024, 1 mul + 2 fma = 5; split t + M - M, t - k = 3; z = f^2
-# 1; the pixel weight folded into the coefficients: w cos = w0 + z*w2, 1 fma
-# = 2, w sin = f*(w1 + z*w3), fma + mul = 3; rotation by the table entry
-# accumulated directly, 4 fma = 8: 22 flops, 14 instructions.  Recon: phase
-# 1 mul + 1 fma = 3; split 3; z 1; sin fma + mul = 3; cos 1 fma = 2;
-# rotation 2 mul + 2 fma = 6; accumulation 2 fma = 4: 22 flops, 15
-# instructions.
+# table index not counted).  Per-row Viss (k_viss_plain): phase u*l + v*m +
+# w*(n-1) on operands pre-scaled by 1024, 1 mul + 2 fma = 5; split t + M - M,
+# t - k = 3; z = f^2 1; the pixel weight folded into the coefficients: w cos =
+# w0 + z*w2, 1 fma = 2, w sin = f*(w1 + z*w3), fma + mul = 3; rotation by the
+# table entry accumulated directly, 4 fma = 8: 22 flops, 14 instructions.
+# Recon (polar terms): phase 2 fma = 4; fract 1; w = q^2 - q 1 fma = 2;
+# polynomial 5 fma = 10; u = c^2 1; u^2 - u 1 fma = 2; accumulation 1 fma = 2:
+# 22 flops, 12 instructions.
 VISS_TERM_FLOPS_PLAIN, VISS_TERM_INSTR_PLAIN = 22, 14
-RECON_TERM_FLOPS_PLAIN, RECON_TERM_INSTR_PLAIN = 22, 15
+RECON_TERM_FLOPS_PLAIN, RECON_TERM_INSTR_PLAIN = 22, 12
 # instructions of one evaluated term of the mixed recon as written
-# (ReconAccF32::term): phase mul_f64 + fma_f64, fract_f64, cvt_f32_f64,
-# sin_f32, cos_f32, 2 fma_f32; weighted by their measured issue costs
-MIXED_RECON_TERM = {"mul_f64": 1, "fma_f64": 1, "fract_f64": 1, "cvt_f32_f64": 1, "sin_f32": 1, "cos_f32": 1,
-                    "fma_f32": 2}
+# (ReconAccF32::term): phase 2 fma_f64, fract_f64, cvt_f32_f64, cos_f32,
+# fma_f32; weighted by their measured issue costs
+MIXED_RECON_TERM = {"fma_f64": 2, "fract_f64": 1, "cvt_f32_f64": 1, "cos_f32": 1, "fma_f32": 1}
 BATCH_TERM_FLOPS = 12  # per (term, sky): 2 real multiply-adds, each 3 BF16 products (hi*hi, hi*lo, lo*hi)
 
 TRAFFIC_FILES = {"nside128": os.path.join(ROOT, "profiles", "pmc_traffic_nside128_16ant_512ep.json"),
@@ -141,6 +143,9 @@ def _plan_counts(pipe, classes=True):
         if classes:
             cls = pipe.tile_classes()
             d["evaluated"] = int(np.dot((cls != 2).sum(axis=0, dtype=np.int64), tsz))
+            # (epoch, pixel) pairs of tiles that two antennas or more see any of
+            P = cls.shape[0] // tl
+            d["epoch_pixels"] = int(np.dot((cls.reshape(tl, P, -1) != 2).any(axis=1).sum(axis=0, dtype=np.int64), tsz))
         d["vraw"] = pipe.viss_half()
         pipe.conj_fill()
         info = pipe.recon_segment()
@@ -204,10 +209,35 @@ def _roof(kernel, bound, pipe_desc, work_per_launch, avg_ms, peak, unit, basis, 
 
 def _slots_per_term(rates, term):
     s = rates["slots"]
-    cost = {"mul_f64": s["mul_f64"], "fma_f64": s["fma_f64"], "fract_f64": s["fract_f64"],
-            "cvt_f32_f64": s["cvt_f32_f64_pair"] / 2, "sin_f32": s["sin_f32"], "cos_f32": s["cos_f32"],
-            "fma_f32": s["fma_f32"]}
+    cost = {"fma_f64": s["fma_f64"], "fract_f64": s["fract_f64"], "cvt_f32_f64": s["cvt_f32_f64_pair"] / 2,
+            "cos_f32": s["cos_f32"], "fma_f32": s["fma_f32"]}
     return sum(cost[k] * n for k, n in term.items())
+
+
+def _viss_roof(W, per_seg, nv, avg_ms, workload):
+    """The plain Viss kernel that the library's automatic choice runs: with
+    13-16 or 22-32 antennas and baselines of up to 1.5e6 wavelengths the
+    antenna-factorized one (products of 16 x 16 antennas on the FP64 matrix
+    cores: 3 a step of 4 pixels up to 16 antennas, 10 up to 32), else the
+    per-row one."""
+    A = W["n_ant"]
+    turns = 2 * 7100e3 * W["freq_hz"] / 3e8
+    if (13 <= A <= 16 or 22 <= A <= 32) and turns <= 1.5e6:
+        groups, products = (1, 3) if A <= 16 else (2, 10)
+        px = sum(s["epoch_pixels"] for s in per_seg) / nv
+        return _roof(
+            f"k_vissf<{W['tile_pix']},{groups},false> (plain antenna-factorized Viss)", "mfma_fp64",
+            "FP64 matrix cores (published peak)", 512 * products * px, avg_ms, FP64_MATRIX_PEAK_TFLOPS, "TFLOP/s",
+            f"{products} products of 16 x 16 x 4 (2,048 flops) per 4 pixels x {px:.6g} (epoch, pixel) pairs per launch "
+            "in tiles that two antennas or more see", _traffic(workload, "k_vissf_plain"), launches_per_step=nv)
+    ev = sum(s["evaluated"] for s in per_seg) / nv
+    return _roof(
+        f"k_viss_plain<{W['tile_pix']},8,false> (plain per-row Viss)", "valu_fp64",
+        "FP64 vector ALU (published FP64 peak)", VISS_TERM_FLOPS_PLAIN * ev, avg_ms, FP64_PEAK_TFLOPS, "TFLOP/s",
+        f"{VISS_TERM_FLOPS_PLAIN} FP64 flops x {ev:.6g} evaluated (half row, pixel) terms per launch",
+        _traffic(workload, "k_viss_plain"),
+        fp64_instr_issue_frac=round(VISS_TERM_INSTR_PLAIN * ev / (avg_ms * 1e-3) / 1e12 / FP64_INSTR_PEAK_T, 4),
+        launches_per_step=nv)
 
 
 def issue_rates():
@@ -243,7 +273,6 @@ def one_sky_leg(workload, steps, warmup, serial, rates, mixed=True, plain_ant=Fa
     nv, nr = tim["n_viss_launch"] // steps, tim["n_recon_launch"] // steps
     viss_avg = tim["viss_kernel_ms"] / (nv * steps)
     recon_avg = tim["recon_kernel_ms"] / (nr * steps)
-    ev_viss = sum(s["evaluated"] for s in per_seg) / nv
     ev_recon = sum(s["rec_evaluated"] for s in per_seg) / nr
     out["plain"] = {
         "value": round(terms / sec / 1e9, 4), "unit": "Gterms/s", "ms_per_step": round(sec * 1e3, 4),
@@ -254,17 +283,11 @@ def one_sky_leg(workload, steps, warmup, serial, rates, mixed=True, plain_ant=Fa
             "k_recon<4,false,0> (plain recon, uv mirror, representative classes)", "valu_fp64",
             "FP64 vector ALU (published FP64 peak)", RECON_TERM_FLOPS_PLAIN * ev_recon, recon_avg, FP64_PEAK_TFLOPS,
             "TFLOP/s", f"{RECON_TERM_FLOPS_PLAIN} FP64 flops x {ev_recon:.6g} evaluated (point, group) terms per launch "
-            f"({nr} launches per step: HEALPix map and lm image per segment)",
+            f"({nr} launches per step, each for the HEALPix map and the lm image of a segment)",
             _traffic(workload, "k_recon_plain"),
             fp64_instr_issue_frac=round(RECON_TERM_INSTR_PLAIN * ev_recon / (recon_avg * 1e-3) / 1e12 / FP64_INSTR_PEAK_T, 4),
             launches_per_step=nr),
-        "roofline_viss": _roof(
-            "k_viss_plain<256,8,false> (plain per-row Viss)", "valu_fp64", "FP64 vector ALU (published FP64 peak)",
-            VISS_TERM_FLOPS_PLAIN * ev_viss, viss_avg, FP64_PEAK_TFLOPS, "TFLOP/s",
-            f"{VISS_TERM_FLOPS_PLAIN} FP64 flops x {ev_viss:.6g} evaluated (half row, pixel) terms per launch",
-            _traffic(workload, "k_viss_plain"),
-            fp64_instr_issue_frac=round(VISS_TERM_INSTR_PLAIN * ev_viss / (viss_avg * 1e-3) / 1e12 / FP64_INSTR_PEAK_T, 4),
-            launches_per_step=nv),
+        "roofline_viss": _viss_roof(W, per_seg, nv, viss_avg, workload),
     }
     dom = "roofline_recon" if tim["recon_kernel_ms"] >= tim["viss_kernel_ms"] else "roofline_viss"
     out["plain"]["dominant"] = dom
@@ -293,17 +316,20 @@ def one_sky_leg(workload, steps, warmup, serial, rates, mixed=True, plain_ant=Fa
                 "k_recon<4,true,0> (mixed recon)", "valu", "vector ALU issue in FP32-FMA slots (2 flops each) "
                 "against the published 157.3 TFLOP/s vector FP32 rate",
                 2 * slots * ev_recon, rec_avg_m, FP32_PEAK_TFLOPS, "TFLOP/s",
-                f"{slots:.3f} issue slots per evaluated term (mul_f64 + fma_f64 + fract_f64 + cvt + sin_f32 + cos_f32 + "
-                f"2 fma_f32, weighted by the issue costs measured by vw_issue_rates) x {ev_recon:.6g} terms per "
-                "launch, 2 flops per slot", launches_per_step=nrm),
+                f"{slots:.3f} issue slots per evaluated term (2 fma_f64 + fract_f64 + cvt + cos_f32 + fma_f32, weighted "
+                f"by the issue costs measured by vw_issue_rates) x {ev_recon:.6g} terms per launch, 2 flops per slot",
+                launches_per_step=nrm),
         }
     if plain_ant:
         with Pipeline(_cfg(workload, serial, viss_form=2)) as ant:
             ant.set_sky(sky)
             per_seg_a, _ = _plan_counts(ant, classes=False)
             sec_a, _ = _time_steps(ant, steps, warmup)
+        with Pipeline(_cfg(workload, serial, viss_form=1)) as rows:
+            rows.set_sky(sky)
+            per_seg_r, _ = _plan_counts(rows, classes=False)
         vr_a = np.concatenate([s["vraw"] for s in per_seg_a])
-        vr_p = np.concatenate([s["vraw"] for s in per_seg])
+        vr_p = np.concatenate([s["vraw"] for s in per_seg_r])
         out["plain_ant"] = {"value": round(terms / sec_a / 1e9, 4), "unit": "Gterms/s",
                             "ms_per_step": round(sec_a * 1e3, 4), "dtype": "f64",
                             "viss_max_rel_err_vs_per_row": _err(vr_a, vr_p)["max_rel"]}
