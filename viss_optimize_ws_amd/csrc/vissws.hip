@@ -1094,7 +1094,7 @@ int enq_frame_vis(Ctx* c, bool img, int64_t tile0, int64_t nt, uint32_t* out, hi
  * only pay for (lunar segment of 2,796 epochs at Nside 64: 0.88 -> 0.93 ms): it
  * shares a tile's groups where the bits come from their table.  With one
  * workgroup a tile throughout, mixed recons of few tiles and many frames waited for
- * one wave's walk over the frames.  Mixed recon stage, ms, one workgroup against
+ * one wave's walk over the frames.  A vw_recon_segment, ms, one workgroup against
  * shared: lunar segments of 699 epochs at Nside 16, 64, 128 0.36 0.20, 0.43 0.32,
  * 0.69 0.59, of 2,796 at Nside 64 1.27 0.85; 2 antennas and a 64^2 image, 16,384
  * epochs at Nside 8 1.25 0.32, 60,000 at Nside 32 4.89 0.91, 400,000 at Nside 8
