@@ -1630,6 +1630,26 @@ int enq_recon(Ctx* c, bool keys_done = false) {
   return VW_OK;
 }
 
+/* Grouping after the Viss of its segment, beside the next one's, instead of
+ * before it.  The groups' keys need the rows only, and done early they leave the
+ * recon to start with the next segment's Viss.  Where the Viss is by far the longer
+ * (the mixed factorized form's matrix products cost the same for few antennas as
+ * for 16, its recon needs a third of the registers it once had) the recon's waves
+ * then take slots from the Viss for as long as it runs and nothing is gained over
+ * one stream; started later, behind a grouping that waits for slots itself, it
+ * fills the end of the Viss.  Whole steps, ms, early / late: lunar formation at
+ * Nside 128, 100 segments 313 / 275 (one stream 314), at Nside 64, 25 segments 73.5
+ * / 70.9; circular orbits at Nside 128, 8 segments, 128^2 image: 4 antennas 29.8 /
+ * 26.8, 6 13.4 / 12.2, 7 9.9 / 9.4, 8 7.79 / 7.82, 12 4.62 / 4.74; with a 512^2 image
+ * 4 antennas 30.0 / 27.8, 6 13.7 / 13.7, 8 9.17 / 9.19.  So up to 28 pairs, image
+ * points counted with the map's.  Short segments need the overlap with the grouping
+ * (lunar formation at Nside 64, 400 segments of 0.2 ms of Viss 99.7 / 106). */
+bool keys_late(const Ctx* c, int r) {
+  if (c->batch || !c->vfact || c->cfg.precision != VW_PREC_MIXED || c->runs[r].second > 1) return false;
+  const int64_t tl = run_tlen(c, r), pts = (c->cfg.healpix_out ? c->npix : 0) + c->ngp;
+  return c->P * pts <= 28 * c->npix && tl * c->npix >= (int64_t)1 << 24;
+}
+
 /* one step over the segment schedule (enqueue only): every segment's
  * geometry, Viss, conjugate fill and recon; with per-sky schedules the
  * Viss of the base segments for every sky into the day buffer, then per
@@ -1642,11 +1662,14 @@ int enq_step(Ctx* c) {
     for (int r = 0; r < (int)c->runs.size(); ++r) {
       const int s = c->runs[r].first;
       if ((rc = enq_gen_rows(c, c->seg_t0[s], run_tlen(c, r), merge_of(c, &c->seg_tlen[s], c->runs[r].second)))) return rc;
-      /* the groups' keys and order need the rows only: beside the Viss */
-      HC(hipEventRecord(c->ev_gen, c->st));
-      HC(hipStreamWaitEvent(c->stB, c->ev_gen, 0));
-      if ((rc = enq_group_keys(c))) return rc;
-      if ((rc = enq_viss(c, false, true)) || (c->batch && (rc = enq_conj(c))) || (rc = enq_recon(c, true))) return rc;
+      const bool late = keys_late(c, r);
+      if (!late) {
+        /* the groups' keys and order need the rows only: beside the Viss */
+        HC(hipEventRecord(c->ev_gen, c->st));
+        HC(hipStreamWaitEvent(c->stB, c->ev_gen, 0));
+        if ((rc = enq_group_keys(c))) return rc;
+      }
+      if ((rc = enq_viss(c, false, true)) || (c->batch && (rc = enq_conj(c))) || (rc = enq_recon(c, !late))) return rc;
     }
     return VW_OK;
   }
