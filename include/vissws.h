@@ -84,10 +84,11 @@ typedef struct {
   double r_min_km, r_max_km; /* circular: orbit radius range                     */
   double gm_km3_s2;    /* circular: gravitational parameter of the central body */
   int64_t class_budget_bytes; /* device bytes for the per-(tile, row) class tables of
-                               * one tile pass (0 = 2 GiB), and as much again per
-                               * output set for the occlusion bits of the mixed and
-                               * batched forms; a smaller budget splits the Viss and
-                               * recon stages into more tile passes               */
+                               * one tile pass (0 = 2 GiB), and as much again, or
+                               * 256 MiB if that is more, per output set for the
+                               * occlusion bits of the mixed and batched forms; a
+                               * smaller budget splits the Viss and recon stages into
+                               * more tile passes                                 */
   int32_t serial_stages;       /* 1: run every stage on one stream (no overlap of the
                                 * recon of a segment with the next segment's Viss;
                                 * for profiling single kernels)                     */
