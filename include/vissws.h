@@ -44,8 +44,8 @@ extern "C" {
 /* Viss summation form (vw_config.viss_form) */
 #define VW_VISS_AUTO 0      /* antenna-factorized in the mixed form for n_ant <= 32; in the plain form
                              * for circular orbits with 13-16 or 22-32 antennas, baselines
-                             * (2 r_max) of up to 1.5e6 wavelengths and a finite sky; else per-row
-                             * sums                                                              */
+                             * (2 r_max) of up to 1.5e6 wavelengths, a finite sky and epochs enough
+                             * in the longest launch to gain by it; else per-row sums            */
 #define VW_VISS_ROWS 1      /* one phase / sin / cos term per (half row, pixel): the reference's
                              * phase rounding, bit for bit                                       */
 #define VW_VISS_ANT 2       /* antenna-factorized on the matrix cores in either form (n_ant <= 32);

@@ -319,6 +319,26 @@ bool fact_auto_plain(const vw_config* cfg, double lambda) {
   return 2.0 * cfg->r_max_km * 1e3 / lambda <= VW_FACT_MAX_TURNS;
 }
 
+/* Where that choice does not pay for the epochs a launch has: the longest run's.
+ * The factorized form costs the same for 16 antennas as for 13, or for 32 as for
+ * 17, and for four epochs as for one, so where the points fill the chip the rows
+ * have to outweigh 70 or 205 pairs an epoch of these quads, and a part of a quad
+ * again for its start.  Factorized / rows, us a step: Nside 256, 13 antennas, 5
+ * epochs 393 / 290, 9 494 / 403, 16 antennas, 2 301 / 245, 6 393 / 407, 22
+ * antennas, 5 829 / 563, 28 antennas, 2 499 / 421, 3 503 / 569; Nside 128, 22
+ * antennas, 2 218 / 182, 16 476 / 505.  At Nside 64 the rows' waves are too few to
+ * gain by it (24 antennas, 9 epochs 220 / 225), nor are they for one epoch at Nside
+ * 128 (32 antennas 160 / 185).  And the smallest sums are one pass of the kernel,
+ * 33 us against 10: Nside 32, 32 antennas, 2 epochs 125 / 116, 8 157 / 189; 13
+ * antennas, 6 102 / 100, 9 104 / 107; Nside 16, 28 antennas, one 120 / 94. */
+bool fact_pays(int A, int64_t tlen, int64_t npix) {
+  const bool one = A <= 16;
+  const int64_t rows = tlen * (A * (A - 1) / 2), quads = (tlen + 3) / 4 * 4, terms = rows * npix;
+  if (terms < (one ? 7 : 16) << 20) return false;
+  const bool full = npix >= 1 << 19 || (tlen > 1 && npix >= 1 << 17 && terms >= 1 << 26);
+  return !full || rows >= (one ? 70 * quads + 75 : 205 * quads + 172);
+}
+
 /* ---------------- plan ---------------- */
 #define VW_BITS_MIN ((int64_t)256 << 20) /* bytes an output set's occlusion bits may take under any class budget */
 int64_t class_budget(const Ctx* c) {
@@ -534,6 +554,7 @@ int make_plan(Ctx* c, const vw_config* cfg) {
     c->nsky_pad = c->nsg * c->nbw * 16;
   }
   plan_runs(c);
+  if (c->fact_auto && !fact_pays(c->A, c->buf_tlen, c->npix)) c->vfact = c->fact_auto = false;
   if (c->max_nh > (int64_t)INT32_MAX / 4) return c->fail(VW_ERR_RANGE, "segment too long for 32-bit row indices");
   return VW_OK;
 }
